@@ -150,7 +150,62 @@ quant_rows_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __res
 }
 
 
-// Vectorised variant: LPR lanes per row (LPR = 256: one workgroup per row),
+// Eight codes clamp(rint(fl(x / safe))) without a division per element.
+// |x| <= amax, so |x / safe| <= 127 * (1 + 2^-23) and, with inv = v_rcp_f32(safe)
+// (at most 1 ulp from 1 / safe; safe is normal and above 2^-120: fp16 rows always
+// are, 2^-24 / 127 at least, bf16 callers check),
+// r = fl(x * inv) is within 128 * (2^-23 + 2^-24) = 1.5 * 2^-16 of x / safe,
+// and fl(x / safe) within 2^-17 of it: |r - fl(x / safe)| < 2^-14. n = r
+// rounded to nearest-even by the 1.5 * 2^23 magic constant; unless
+// |r - n| > 0.5 - 2^-14 (r near a half-integer) both r and fl(x / safe)
+// round to n. Lanes holding such an element (about 1e-4 of them) take the
+// IEEE division, under a wave-uniform branch so the common path never
+// executes it.
+__device__ __forceinline__ uint2 codes8(const float* f, float safe) {
+  const float inv = __builtin_amdgcn_rcpf(safe);
+  constexpr float MAGIC = 12582912.f;  // 1.5 * 2^23
+  float n[8];
+  bool amb = false;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float r = f[e] * inv;
+    n[e] = (r + MAGIC) - MAGIC;
+    amb |= !(fabsf(r - n[e]) <= 0.5f - 0x1p-14f);  // also catches inf / NaN
+  }
+  if (__builtin_expect(__ballot(amb) != 0, 0)) {
+    if (amb) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        n[e] = rintf(__fdiv_rn(f[e], safe));
+        if (n[e] != n[e]) n[e] = -127.f;  // NaN: the clamp of fmaxf / fminf gives -127
+      }
+    }
+  }
+  // n is an integer in [-128, 128] (or the division's result): clamp as int
+  uint32_t w[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    int c[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) c[e] = __builtin_amdgcn_fmed3f(n[4 * i + e], -127.f, 127.f);
+    // bytes 0 of c0..c3 -> one dword (v_perm_b32: selectors 0-3 pick the
+    // second operand's bytes, 4-7 the first's, 0x0c a zero byte)
+    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)c[1], (uint32_t)c[0], 0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)c[3], (uint32_t)c[2], 0x04000c0cu);
+    w[i] = lo | hi;
+  }
+  return make_uint2(w[0], w[1]);
+}
+
+// The same codes by IEEE division (any safe).
+__device__ __forceinline__ uint2 codes8_exact(const float* f, float safe) {
+  uint32_t w[2] = {0, 0};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) w[e / 4] |= (uint32_t)(uint8_t)code_of(f[e], safe) << (8 * (e % 4));
+  return make_uint2(w[0], w[1]);
+}
+
+// Vectorised variant: LPR lanes per row (LPR = BT: one workgroup per row),
 // each lane holding NV 16-byte vectors of the row in registers for both the
 // amax and the code pass (one HBM read per element). Needs K a multiple of
 // the elements per 16 bytes (EPV) and a 16-byte aligned base.
@@ -179,31 +234,37 @@ template <> struct VecIO<SL8_DTYPE_F32> {
   }
 };
 
-template <int DT, int LPR, int NV, bool MEAN>
-__global__ void __launch_bounds__(QTHREADS)
+template <int DT, int BT, int LPR, int NV, bool MEAN>
+__global__ void __launch_bounds__(BT)
 quant_rows_vec_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __restrict__ mean,
                       int8_t* __restrict__ q, float* __restrict__ scale, int64_t rows,
                       int64_t rows_per_mean, int K, float scale_mul) {
   using T = typename Elem<DT>::T;
   constexpr int EPV = VecIO<DT>::EPV;
+  static_assert(LPR <= 64 || LPR == BT, "a row is a lane group or the whole workgroup");
   const int lane = threadIdx.x % LPR;
-  const int64_t row = (int64_t)blockIdx.x * (QTHREADS / LPR) + threadIdx.x / LPR;
+  const int64_t row = (int64_t)blockIdx.x * (BT / LPR) + threadIdx.x / LPR;
   const bool live = row < rows;
   const int64_t r = live ? row : 0;
   const T* xr = x + r * K;
   const float* mr = MEAN ? mean + (r / rows_per_mean) * K : nullptr;
   const int nvec = K / EPV;
 
+  uint4 raw[NV];  // every load of the thread's row part is in flight before any is used
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const int vi = v * LPR + lane;
+    raw[v] = make_uint4(0, 0, 0, 0);
+    if (live && vi < nvec) raw[v] = reinterpret_cast<const uint4*>(xr)[vi];
+  }
   float f[NV][EPV];
   float amax = 0.f;
 #pragma unroll
   for (int v = 0; v < NV; ++v) {
-    const int vi = v * LPR + lane;
-    const bool ok = live && vi < nvec;
-    uint4 raw = make_uint4(0, 0, 0, 0);
-    if (ok) raw = reinterpret_cast<const uint4*>(xr)[vi];
-    VecIO<DT>::unpack(raw, f[v]);
+    VecIO<DT>::unpack(raw[v], f[v]);
     if constexpr (MEAN) {
+      const int vi = v * LPR + lane;
+      const bool ok = live && vi < nvec;
 #pragma unroll
       for (int e = 0; e < EPV; ++e)
         f[v][e] = ok ? Elem<DT>::round(f[v][e] - mr[vi * EPV + e]) : 0.f;
@@ -214,13 +275,12 @@ quant_rows_vec_kernel(const typename Elem<DT>::T* __restrict__ x, const float* _
   if constexpr (LPR <= 64) {
     amax = lane_group_max<LPR>(amax);
   } else {
-    __shared__ float red[QTHREADS / 64];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, 64));
+    __shared__ float red[BT / 64];
+    amax = lane_group_max<64>(amax);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < QTHREADS / 64; ++w) amax = fmaxf(amax, red[w]);
+    for (int w = 0; w < BT / 64; ++w) amax = fmaxf(amax, red[w]);
   }
   if (!live) return;
   const float s = amax * (1.0f / 127.0f);
@@ -231,16 +291,17 @@ quant_rows_vec_kernel(const typename Elem<DT>::T* __restrict__ x, const float* _
   for (int v = 0; v < NV; ++v) {
     const int vi = v * LPR + lane;
     if (vi < nvec) {
-      uint32_t w[EPV / 4];
+      if constexpr (EPV == 8) {
+        // codes8's error bound needs safe normal; bf16 rows may be smaller than that
+        const uint2 w = DT == SL8_DTYPE_F16 || safe >= 0x1p-120f ? codes8(f[v], safe)
+                                                                 : codes8_exact(f[v], safe);
+        *reinterpret_cast<uint2*>(qr + vi * EPV) = w;
+      } else {
+        uint32_t w = 0;
 #pragma unroll
-      for (int i = 0; i < EPV / 4; ++i) {
-        w[i] = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          w[i] |= (uint32_t)(uint8_t)code_of(f[v][4 * i + e], safe) << (8 * e);
+        for (int e = 0; e < 4; ++e) w |= (uint32_t)(uint8_t)code_of(f[v][e], safe) << (8 * e);
+        *reinterpret_cast<uint32_t*>(qr + vi * EPV) = w;
       }
-      if constexpr (EPV == 8) *reinterpret_cast<uint2*>(qr + vi * EPV) = make_uint2(w[0], w[1]);
-      else *reinterpret_cast<uint32_t*>(qr + vi * EPV) = w[0];
     }
   }
 }
@@ -258,24 +319,36 @@ int launch_quant(const void* x, const float* mean, int8_t* q, float* scale, int6
                                                                 rows_per_mean, (int)K, scale_mul);
   };
   constexpr int EPV = VecIO<DT>::EPV;
-  if (K % EPV == 0 && aligned(x, 16) && aligned(q, EPV) && K / EPV <= 8 * QTHREADS) {
+  constexpr int LT = 1024;  // threads of a long row's workgroup
+  if (K % EPV == 0 && aligned(x, 16) && aligned(q, EPV) && K / EPV <= 8 * LT) {
     const int64_t nvec = K / EPV;
-    auto gv = [&](auto lpr_tag, auto nv_tag) {
-      constexpr int LPR = decltype(lpr_tag)::value, NV = decltype(nv_tag)::value;
-      const int64_t rpb = QTHREADS / LPR;
+    auto gv = [&](auto bt_tag, auto lpr_tag, auto nv_tag) {
+      constexpr int BT = decltype(bt_tag)::value, LPR = decltype(lpr_tag)::value,
+                    NV = decltype(nv_tag)::value;
+      const int64_t rpb = BT / LPR;
       const dim3 grid((unsigned)((rows + rpb - 1) / rpb));
-      quant_rows_vec_kernel<DT, LPR, NV, MEAN><<<grid, QTHREADS, 0, st>>>(
+      quant_rows_vec_kernel<DT, BT, LPR, NV, MEAN><<<grid, BT, 0, st>>>(
           xp, mean, q, scale, rows, rows_per_mean, (int)K, scale_mul);
     };
-    using I = std::integral_constant<int, 1>;
-    if (nvec <= 16) gv(std::integral_constant<int, 16>{}, I{});
-    else if (nvec <= 32) gv(std::integral_constant<int, 32>{}, I{});
-    else if (nvec <= 64) gv(std::integral_constant<int, 64>{}, I{});
-    else if (nvec <= 128) gv(std::integral_constant<int, 64>{}, std::integral_constant<int, 2>{});
-    else if (nvec <= 256) gv(std::integral_constant<int, 256>{}, I{});
-    else if (nvec <= 512) gv(std::integral_constant<int, 256>{}, std::integral_constant<int, 2>{});
-    else if (nvec <= 1024) gv(std::integral_constant<int, 256>{}, std::integral_constant<int, 4>{});
-    else gv(std::integral_constant<int, 256>{}, std::integral_constant<int, 8>{});
+    using B = std::integral_constant<int, QTHREADS>;
+    using L = std::integral_constant<int, LT>;
+    using N1 = std::integral_constant<int, 1>;
+    using N2 = std::integral_constant<int, 2>;
+    using N4 = std::integral_constant<int, 4>;
+    using N8 = std::integral_constant<int, 8>;
+    if (nvec <= 16) gv(B{}, std::integral_constant<int, 16>{}, N1{});
+    else if (nvec <= 32) gv(B{}, std::integral_constant<int, 32>{}, N1{});
+    else if (nvec <= 64) gv(B{}, std::integral_constant<int, 64>{}, N1{});
+    else if (nvec <= 128) gv(B{}, std::integral_constant<int, 64>{}, N2{});
+    else if (nvec <= 256) gv(B{}, B{}, N1{});
+    else if (nvec <= 512) gv(B{}, B{}, N2{});
+    // longer rows: 1024 threads, so the few rows of a decode batch (one CU each) have 16 waves
+    // of loads in flight. 8 bf16 rows of 17408 (past the 16384 that 256 threads of 8 vectors
+    // held): 92.0 us in the element-wise kernel below, about 4 us here
+    else if (nvec <= 1024) gv(L{}, L{}, N1{});
+    else if (nvec <= 2048) gv(L{}, L{}, N2{});
+    else if (nvec <= 4096) gv(L{}, L{}, N4{});
+    else gv(L{}, L{}, N8{});
   } else if (K <= 128) {
     go(std::integral_constant<int, 16>{});
   } else if (K <= 512) {
@@ -751,52 +824,6 @@ __device__ __forceinline__ void unpack_h8(const uint4& raw, float* f) {
   const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
   for (int i = 0; i < 4; ++i) { f[2 * i] = h2f(w[i] & 0xFFFFu); f[2 * i + 1] = h2f(w[i] >> 16); }
-}
-
-// Eight codes clamp(rint(fl(x / safe))) without a division per element.
-// |x| <= amax, so |x / safe| <= 127 * (1 + 2^-23) and, with inv = v_rcp_f32(safe)
-// (at most 1 ulp from 1 / safe; safe >= 2^-24 / 127 here, a normal number),
-// r = fl(x * inv) is within 128 * (2^-23 + 2^-24) = 1.5 * 2^-16 of x / safe,
-// and fl(x / safe) within 2^-17 of it: |r - fl(x / safe)| < 2^-14. n = r
-// rounded to nearest-even by the 1.5 * 2^23 magic constant; unless
-// |r - n| > 0.5 - 2^-14 (r near a half-integer) both r and fl(x / safe)
-// round to n. Lanes holding such an element (about 1e-4 of them) take the
-// IEEE division, under a wave-uniform branch so the common path never
-// executes it.
-__device__ __forceinline__ uint2 codes8(const float* f, float safe) {
-  const float inv = __builtin_amdgcn_rcpf(safe);
-  constexpr float MAGIC = 12582912.f;  // 1.5 * 2^23
-  float n[8];
-  bool amb = false;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float r = f[e] * inv;
-    n[e] = (r + MAGIC) - MAGIC;
-    amb |= !(fabsf(r - n[e]) <= 0.5f - 0x1p-14f);  // also catches inf / NaN
-  }
-  if (__builtin_expect(__ballot(amb) != 0, 0)) {
-    if (amb) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        n[e] = rintf(__fdiv_rn(f[e], safe));
-        if (n[e] != n[e]) n[e] = -127.f;  // NaN: the clamp of fmaxf / fminf gives -127
-      }
-    }
-  }
-  // n is an integer in [-128, 128] (or the division's result): clamp as int
-  uint32_t w[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    int c[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c[e] = __builtin_amdgcn_fmed3f(n[4 * i + e], -127.f, 127.f);
-    // bytes 0 of c0..c3 -> one dword (v_perm_b32: selectors 0-3 pick the
-    // second operand's bytes, 4-7 the first's, 0x0c a zero byte)
-    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)c[1], (uint32_t)c[0], 0x0c0c0400u);
-    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)c[3], (uint32_t)c[2], 0x04000c0cu);
-    w[i] = lo | hi;
-  }
-  return make_uint2(w[0], w[1]);
 }
 
 // A: exact int64 fixed-point K-mean partials of PRO_CHUNK-row chunks (one

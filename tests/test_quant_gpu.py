@@ -87,3 +87,34 @@ def test_smooth_k_matches_oracle(device):
     rks, rm = oqn.smooth_k(_np(k))
     np.testing.assert_array_equal(_np(ks.float()), rks)
     np.testing.assert_array_equal(_np(km), rm)
+
+
+@pytest.mark.parametrize("dtype,tag", [(torch.float16, "f16"), (torch.bfloat16, "bf16"),
+                                       (torch.float32, "f32")])
+@pytest.mark.parametrize("rows,K", [(1, 4096), (3, 4104), (2, 8200), (5, 16384), (8, 17408),
+                                    (1, 32768), (2, 65536), (2, 65544)])
+def test_long_rows_bit_exact(device, dtype, tag, rows, K):
+    """Rows of a whole workgroup: the edges between one, two, four and eight 16-byte
+    vectors per thread, and the first length past them (the element-wise kernel)."""
+    x = torch.randn(rows, K, device=device) * 3
+    x[0, -1] = 40.0   # the row's maximum in the last, partly filled vector
+    x = x.to(dtype)
+    q, s = _C.quantize_i8_rowwise(x)
+    rq, rs = oqn.quantize_rows(_np(x.float()))
+    np.testing.assert_array_equal(_np(q), rq)
+    np.testing.assert_array_equal(_np(s), rs)
+
+
+@pytest.mark.parametrize("K", [128, 4096, 16384])
+def test_bf16_tiny_and_huge_rows_bit_exact(device, K):
+    """bf16 rows whose scale leaves the range of the reciprocal code path (below 2^-120,
+    subnormal scales included), just inside it, and near the largest finite bf16."""
+    x = torch.randn(6, K, device=device)
+    x = x / x.abs().amax(-1, keepdim=True)
+    x = x * torch.tensor([2.0 ** -126, 2.0 ** -113.5, 2.0 ** -112, 2.0 ** -100, 1.0, 3.0e38],
+                         device=device)[:, None]
+    x = x.to(torch.bfloat16)
+    q, s = _C.quantize_i8_rowwise(x)
+    rq, rs = oqn.quantize_rows(_np(x.float()))
+    np.testing.assert_array_equal(_np(s), rs)
+    np.testing.assert_array_equal(_np(q), rq)

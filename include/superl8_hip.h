@@ -57,7 +57,7 @@ int sl8_quantize_i8_rowwise(const void* x, int x_dtype, int64_t M, int64_t K,
  * K-smoothing mean: mean[g, d] = (1/N) * sum_n k[g, n, d], fp32.
  * Replaces the torch reduction in superl8/quant/core.py:29-44,70-95
  * (_mean_k_fp32_bounded / smooth_k). fp16 input is summed exactly in int64
- * fixed point (order-independent); bf16/f32 in fp64, rows in order.
+ * fixed point (order-independent); bf16/f32 in fp64, in a fixed order.
  *   k [G, N, D] (dtype f16/bf16/f32) -> mean fp32 [G, D]
  * workspace: sl8_k_mean_workspace(G, D) bytes, 8-byte aligned (used for fp16:
  * the int64 partial sums; contents need not be initialised).
@@ -91,12 +91,13 @@ int sl8_quantize_i8_row_groups(const void* x, int x_dtype, int64_t G, int64_t N,
                                int8_t* q, float* scale, void* stream);
 
 /* ------------------------------------------------------------------------
- * Fused fp16 attention prologue: quantize_qk (no rotation) plus, optionally,
+ * Fused fp16 / bf16 attention prologue: quantize_qk (no rotation) plus, optionally,
  * the outlier gate, in two launches (six unfused). Replaces superl8/quant/core.py:164-196
  * (smooth_k + quantize_qk) and detect_q_outlier_domination (core.py:113-145)
  * as called from superl8/ops.py:115-150; results equal sl8_k_mean,
  * sl8_quantize_i8_rows_centered and sl8_q_outlier_gate bit for bit.
- *   q [qrows, D] fp16 (qrows = B*Hq*M), k [G, N, D] fp16 (G = B*Hkv), D in {64,128,256}
+ *   q [qrows, D] (qrows = B*Hq*M), k [G, N, D] (G = B*Hkv), both dtype f16 or bf16,
+ *   D in {32,64,72,80,128,256}
  *   -> q_i8 [qrows, D], q_scale [qrows] (x q_scale_mul), k_i8 [G, N, D],
  *      k_scale [G, N], k_mean fp32 [G, D]
  * gate_ratio > 0: *gate_flag = 1 if some Q row has max/(median+1e-10) > ratio,

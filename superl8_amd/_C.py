@@ -137,14 +137,14 @@ def quantize_row_groups(x: torch.Tensor, rows_per_group: int, mean: torch.Tensor
 
 def quantize_qk_fused(q: torch.Tensor, k: torch.Tensor, q_scale_mul: float,
                       gate_ratio: float = 0.0):
-    """Fused fp16 prologue: q [B,Hq,M,D], k [B,Hkv,N,D] -> (q_i8, q_scale [B,Hq,M],
+    """Fused fp16 / bf16 prologue: q [B,Hq,M,D], k [B,Hkv,N,D] -> (q_i8, q_scale [B,Hq,M],
     k_i8, k_scale [B,Hkv,N], k_mean fp32 [B,Hkv,1,D], flag int32 [1] or None).
 
-    K is smoothed by its exact per-channel mean, q_scale carries q_scale_mul;
+    K is smoothed by its per-channel mean (see k_mean), q_scale carries q_scale_mul;
     with gate_ratio > 0, flag = 1 when some Q row has max/(median+1e-10) above it."""
     _on_gpu(q, k)
-    _check(q.dtype == torch.float16 and k.dtype == torch.float16,
-           "fused prologue expects float16 q and k")
+    _check(q.dtype == k.dtype and q.dtype in (torch.float16, torch.bfloat16),
+           "fused prologue expects float16 or bfloat16 q and k")
     _check(q.dim() == 4 and k.dim() == 4 and q.shape[-1] == k.shape[-1],
            "fused prologue expects q[B,Hq,M,D], k[B,Hkv,N,D]")
     q, k = q.contiguous(), k.contiguous()

@@ -205,6 +205,12 @@ __device__ __forceinline__ uint2 codes8_exact(const float* f, float safe) {
   return make_uint2(w[0], w[1]);
 }
 
+// Eight codes of a 16-bit row (see codes8; bf16 rows may have scales below its range).
+template <int DT>
+__device__ __forceinline__ uint2 row_codes8(const float* f, float safe) {
+  return DT == SL8_DTYPE_F16 || safe >= 0x1p-120f ? codes8(f, safe) : codes8_exact(f, safe);
+}
+
 // Vectorised variant: LPR lanes per row (LPR = BT: one workgroup per row),
 // each lane holding NV 16-byte vectors of the row in registers for both the
 // amax and the code pass (one HBM read per element). Needs K a multiple of
@@ -292,10 +298,7 @@ quant_rows_vec_kernel(const typename Elem<DT>::T* __restrict__ x, const float* _
     const int vi = v * LPR + lane;
     if (vi < nvec) {
       if constexpr (EPV == 8) {
-        // codes8's error bound needs safe normal; bf16 rows may be smaller than that
-        const uint2 w = DT == SL8_DTYPE_F16 || safe >= 0x1p-120f ? codes8(f[v], safe)
-                                                                 : codes8_exact(f[v], safe);
-        *reinterpret_cast<uint2*>(qr + vi * EPV) = w;
+        *reinterpret_cast<uint2*>(qr + vi * EPV) = row_codes8<DT>(f[v], safe);
       } else {
         uint32_t w = 0;
 #pragma unroll
@@ -426,18 +429,32 @@ k_mean_finish_kernel(const unsigned long long* __restrict__ acc, float* __restri
   if (i < n) mean[i] = (float)(((double)(long long)acc[i] * 0x1p-24) / (double)N);
 }
 
-// bf16 / f32: fp64 running sum over rows in index order (one thread per column).
+// bf16 / f32: fp64 sums in a fixed order (the rows of a phase, then the phases). One block per
+// (group, 16 columns) with 64 row phases: one thread per column over all N rows in turn took
+// 1439 us for 8 groups of 6121 bf16 rows of 128.
+constexpr int SEQ_COLS = 16, SEQ_PHASES = 64;
 template <int DT>
-__global__ void __launch_bounds__(MEAN_COLS)
+__global__ void __launch_bounds__(SEQ_COLS * SEQ_PHASES)
 k_mean_seq_kernel(const typename Elem<DT>::T* __restrict__ k, float* __restrict__ mean,
                   int64_t N, int D) {
+  __shared__ double part[SEQ_PHASES][SEQ_COLS];
   const int64_t g = blockIdx.y;
-  const int d = blockIdx.x * MEAN_COLS + threadIdx.x;
-  if (d >= D) return;
-  const typename Elem<DT>::T* kg = k + g * N * D + d;
+  const int col = threadIdx.x % SEQ_COLS, ph = threadIdx.x / SEQ_COLS;
+  const int d = blockIdx.x * SEQ_COLS + col;
   double s = 0.0;
-  for (int64_t n = 0; n < N; ++n) s += (double)Elem<DT>::ld(kg, n * D);
-  mean[g * D + d] = (float)(s / (double)N);
+  if (d < D) {
+    const typename Elem<DT>::T* kg = k + g * N * D + d;
+#pragma unroll 8
+    for (int64_t n = ph; n < N; n += SEQ_PHASES) s += (double)Elem<DT>::ld(kg, n * D);
+  }
+  part[ph][col] = s;
+  __syncthreads();
+  if (ph == 0 && d < D) {
+    double t = 0.0;
+#pragma unroll 8
+    for (int p = 0; p < SEQ_PHASES; ++p) t += part[p][col];
+    mean[g * D + d] = (float)(t / (double)N);
+  }
 }
 
 // ---- per-channel (column) quantisation over the key axis ----------------
@@ -678,13 +695,14 @@ extern "C" int sl8_k_mean(const void* k, int dtype, int64_t G, int64_t N, int64_
                                                                  acc, N, (int)D);
     k_mean_finish_kernel<<<ng, 256, 0, st>>>(acc, mean, n, N);
   } else {
-    const dim3 grid((unsigned)((D + MEAN_COLS - 1) / MEAN_COLS), (unsigned)G);
+    const dim3 grid((unsigned)((D + SEQ_COLS - 1) / SEQ_COLS), (unsigned)G);
+    constexpr int BT = SEQ_COLS * SEQ_PHASES;
     if (dtype == SL8_DTYPE_BF16)
-      k_mean_seq_kernel<SL8_DTYPE_BF16><<<grid, MEAN_COLS, 0, st>>>(static_cast<const uint16_t*>(k),
-                                                                    mean, N, (int)D);
+      k_mean_seq_kernel<SL8_DTYPE_BF16><<<grid, BT, 0, st>>>(static_cast<const uint16_t*>(k), mean,
+                                                             N, (int)D);
     else
-      k_mean_seq_kernel<SL8_DTYPE_F32><<<grid, MEAN_COLS, 0, st>>>(static_cast<const float*>(k),
-                                                                   mean, N, (int)D);
+      k_mean_seq_kernel<SL8_DTYPE_F32><<<grid, BT, 0, st>>>(static_cast<const float*>(k), mean, N,
+                                                            (int)D);
   }
   SL8_CHECK_LAUNCH("k_mean");
   return SL8_OK;
@@ -777,20 +795,22 @@ extern "C" int sl8_q_outlier_gate(const void* q, int dtype, int64_t rows, int64_
 }
 
 // ---------------------------------------------------------------------------
-// Fused attention prologue for fp16 Q/K (reference superl8/quant/core.py
+// Fused attention prologue for fp16 / bf16 Q/K (reference superl8/quant/core.py
 // quantize_qk + smooth_k, and the outlier gate of superl8/ops.py:115-147):
 // two launches instead of six, Q read once, K read twice, no zeroing pass.
 //
-// Launch A: K-mean partials. Block (g, c) sums key rows [128c, 128c + 128)
-//   of group g exactly in int64 fixed point (value * 2^24, decoded from the
-//   fp16 bits) with 16-byte loads, all of a thread's rows in flight at once,
-//   and stores its D partial sums; the mean is exact, hence independent of
-//   the summation order. Block 0 also clears the gate flag.
+// Launch A: K-mean partials. Block (g, c) sums the key rows of chunk c of
+//   group g with 16-byte loads, a pass of a thread's rows in flight at once,
+//   and stores its D partial sums: fp16 exactly in int64 fixed point (value *
+//   2^24, decoded from the fp16 bits), hence independent of the summation
+//   order; bf16 in fp64, whose 53 bits hold sums of 8-bit significands exactly
+//   unless one column spans more than about 2^30 in magnitude (then the order
+//   is fixed: rows of a thread, threads, chunks). Block 0 clears the gate flag.
 // Launch B, two roles chosen per block:
 //   * K: issues its key rows' loads, forms the group's mean from the C
-//     partials meanwhile (int64 -> fp64 -> / N -> fp32, as sl8_k_mean; the
-//     first block of each group also stores it), subtracts it from each row
-//     with the fp16 rounding of torch.sub and quantises the row;
+//     partials meanwhile (as sl8_k_mean; the first block of each group also
+//     stores it), subtracts it from each row with the rounding of torch.sub
+//     and quantises the row;
 //   * Q: per-row int8 quantisation (scale * q_scale_mul) and, with a gate
 //     ratio, the outlier decision for every row. f(x) = fl(max / fl(x + 1e-10))
 //     is non-increasing in x >= 0, so f(median) > ratio iff more than (D-1)/2
@@ -799,14 +819,28 @@ extern "C" int sl8_q_outlier_gate(const void* q, int dtype, int64_t rows, int64_
 //     2^-18 of max / ratio). A row holding a NaN never fires (torch's amax and
 //     median are NaN there). A block with a firing row ORs 1 into the flag
 //     (atomicOr), so the flag is set iff some row fires.
+// Head dims 72 and 80 take the 16 lanes per row of 128 with 9 and 10 of them
+// holding elements.
 // ---------------------------------------------------------------------------
 namespace sl8 {
 namespace {
 
-constexpr int PRO_CHUNK = 128;      // key rows per mean partial
+constexpr int PRO_CHUNK = 128;      // key rows per mean partial, up to PRO_CHUNKS_MAX partials;
+// beyond, the chunks grow: every K block of B reads all its group's partials, which at 128 rows
+// a partial would be more bytes than its own rows from N = 2048 on (16-bit D = 128: 1 KB a
+// partial, 16 KB of rows) and grow with N * N
+constexpr int PRO_CHUNKS_MAX = 48;
 constexpr int PRO_KROWS = 64;       // key rows per quantise block (each K block also forms its group's mean: 32 measured 1 us slower at config 2, 128 0.3 us)
 constexpr int PRO_QBLOCKS_MAX = 16384;
 constexpr int PRO_QP = 1;           // Q rows per thread per pass (1: measured fastest; more rows per thread cost occupancy)
+
+int64_t pro_chunk_rows(int64_t N) {
+  const int64_t per = (N + PRO_CHUNKS_MAX - 1) / PRO_CHUNKS_MAX;
+  return std::max<int64_t>(PRO_CHUNK, (per + PRO_CHUNK - 1) / PRO_CHUNK * PRO_CHUNK);
+}
+
+// Lanes per row (8 elements, 16 bytes each); the first D / 8 of them hold elements.
+constexpr int pro_lpr(int D) { return D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 16 : 32; }
 
 // fp16 bits -> value * 2^24 as an exact integer (finite inputs: |result| < 2^40)
 __device__ __forceinline__ long long f16_fixed24(uint32_t h) {
@@ -815,137 +849,160 @@ __device__ __forceinline__ long long f16_fixed24(uint32_t h) {
   return (h & 0x8000u) ? -v : v;
 }
 
-template <int LPR>
-__device__ __forceinline__ float group_max(float v) { return lane_group_max<LPR>(v); }
-template <int LPR>
-__device__ __forceinline__ int group_sum(int v) { return lane_group_sum<LPR>(v); }
+// The K-mean partial sums of a storage type.
+template <int DT> struct MeanSum;
+template <> struct MeanSum<SL8_DTYPE_F16> {
+  using T = long long;
+  __device__ static T of(uint32_t bits) { return f16_fixed24(bits); }
+  __device__ static float mean(T sum, int64_t N) {
+    return (float)(((double)sum * 0x1p-24) / (double)N);
+  }
+};
+template <> struct MeanSum<SL8_DTYPE_BF16> {
+  using T = double;
+  __device__ static T of(uint32_t bits) { return (double)bf2f((uint16_t)bits); }
+  __device__ static float mean(T sum, int64_t N) { return (float)(sum / (double)N); }
+};
 
-__device__ __forceinline__ void unpack_h8(const uint4& raw, float* f) {
-  const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) { f[2 * i] = h2f(w[i] & 0xFFFFu); f[2 * i + 1] = h2f(w[i] >> 16); }
-}
-
-// A: exact int64 fixed-point K-mean partials of PRO_CHUNK-row chunks (one
-// block per (group, chunk)); block 0 also clears the gate flag, which the Q
-// blocks of B set.
-template <int D>
-__global__ void __launch_bounds__(256, 8)
-prologue_a_kernel(const uint16_t* __restrict__ k, int64_t N, int C,
-                  long long* __restrict__ part, int32_t* __restrict__ flag) {
-  constexpr int LPR = D / 8;       // lanes per row, 8 elements (16 bytes) each
-  constexpr int RPP = 256 / LPR;   // rows per block pass
+// Partial sums over rows [n0, n1) of k[., D] by a 256-thread block -> part[0, D).
+template <int DT, int D>
+__device__ __forceinline__ void mean_chunk(const uint16_t* __restrict__ kg, int64_t n0, int64_t n1,
+                                           typename MeanSum<DT>::T* __restrict__ part) {
+  using S = MeanSum<DT>;
+  constexpr int LPR = pro_lpr(D), NL = D / 8;
+  constexpr int RPP = 256 / LPR;                     // rows per pass
+  constexpr int NIT = PRO_CHUNK / RPP < 8 ? PRO_CHUNK / RPP : 8;  // passes in flight
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
-  if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
-  __shared__ long long red[RPP][D];
-  const int64_t g = blockIdx.x / C;
-  const int c = blockIdx.x % C;
-  const int64_t n0 = (int64_t)c * PRO_CHUNK, n1 = min(N, n0 + PRO_CHUNK);
-  const uint16_t* kg = k + g * N * D + lane * 8;
-  long long acc[8];
+  const bool on = lane < NL;
+  __shared__ typename S::T red[RPP][D];
+  typename S::T acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0;
-  // every row load of the chunk is issued before any is summed (one round trip)
-  constexpr int NIT = PRO_CHUNK / RPP;
-  uint4 raw[NIT];
+  for (int64_t b = n0; b < n1; b += NIT * RPP) {
+    uint4 raw[NIT];
 #pragma unroll
-  for (int i = 0; i < NIT; ++i) {
-    const int64_t n = n0 + sub + (int64_t)i * RPP;
-    raw[i] = n < n1 ? *reinterpret_cast<const uint4*>(kg + n * D) : make_uint4(0, 0, 0, 0);
-  }
+    for (int i = 0; i < NIT; ++i) {
+      const int64_t n = b + sub + i * RPP;
+      raw[i] = on && n < n1 ? reinterpret_cast<const uint4*>(kg + n * D)[lane] : make_uint4(0, 0, 0, 0);
+    }
 #pragma unroll
-  for (int it = 0; it < NIT; ++it) {
-    const uint32_t w[4] = {raw[it].x, raw[it].y, raw[it].z, raw[it].w};
+    for (int it = 0; it < NIT; ++it) {
+      const uint32_t w[4] = {raw[it].x, raw[it].y, raw[it].z, raw[it].w};
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      acc[2 * i] += f16_fixed24(w[i] & 0xFFFFu);
-      acc[2 * i + 1] += f16_fixed24(w[i] >> 16);
+      for (int i = 0; i < 4; ++i) {
+        acc[2 * i] += S::of(w[i] & 0xFFFFu);
+        acc[2 * i + 1] += S::of(w[i] >> 16);
+      }
     }
   }
+  if (on) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) red[sub][lane * 8 + e] = acc[e];
+    for (int e = 0; e < 8; ++e) red[sub][lane * 8 + e] = acc[e];
+  }
   __syncthreads();
   for (int d = threadIdx.x; d < D; d += 256) {
-    long long t = 0;
+    typename S::T t = 0;
 #pragma unroll 8
     for (int p = 0; p < RPP; ++p) t += red[p][d];
-    part[(g * C + c) * D + d] = t;
+    part[d] = t;
   }
+}
+
+// Smooth + quantise PRO_KROWS key rows from n0 on, by a 256-thread block: the rows' loads are
+// issued first, the group's mean is formed from its C partials under them.
+template <int DT, int D>
+__device__ __forceinline__ void smooth_rows(const uint16_t* __restrict__ kg, int64_t n0, int64_t N,
+                                            const typename MeanSum<DT>::T* __restrict__ part, int C,
+                                            float* __restrict__ mean_out,
+                                            int8_t* __restrict__ kq, float* __restrict__ kscale) {
+  using S = MeanSum<DT>;
+  constexpr int LPR = pro_lpr(D), NL = D / 8, RPP = 256 / LPR, NP = PRO_KROWS / RPP;
+  const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
+  const bool on = lane < NL;
+  uint4 raw[NP];
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int64_t n = n0 + i * RPP + sub;
+    raw[i] = on && n < N ? reinterpret_cast<const uint4*>(kg + n * D)[lane] : make_uint4(0, 0, 0, 0);
+  }
+  // column d summed by PS threads over every PS-th partial, then in LDS
+  constexpr int PS = 256 / D;
+  __shared__ typename S::T mred[PS][D];
+  __shared__ float mean_s[D];
+  if (threadIdx.x < PS * D) {
+    const int d = threadIdx.x % D, ps = threadIdx.x / D;
+    typename S::T t = 0;
+#pragma unroll 8
+    for (int c = ps; c < C; c += PS) t += part[(int64_t)c * D + d];
+    mred[ps][d] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    typename S::T t = 0;
+#pragma unroll
+    for (int p = 0; p < PS; ++p) t += mred[p][threadIdx.x];
+    const float m = S::mean(t, N);
+    mean_s[threadIdx.x] = m;
+    if (mean_out) mean_out[threadIdx.x] = m;
+  }
+  __syncthreads();
+  float mv[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) mv[e] = on ? mean_s[lane * 8 + e] : 0.f;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int64_t n = n0 + i * RPP + sub;
+    float f[8];
+    VecIO<DT>::unpack(raw[i], f);
+    float mx = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      f[e] = Elem<DT>::round(f[e] - mv[e]);
+      mx = fmaxf(mx, fabsf(f[e]));
+    }
+    mx = lane_group_max<LPR>(mx);
+    const float s = mx * (1.0f / 127.0f);
+    const float safe = (s == 0.f) ? 1.f : s;
+    if (on && n < N) {
+      if (lane == 0) kscale[n] = safe;
+      reinterpret_cast<uint2*>(kq + n * D)[lane] = row_codes8<DT>(f, safe);
+    }
+  }
+}
+
+// A: K-mean partials of `chunk`-row chunks, one block per (group, chunk).
+template <int DT, int D>
+__global__ void __launch_bounds__(256)
+prologue_a_kernel(const uint16_t* __restrict__ k, int64_t N, int C, int64_t chunk,
+                  typename MeanSum<DT>::T* __restrict__ part, int32_t* __restrict__ flag) {
+  if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
+  const int64_t g = blockIdx.x / C, c = blockIdx.x % C;
+  mean_chunk<DT, D>(k + g * N * D, c * chunk, min(N, (c + 1) * chunk), part + (g * C + c) * D);
 }
 
 // B: the smoothed K rows (blocks [0, nkb): PRO_KROWS rows of group
 // blockIdx / kbg each) and the Q rows with the outlier gate (the rest). The Q
 // work does not depend on the mean, but sharing this launch keeps it off the
 // critical path A -> mean -> B of the K side.
-template <int D, bool GATE>
+template <int DT, int D, bool GATE>
 __global__ void __launch_bounds__(256)
-prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N, const long long* __restrict__ part,
+prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
+                  const typename MeanSum<DT>::T* __restrict__ part,
                   int C, float* __restrict__ k_mean,
                   int8_t* __restrict__ k_i8, float* __restrict__ k_scale, int kbg, int nkb,
                   const uint16_t* __restrict__ q, int64_t qrows, float qmul, float ratio,
                   int8_t* __restrict__ q_i8, float* __restrict__ q_scale,
                   int32_t* __restrict__ flag) {
-  constexpr int LPR = D / 8, RPP = 256 / LPR;
+  constexpr int LPR = pro_lpr(D), NL = D / 8, RPP = 256 / LPR;
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
   if ((int)blockIdx.x < nkb) {
-    constexpr int NP = PRO_KROWS / RPP;
     const int64_t g = blockIdx.x / kbg;
-    const int64_t n0 = (int64_t)(blockIdx.x % kbg) * PRO_KROWS;
-    const uint16_t* kg = k + g * N * D;
-    uint4 raw[NP];
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int64_t n = n0 + i * RPP + sub;
-      raw[i] = n < N ? reinterpret_cast<const uint4*>(kg + n * D)[lane] : make_uint4(0, 0, 0, 0);
-    }
-    // the group's mean from A's partials while the rows are in flight:
-    // column d summed by PS threads over every PS-th partial, then in LDS
-    constexpr int PS = 256 / D;
-    __shared__ long long mred[PS][D];
-    __shared__ float mean_s[D];
-    {
-      const int d = threadIdx.x % D, ps = threadIdx.x / D;
-      const long long* pg = part + g * C * D + d;
-      long long t = 0;
-#pragma unroll 8
-      for (int c = ps; c < C; c += PS) t += pg[(int64_t)c * D];
-      mred[ps][d] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x < D) {
-      long long t = 0;
-#pragma unroll
-      for (int p = 0; p < PS; ++p) t += mred[p][threadIdx.x];
-      const float m = (float)(((double)t * 0x1p-24) / (double)N);
-      mean_s[threadIdx.x] = m;
-      if (blockIdx.x % kbg == 0) k_mean[g * D + threadIdx.x] = m;
-    }
-    __syncthreads();
-    float mv[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) mv[e] = mean_s[lane * 8 + e];
-#pragma unroll
-    for (int i = 0; i < NP; ++i) {
-      const int64_t n = n0 + i * RPP + sub;
-      const bool live = n < N;
-      float f[8];
-      unpack_h8(raw[i], f);
-      float mx = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        f[e] = Elem<SL8_DTYPE_F16>::round(f[e] - mv[e]);
-        mx = fmaxf(mx, fabsf(f[e]));
-      }
-      mx = group_max<LPR>(mx);
-      const float s = mx * (1.0f / 127.0f);
-      const float safe = (s == 0.f) ? 1.f : s;
-      if (live) {
-        if (lane == 0) k_scale[g * N + n] = safe;
-        reinterpret_cast<uint2*>(k_i8 + (g * N + n) * D)[lane] = codes8(f, safe);
-      }
-    }
+    const int b = blockIdx.x % kbg;
+    smooth_rows<DT, D>(k + g * N * D, (int64_t)b * PRO_KROWS, N, part + g * C * D, C,
+                       b == 0 ? k_mean + g * D : nullptr, k_i8 + g * N * D, k_scale + g * N);
     return;
   }
+  const bool on = lane < NL;
   const int qb = blockIdx.x - nkb, nqb = gridDim.x - nkb;
   int fired = 0;
   const float rinv = 1.f / ratio;
@@ -955,23 +1012,24 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N, const long long* __
 #pragma unroll
     for (int p = 0; p < PRO_QP; ++p) {
       const int64_t r = base + p * RPP + sub;
-      raw[p] = r < qrows ? reinterpret_cast<const uint4*>(q + r * D)[lane] : make_uint4(0, 0, 0, 0);
+      raw[p] = on && r < qrows ? reinterpret_cast<const uint4*>(q + r * D)[lane]
+                               : make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
     for (int p = 0; p < PRO_QP; ++p) {
       const int64_t r = base + p * RPP + sub;
       const bool live = r < qrows;
       float f[8];
-      unpack_h8(raw[p], f);
+      VecIO<DT>::unpack(raw[p], f);
       float mx = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
-      mx = group_max<LPR>(mx);
+      mx = lane_group_max<LPR>(mx);
       const float s = mx * (1.0f / 127.0f);
       const float safe = (s == 0.f) ? 1.f : s;
-      if (live) {
+      if (live && on) {
         if (lane == 0) q_scale[r] = safe * qmul;
-        reinterpret_cast<uint2*>(q_i8 + r * D)[lane] = codes8(f, safe);
+        reinterpret_cast<uint2*>(q_i8 + r * D)[lane] = row_codes8<DT>(f, safe);
       }
       if constexpr (GATE) {
         // y = fl(|x| + 1e-10) against t = max / ratio: far from t the exact test
@@ -1001,7 +1059,8 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N, const long long* __
             }
           }
         }
-        cnt = group_sum<LPR>(cnt + (nan << 16));  // NaN count in the high half
+        if (!on) cnt = 0;  // a lane without elements
+        cnt = lane_group_sum<LPR>(cnt + (nan << 16));  // NaN count in the high half
         if (live && (cnt >> 16) == 0 && (cnt & 0xFFFF) > (D - 1) / 2) fired = 1;
       }
     }
@@ -1012,17 +1071,59 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N, const long long* __
   }
 }
 
-int prologue_nqb(int64_t qrows, int64_t D) {
-  const int64_t rpp = 256 / (D / 8) * PRO_QP;
+int prologue_nqb(int64_t qrows, int D) {
+  const int64_t rpp = 256 / pro_lpr(D) * PRO_QP;
   return (int)std::min<int64_t>(PRO_QBLOCKS_MAX, (qrows + rpp - 1) / rpp);
 }
+
+// The sizes of one prologue call and its launches for a storage type and head dim.
+struct Prologue {
+  const uint16_t *q, *k;
+  int64_t qrows, G, N;
+  float q_scale_mul, gate_ratio;
+  int8_t *q_i8, *k_i8;
+  float *q_scale, *k_scale, *k_mean;
+  int32_t* flag;
+  void* part;
+  hipStream_t st;
+  int64_t chunk;
+  int C, kbg;
+
+  // A (K-mean partials) -> B (the mean, K and Q rows, gate): the Q rows, the
+  // bulk of the bytes, run beside the K rows in B instead of ahead of the mean
+  template <int DT, int D>
+  void go() const {
+    using S = typename MeanSum<DT>::T;
+    const int nkb = (int)(G * kbg), nqb = prologue_nqb(qrows, D);
+    S* pt = static_cast<S*>(part);
+    prologue_a_kernel<DT, D><<<(unsigned)(G * C), 256, 0, st>>>(k, N, C, chunk, pt, flag);
+    auto b = [&](auto gate) {
+      prologue_b_kernel<DT, D, decltype(gate)::value><<<nkb + nqb, 256, 0, st>>>(
+          k, N, pt, C, k_mean, k_i8, k_scale, kbg, nkb, q, qrows, q_scale_mul, gate_ratio, q_i8,
+          q_scale, flag);
+    };
+    if (flag) b(std::true_type{});
+    else b(std::false_type{});
+  }
+  template <int DT>
+  void go(int64_t D) const {
+    switch (D) {
+      case 32: return go<DT, 32>();
+      case 64: return go<DT, 64>();
+      case 72: return go<DT, 72>();
+      case 80: return go<DT, 80>();
+      case 128: return go<DT, 128>();
+      default: return go<DT, 256>();
+    }
+  }
+};
 
 }  // namespace
 }  // namespace sl8
 
 extern "C" size_t sl8_quantize_qk_workspace(int64_t BHq_M, int64_t G, int64_t N, int64_t D) {
   if (G <= 0 || N <= 0 || D <= 0) return 0;
-  const int64_t C = (N + PRO_CHUNK - 1) / PRO_CHUNK;
+  const int64_t chunk = pro_chunk_rows(N), C = (N + chunk - 1) / chunk;
   (void)BHq_M;  // the Q rows need no workspace (the gate sets the flag directly)
   return (size_t)(G * C * D) * sizeof(long long);  // the K-mean partials
 }
@@ -1033,9 +1134,10 @@ extern "C" int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t 
                                float* k_mean, int32_t* gate_flag, void* workspace,
                                size_t workspace_bytes, void* stream) {
   clear_error();
-  SL8_CHECK_ARG(dtype == SL8_DTYPE_F16, "fused prologue: q and k must be float16");
-  SL8_CHECK_ARG(D == 64 || D == 128 || D == 256,
-                "fused prologue: head dim must be 64/128/256, got %lld", (long long)D);
+  SL8_CHECK_ARG(dtype == SL8_DTYPE_F16 || dtype == SL8_DTYPE_BF16,
+                "fused prologue: q and k must be float16 or bfloat16");
+  SL8_CHECK_ARG(D == 32 || D == 64 || D == 72 || D == 80 || D == 128 || D == 256,
+                "fused prologue: head dim must be 32/64/72/80/128/256, got %lld", (long long)D);
   SL8_CHECK_ARG(qrows > 0 && G > 0 && N > 0 && N < (1LL << 23),
                 "fused prologue: bad shape (rows %lld, groups %lld, keys %lld)", (long long)qrows,
                 (long long)G, (long long)N);
@@ -1047,32 +1149,16 @@ extern "C" int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t 
   const size_t need = sl8_quantize_qk_workspace(qrows, G, N, D);
   SL8_CHECK_ARG(workspace && workspace_bytes >= need && aligned(workspace, 8),
                 "fused prologue: workspace needs %zu bytes", need);
-  const int C = (int)((N + PRO_CHUNK - 1) / PRO_CHUNK);
+  const int64_t chunk = pro_chunk_rows(N), C = (N + chunk - 1) / chunk;
   const int64_t kbg = (N + PRO_KROWS - 1) / PRO_KROWS;  // quantise blocks per group
   SL8_CHECK_ARG(G * C < (1LL << 30) && G * kbg < (1LL << 30) && G < 65536,
                 "fused prologue: too many key groups");
-  const int nka = (int)(G * C), nkb = (int)(G * kbg), nqb = prologue_nqb(qrows, D);
-  long long* part = static_cast<long long*>(workspace);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const uint16_t* qh = static_cast<const uint16_t*>(q);
-  const uint16_t* kh = static_cast<const uint16_t*>(k);
-  int32_t* fl = gate ? gate_flag : nullptr;
-  // A (K-mean partials) -> B (the mean, K and Q rows, gate): the Q rows, the
-  // bulk of the bytes, run beside the K rows in B instead of ahead of the mean
-#define SL8_PRO(DD)                                                                              \
-  do {                                                                                          \
-    prologue_a_kernel<DD><<<nka, 256, 0, st>>>(kh, N, C, part, fl);                              \
-    if (gate)                                                                                   \
-      prologue_b_kernel<DD, true><<<nkb + nqb, 256, 0, st>>>(kh, N, part, C, k_mean, k_i8,      \
-          k_scale, (int)kbg, nkb, qh, qrows, q_scale_mul, gate_ratio, q_i8, q_scale, fl);       \
-    else                                                                                        \
-      prologue_b_kernel<DD, false><<<nkb + nqb, 256, 0, st>>>(kh, N, part, C, k_mean, k_i8,     \
-          k_scale, (int)kbg, nkb, qh, qrows, q_scale_mul, gate_ratio, q_i8, q_scale, fl);       \
-  } while (0)
-  if (D == 64) SL8_PRO(64);
-  else if (D == 128) SL8_PRO(128);
-  else SL8_PRO(256);
-#undef SL8_PRO
+  const Prologue p{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), qrows, G, N,
+                   q_scale_mul, gate_ratio, q_i8, k_i8, q_scale, k_scale, k_mean,
+                   gate ? gate_flag : nullptr, workspace, static_cast<hipStream_t>(stream), chunk,
+                   (int)C, (int)kbg};
+  if (dtype == SL8_DTYPE_F16) p.go<SL8_DTYPE_F16>(D);
+  else p.go<SL8_DTYPE_BF16>(D);
   SL8_CHECK_LAUNCH("fused prologue");
   return SL8_OK;
 }

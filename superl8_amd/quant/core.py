@@ -92,11 +92,14 @@ def detect_q_outlier_domination(q: torch.Tensor, *, ratio_threshold: float = 12.
 
 
 def _fused_ok(q: torch.Tensor, k: torch.Tensor) -> bool:
-    """Shapes the fused fp16 prologue (sl8_quantize_qk) serves."""
-    return (q.dtype == torch.float16 and k.dtype == torch.float16 and q.dim() == 4
-            and k.dim() == 4 and q.shape[-1] == k.shape[-1] and q.shape[-1] in (64, 128, 256)
+    """Shapes the fused prologue (sl8_quantize_qk) serves."""
+    return (q.dtype == k.dtype and q.dtype in (torch.float16, torch.bfloat16) and q.dim() == 4
+            and k.dim() == 4 and q.shape[-1] == k.shape[-1]
+            and q.shape[-1] in (32, 64, 72, 80, 128, 256)
             and q.shape[0] == k.shape[0] and q.numel() > 0 and k.numel() > 0
-            and k.shape[-2] < (1 << 23))
+            and k.shape[-2] < (1 << 23)
+            # 16-byte loads: a contiguous view at an odd offset takes the separate kernels
+            and all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (q, k)))
 
 
 def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float | None = None,
@@ -105,7 +108,7 @@ def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float 
 
     Returns (fired, quantize_qk's five outputs or None). fired is
     detect_q_outlier_domination(q); when it holds the quantised tensors are
-    not needed (the caller routes to full precision). For fp16 Q/K without
+    not needed (the caller routes to full precision). For fp16 / bf16 Q/K without
     rotation the gate is decided inside the fused prologue (one flag read);
     otherwise it is evaluated first and quantize_qk runs only when it passes.
     Under graph capture the gate is skipped (False), as in
@@ -137,8 +140,8 @@ def quantize_qk(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float | None
     """Quantise Q and smoothed K for the int8 QK^T.
 
     Returns (q_int8, q_scale[..., m, 1] folded with softmax_scale*log2(e),
-    k_int8, k_scale[..., n, 1], k_mean[..., 1, d]). fp16 Q/K without rotation
-    take the fused prologue (three launches); otherwise the K mean and the
+    k_int8, k_scale[..., n, 1], k_mean[..., 1, d]). fp16 / bf16 Q/K without rotation
+    take the fused prologue (two launches); otherwise the K mean and the
     smooth-and-quantise of each side are separate kernels (the smoothed K is
     never written either way).
     """

@@ -102,6 +102,33 @@ def test_fused_gate_decisions(device, D):
             assert bool(flag.item()) == bool(ref.item()) == _torch_gate(c, thr), (thr,)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("B,Hq,Hkv,M,N,D", [(1, 4, 2, 37, 129, 32), (2, 3, 3, 196, 196, 72),
+                                            (1, 2, 1, 61, 6145, 80), (1, 4, 2, 5, 777, 64),
+                                            (1, 2, 2, 130, 6300, 128), (1, 2, 1, 33, 12400, 256)])
+def test_fused_prologue_types_and_head_dims(device, dtype, B, Hq, Hkv, M, N, D):
+    """Both storage types at every head dim, key counts around the growing mean chunks
+    (6144 keys on), against the separate kernels and the torch gate, bit for bit."""
+    g = torch.Generator(device="cpu").manual_seed(N + D)
+    q = (torch.randn(B, Hq, M, D, generator=g) * 1.5).to(dtype).to(device)
+    k = (torch.randn(B, Hkv, N, D, generator=g) * 2 + 3).to(dtype).to(device)
+    q[0, 0, 0, :] = 0
+    m_ref = _C.k_mean(k)
+    qi_ref, qs_ref = _C.quantize_rows_centered(q, None, 0.3)
+    ki_ref, ks_ref = _C.quantize_rows_centered(k, m_ref, 1.0)
+    for spike in (False, True):
+        if spike:
+            q[-1, -1, -1, :] = 0.01
+            q[-1, -1, -1, D - 1] = 90.0
+            qi_ref, qs_ref = _C.quantize_rows_centered(q, None, 0.3)
+        thr = 12.0 if D > 32 else 40.0   # 32 Gaussian values: the median is too loose for 12
+        qi, qs, ki, ks, km, flag = _C.quantize_qk_fused(q, k, 0.3, thr)
+        assert torch.equal(km, m_ref)
+        assert torch.equal(qi, qi_ref) and torch.equal(qs, qs_ref)
+        assert torch.equal(ki, ki_ref) and torch.equal(ks, ks_ref)
+        assert bool(flag.item()) == _torch_gate(q, thr) == spike
+
+
 def test_gate_boundary_exact(device):
     """Rows built so that max/median lands on either side of the threshold by one ulp."""
     D = 128
@@ -128,6 +155,21 @@ def test_attn_fwd_routes_on_fused_gate(device):
     ref = torch.nn.functional.scaled_dot_product_attention(q, k, v, is_causal=True, enable_gqa=True)
     o = ops.attn_int8_fwd(q, k, v, causal=True)
     assert torch.equal(o, ref)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.bfloat16, 72), (torch.float16, 80)])
+def test_attn_fwd_gate_of_new_prologue_forms(device, dtype, D):
+    """bf16 and the head dims 72 / 80 take the deferred gate: quiet and firing calls, and
+    inputs at an odd offset (the separate kernels) give the same codes and the same output."""
+    torch.manual_seed(12)
+    q, k, v = (torch.randn(1, h, 200, D, device=device).to(dtype) for h in (4, 2, 2))
+    o = ops.attn_int8_fwd(q, k, v, causal=True)
+    flat = torch.empty(q.numel() + 1, device=device, dtype=dtype)
+    flat[1:] = q.reshape(-1)
+    assert torch.equal(ops.attn_int8_fwd(flat[1:].view_as(q), k, v, causal=True), o)
+    q[0, 1, 100, 7] = 300.0
+    ref = torch.nn.functional.scaled_dot_product_attention(q, k, v, is_causal=True, enable_gqa=True)
+    assert torch.equal(ops.attn_int8_fwd(q, k, v, causal=True), ref)
 
 
 def test_fused_rejects(device):

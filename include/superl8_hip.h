@@ -306,6 +306,13 @@ int sl8_kv_write_paged(const void* k_new, const void* v_new, const int32_t* slot
                        int8_t* k_cache, float* k_scale, int8_t* v_cache, float* v_scale,
                        int64_t B, int64_t Hkv, int64_t D, int64_t num_blocks,
                        int64_t block_size, void* stream);
+/* sl8_kv_write_paged with every K row multiplied by the normalised Hadamard matrix of order D
+ * first (fp32, rounded to fp16; superl8/quant/rotation.py:28-51 as called from
+ * superl8/ops.py:730-775). k_new / v_new 16-byte, caches 8-byte aligned. */
+int sl8_kv_write_paged_rotated(const void* k_new, const void* v_new, const int32_t* slot_mapping,
+                               int8_t* k_cache, float* k_scale, int8_t* v_cache, float* v_scale,
+                               int64_t B, int64_t Hkv, int64_t D, int64_t num_blocks,
+                               int64_t block_size, void* stream);
 
 /* ------------------------------------------------------------------------
  * Q4_K GEMM/GEMV over native GGUF super-blocks (144 B per 256 weights:

@@ -527,9 +527,13 @@ def attn_paged_decode_k8v3(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_cod
     return out
 
 
-def kv_write_paged(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scale):
+def kv_write_paged(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scale, *,
+                   rotate=False):
     """Quantize-on-write of one new token per (batch, KV head) into the paged int8
-    cache, in place (reference csrc/kernel/attn_paged_decode.cu:360-421)."""
+    cache, in place (reference csrc/kernel/attn_paged_decode.cu:360-421).
+
+    rotate (keyword of this build only): K rows pass through the normalised Hadamard
+    transform first, inside the same launch."""
     _on_gpu(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scale)
     _check(k_new.dtype == torch.float16 and v_new.dtype == torch.float16,
            "kv_write_paged: k_new/v_new must be float16")
@@ -554,8 +558,12 @@ def kv_write_paged(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scal
     _check(D in _HEAD_DIMS_DECODE, f"kv_write_paged: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
     if B == 0:
         return
+    if rotate and any(t.data_ptr() % 16 for t in (k_new, v_new, k_cache, v_cache)):
+        from .quant.rotation import rotate_last
+
+        k_new, rotate = rotate_last(k_new), False
     with torch.cuda.device(k_new.device):
-        call("sl8_kv_write_paged", k_new.data_ptr(), v_new.data_ptr(), slot_mapping.data_ptr(),
+        call("sl8_kv_write_paged_rotated" if rotate else "sl8_kv_write_paged", k_new.data_ptr(), v_new.data_ptr(), slot_mapping.data_ptr(),
              k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(), v_scale.data_ptr(),
              B, Hkv, D, k_cache.shape[0], k_cache.shape[2], stream_of(k_new))
 

@@ -25,6 +25,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "rowquant.hpp"
 
 namespace sl8 {
 namespace {
@@ -1222,6 +1223,45 @@ kv_write_paged_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __rest
   }
 }
 
+// The same write with 16-byte loads, 8 elements per lane and K and V rows side by side (rows
+// [0, rows) are K, the rest V); ROT: the K rows pass through the normalised Hadamard transform
+// first, rounded to fp16 as the separate rotation is. Bound by latency and launches (a batch of
+// 32: 198 KB): the rotation as a matrix product in front (two conversions and a one-workgroup
+// GEMM of 19 us) made 4 launches, 43 us a call; here it is one launch of about 4 us.
+template <int D, bool ROT>
+__global__ void __launch_bounds__(256)
+kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __restrict__ v_new,
+                          const int32_t* __restrict__ slot_mapping, int8_t* __restrict__ k_cache,
+                          float* __restrict__ k_scale, int8_t* __restrict__ v_cache,
+                          float* __restrict__ v_scale, int64_t rows, int h_kv, int bs) {
+  constexpr int LPR = row_lanes(D), RPB = 256 / LPR;
+  const int lane = threadIdx.x % LPR;
+  const int64_t i = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+  const bool live = i < 2 * rows;
+  const bool is_v = live && i >= rows;
+  const int64_t r = live ? (is_v ? i - rows : i) : 0;
+  const int64_t slot = slot_mapping[r / h_kv];
+  float f[8];
+  VecIO<SL8_DTYPE_F16>::unpack(reinterpret_cast<const uint4*>((is_v ? v_new : k_new) + r * D)[lane], f);
+  if constexpr (ROT) {
+    float h[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) h[e] = f[e];
+    hadamard_row<D>(h, lane);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = is_v ? f[e] : Elem<SL8_DTYPE_F16>::round(h[e]);
+  }
+  float amax = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(f[e]));
+  amax = lane_group_max<LPR>(amax);
+  if (!live) return;
+  const float s = amax > 0.f ? __fdiv_rn(amax, 127.f) : 1.f;
+  const int64_t row = ((slot / bs) * h_kv + r % h_kv) * bs + slot % bs;
+  reinterpret_cast<uint2*>((is_v ? v_cache : k_cache) + row * D)[lane] = codes8(f, s);
+  if (lane == 0) (is_v ? v_scale : k_scale)[row] = s;
+}
+
 // ---------------------------------------------------------------------------
 // K8V3 paged decode (reference attn_paged_decode.cuh:114-257 with LowbitV,
 // attn_paged_decode.cu:229-330). K and the split / softmax / merge contract are
@@ -1821,10 +1861,11 @@ extern "C" int sl8_attn_paged_decode_k8v3(const int8_t* q, const float* q_scale,
   return SL8_OK;
 }
 
-extern "C" int sl8_kv_write_paged(const void* k_new, const void* v_new, const int32_t* slot_mapping,
-                                  int8_t* k_cache, float* k_scale, int8_t* v_cache, float* v_scale,
-                                  int64_t B, int64_t Hkv, int64_t D, int64_t num_blocks,
-                                  int64_t block_size, void* stream) {
+namespace sl8 {
+namespace {
+int kv_write(const void* k_new, const void* v_new, const int32_t* slot_mapping, int8_t* k_cache,
+             float* k_scale, int8_t* v_cache, float* v_scale, int64_t B, int64_t Hkv, int64_t D,
+             int64_t num_blocks, int64_t block_size, bool rotate, void* stream) {
   clear_error();
   SL8_CHECK_ARG(B >= 0 && Hkv > 0 && num_blocks >= 0 && block_size > 0,
                 "fni8 kv_write_paged: bad shape");
@@ -1833,14 +1874,54 @@ extern "C" int sl8_kv_write_paged(const void* k_new, const void* v_new, const in
   if (B == 0) return SL8_OK;
   SL8_CHECK_ARG(k_new && v_new && slot_mapping && k_cache && k_scale && v_cache && v_scale,
                 "fni8 kv_write_paged: null pointer");
+  // 16-byte loads and 8-byte stores; inputs or caches at other offsets (views) take the
+  // element-wise kernel, which has no rotation
+  const bool vec = aligned(k_new, 16) && aligned(v_new, 16) && aligned(k_cache, 8) && aligned(v_cache, 8);
+  SL8_CHECK_ARG(vec || !rotate,
+                "fni8 kv_write_paged_rotated: k_new/v_new must be 16-byte and the caches 8-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)(B * Hkv));
   const uint16_t* kn = static_cast<const uint16_t*>(k_new);
   const uint16_t* vn = static_cast<const uint16_t*>(v_new);
-  if (D == 32) kv_write_paged_kernel<32><<<grid, 64, 0, st>>>(kn, vn, slot_mapping, k_cache, k_scale, v_cache, v_scale, (int)Hkv, (int)block_size);
-  else if (D == 64) kv_write_paged_kernel<64><<<grid, 64, 0, st>>>(kn, vn, slot_mapping, k_cache, k_scale, v_cache, v_scale, (int)Hkv, (int)block_size);
-  else if (D == 128) kv_write_paged_kernel<128><<<grid, 64, 0, st>>>(kn, vn, slot_mapping, k_cache, k_scale, v_cache, v_scale, (int)Hkv, (int)block_size);
-  else kv_write_paged_kernel<256><<<grid, 64, 0, st>>>(kn, vn, slot_mapping, k_cache, k_scale, v_cache, v_scale, (int)Hkv, (int)block_size);
+  auto go = [&](auto d_tag) {
+    constexpr int DD = decltype(d_tag)::value;
+    const int64_t rows = B * Hkv;
+    if (!vec) {
+      kv_write_paged_kernel<DD><<<(unsigned)rows, 64, 0, st>>>(
+          kn, vn, slot_mapping, k_cache, k_scale, v_cache, v_scale, (int)Hkv, (int)block_size);
+      return;
+    }
+    constexpr int RPB = 256 / row_lanes(DD);
+    const unsigned grid = (unsigned)((2 * rows + RPB - 1) / RPB);
+    if (rotate)
+      kv_write_paged_vec_kernel<DD, true><<<grid, 256, 0, st>>>(
+          kn, vn, slot_mapping, k_cache, k_scale, v_cache, v_scale, rows, (int)Hkv, (int)block_size);
+    else
+      kv_write_paged_vec_kernel<DD, false><<<grid, 256, 0, st>>>(
+          kn, vn, slot_mapping, k_cache, k_scale, v_cache, v_scale, rows, (int)Hkv, (int)block_size);
+  };
+  if (D == 32) go(std::integral_constant<int, 32>{});
+  else if (D == 64) go(std::integral_constant<int, 64>{});
+  else if (D == 128) go(std::integral_constant<int, 128>{});
+  else go(std::integral_constant<int, 256>{});
   SL8_CHECK_LAUNCH("kv_write_paged");
   return SL8_OK;
+}
+}  // namespace
+}  // namespace sl8
+
+extern "C" int sl8_kv_write_paged(const void* k_new, const void* v_new, const int32_t* slot_mapping,
+                                  int8_t* k_cache, float* k_scale, int8_t* v_cache, float* v_scale,
+                                  int64_t B, int64_t Hkv, int64_t D, int64_t num_blocks,
+                                  int64_t block_size, void* stream) {
+  return kv_write(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scale, B, Hkv, D,
+                  num_blocks, block_size, false, stream);
+}
+
+extern "C" int sl8_kv_write_paged_rotated(const void* k_new, const void* v_new,
+                                          const int32_t* slot_mapping, int8_t* k_cache,
+                                          float* k_scale, int8_t* v_cache, float* v_scale,
+                                          int64_t B, int64_t Hkv, int64_t D, int64_t num_blocks,
+                                          int64_t block_size, void* stream) {
+  return kv_write(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scale, B, Hkv, D,
+                  num_blocks, block_size, true, stream);
 }

@@ -14,6 +14,7 @@
 // pass); the second read is served by L2 for the row sizes used here.
 
 #include "common.hpp"
+#include "rowquant.hpp"
 
 #include <cmath>
 #include <type_traits>
@@ -37,76 +38,12 @@ namespace {
 
 constexpr int QTHREADS = 256;
 
-// Reduction over aligned groups of LPR lanes (a power of two <= 64) with no
-// LDS round trip: DPP inside a 16-lane row (quad_perm [1,0,3,2], quad_perm
-// [2,3,0,1], row_half_mirror, row_mirror: after each step a lane holds the
-// reduction over 2, 4, 8, 16 lanes), then v_permlane16_swap across the row
-// pair and v_permlane32_swap across the wave halves. Every lane of the group
-// ends with the result; op must be associative and commutative (max, integer
-// add: exact in any order).
-template <int LPR, typename F>
-__device__ __forceinline__ uint32_t lane_group_reduce(uint32_t v, F op) {
-  static_assert(LPR >= 1 && LPR <= 64 && (LPR & (LPR - 1)) == 0, "LPR: a power of two <= 64");
-  auto dpp = [](uint32_t x, auto ctrl) __attribute__((always_inline)) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, 0xF, 0xF, false);
-  };
-  if constexpr (LPR >= 2) v = op(v, dpp(v, std::integral_constant<int, 0xB1>{}));
-  if constexpr (LPR >= 4) v = op(v, dpp(v, std::integral_constant<int, 0x4E>{}));
-  if constexpr (LPR >= 8) v = op(v, dpp(v, std::integral_constant<int, 0x141>{}));
-  if constexpr (LPR >= 16) v = op(v, dpp(v, std::integral_constant<int, 0x140>{}));
-  if constexpr (LPR >= 32) {
-    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    v = op(r[0], r[1]);
-  }
-  if constexpr (LPR >= 64) {
-    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    v = op(r[0], r[1]);
-  }
-  return v;
-}
-// v >= 0 and not NaN (an amax started at 0 and grown by fmaxf, which drops
-// NaN): the unsigned order of the bit patterns is the float order, and 0 is
-// the identity of the unsigned max the DPP moves fold into
-template <int LPR>
-__device__ __forceinline__ float lane_group_max(float v) {
-  return __uint_as_float(lane_group_reduce<LPR>(__float_as_uint(v), [](uint32_t a, uint32_t b) {
-    return a > b ? a : b;
-  }));
-}
-template <int LPR>
-__device__ __forceinline__ int lane_group_sum(int v) {
-  return (int)lane_group_reduce<LPR>((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
-}
-
-template <int DT> struct Elem;
-template <> struct Elem<SL8_DTYPE_F16> {
-  using T = uint16_t;
-  __device__ static float ld(const T* p, int64_t i) { return h2f(p[i]); }
-  __device__ static float round(float v) { return h2f(f2h_bits(v)); }
-};
-template <> struct Elem<SL8_DTYPE_BF16> {
-  using T = uint16_t;
-  __device__ static float ld(const T* p, int64_t i) { return bf2f(p[i]); }
-  __device__ static float round(float v) { return bf2f(f2bf_bits(v)); }
-};
-template <> struct Elem<SL8_DTYPE_F32> {
-  using T = float;
-  __device__ static float ld(const T* p, int64_t i) { return p[i]; }
-  __device__ static float round(float v) { return v; }
-};
-
 // Value of element d of a row after the optional mean shift.
 template <int DT, bool MEAN>
 __device__ __forceinline__ float row_val(const typename Elem<DT>::T* xr, const float* mr, int d) {
   float v = Elem<DT>::ld(xr, d);
   if constexpr (MEAN) v = Elem<DT>::round(v - mr[d]);
   return v;
-}
-
-__device__ __forceinline__ int8_t code_of(float v, float safe) {
-  float r = rintf(__fdiv_rn(v, safe));
-  r = fminf(fmaxf(r, -127.f), 127.f);
-  return static_cast<int8_t>(r);
 }
 
 // rows = G*N; row r uses mean row r / rows_per_mean.
@@ -150,96 +87,10 @@ quant_rows_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __res
 }
 
 
-// Eight codes clamp(rint(fl(x / safe))) without a division per element.
-// |x| <= amax, so |x / safe| <= 127 * (1 + 2^-23) and, with inv = v_rcp_f32(safe)
-// (at most 1 ulp from 1 / safe; safe is normal and above 2^-120: fp16 rows always
-// are, 2^-24 / 127 at least, bf16 callers check),
-// r = fl(x * inv) is within 128 * (2^-23 + 2^-24) = 1.5 * 2^-16 of x / safe,
-// and fl(x / safe) within 2^-17 of it: |r - fl(x / safe)| < 2^-14. n = r
-// rounded to nearest-even by the 1.5 * 2^23 magic constant; unless
-// |r - n| > 0.5 - 2^-14 (r near a half-integer) both r and fl(x / safe)
-// round to n. Lanes holding such an element (about 1e-4 of them) take the
-// IEEE division, under a wave-uniform branch so the common path never
-// executes it.
-__device__ __forceinline__ uint2 codes8(const float* f, float safe) {
-  const float inv = __builtin_amdgcn_rcpf(safe);
-  constexpr float MAGIC = 12582912.f;  // 1.5 * 2^23
-  float n[8];
-  bool amb = false;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float r = f[e] * inv;
-    n[e] = (r + MAGIC) - MAGIC;
-    amb |= !(fabsf(r - n[e]) <= 0.5f - 0x1p-14f);  // also catches inf / NaN
-  }
-  if (__builtin_expect(__ballot(amb) != 0, 0)) {
-    if (amb) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        n[e] = rintf(__fdiv_rn(f[e], safe));
-        if (n[e] != n[e]) n[e] = -127.f;  // NaN: the clamp of fmaxf / fminf gives -127
-      }
-    }
-  }
-  // n is an integer in [-128, 128] (or the division's result): clamp as int
-  uint32_t w[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    int c[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c[e] = __builtin_amdgcn_fmed3f(n[4 * i + e], -127.f, 127.f);
-    // bytes 0 of c0..c3 -> one dword (v_perm_b32: selectors 0-3 pick the
-    // second operand's bytes, 4-7 the first's, 0x0c a zero byte)
-    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)c[1], (uint32_t)c[0], 0x0c0c0400u);
-    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)c[3], (uint32_t)c[2], 0x04000c0cu);
-    w[i] = lo | hi;
-  }
-  return make_uint2(w[0], w[1]);
-}
-
-// The same codes by IEEE division (any safe).
-__device__ __forceinline__ uint2 codes8_exact(const float* f, float safe) {
-  uint32_t w[2] = {0, 0};
-#pragma unroll
-  for (int e = 0; e < 8; ++e) w[e / 4] |= (uint32_t)(uint8_t)code_of(f[e], safe) << (8 * (e % 4));
-  return make_uint2(w[0], w[1]);
-}
-
-// Eight codes of a 16-bit row (see codes8; bf16 rows may have scales below its range).
-template <int DT>
-__device__ __forceinline__ uint2 row_codes8(const float* f, float safe) {
-  return DT == SL8_DTYPE_F16 || safe >= 0x1p-120f ? codes8(f, safe) : codes8_exact(f, safe);
-}
-
 // Vectorised variant: LPR lanes per row (LPR = BT: one workgroup per row),
 // each lane holding NV 16-byte vectors of the row in registers for both the
 // amax and the code pass (one HBM read per element). Needs K a multiple of
 // the elements per 16 bytes (EPV) and a 16-byte aligned base.
-template <int DT> struct VecIO;
-template <> struct VecIO<SL8_DTYPE_F16> {
-  static constexpr int EPV = 8;
-  __device__ static void unpack(uint4 v, float* f) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { f[2 * i] = h2f(w[i] & 0xFFFF); f[2 * i + 1] = h2f(w[i] >> 16); }
-  }
-};
-template <> struct VecIO<SL8_DTYPE_BF16> {
-  static constexpr int EPV = 8;
-  __device__ static void unpack(uint4 v, float* f) {
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { f[2 * i] = bf2f(w[i] & 0xFFFF); f[2 * i + 1] = bf2f(w[i] >> 16); }
-  }
-};
-template <> struct VecIO<SL8_DTYPE_F32> {
-  static constexpr int EPV = 4;
-  __device__ static void unpack(uint4 v, float* f) {
-    f[0] = __uint_as_float(v.x); f[1] = __uint_as_float(v.y);
-    f[2] = __uint_as_float(v.z); f[3] = __uint_as_float(v.w);
-  }
-};
-
 template <int DT, int BT, int LPR, int NV, bool MEAN>
 __global__ void __launch_bounds__(BT)
 quant_rows_vec_kernel(const typename Elem<DT>::T* __restrict__ x, const float* __restrict__ mean,
@@ -839,9 +690,6 @@ int64_t pro_chunk_rows(int64_t N) {
   return std::max<int64_t>(PRO_CHUNK, (per + PRO_CHUNK - 1) / PRO_CHUNK * PRO_CHUNK);
 }
 
-// Lanes per row (8 elements, 16 bytes each); the first D / 8 of them hold elements.
-constexpr int pro_lpr(int D) { return D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 16 : 32; }
-
 // fp16 bits -> value * 2^24 as an exact integer (finite inputs: |result| < 2^40)
 __device__ __forceinline__ long long f16_fixed24(uint32_t h) {
   const uint32_t e = (h >> 10) & 31u, m = h & 1023u;
@@ -869,7 +717,7 @@ template <int DT, int D>
 __device__ __forceinline__ void mean_chunk(const uint16_t* __restrict__ kg, int64_t n0, int64_t n1,
                                            typename MeanSum<DT>::T* __restrict__ part) {
   using S = MeanSum<DT>;
-  constexpr int LPR = pro_lpr(D), NL = D / 8;
+  constexpr int LPR = row_lanes(D), NL = D / 8;
   constexpr int RPP = 256 / LPR;                     // rows per pass
   constexpr int NIT = PRO_CHUNK / RPP < 8 ? PRO_CHUNK / RPP : 8;  // passes in flight
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
@@ -916,7 +764,7 @@ __device__ __forceinline__ void smooth_rows(const uint16_t* __restrict__ kg, int
                                             float* __restrict__ mean_out,
                                             int8_t* __restrict__ kq, float* __restrict__ kscale) {
   using S = MeanSum<DT>;
-  constexpr int LPR = pro_lpr(D), NL = D / 8, RPP = 256 / LPR, NP = PRO_KROWS / RPP;
+  constexpr int LPR = row_lanes(D), NL = D / 8, RPP = 256 / LPR, NP = PRO_KROWS / RPP;
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
   const bool on = lane < NL;
   uint4 raw[NP];
@@ -993,7 +841,7 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
                   const uint16_t* __restrict__ q, int64_t qrows, float qmul, float ratio,
                   int8_t* __restrict__ q_i8, float* __restrict__ q_scale,
                   int32_t* __restrict__ flag) {
-  constexpr int LPR = pro_lpr(D), NL = D / 8, RPP = 256 / LPR;
+  constexpr int LPR = row_lanes(D), NL = D / 8, RPP = 256 / LPR;
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
   if ((int)blockIdx.x < nkb) {
     const int64_t g = blockIdx.x / kbg;
@@ -1072,7 +920,7 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
 }
 
 int prologue_nqb(int64_t qrows, int D) {
-  const int64_t rpp = 256 / pro_lpr(D) * PRO_QP;
+  const int64_t rpp = 256 / row_lanes(D) * PRO_QP;
   return (int)std::min<int64_t>(PRO_QBLOCKS_MAX, (qrows + rpp - 1) / rpp);
 }
 

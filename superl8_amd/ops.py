@@ -14,6 +14,7 @@ import math
 import torch
 
 from . import _C
+from .quant.rotation import hadamard_dim
 
 # Decode-shape M cap for the k-quant linear (reference ops.py:1289).
 _KQUANT_DECODE_MAX_M = 16
@@ -162,12 +163,10 @@ def quantize_kv_write_paged(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: t
     """Quantise-on-write of one new token per sequence into the paged int8 KV pool,
     in place (reference ops.py:730-775): per-token scales for K and V; `rotate`
     applies the Hadamard rotation to K (the smoothing usable one token at a time)."""
-    from .quant.rotation import rotate_last
-
     if rotate:
-        k_new = rotate_last(k_new)
+        hadamard_dim(k_new.shape[-1])
     _C.kv_write_paged(k_new.contiguous(), v_new.contiguous(), slot_mapping.contiguous(),
-                      k_cache, k_scale, v_cache, v_scale)
+                      k_cache, k_scale, v_cache, v_scale, rotate=rotate)
 
 
 def attn_paged_decode_cached(q: torch.Tensor, k_cache: torch.Tensor, k_scale: torch.Tensor,

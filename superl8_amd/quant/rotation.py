@@ -6,11 +6,17 @@ import functools
 import torch
 
 
+def hadamard_dim(d: int) -> int:
+    """d, if a Sylvester-Hadamard matrix of that order exists."""
+    if d <= 0 or d & (d - 1):
+        raise ValueError(f"Hadamard needs a power-of-two dim, got {d}")
+    return d
+
+
 @functools.lru_cache(maxsize=8)
 def hadamard_matrix(d: int, device: str = "cpu", dtype: torch.dtype = torch.float32):
     """Normalised Sylvester-Hadamard M [d, d] (M @ M.T == I); d a power of two."""
-    if d <= 0 or d & (d - 1):
-        raise ValueError(f"Hadamard needs a power-of-two dim, got {d}")
+    hadamard_dim(d)
     h = torch.ones(1, 1, dtype=torch.float32)
     while h.shape[0] < d:
         h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)

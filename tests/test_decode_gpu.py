@@ -303,6 +303,53 @@ def test_kv_write_paged_bit_exact(device, D):
     np.testing.assert_array_equal(_np(tens[6]), rvs)
 
 
+@pytest.mark.parametrize("B,Hkv,D,bs", [(1, 1, 32, 16), (5, 3, 64, 8), (33, 8, 128, 16), (2, 2, 256, 24)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_kv_write_paged_forms(device, B, Hkv, D, bs, offset):
+    """The vector and the element-wise write (inputs at an odd offset) and the fused rotation.
+
+    Rotation: the kernel's 32-bit butterflies and the 64-bit product may round to neighbouring
+    fp16 values (2^-11 relative), which moves a scale by at most that and a code by at most one
+    step; the rows' error against 64 bits is no larger than the matrix product's."""
+    g = torch.Generator(device="cpu").manual_seed(B * 100 + D)
+
+    def shifted(x):
+        flat = torch.empty(x.numel() + offset, device=device, dtype=x.dtype)
+        flat[offset:] = x.to(device).reshape(-1)
+        return flat[offset:].view(x.shape)
+
+    kn, vn = (shifted((torch.randn(B, Hkv, D, generator=g) * 2).half()) for _ in range(2))
+    kn[0, 0] = 0
+    slots = torch.randperm(4 * B * bs, generator=g)[:B].to(torch.int32).to(device)
+    pool = (4 * B, Hkv, bs)
+
+    def caches():
+        return [torch.zeros(*pool, D, device=device, dtype=torch.int8), torch.zeros(pool, device=device),
+                torch.zeros(*pool, D, device=device, dtype=torch.int8), torch.zeros(pool, device=device)]
+
+    got = caches()
+    _C.kv_write_paged(kn, vn, slots, *got)
+    want = [_np(x) for x in caches()]
+    oqn.kv_write_paged(_np(kn.float()), _np(vn.float()), _np(slots), *want)
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(_np(a), b)
+    rot = caches()
+    _C.kv_write_paged(kn, vn, slots, *rot, rotate=True)
+    assert torch.equal(rot[2], got[2]) and torch.equal(rot[3], got[3])  # V is not rotated
+    i = slots.long()
+    codes, scale = rot[0][i // bs, :, i % bs], rot[1][i // bs, :, i % bs]
+    h = torch.ones(1, 1, dtype=torch.float64, device=device)
+    while h.shape[0] < D:
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+    ref = (kn.double() @ h / D ** 0.5).half()
+    s_ref = ref.double().abs().amax(-1) / 127
+    s_ref = torch.where(s_ref == 0, torch.ones_like(s_ref), s_ref)
+    assert ((scale.double() / s_ref - 1).abs() <= 2.0 ** -10).all()
+    c_ref = (ref.double() / s_ref[..., None]).round().clamp(-127, 127)
+    assert ((codes.double() - c_ref).abs() <= 1).all()
+    assert (codes.double() != c_ref).float().mean() <= 0.01
+
+
 @pytest.mark.parametrize("D,lens", [(128, (40, 97, 1)), (64, (130,)), (32, (70, 5))])
 def test_paged_end_to_end(device, D, lens):
     """Token-by-token quantize-on-write into a shuffled block pool, then one paged

@@ -302,6 +302,39 @@ int sl8_attn_paged_decode_k8v3(const int8_t* q, const float* q_scale, const int8
                                int64_t max_blocks_per_seq, int64_t max_context_len,
                                int64_t num_splits, void* workspace, size_t workspace_bytes,
                                void* stream);
+/* Decode steps that start from the fp16 / bf16 query [B,Hq,1,D] (16-byte aligned): the query is
+ * rotated (rotate != 0: times the normalised Hadamard matrix, in fp32, rounded to its type),
+ * quantised per row and its scale multiplied by q_scale_mul (softmax_scale * log2 e) in a launch
+ * of their own, in place of the caller's (reference superl8/ops.py:671-727,778-915).
+ * The paged forms also plan their splits on the device from context_lens (there is no num_splits):
+ * equal work per workgroup over a batch of mixed lengths. Workspace of the paged forms:
+ * sl8_attn_paged_decode_q16_workspace() bytes, 0 if the call cannot be planned (B > 1024, or
+ * contexts of more than 256 splits that the streaming kernel's block-table staging can hold): use
+ * sl8_attn_paged_decode / _k8v3 then. */
+size_t sl8_attn_paged_decode_q16_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t D,
+                                           int64_t num_blocks, int64_t block_size,
+                                           int64_t max_context_len, int k8v3);
+int sl8_attn_paged_decode_q16(const void* q, int q_dtype, int rotate, float q_scale_mul,
+                              const int8_t* k_cache, const float* k_scale, const int8_t* v_cache,
+                              const float* v_scale, const int32_t* block_table,
+                              const int32_t* context_lens, void* out, int64_t B, int64_t Hq,
+                              int64_t Hkv, int64_t D, int64_t num_blocks, int64_t block_size,
+                              int64_t max_blocks_per_seq, int64_t max_context_len, void* workspace,
+                              size_t workspace_bytes, void* stream);
+int sl8_attn_paged_decode_k8v3_q16(const void* q, int q_dtype, int rotate, float q_scale_mul,
+                                   const int8_t* k_cache, const float* k_scale,
+                                   const int32_t* v_packed, const float* v_norm,
+                                   const float* v_codebook, const int32_t* block_table,
+                                   const int32_t* context_lens, void* out, int64_t B, int64_t Hq,
+                                   int64_t Hkv, int64_t D, int64_t num_blocks, int64_t block_size,
+                                   int64_t max_blocks_per_seq, int64_t max_context_len,
+                                   void* workspace, size_t workspace_bytes, void* stream);
+size_t sl8_attn_int8_decode_kv8_q16_workspace(int64_t B, int64_t Hq, int64_t D, int64_t num_splits);
+int sl8_attn_int8_decode_kv8_q16(const void* q, int q_dtype, int rotate, float q_scale_mul,
+                                 const int8_t* k, const float* k_scale, const int8_t* v,
+                                 const float* v_scale, void* out, int64_t B, int64_t Hq,
+                                 int64_t Hkv, int64_t N, int64_t D, int64_t num_splits,
+                                 void* workspace, size_t workspace_bytes, void* stream);
 int sl8_kv_write_paged(const void* k_new, const void* v_new, const int32_t* slot_mapping,
                        int8_t* k_cache, float* k_scale, int8_t* v_cache, float* v_scale,
                        int64_t B, int64_t Hkv, int64_t D, int64_t num_blocks,

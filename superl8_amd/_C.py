@@ -372,36 +372,46 @@ def attn_int8_decode(q, q_scale, k, k_scale, v, num_splits=-1):
     return out
 
 
-def attn_int8_decode_kv8(q, q_scale, k, k_scale, v, v_scale, num_splits=-1):
-    """Decode over an int8 K/V cache (reference csrc/kernel/attn_decode.cu:245-320):
-    q int8 [B,Hq,1,D], q_scale fp32 [B,Hq,1], k int8 [B,Hkv,N,D], k_scale fp32 [B,Hkv,N],
-    v int8 [B,Hkv,N,D], v_scale fp32 [B,Hkv,D] (per channel) -> fp16 [B,Hq,1,D]."""
-    _on_gpu(q, q_scale, k, k_scale, v, v_scale)
-    _check(q.dtype == torch.int8 and k.dtype == torch.int8 and v.dtype == torch.int8,
-           "decode_kv8: q/k/v must be int8")
-    _check(q_scale.dtype == torch.float32 and k_scale.dtype == torch.float32 and
-           v_scale.dtype == torch.float32, "decode_kv8: scales must be float32")
+def _kv8_checks(q, k, k_scale, v, v_scale, num_splits):
+    """The checks of the int8-V decode but those on q's type and scale; sizes and split count."""
+    _on_gpu(q, k, k_scale, v, v_scale)
+    _check(k.dtype == torch.int8 and v.dtype == torch.int8, "decode_kv8: q/k/v must be int8")
+    _check(k_scale.dtype == torch.float32 and v_scale.dtype == torch.float32,
+           "decode_kv8: scales must be float32")
     _check(q.dim() == 4 and k.dim() == 4 and v.dim() == 4, "decode_kv8: expect [B,H,S,D]")
     _check(q.shape[2] == 1, "decode_kv8: query length M must be 1 (decode)")
-    _contig(q, q_scale, k, k_scale, v, v_scale)
+    _contig(q, k, k_scale, v, v_scale)
     B, H, _, D = q.shape
     Hkv, N = k.shape[1], k.shape[2]
     _check(k.shape[0] == B and v.shape[0] == B and v.shape[1] == Hkv,
            "decode_kv8: batch/head mismatch")
     _check(Hkv > 0 and H % Hkv == 0, "decode_kv8: H_q must be divisible by H_kv (GQA)")
     _check(k.shape[3] == D and v.shape[3] == D and v.shape[2] == N, "decode_kv8: K/V shape mismatch")
-    _check(q_scale.numel() == B * H and k_scale.numel() == B * Hkv * N and
-           v_scale.numel() == B * Hkv * D, "decode_kv8: scale shape mismatch")
+    _check(k_scale.numel() == B * Hkv * N and v_scale.numel() == B * Hkv * D,
+           "decode_kv8: scale shape mismatch")
     _check(D in _HEAD_DIMS_DECODE, f"decode_kv8: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
     num_splits = int(num_splits)
     _check(num_splits != 0,
            f"decode_kv8: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
+    ns = choose_n_splits(N, B, Hkv) if num_splits < 0 else num_splits
+    return B, H, Hkv, N, D, ns
+
+
+def attn_int8_decode_kv8(q, q_scale, k, k_scale, v, v_scale, num_splits=-1):
+    """Decode over an int8 K/V cache (reference csrc/kernel/attn_decode.cu:245-320):
+    q int8 [B,Hq,1,D], q_scale fp32 [B,Hq,1], k int8 [B,Hkv,N,D], k_scale fp32 [B,Hkv,N],
+    v int8 [B,Hkv,N,D], v_scale fp32 [B,Hkv,D] (per channel) -> fp16 [B,Hq,1,D]."""
+    _on_gpu(q, q_scale, k)
+    _check(q.dtype == torch.int8, "decode_kv8: q/k/v must be int8")
+    _check(q_scale.dtype == torch.float32, "decode_kv8: scales must be float32")
+    B, H, Hkv, N, D, ns = _kv8_checks(q, k, k_scale, v, v_scale, num_splits)
+    _contig(q_scale)
+    _check(q_scale.numel() == B * H, "decode_kv8: scale shape mismatch")
     out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
     if B == 0 or H == 0:
         return out
     if N == 0:
         return out.zero_()
-    ns = choose_n_splits(N, B, Hkv) if num_splits < 0 else num_splits
     _check(1 <= ns <= DEC_MAX_SPLITS, f"decode_kv8: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
     ws_bytes = _lib.load().sl8_attn_int8_decode_workspace(B, H, D, ns)
     ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
@@ -412,37 +422,50 @@ def attn_int8_decode_kv8(q, q_scale, k, k_scale, v, v_scale, num_splits=-1):
     return out
 
 
+def attn_int8_decode_kv8_q16(q, q_mul, rotate, k, k_scale, v, v_scale, num_splits=-1):
+    """attn_int8_decode_kv8 from the fp16/bf16 query [B,Hq,1,D] (see q16_ok): rotated and
+    quantised (scale times q_mul) in the same call."""
+    B, H, Hkv, N, D, ns = _kv8_checks(q, k, k_scale, v, v_scale, num_splits)
+    out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
+    if N == 0:
+        return out.zero_()
+    _check(1 <= ns <= DEC_MAX_SPLITS, f"decode_kv8: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
+    ws_bytes = _lib.load().sl8_attn_int8_decode_kv8_q16_workspace(B, H, D, ns)
+    ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
+    with torch.cuda.device(q.device):
+        call("sl8_attn_int8_decode_kv8_q16", q.data_ptr(), dtype_code(q.dtype), int(bool(rotate)),
+             float(q_mul), k.data_ptr(), k_scale.data_ptr(), v.data_ptr(), v_scale.data_ptr(),
+             out.data_ptr(), B, H, Hkv, N, D, ns, ws.data_ptr(), ws_bytes, stream_of(q))
+    return out
+
+
 def paged_choose_n_splits(n_len_max, bhq):
     """Auto split count of the paged decode (reference attn_paged_decode.cu:14-31)."""
     return int(_lib.load().sl8_paged_choose_num_splits(int(n_len_max), int(bhq)))
 
 
-def attn_paged_decode(q, q_scale, k_cache, k_scale, v_cache, v_scale, block_table, context_lens,
-                      block_size, max_context_len, num_splits=-1):
-    """Paged-KV decode (reference csrc/kernel/attn_paged_decode.cu:107-240): q int8
-    [B,Hq,1,D], q_scale fp32 [B,Hq,1], k_cache/v_cache int8 [num_blocks,Hkv,bs,D],
-    k_scale/v_scale fp32 [num_blocks,Hkv,bs], block_table int32 [B,max_blocks],
-    context_lens int32 [B] -> fp16 [B,Hq,1,D]."""
-    _on_gpu(q, q_scale, k_cache, k_scale, v_cache, v_scale, block_table, context_lens)
-    _check(q.dtype == torch.int8 and k_cache.dtype == torch.int8 and v_cache.dtype == torch.int8,
+def _paged_checks(q, k_cache, k_scale, v_cache, v_scale, block_table, context_lens, block_size,
+                  max_context_len):
+    """The checks of the paged int8 decode but those on q's type and scale; the call's sizes."""
+    _on_gpu(q, k_cache, k_scale, v_cache, v_scale, block_table, context_lens)
+    _check(k_cache.dtype == torch.int8 and v_cache.dtype == torch.int8,
            "paged_decode: q/k_cache/v_cache must be int8")
-    _check(q_scale.dtype == torch.float32 and k_scale.dtype == torch.float32 and
-           v_scale.dtype == torch.float32, "paged_decode: scales must be float32")
+    _check(k_scale.dtype == torch.float32 and v_scale.dtype == torch.float32,
+           "paged_decode: scales must be float32")
     _check(block_table.dtype == torch.int32 and context_lens.dtype == torch.int32,
            "paged_decode: block_table/context_lens must be int32")
     _check(q.dim() == 4 and q.shape[2] == 1, "paged_decode: q must be [B,H_q,1,D]")
     _check(k_cache.dim() == 4 and v_cache.dim() == 4,
            "paged_decode: k_cache/v_cache must be [num_blocks,H_kv,block_size,D]")
-    _contig(q, q_scale, k_cache, k_scale, v_cache, v_scale, block_table, context_lens)
+    _contig(q, k_cache, k_scale, v_cache, v_scale, block_table, context_lens)
     B, H, _, D = q.shape
-    nblk, Hkv, bs = k_cache.shape[0], k_cache.shape[1], k_cache.shape[2]
+    nblk, Hkv, bs, Dk = k_cache.shape
     _check(bs == block_size, "paged_decode: block_size mismatch vs k_cache.size(2)")
-    _check(k_cache.shape[3] == D and v_cache.shape == k_cache.shape,
+    _check(Dk == D and v_cache.shape == k_cache.shape,
            "paged_decode: k_cache/v_cache shape mismatch")
     _check(Hkv > 0 and H % Hkv == 0, "paged_decode: H_q must be divisible by H_kv (GQA)")
     _check(k_cache.numel() == k_scale.numel() * D and v_cache.numel() == v_scale.numel() * D,
            "paged_decode: scale shape mismatch vs cache")
-    _check(q_scale.numel() == B * H, "paged_decode: q_scale shape mismatch")
     _check(block_table.dim() == 2 and block_table.shape[0] == B,
            "paged_decode: block_table must be [B, max_blocks_per_seq]")
     _check(context_lens.dim() == 1 and context_lens.shape[0] == B,
@@ -451,6 +474,22 @@ def attn_paged_decode(q, q_scale, k_cache, k_scale, v_cache, v_scale, block_tabl
     maxb = block_table.shape[1]
     _check(0 <= max_context_len <= maxb * bs,
            "paged_decode: max_context_len exceeds block_table capacity")
+    return B, H, Hkv, D, nblk, bs, maxb
+
+
+def attn_paged_decode(q, q_scale, k_cache, k_scale, v_cache, v_scale, block_table, context_lens,
+                      block_size, max_context_len, num_splits=-1):
+    """Paged-KV decode (reference csrc/kernel/attn_paged_decode.cu:107-240): q int8
+    [B,Hq,1,D], q_scale fp32 [B,Hq,1], k_cache/v_cache int8 [num_blocks,Hkv,bs,D],
+    k_scale/v_scale fp32 [num_blocks,Hkv,bs], block_table int32 [B,max_blocks],
+    context_lens int32 [B] -> fp16 [B,Hq,1,D]."""
+    _on_gpu(q, q_scale, k_cache)
+    _check(q.dtype == torch.int8, "paged_decode: q/k_cache/v_cache must be int8")
+    _check(q_scale.dtype == torch.float32, "paged_decode: scales must be float32")
+    B, H, Hkv, D, nblk, bs, maxb = _paged_checks(q, k_cache, k_scale, v_cache, v_scale, block_table,
+                                                 context_lens, block_size, max_context_len)
+    _contig(q_scale)
+    _check(q_scale.numel() == B * H, "paged_decode: q_scale shape mismatch")
     num_splits = int(num_splits)
     _check(num_splits != 0,
            f"paged_decode: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
@@ -469,31 +508,53 @@ def attn_paged_decode(q, q_scale, k_cache, k_scale, v_cache, v_scale, block_tabl
     return out
 
 
-def attn_paged_decode_k8v3(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_codebook,
-                           block_table, context_lens, block_size, max_context_len,
-                           num_splits=-1):
-    """Paged decode over a K8V3 store (reference csrc/kernel/attn_paged_decode.cu:229-330):
-    K as attn_paged_decode; V as 3-bit Lloyd-Max codes v_packed int32
-    [num_blocks,Hkv,bs,3D/32], per-128-channel norms v_norm fp32 [num_blocks,Hkv,bs,D/128]
-    and a codebook fp32 [8]; D 128 or 256 -> fp16 [B,Hq,1,D]."""
+def q16_ok(q) -> bool:
+    """Whether the decode entries that quantise the 16-bit query themselves serve q."""
+    return (q.is_cuda and q.dtype in (torch.float16, torch.bfloat16) and q.numel() > 0
+            and q.shape[-1] in _HEAD_DIMS_DECODE and q.data_ptr() % 16 == 0)
+
+
+def attn_paged_decode_q16(q, q_mul, rotate, k_cache, k_scale, v_cache, v_scale, block_table,
+                          context_lens, block_size, max_context_len):
+    """attn_paged_decode from the fp16/bf16 query [B,Hq,1,D] (see q16_ok): rotated, quantised
+    (scale times q_mul) and its splits planned on the device. None if the batch or the
+    contexts are too large to plan."""
+    B, H, Hkv, D, nblk, bs, maxb = _paged_checks(q, k_cache, k_scale, v_cache, v_scale, block_table,
+                                                 context_lens, block_size, max_context_len)
+    with torch.cuda.device(q.device):
+        ws_bytes = _lib.load().sl8_attn_paged_decode_q16_workspace(B, H, Hkv, D, nblk, bs,
+                                                                   max_context_len, 0)
+        if not ws_bytes:
+            return None
+        out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
+        ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
+        call("sl8_attn_paged_decode_q16", q.data_ptr(), dtype_code(q.dtype), int(bool(rotate)),
+             float(q_mul), k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(),
+             v_scale.data_ptr(), block_table.data_ptr(), context_lens.data_ptr(), out.data_ptr(),
+             B, H, Hkv, D, nblk, bs, maxb, int(max_context_len), ws.data_ptr(), ws_bytes,
+             stream_of(q))
+    return out
+
+
+def _k8v3_checks(q, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table, context_lens,
+                 block_size, max_context_len):
+    """The checks of the K8V3 decode but those on q's type and scale; the call's sizes."""
     tag = "paged_decode_k8v3"
-    _on_gpu(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table,
-            context_lens)
-    _check(q.dtype == torch.int8 and k_cache.dtype == torch.int8, f"{tag}: q/k_cache must be int8")
+    _on_gpu(q, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table, context_lens)
+    _check(k_cache.dtype == torch.int8, f"{tag}: q/k_cache must be int8")
     _check(v_packed.dtype == torch.int32, f"{tag}: v_packed must be int32")
-    _check(q_scale.dtype == torch.float32 and k_scale.dtype == torch.float32 and
-           v_norm.dtype == torch.float32 and v_codebook.dtype == torch.float32,
-           f"{tag}: scales/norms/codebook must be float32")
+    _check(k_scale.dtype == torch.float32 and v_norm.dtype == torch.float32 and
+           v_codebook.dtype == torch.float32, f"{tag}: scales/norms/codebook must be float32")
     _check(block_table.dtype == torch.int32 and context_lens.dtype == torch.int32,
            f"{tag}: block_table/context_lens must be int32")
     _check(q.dim() == 4 and q.shape[2] == 1, f"{tag}: q must be [B,H_q,1,D]")
     _check(k_cache.dim() == 4 and v_packed.dim() == 4 and v_norm.dim() == 4,
            f"{tag}: caches must be [num_blocks,H_kv,block_size,...]")
-    _contig(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table, context_lens)
+    _contig(q, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table, context_lens)
     B, H, _, D = q.shape
-    nblk, Hkv, bs = k_cache.shape[0], k_cache.shape[1], k_cache.shape[2]
+    nblk, Hkv, bs, Dk = k_cache.shape
     _check(bs == block_size, f"{tag}: block_size mismatch vs k_cache.size(2)")
-    _check(k_cache.shape[3] == D and tuple(v_packed.shape[:3]) == (nblk, Hkv, bs) and
+    _check(Dk == D and tuple(v_packed.shape[:3]) == (nblk, Hkv, bs) and
            tuple(v_norm.shape[:3]) == (nblk, Hkv, bs),
            f"{tag}: k_cache/v_packed/v_norm shape mismatch")
     _check(Hkv > 0 and H % Hkv == 0, f"{tag}: H_q must be divisible by H_kv (GQA)")
@@ -503,12 +564,30 @@ def attn_paged_decode_k8v3(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_cod
            f"{tag}: v_packed last dim must be D*3/32, got {v_packed.shape[3]}")
     _check(v_norm.shape[3] == D // 128, f"{tag}: v_norm last dim must be D/128, got {v_norm.shape[3]}")
     _check(v_codebook.dim() == 1 and v_codebook.numel() == 8, f"{tag}: v_codebook must be [8] fp32")
-    _check(q_scale.numel() == B * H, f"{tag}: q_scale shape mismatch")
     _check(block_table.dim() == 2 and block_table.shape[0] == B,
            f"{tag}: block_table must be [B, max_blocks_per_seq]")
     _check(context_lens.dim() == 1 and context_lens.shape[0] == B, f"{tag}: context_lens must be [B]")
     maxb = block_table.shape[1]
     _check(0 <= max_context_len <= maxb * bs, f"{tag}: max_context_len exceeds block_table capacity")
+    return B, H, Hkv, D, nblk, bs, maxb
+
+
+def attn_paged_decode_k8v3(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_codebook,
+                           block_table, context_lens, block_size, max_context_len,
+                           num_splits=-1):
+    """Paged decode over a K8V3 store (reference csrc/kernel/attn_paged_decode.cu:229-330):
+    K as attn_paged_decode; V as 3-bit Lloyd-Max codes v_packed int32
+    [num_blocks,Hkv,bs,3D/32], per-128-channel norms v_norm fp32 [num_blocks,Hkv,bs,D/128]
+    and a codebook fp32 [8]; D 128 or 256 -> fp16 [B,Hq,1,D]."""
+    tag = "paged_decode_k8v3"
+    _on_gpu(q, q_scale, k_cache)
+    _check(q.dtype == torch.int8, f"{tag}: q/k_cache must be int8")
+    _check(q_scale.dtype == torch.float32, f"{tag}: scales/norms/codebook must be float32")
+    B, H, Hkv, D, nblk, bs, maxb = _k8v3_checks(q, k_cache, k_scale, v_packed, v_norm, v_codebook,
+                                                block_table, context_lens, block_size,
+                                                max_context_len)
+    _contig(q_scale)
+    _check(q_scale.numel() == B * H, f"{tag}: q_scale shape mismatch")
     num_splits = int(num_splits)
     _check(num_splits != 0,
            f"{tag}: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
@@ -524,6 +603,27 @@ def attn_paged_decode_k8v3(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_cod
              k_scale.data_ptr(), v_packed.data_ptr(), v_norm.data_ptr(), v_codebook.data_ptr(),
              block_table.data_ptr(), context_lens.data_ptr(), out.data_ptr(), B, H, Hkv, D, nblk,
              bs, maxb, int(max_context_len), ns, ws.data_ptr(), ws_bytes, stream_of(q))
+    return out
+
+
+def attn_paged_decode_k8v3_q16(q, q_mul, rotate, k_cache, k_scale, v_packed, v_norm, v_codebook,
+                               block_table, context_lens, block_size, max_context_len):
+    """attn_paged_decode_k8v3 from the 16-bit query, as attn_paged_decode_q16."""
+    B, H, Hkv, D, nblk, bs, maxb = _k8v3_checks(q, k_cache, k_scale, v_packed, v_norm, v_codebook,
+                                                block_table, context_lens, block_size,
+                                                max_context_len)
+    with torch.cuda.device(q.device):
+        ws_bytes = _lib.load().sl8_attn_paged_decode_q16_workspace(B, H, Hkv, D, nblk, bs,
+                                                                   max_context_len, 1)
+        if not ws_bytes:
+            return None
+        out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
+        ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
+        call("sl8_attn_paged_decode_k8v3_q16", q.data_ptr(), dtype_code(q.dtype), int(bool(rotate)),
+             float(q_mul), k_cache.data_ptr(), k_scale.data_ptr(), v_packed.data_ptr(),
+             v_norm.data_ptr(), v_codebook.data_ptr(), block_table.data_ptr(),
+             context_lens.data_ptr(), out.data_ptr(), B, H, Hkv, D, nblk, bs, maxb,
+             int(max_context_len), ws.data_ptr(), ws_bytes, stream_of(q))
     return out
 
 

@@ -59,6 +59,12 @@ SIGNATURES = {
                                    _I64, _I64, _I64, _I64, _I64, _P, _SZ, _P]),
     "sl8_attn_paged_decode_k8v3": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64,
                                         _I64, _I64, _I64, _I64, _I64, _I64, _P, _SZ, _P]),
+    "sl8_attn_paged_decode_q16_workspace": (_SZ, [_I64] * 7 + [_I]),
+    "sl8_attn_paged_decode_q16": (_I, [_P, _I, _I, _F] + [_P] * 7 + [_I64] * 8 + [_P, _SZ, _P]),
+    "sl8_attn_paged_decode_k8v3_q16": (_I, [_P, _I, _I, _F] + [_P] * 8 + [_I64] * 8
+                                       + [_P, _SZ, _P]),
+    "sl8_attn_int8_decode_kv8_q16_workspace": (_SZ, [_I64] * 4),
+    "sl8_attn_int8_decode_kv8_q16": (_I, [_P, _I, _I, _F] + [_P] * 5 + [_I64] * 6 + [_P, _SZ, _P]),
     "sl8_kv_write_paged": (_I, [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P]),
     "sl8_kv_write_paged_rotated": (_I, [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64,
                                         _P]),

@@ -21,6 +21,7 @@
 //     are deterministic).
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <type_traits>
 
@@ -69,7 +70,39 @@ struct PagedArgs {
   int maxb, bs;
   int bs_sh;           // log2(bs) (streaming kernels: bs a power of two; K8V3: -1 if not)
   int cache_rows;      // num_blocks * Hkv * bs (streaming kernel, block-aligned tiles)
+  // splits planned on the device (see decode_prep_kernel): workgroup x serves keys [y, z) of
+  // (batch, KV head) x of items[x] and writes partial rows x * gsz ..; null = the grid's
+  // (split, batch * KV head) with equal splits of the launch's maximum
+  const int4* items;
 };
+
+// The keys and partial rows of one workgroup.
+struct SplitWork {
+  int bkv, n0, n1;
+  int64_t row;  // partial row of the group's first query head
+};
+__device__ __forceinline__ SplitWork split_work(int n_len, int n_splits, int h_q, int h_kv, int gsz,
+                                                int bhq, bool paged, const PagedArgs& pg) {
+  SplitWork w;
+  if (paged && pg.items) {
+    const int4 it = pg.items[blockIdx.x];
+    w.bkv = __builtin_amdgcn_readfirstlane(it.x);
+    w.n0 = __builtin_amdgcn_readfirstlane(it.y);
+    w.n1 = __builtin_amdgcn_readfirstlane(it.z);
+    w.row = (int64_t)blockIdx.x * gsz;
+    return w;
+  }
+  const int split = blockIdx.x;
+  w.bkv = blockIdx.y;  // b * h_kv + kvh
+  const int b = w.bkv / h_kv, kvh = w.bkv % h_kv;
+  const int per = (n_len + n_splits - 1) / n_splits;
+  w.n0 = split * per;
+  // paged: a context length above max_context_len (n_len) is read as
+  // max_context_len, so no block-table entry past the table's capacity is used
+  w.n1 = min(paged ? min(pg.ctx[b], n_len) : n_len, w.n0 + per);
+  w.row = (int64_t)split * bhq + (int64_t)b * h_q + (int64_t)kvh * gsz;
+  return w;
+}
 // block-table entries of one split staged in LDS by the streaming paged kernel
 constexpr int DEC_BT_MAX = 1024;
 
@@ -97,8 +130,9 @@ decode_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sc
   __shared__ DecSmem<D, G> sm;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int split = blockIdx.x;
-  const int bkv = blockIdx.y;  // b * h_kv + kvh
+  const SplitWork sw = split_work(n_len, n_splits, h_q, h_kv, gsz, bhq, PG, pg);
+  const int bkv = sw.bkv, n0 = sw.n0, n1 = sw.n1;
+  if (PG && pg.items && n1 <= n0) return;  // an unused item
   const int b = bkv / h_kv, kvh = bkv % h_kv;
   const int j0 = blockIdx.z * G;  // first head of this chunk within the group
   const int ng = min(G, gsz - j0);
@@ -119,11 +153,6 @@ decode_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sc
   }
   __syncthreads();
 
-  const int per = (n_len + n_splits - 1) / n_splits;
-  const int n0 = split * per;
-  // paged: a context length above max_context_len (n_len) is read as
-  // max_context_len, so no block-table entry past the table's capacity is used
-  const int n1 = min(PG ? min(pg.ctx[b], n_len) : n_len, n0 + per);
   // cache row of key n (contiguous: relative to this (batch, KV head))
   const int32_t* btb = PG ? pg.bt + (int64_t)b * pg.maxb : nullptr;
   auto krow = [&](int n) -> int64_t {
@@ -265,8 +294,7 @@ decode_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sc
         den += sm.l[w][g] * wt;
       }
     }
-    const int64_t hq = (int64_t)b * h_q + kvh * gsz + j0 + g;
-    const int64_t row = (int64_t)split * bhq + hq;
+    const int64_t row = sw.row + j0 + g;
     o_part[row * D + d] = (VI8 && !PG) ? acc * vsc[(int64_t)bkv * D + d] : acc;
     if (d == 0) {
       m_part[row] = (mm == -INFINITY) ? DEC_NEG_INF : mm;
@@ -282,11 +310,15 @@ decode_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sc
 // before any is used; the split weights 2^(m_s - gm) are formed once per
 // split by the lane that loaded m_s and broadcast, and the sums run over the
 // splits in index order (deterministic).
+//
+// With planned splits (seq: first item and splits per KV head of each sequence) the partial rows
+// of a head are gsz apart and a sequence has as many as it needs, none if it is empty.
 template <int D>
 __global__ void __launch_bounds__(CMB_WAVES * 64)
 decode_combine_wave_kernel(const float* __restrict__ o_part, const float* __restrict__ m_part,
                            const float* __restrict__ l_part, uint16_t* __restrict__ out,
-                           int n_splits, int bhq) {
+                           int n_splits, int bhq, const int2* __restrict__ seq = nullptr,
+                           int h_q = 1, int gsz = 1) {
   // D = 32: one channel per lane, lanes 32..63 idle
   constexpr int CPL = D >= 64 ? D / 64 : 1;
   const int lane = threadIdx.x & 63;
@@ -294,13 +326,27 @@ decode_combine_wave_kernel(const float* __restrict__ o_part, const float* __rest
   if (hq >= bhq) return;  // wave-uniform
   constexpr int SCH = 16;  // splits whose partials are in flight together
   const bool act = CPL * lane < D;
-  const float* ob = o_part + hq * D + (act ? CPL * lane : 0);
+  int64_t row0 = hq, rstride = bhq;  // partial row of split s: row0 + s * rstride
+  if (seq) {
+    const int b = (int)(hq / h_q), h = (int)(hq % h_q);
+    const int2 s2 = seq[b];
+    n_splits = __builtin_amdgcn_readfirstlane(s2.y);
+    row0 = ((int64_t)__builtin_amdgcn_readfirstlane(s2.x) + (int64_t)(h / gsz) * n_splits) * gsz + h % gsz;
+    rstride = gsz;
+    if (n_splits == 0) {
+#pragma unroll
+      for (int e = 0; e < CPL; ++e)
+        if (act) out[hq * D + CPL * lane + e] = 0;
+      return;
+    }
+  }
+  const float* ob = o_part + row0 * D + (act ? CPL * lane : 0);
   // partial O of splits s0 .. s0 + SCH - 1 (clamped to the last split)
   auto load_o = [&](int s0, float (&ov)[SCH][CPL]) {
 #pragma unroll
     for (int i = 0; i < SCH; ++i) {
       const int sp = min(s0 + i, n_splits - 1);
-      const float* src = ob + (int64_t)sp * bhq * D;
+      const float* src = ob + (int64_t)sp * rstride * D;
       if constexpr (CPL == 4) {
         const float4 v4 = *reinterpret_cast<const float4*>(src);
         ov[i][0] = v4.x; ov[i][1] = v4.y; ov[i][2] = v4.z; ov[i][3] = v4.w;
@@ -322,8 +368,8 @@ decode_combine_wave_kernel(const float* __restrict__ o_part, const float* __rest
 #pragma unroll
   for (int c = 0; c < DEC_MAX_SPLITS / 64; ++c) {
     const int sp = c * 64 + lane;
-    ms[c] = sp < n_splits ? m_part[(int64_t)sp * bhq + hq] : DEC_NEG_INF;
-    ls[c] = sp < n_splits ? l_part[(int64_t)sp * bhq + hq] : 0.f;
+    ms[c] = sp < n_splits ? m_part[row0 + sp * rstride] : DEC_NEG_INF;
+    ls[c] = sp < n_splits ? l_part[row0 + sp * rstride] : 0.f;
     gm = fmaxf(gm, ms[c]);
   }
 #pragma unroll
@@ -445,7 +491,7 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
                    const void* __restrict__ v, const float* __restrict__ vsc,
                    float* __restrict__ o_part,
                    float* __restrict__ m_part, float* __restrict__ l_part, int n_len,
-                   int n_splits, int h_q, int h_kv, int bhq, const PagedArgs pg) {
+                   int n_splits, int h_q, int h_kv, int gsz, int bhq, const PagedArgs pg) {
   static_assert(!PG || VI8, "the paged cache holds int8 V");
   using C = WaveCfg<D, GS, VI8, PG>;
   constexpr int KL = C::KL, SUB = C::SUB, T = C::T, CPL = C::CPL, KC = C::KC, KSW = C::KSW;
@@ -467,14 +513,10 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
     return s + wave * STAGE;
   };
 
-  const int split = blockIdx.x;
-  const int bkv = blockIdx.y;
+  const SplitWork sw = split_work(n_len, n_splits, h_q, h_kv, GS, bhq, PG, pg);
+  const int bkv = sw.bkv, n0 = sw.n0, n1 = sw.n1;
+  if (PG && pg.items && n1 <= n0) return;  // an unused item
   const int b = bkv / h_kv, kvh = bkv % h_kv;
-  const int per = (n_len + n_splits - 1) / n_splits;
-  const int n0 = split * per;
-  // paged: a context length above max_context_len (n_len) is read as
-  // max_context_len, so no block-table entry past the table's capacity is used
-  const int n1 = min(PG ? min(pg.ctx[b], n_len) : n_len, n0 + per);
   const int ntiles = n1 > n0 ? (n1 - n0 + T - 1) / T : 0;
   const int nt = ntiles > wave ? (ntiles - wave + DEC_WAVES - 1) / DEC_WAVES : 0;  // this wave's
   const int8_t* kb = k + (PG ? 0 : (int64_t)bkv * n_len * D);
@@ -908,13 +950,145 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
         den += red[DEC_WAVES * GS * D + DEC_WAVES * GS + w * GS + hh] * wt;
       }
     }
-    const int64_t row = (int64_t)split * bhq + (int64_t)b * h_q + (int64_t)kvh * GS + hh;
+    const int64_t row = sw.row + hh;
     o_part[row * D + d] = acc;
     if (d == 0) {
       m_part[row] = mm == -INFINITY ? DEC_NEG_INF : mm;
       l_part[row] = den;
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Preparation of a decode step that starts from the 16-bit query, one launch: the query rows
+// (optionally rotated, rounded to their type, quantised; the scale carries q_mul) and, for a
+// paged cache, the split plan, made by block 0.
+//
+// The plan: keys per split L is the smallest multiple of `unit` with no more than `target` splits
+// over all (sequence, KV head) pairs (target: the workgroups that are resident at once), within
+// [lmin, lcap]; each sequence of n keys then gets ceil(n / L) splits of equal length. Splits
+// sized on the longest sequence alone (256 keys and up to 256 splits of every sequence) left most
+// workgroups of a batch of mixed lengths empty and the rest too short to stream: 32 sequences of
+// 512..8192 keys, 8 KV heads, D = 128: 95 us for 191 MB.
+// ---------------------------------------------------------------------------
+constexpr int PLAN_MAX_B = 1024;  // sequences (LDS of the plan block); larger batches: no plan
+struct PlanArgs {
+  const int32_t* ctx;  // null: no plan
+  int B, h_kv, n_len;
+  int target, unit, lmin, lcap;
+  int max_items;
+  int4* items;  // [max_items]: (b * h_kv + kvh, first key, end, -), empty past the last
+  int2* seq;    // [B]: (first item, splits per KV head)
+};
+
+__device__ __forceinline__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+__device__ __forceinline__ void plan_block(const PlanArgs& p) {
+  __shared__ int n_s[PLAN_MAX_B], pre_s[PLAN_MAX_B + 1];
+  for (int b = threadIdx.x; b < p.B; b += 256) n_s[b] = max(0, min(p.ctx[b], p.n_len));
+  __syncthreads();
+  const int lane = threadIdx.x & 63;
+  // every wave searches for itself (no barriers): smallest L = unit * u in the bounds with
+  // splits(L) <= target
+  auto splits = [&](int L) {
+    int s = 0;
+    for (int b = lane; b < p.B; b += 64) s += ceil_div(n_s[b], L);
+    return __builtin_amdgcn_readfirstlane(lane_group_sum<64>(s)) * p.h_kv;
+  };
+  int lo = p.lmin / p.unit, hi = p.lcap / p.unit;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (splits(mid * p.unit) <= p.target) hi = mid;
+    else lo = mid + 1;
+  }
+  const int L = lo * p.unit;
+  if (threadIdx.x < 64) {
+    int base = 0;
+    for (int b0 = 0; b0 < p.B; b0 += 64) {
+      const int b = b0 + lane;
+      const int c = b < p.B ? ceil_div(n_s[b], L) : 0;
+      int x = c;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+      }
+      if (b < p.B) {
+        pre_s[b] = base + x - c;
+        p.seq[b] = make_int2((base + x - c) * p.h_kv, c);
+      }
+      base += __shfl(x, 63, 64);
+    }
+    if (lane == 0) pre_s[p.B] = base;
+  }
+  __syncthreads();
+  const int total = pre_s[p.B] * p.h_kv;
+  for (int i = threadIdx.x; i < p.max_items; i += 256) {
+    int4 it = make_int4(0, 0, 0, 0);
+    if (i < total) {
+      int a = 0, z = p.B;  // the sequence with pre[b] * h_kv <= i < pre[b + 1] * h_kv
+      while (z - a > 1) {
+        const int m = (a + z) >> 1;
+        if (pre_s[m] * p.h_kv <= i) a = m;
+        else z = m;
+      }
+      const int n = n_s[a], cnt = pre_s[a + 1] - pre_s[a];
+      const int r = i - pre_s[a] * p.h_kv;
+      const int len = ceil_div(ceil_div(n, cnt), p.unit) * p.unit;
+      const int n0 = (r % cnt) * len;
+      it = make_int4(a * p.h_kv + r / cnt, n0, min(n, n0 + len), 0);
+    }
+    p.items[i] = it;
+  }
+}
+
+template <int DT, int D, bool ROT>
+__global__ void __launch_bounds__(256)
+decode_prep_kernel(const uint16_t* __restrict__ q, int64_t rows, float q_mul,
+                   int8_t* __restrict__ q_i8, float* __restrict__ q_scale, const PlanArgs plan) {
+  if (plan.ctx && blockIdx.x == 0) return plan_block(plan);
+  constexpr int LPR = row_lanes(D), RPB = 256 / LPR;
+  const int lane = threadIdx.x % LPR;
+  const int64_t r = (int64_t)(blockIdx.x - (plan.ctx ? 1 : 0)) * RPB + threadIdx.x / LPR;
+  const bool live = r < rows;
+  float f[8];
+  VecIO<DT>::unpack(reinterpret_cast<const uint4*>(q + (live ? r : 0) * D)[lane], f);
+  if constexpr (ROT) {
+    hadamard_row<D>(f, lane);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] = Elem<DT>::round(f[e]);
+  }
+  float amax = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(f[e]));
+  amax = lane_group_max<LPR>(amax);
+  if (!live) return;
+  const float s = amax * (1.0f / 127.0f);
+  const float safe = (s == 0.f) ? 1.f : s;
+  if (lane == 0) q_scale[r] = safe * q_mul;
+  reinterpret_cast<uint2*>(q_i8 + r * D)[lane] = row_codes8<DT>(f, safe);
+}
+
+int launch_prep(const void* q, int dtype, int64_t rows, int64_t D, bool rotate, float q_mul,
+                int8_t* q_i8, float* q_scale, const PlanArgs& plan, hipStream_t st) {
+  auto go = [&](auto dt, auto d) {
+    constexpr int DT = decltype(dt)::value, DD = decltype(d)::value;
+    constexpr int RPB = 256 / row_lanes(DD);
+    const unsigned grid = (unsigned)((rows + RPB - 1) / RPB) + (plan.ctx ? 1 : 0);
+    const uint16_t* qh = static_cast<const uint16_t*>(q);
+    if (rotate) decode_prep_kernel<DT, DD, true><<<grid, 256, 0, st>>>(qh, rows, q_mul, q_i8, q_scale, plan);
+    else decode_prep_kernel<DT, DD, false><<<grid, 256, 0, st>>>(qh, rows, q_mul, q_i8, q_scale, plan);
+  };
+  auto by_d = [&](auto dt) {
+    if (D == 32) go(dt, std::integral_constant<int, 32>{});
+    else if (D == 64) go(dt, std::integral_constant<int, 64>{});
+    else if (D == 128) go(dt, std::integral_constant<int, 128>{});
+    else go(dt, std::integral_constant<int, 256>{});
+  };
+  if (dtype == SL8_DTYPE_F16) by_d(std::integral_constant<int, SL8_DTYPE_F16>{});
+  else by_d(std::integral_constant<int, SL8_DTYPE_BF16>{});
+  SL8_CHECK_LAUNCH("decode prep");
+  return SL8_OK;
 }
 
 template <int D, int G, bool VI8, bool PG, bool KS16>
@@ -929,7 +1103,7 @@ template <int D, bool VI8, bool PG = false, bool KS16 = false>
 void launch_d(int G, dim3 grid, const int8_t* q, const float* qs, const int8_t* k,
               const void* ks, const void* v, const float* vsc, float* op, float* mp, float* lp,
               int N, int ns, int hq, int hkv, int gsz, int bhq, hipStream_t st,
-              const PagedArgs& pg = PagedArgs{nullptr, nullptr, 0, 1, 0, 0}) {
+              const PagedArgs& pg = PagedArgs{nullptr, nullptr, 0, 1, 0, 0, nullptr}) {
 #define SL8_SPLIT(GG) \
   launch_split<D, GG, VI8, PG, KS16>(grid, q, qs, k, ks, v, vsc, op, mp, lp, N, ns, hq, hkv, gsz, bhq, pg, st)
   switch (G) {
@@ -991,8 +1165,8 @@ int decode_launch(const int8_t* q, const float* q_scale, const int8_t* k, const 
     const dim3 g2((unsigned)ns, (unsigned)(B * Hkv));
 #define SL8_WAVE(DD, GS, NB)                                                                     \
     decode_wave_kernel<DD, GS, NB, VI8, false, KS16><<<g2, DEC_THREADS, 0, st>>>(                    \
-        q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, bhq,       \
-        PagedArgs{nullptr, nullptr, 0, 1, 0, 0})
+        q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, GS, bhq,   \
+        PagedArgs{nullptr, nullptr, 0, 1, 0, 0, nullptr})
 #define SL8_WAVE_D(GS)                         \
     if (D == 64) SL8_WAVE(64, GS, 4);          \
     else if (D == 128) SL8_WAVE(128, GS, 3);   \
@@ -1373,8 +1547,9 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
   __shared__ SM sm;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int split = blockIdx.x;
-  const int bkv = blockIdx.y;
+  const SplitWork sw = split_work(n_len, n_splits, h_q, h_kv, gsz, bhq, true, pg);
+  const int bkv = sw.bkv, n0 = sw.n0, n1 = sw.n1;
+  if (pg.items && n1 <= n0) return;  // an unused item
   const int b = bkv / h_kv, kvh = bkv % h_kv;
   const int j0 = blockIdx.z * G;
   const int ng = min(G, gsz - j0);
@@ -1409,10 +1584,6 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
   // (at least FLT_MIN: a masked key's -inf logit must stay -inf, never 0 * -inf)
   const float qsl = col < G ? fmaxf(sm.qs[col], 1.17549435e-38f) : 0.f;
 
-  const int per = (n_len + n_splits - 1) / n_splits;
-  const int n0 = split * per;
-  // a context length above max_context_len (n_len) is read as max_context_len
-  const int n1 = min(min(pg.ctx[b], n_len), n0 + per);
   const int32_t* btb = pg.bt + (int64_t)b * pg.maxb;
 
   // 32-byte chunk swizzle of V row r: 8 distinct values over the 16 rows one
@@ -1662,8 +1833,7 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
         den += sm.r.l[w][g] * wt;
       }
     }
-    const int64_t hq = (int64_t)b * h_q + kvh * gsz + j0 + g;
-    const int64_t orow = (int64_t)split * bhq + hq;
+    const int64_t orow = sw.row + j0 + g;
     o_part[orow * D + d] = acc;
     if (d == 0) {
       m_part[orow] = (mm == -INFINITY) ? DEC_NEG_INF : mm;
@@ -1690,6 +1860,275 @@ extern "C" int sl8_paged_choose_num_splits(int64_t n_len_max, int64_t bhq) {
   return (int)s;
 }
 
+namespace sl8 {
+namespace {
+
+// A paged decode call: the cache and the sequences (everything but the query).
+struct Paged {
+  const char* tag;
+  const int8_t* k;
+  const float* ks;
+  const void* v;         // int8 cache, or the packed codes (k8v3)
+  const float* vs;       // per-token V scale, or the norms (k8v3)
+  const float* codebook; // k8v3 only
+  const int32_t *bt, *ctx;
+  int64_t B, Hq, Hkv, D, num_blocks, bs, maxb, nmax;
+  bool k8v3;
+
+  int check() const {
+    SL8_CHECK_ARG(B >= 0 && Hq >= 0 && Hkv > 0 && num_blocks >= 0 && bs > 0 && maxb >= 0,
+                  "fni8 %s: bad shape", tag);
+    SL8_CHECK_ARG(Hq % Hkv == 0, "fni8 %s: H_q must be divisible by H_kv (GQA)", tag);
+    if (k8v3)
+      SL8_CHECK_ARG(D == 128 || D == 256, "fni8 %s: lloydmax3 requires head dim 128 or 256, got %lld",
+                    tag, (long long)D);
+    else
+      SL8_CHECK_ARG(D == 32 || D == 64 || D == 128 || D == 256,
+                    "fni8 %s: head dim must be 32/64/128/256, got %lld", tag, (long long)D);
+    SL8_CHECK_ARG(nmax >= 0 && nmax <= maxb * bs,
+                  "fni8 %s: max_context_len exceeds block_table capacity", tag);
+    SL8_CHECK_ARG(B * Hq < (1LL << 31) && num_blocks * Hkv * bs < (1LL << 40) && nmax < (1LL << 31),
+                  "fni8 %s: shape too large", tag);
+    return SL8_OK;
+  }
+  int check_pointers(const void* q, const void* out) const {
+    SL8_CHECK_ARG(q && bt && ctx && out && (!k8v3 || codebook) &&
+                      (num_blocks == 0 || (k && ks && v && vs)),
+                  "fni8 %s: null pointer", tag);
+    if (k8v3) {
+      SL8_CHECK_ARG(num_blocks * Hkv * bs < (1LL << 31),
+                    "fni8 %s: cache too large (rows must fit in 31 bits)", tag);
+      SL8_CHECK_ARG(aligned(q, 4) && aligned(k, 16) && aligned(v, 16),
+                    "fni8 %s: q must be 4-byte aligned, k_cache/v_packed 16-byte aligned", tag);
+    } else {
+      SL8_CHECK_ARG(aligned(q, 16) && aligned(k, 16) && aligned(v, 16),
+                    "fni8 %s: q/k_cache/v_cache must be 16-byte aligned", tag);
+    }
+    return SL8_OK;
+  }
+  int gsz() const { return (int)(Hq / Hkv); }
+  // log2 of the block size, -1 if not a power of two
+  int bs_shift() const {
+    int s = 0;
+    while ((1LL << s) < bs) ++s;
+    return (1LL << s) == bs ? s : -1;
+  }
+  int64_t cache_rows() const { return num_blocks * Hkv * bs; }
+  // streaming kernel (keys per split: per)
+  bool streams(int64_t per) const {
+    return D != 32 && bs_shift() >= 0 && per / bs + 2 <= DEC_BT_MAX &&
+           ((gsz() == 2 && D == 128) || gsz() == 4 || gsz() == 8);
+  }
+  // streaming tiles hold T = 32 (2 heads per KV head) or 16 keys; when blocks
+  // and split boundaries are multiples of T, each tile sits in one block
+  int64_t tile_keys() const { return gsz() == 2 ? 32 : 16; }
+  bool aligned_tiles(int64_t per) const {
+    return bs % tile_keys() == 0 && per % tile_keys() == 0 && cache_rows() * D < (1LL << 31);
+  }
+};
+
+// A kernel as a type, so that a visitor can launch it or ask for its occupancy.
+template <auto K> struct KernelTag {
+  static constexpr auto kernel = K;
+  // workgroups resident on one CU (queried once)
+  static int wgs_per_cu() {
+    static std::atomic<int> n{0};
+    int v = n.load(std::memory_order_relaxed);
+    if (v == 0) {
+      if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, reinterpret_cast<const void*>(K),
+                                                       DEC_THREADS, 0) != hipSuccess || v < 1) {
+        (void)hipGetLastError();
+        return 2;  // no device: any figure (nothing is launched)
+      }
+      n.store(v, std::memory_order_relaxed);
+    }
+    return v;
+  }
+};
+
+// f(KernelTag) of the int8-V paged kernel that serves p with splits of `per` keys.
+template <typename F>
+auto with_paged_kernel(const Paged& p, int64_t per, F&& f) {
+  const int gsz = p.gsz();
+  if (p.streams(per)) {
+    const bool al = p.aligned_tiles(per);
+#define SL8_PWAVE(DD, GS, NB)                                                                 \
+    return al ? f(KernelTag<decode_wave_kernel<DD, GS, NB, true, true, false, true>>{})       \
+              : f(KernelTag<decode_wave_kernel<DD, GS, NB, true, true>>{})
+// D = 128: a two-stage ring (37 KB of LDS per workgroup, so 4 workgroups
+// per CU instead of 2) measured 210 us against 227 us with three stages at
+// config 3's shape with 16-key blocks scattered over the pool: more
+// independent block streams in flight beat a deeper ring per wave.
+#define SL8_PWAVE_D(GS)                        \
+    if (p.D == 64) SL8_PWAVE(64, GS, 4);       \
+    if (p.D == 128) SL8_PWAVE(128, GS, 2);     \
+    SL8_PWAVE(256, GS, 3)
+    if (gsz == 2) SL8_PWAVE(128, 2, 3);
+    if (gsz == 4) { SL8_PWAVE_D(4); }
+    SL8_PWAVE_D(8);
+#undef SL8_PWAVE_D
+#undef SL8_PWAVE
+  }
+  const int G = group_width(gsz);
+#define SL8_PSPLIT(DD)                                                                   \
+  switch (G) {                                                                           \
+    case 1: return f(KernelTag<decode_split_kernel<DD, 1, true, true>>{});               \
+    case 2: return f(KernelTag<decode_split_kernel<DD, 2, true, true>>{});               \
+    case 4: return f(KernelTag<decode_split_kernel<DD, 4, true, true>>{});               \
+    default: return f(KernelTag<decode_split_kernel<DD, 8, true, true>>{});              \
+  }
+  switch (p.D) {
+    case 32: SL8_PSPLIT(32)
+    case 64: SL8_PSPLIT(64)
+    case 128: SL8_PSPLIT(128)
+    default: SL8_PSPLIT(256)
+  }
+#undef SL8_PSPLIT
+}
+
+template <typename F>
+auto with_k8v3_kernel(const Paged& p, F&& f) {
+  const int G = group_width(p.gsz());
+#define SL8_K3D(DD)                                                  \
+  switch (G) {                                                       \
+    case 1: return f(KernelTag<k8v3_split_kernel<DD, 1>>{});         \
+    case 2: return f(KernelTag<k8v3_split_kernel<DD, 2>>{});         \
+    case 4: return f(KernelTag<k8v3_split_kernel<DD, 4>>{});         \
+    default: return f(KernelTag<k8v3_split_kernel<DD, 8>>{});        \
+  }
+  if (p.D == 128) { SL8_K3D(128) }
+  SL8_K3D(256)
+#undef SL8_K3D
+}
+
+// Split kernels + merge. Equal splits of nmax (ns of them) with partials for every (split, head),
+// or, with items, the planned ones (grid: max_items).
+int paged_launch(const Paged& p, const int8_t* q, const float* q_scale, void* out, int ns,
+                 const int4* items, const int2* seq, int max_items, float* op, hipStream_t st) {
+  const int bhq = (int)(p.B * p.Hq), gsz = p.gsz(), G = group_width(gsz);
+  const int64_t rows = items ? (int64_t)max_items * gsz : (int64_t)ns * bhq;
+  float* mp = op + rows * p.D;
+  float* lp = mp + rows;
+  const int sh = p.bs_shift();
+  PagedArgs pg{p.bt, p.ctx, (int)p.maxb, (int)p.bs, sh,
+               (int)std::min<int64_t>(p.cache_rows(), (int64_t)0x7fffffff), items};
+  const int nmax = (int)p.nmax;
+  dim3 grid = items ? dim3((unsigned)max_items) : dim3((unsigned)ns, (unsigned)(p.B * p.Hkv));
+  if (p.k8v3) {
+    grid.z = (unsigned)((gsz + G - 1) / G);
+    with_k8v3_kernel(p, [&](auto kt) {
+      decltype(kt)::kernel<<<grid, DEC_THREADS, 0, st>>>(
+          q, q_scale, p.k, p.ks, static_cast<const uint32_t*>(p.v), p.vs, p.codebook, op, mp, lp,
+          nmax, ns, (int)p.Hq, (int)p.Hkv, gsz, bhq, pg);
+    });
+  } else {
+    // planned splits are multiples of the streaming tiles and bounded by its block-table staging
+    const int64_t per = items ? 256 : (p.nmax + ns - 1) / ns;
+    if (!p.streams(per)) grid.z = (unsigned)((gsz + G - 1) / G);
+    with_paged_kernel(p, per, [&](auto kt) {
+      decltype(kt)::kernel<<<grid, DEC_THREADS, 0, st>>>(q, q_scale, p.k, p.ks, p.v, p.vs, op, mp,
+                                                         lp, nmax, ns, (int)p.Hq, (int)p.Hkv, gsz,
+                                                         bhq, pg);
+    });
+  }
+  SL8_CHECK_LAUNCH(p.tag);
+  launch_combine((int)p.D, bhq, st, op, mp, lp, static_cast<uint16_t*>(out), ns, bhq, seq,
+                 (int)p.Hq, gsz);
+  SL8_CHECK_LAUNCH(p.tag);
+  return SL8_OK;
+}
+
+int paged_decode(const Paged& p, const int8_t* q, const float* q_scale, void* out,
+                 int64_t num_splits, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  if (const int rc = p.check()) return rc;
+  if (num_splits < 0) num_splits = sl8_paged_choose_num_splits(p.nmax, p.B * p.Hq);
+  SL8_CHECK_ARG(num_splits >= 1 && num_splits <= DEC_MAX_SPLITS,
+                "fni8 %s: num_splits must be 1..%d, got %lld", p.tag, DEC_MAX_SPLITS,
+                (long long)num_splits);
+  if (p.B == 0 || p.Hq == 0) return SL8_OK;
+  if (const int rc = p.check_pointers(q, out)) return rc;
+  SL8_CHECK_ARG(q_scale, "fni8 %s: null pointer", p.tag);
+  const size_t need = sl8_attn_int8_decode_workspace(p.B, p.Hq, p.D, num_splits);
+  SL8_CHECK_ARG(workspace && workspace_bytes >= need && aligned(workspace, 16),
+                "fni8 %s: workspace needs %zu bytes", p.tag, need);
+  return paged_launch(p, q, q_scale, out, (int)num_splits, nullptr, nullptr, 0,
+                      static_cast<float*>(workspace), static_cast<hipStream_t>(stream));
+}
+
+// The planned call's bounds and its workspace: partials, items, seq, query codes and scales.
+struct PagedPlan {
+  PlanArgs a;
+  size_t items_at, seq_at, q_at, qs_at, bytes;
+};
+PagedPlan paged_plan(const Paged& p) {
+  const int gsz = p.gsz(), G = group_width(gsz);
+  const int64_t groups = p.B * p.Hkv;
+  const bool streams = !p.k8v3 && p.streams(256);
+  // keys a workgroup's 4 waves take in one round of tiles
+  const int64_t unit = streams ? 4 * p.tile_keys() : 4 * DEC_TILE;
+  const int chunks = streams ? 1 : (gsz + G - 1) / G;
+  const int wgs = p.k8v3 ? with_k8v3_kernel(p, [](auto kt) { return decltype(kt)::wgs_per_cu(); })
+                         : with_paged_kernel(p, 256, [](auto kt) { return decltype(kt)::wgs_per_cu(); });
+  auto up = [&](int64_t n) { return (n + unit - 1) / unit * unit; };
+  const int64_t nmax = std::max<int64_t>(p.nmax, 1);
+  PagedPlan r{};
+  // one round of resident workgroups; a batch whose (sequence, KV head) pairs nearly fill that
+  // alone gets two splits per pair on average, so that its longest sequences are still cut
+  const int64_t target = std::max<int64_t>((int64_t)cu_count() * wgs / chunks, 2 * groups);
+  int64_t lmin = std::max<int64_t>(256, up((nmax + DEC_MAX_SPLITS - 1) / DEC_MAX_SPLITS));
+  int64_t lcap = up(nmax);
+  if (streams) lcap = std::min<int64_t>(lcap, (DEC_BT_MAX - 2) * p.bs / unit * unit);
+  lcap = std::max(lcap, lmin);
+  const int64_t items = std::min(groups * ((nmax + lmin - 1) / lmin),
+                                 std::max(target, groups * ((nmax + lcap - 1) / lcap)));
+  r.a = PlanArgs{p.ctx, (int)p.B, (int)p.Hkv, (int)p.nmax, (int)target, (int)unit, (int)lmin,
+                 (int)lcap, (int)items, nullptr, nullptr};
+  auto at = [&](size_t n) { const size_t o = r.bytes; r.bytes += (n + 15) / 16 * 16; return o; };
+  at((size_t)items * gsz * (p.D + 2) * sizeof(float));
+  r.items_at = at((size_t)items * sizeof(int4));
+  r.seq_at = at((size_t)p.B * sizeof(int2));
+  r.q_at = at((size_t)(p.B * p.Hq * p.D));
+  r.qs_at = at((size_t)(p.B * p.Hq) * sizeof(float));
+  return r;
+}
+
+bool plan_ok(const Paged& p) {
+  if (p.B > PLAN_MAX_B) return false;
+  // the streaming kernel's staging bound against the smallest split (tiny blocks, huge contexts)
+  if (p.k8v3 || !p.streams(256)) return true;
+  const int64_t lmin = std::max<int64_t>(256, (p.nmax + DEC_MAX_SPLITS - 1) / DEC_MAX_SPLITS + 128);
+  return lmin / p.bs + 2 <= DEC_BT_MAX;
+}
+
+int paged_decode_q16(const Paged& p, const void* q, int q_dtype, int rotate, float q_mul, void* out,
+                     void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  if (const int rc = p.check()) return rc;
+  SL8_CHECK_ARG(q_dtype == SL8_DTYPE_F16 || q_dtype == SL8_DTYPE_BF16,
+                "fni8 %s: q must be float16 or bfloat16", p.tag);
+  SL8_CHECK_ARG(plan_ok(p), "fni8 %s: batch or context too large for planned splits", p.tag);
+  if (p.B == 0 || p.Hq == 0) return SL8_OK;
+  if (const int rc = p.check_pointers(q, out)) return rc;
+  SL8_CHECK_ARG(aligned(q, 16), "fni8 %s: q must be 16-byte aligned", p.tag);
+  PagedPlan plan = paged_plan(p);
+  SL8_CHECK_ARG(workspace && workspace_bytes >= plan.bytes && aligned(workspace, 16),
+                "fni8 %s: workspace needs %zu bytes", p.tag, plan.bytes);
+  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  plan.a.items = reinterpret_cast<int4*>(ws + plan.items_at);
+  plan.a.seq = reinterpret_cast<int2*>(ws + plan.seq_at);
+  int8_t* qi = reinterpret_cast<int8_t*>(ws + plan.q_at);
+  float* qs = reinterpret_cast<float*>(ws + plan.qs_at);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (const int rc = launch_prep(q, q_dtype, p.B * p.Hq, p.D, rotate != 0, q_mul, qi, qs, plan.a, st))
+    return rc;
+  return paged_launch(p, qi, qs, out, 1, plan.a.items, plan.a.seq, plan.a.max_items,
+                      static_cast<float*>(workspace), st);
+}
+
+}  // namespace
+}  // namespace sl8
+
 extern "C" int sl8_attn_paged_decode(const int8_t* q, const float* q_scale, const int8_t* k_cache,
                                      const float* k_scale, const int8_t* v_cache,
                                      const float* v_scale, const int32_t* block_table,
@@ -1698,96 +2137,10 @@ extern "C" int sl8_attn_paged_decode(const int8_t* q, const float* q_scale, cons
                                      int64_t block_size, int64_t max_blocks_per_seq,
                                      int64_t max_context_len, int64_t num_splits,
                                      void* workspace, size_t workspace_bytes, void* stream) {
-  clear_error();
-  SL8_CHECK_ARG(B >= 0 && Hq >= 0 && Hkv > 0 && num_blocks >= 0 && block_size > 0 &&
-                    max_blocks_per_seq >= 0,
-                "fni8 paged_decode: bad shape");
-  SL8_CHECK_ARG(Hq % Hkv == 0, "fni8 paged_decode: H_q must be divisible by H_kv (GQA)");
-  SL8_CHECK_ARG(D == 32 || D == 64 || D == 128 || D == 256,
-                "fni8 paged_decode: head dim must be 32/64/128/256, got %lld", (long long)D);
-  SL8_CHECK_ARG(max_context_len >= 0 && max_context_len <= max_blocks_per_seq * block_size,
-                "fni8 paged_decode: max_context_len exceeds block_table capacity");
-  SL8_CHECK_ARG(B * Hq < (1LL << 31) && num_blocks * Hkv * block_size < (1LL << 40) &&
-                    max_context_len < (1LL << 31),
-                "fni8 paged_decode: shape too large");
-  const int64_t bhq = B * Hq;
-  if (num_splits < 0) num_splits = sl8_paged_choose_num_splits(max_context_len, bhq);
-  SL8_CHECK_ARG(num_splits >= 1 && num_splits <= DEC_MAX_SPLITS,
-                "fni8 paged_decode: num_splits must be 1..%d, got %lld", DEC_MAX_SPLITS,
-                (long long)num_splits);
-  if (B == 0 || Hq == 0) return SL8_OK;
-  SL8_CHECK_ARG(q && q_scale && block_table && context_lens && out &&
-                    (num_blocks == 0 || (k_cache && k_scale && v_cache && v_scale)),
-                "fni8 paged_decode: null pointer");
-  SL8_CHECK_ARG(aligned(q, 16) && aligned(k_cache, 16) && aligned(v_cache, 16),
-                "fni8 paged_decode: q/k_cache/v_cache must be 16-byte aligned");
-  const size_t need = sl8_attn_int8_decode_workspace(B, Hq, D, num_splits);
-  SL8_CHECK_ARG(workspace && workspace_bytes >= need && aligned(workspace, 16),
-                "fni8 paged_decode: workspace needs %zu bytes", need);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const int ns = (int)num_splits, ibhq = (int)bhq, gsz = (int)(Hq / Hkv);
-  const int G = group_width(gsz);
-  float* op = static_cast<float*>(workspace);
-  float* mp = op + (size_t)ns * ibhq * D;
-  float* lp = mp + (size_t)ns * ibhq;
-  const dim3 grid((unsigned)ns, (unsigned)(B * Hkv), (unsigned)((gsz + G - 1) / G));
-  int bs_sh = 0;
-  while ((1LL << bs_sh) < block_size) ++bs_sh;
-  const bool pow2 = (1LL << bs_sh) == block_size;
-  const int64_t cache_rows = num_blocks * Hkv * block_size;
-  const PagedArgs pg{block_table, context_lens, (int)max_blocks_per_seq, (int)block_size, bs_sh,
-                     (int)std::min<int64_t>(cache_rows, (int64_t)0x7fffffff)};
-  const int nmax = (int)max_context_len;
-  const int64_t per = (max_context_len + ns - 1) / ns;
-  const bool stream_ok = D != 32 && pow2 && per / block_size + 2 <= DEC_BT_MAX &&
-                         ((gsz == 2 && D == 128) || gsz == 4 || gsz == 8);
-  // streaming tiles hold T = 32 (2 heads per KV head) or 16 keys; when blocks
-  // and split boundaries are multiples of T, each tile sits in one block
-  const int64_t tkeys = gsz == 2 ? 32 : 16;
-  const bool aligned_tiles = block_size % tkeys == 0 && per % tkeys == 0 &&
-                             cache_rows * D < (1LL << 31);
-  if (stream_ok) {
-    const dim3 g2((unsigned)ns, (unsigned)(B * Hkv));
-#define SL8_PWAVE(DD, GS, NB)                                                                   \
-    do {                                                                                         \
-      if (aligned_tiles)                                                                         \
-        decode_wave_kernel<DD, GS, NB, true, true, false, true><<<g2, DEC_THREADS, 0, st>>>(     \
-            q, q_scale, k_cache, k_scale, v_cache, v_scale, op, mp, lp, nmax, ns, (int)Hq,       \
-            (int)Hkv, ibhq, pg);                                                                 \
-      else                                                                                       \
-        decode_wave_kernel<DD, GS, NB, true, true><<<g2, DEC_THREADS, 0, st>>>(                  \
-            q, q_scale, k_cache, k_scale, v_cache, v_scale, op, mp, lp, nmax, ns, (int)Hq,       \
-            (int)Hkv, ibhq, pg);                                                                 \
-    } while (0)
-// D = 128: a two-stage ring (37 KB of LDS per workgroup, so 4 workgroups
-// per CU instead of 2) measured 210 us against 227 us with three stages at
-// config 3's shape with 16-key blocks scattered over the pool: more
-// independent block streams in flight beat a deeper ring per wave.
-#define SL8_PWAVE_D(GS)                        \
-    if (D == 64) SL8_PWAVE(64, GS, 4);         \
-    else if (D == 128) SL8_PWAVE(128, GS, 2);  \
-    else SL8_PWAVE(256, GS, 3);
-    switch (gsz) {
-      case 2: SL8_PWAVE(128, 2, 3); break;
-      case 4: SL8_PWAVE_D(4); break;
-      default: SL8_PWAVE_D(8); break;
-    }
-#undef SL8_PWAVE_D
-#undef SL8_PWAVE
-  } else {
-#define SL8_PAGED(DD)                                                                          \
-    launch_d<DD, true, true>(G, grid, q, q_scale, k_cache, k_scale, v_cache, v_scale, op, mp, lp, \
-                             nmax, ns, (int)Hq, (int)Hkv, gsz, ibhq, st, pg)
-    if (D == 32) SL8_PAGED(32);
-    else if (D == 64) SL8_PAGED(64);
-    else if (D == 128) SL8_PAGED(128);
-    else SL8_PAGED(256);
-#undef SL8_PAGED
-  }
-  SL8_CHECK_LAUNCH("attn_paged_decode split");
-  launch_combine((int)D, ibhq, st, op, mp, lp, static_cast<uint16_t*>(out), ns, ibhq);
-  SL8_CHECK_LAUNCH("attn_paged_decode combine");
-  return SL8_OK;
+  const Paged p{"paged_decode", k_cache, k_scale, v_cache, v_scale, nullptr, block_table,
+                context_lens, B, Hq, Hkv, D, num_blocks, block_size, max_blocks_per_seq,
+                max_context_len, false};
+  return paged_decode(p, q, q_scale, out, num_splits, workspace, workspace_bytes, stream);
 }
 
 extern "C" int sl8_attn_paged_decode_k8v3(const int8_t* q, const float* q_scale,
@@ -1799,66 +2152,81 @@ extern "C" int sl8_attn_paged_decode_k8v3(const int8_t* q, const float* q_scale,
                                           int64_t block_size, int64_t max_blocks_per_seq,
                                           int64_t max_context_len, int64_t num_splits,
                                           void* workspace, size_t workspace_bytes, void* stream) {
+  const Paged p{"paged_decode_k8v3", k_cache, k_scale, v_packed, v_norm, v_codebook, block_table,
+                context_lens, B, Hq, Hkv, D, num_blocks, block_size, max_blocks_per_seq,
+                max_context_len, true};
+  return paged_decode(p, q, q_scale, out, num_splits, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t sl8_attn_paged_decode_q16_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t D,
+                                                      int64_t num_blocks, int64_t block_size,
+                                                      int64_t max_context_len, int k8v3) {
+  const Paged p{"paged_decode", nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, Hq,
+                Hkv, D, num_blocks, block_size, 0, max_context_len, k8v3 != 0};
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || D <= 0 || block_size <= 0 || !plan_ok(p)) return 0;
+  return paged_plan(p).bytes;
+}
+
+extern "C" int sl8_attn_paged_decode_q16(const void* q, int q_dtype, int rotate, float q_scale_mul,
+                                         const int8_t* k_cache, const float* k_scale,
+                                         const int8_t* v_cache, const float* v_scale,
+                                         const int32_t* block_table, const int32_t* context_lens,
+                                         void* out, int64_t B, int64_t Hq, int64_t Hkv, int64_t D,
+                                         int64_t num_blocks, int64_t block_size,
+                                         int64_t max_blocks_per_seq, int64_t max_context_len,
+                                         void* workspace, size_t workspace_bytes, void* stream) {
+  const Paged p{"paged_decode", k_cache, k_scale, v_cache, v_scale, nullptr, block_table,
+                context_lens, B, Hq, Hkv, D, num_blocks, block_size, max_blocks_per_seq,
+                max_context_len, false};
+  return paged_decode_q16(p, q, q_dtype, rotate, q_scale_mul, out, workspace, workspace_bytes, stream);
+}
+
+extern "C" int sl8_attn_paged_decode_k8v3_q16(
+    const void* q, int q_dtype, int rotate, float q_scale_mul, const int8_t* k_cache,
+    const float* k_scale, const int32_t* v_packed, const float* v_norm, const float* v_codebook,
+    const int32_t* block_table, const int32_t* context_lens, void* out, int64_t B, int64_t Hq,
+    int64_t Hkv, int64_t D, int64_t num_blocks, int64_t block_size, int64_t max_blocks_per_seq,
+    int64_t max_context_len, void* workspace, size_t workspace_bytes, void* stream) {
+  const Paged p{"paged_decode_k8v3", k_cache, k_scale, v_packed, v_norm, v_codebook, block_table,
+                context_lens, B, Hq, Hkv, D, num_blocks, block_size, max_blocks_per_seq,
+                max_context_len, true};
+  return paged_decode_q16(p, q, q_dtype, rotate, q_scale_mul, out, workspace, workspace_bytes, stream);
+}
+
+extern "C" size_t sl8_attn_int8_decode_kv8_q16_workspace(int64_t B, int64_t Hq, int64_t D,
+                                                         int64_t num_splits) {
+  if (B <= 0 || Hq <= 0 || D <= 0 || num_splits <= 0) return 0;
+  const size_t part = (sl8_attn_int8_decode_workspace(B, Hq, D, num_splits) + 15) / 16 * 16;
+  return part + (size_t)(B * Hq) * (D + sizeof(float));
+}
+
+extern "C" int sl8_attn_int8_decode_kv8_q16(const void* q, int q_dtype, int rotate,
+                                            float q_scale_mul, const int8_t* k,
+                                            const float* k_scale, const int8_t* v,
+                                            const float* v_scale, void* out, int64_t B, int64_t Hq,
+                                            int64_t Hkv, int64_t N, int64_t D, int64_t num_splits,
+                                            void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
-  SL8_CHECK_ARG(B >= 0 && Hq >= 0 && Hkv > 0 && num_blocks >= 0 && block_size > 0 &&
-                    max_blocks_per_seq >= 0,
-                "fni8 paged_decode_k8v3: bad shape");
-  SL8_CHECK_ARG(Hq % Hkv == 0, "fni8 paged_decode_k8v3: H_q must be divisible by H_kv (GQA)");
-  SL8_CHECK_ARG(D == 128 || D == 256,
-                "fni8 paged_decode_k8v3: lloydmax3 requires head dim 128 or 256, got %lld",
-                (long long)D);
-  SL8_CHECK_ARG(max_context_len >= 0 && max_context_len <= max_blocks_per_seq * block_size,
-                "fni8 paged_decode_k8v3: max_context_len exceeds block_table capacity");
-  SL8_CHECK_ARG(B * Hq < (1LL << 31) && num_blocks * Hkv * block_size < (1LL << 40) &&
-                    max_context_len < (1LL << 31),
-                "fni8 paged_decode_k8v3: shape too large");
-  const int64_t bhq = B * Hq;
-  if (num_splits < 0) num_splits = sl8_paged_choose_num_splits(max_context_len, bhq);
-  SL8_CHECK_ARG(num_splits >= 1 && num_splits <= DEC_MAX_SPLITS,
-                "fni8 paged_decode_k8v3: num_splits must be 1..%d, got %lld", DEC_MAX_SPLITS,
-                (long long)num_splits);
+  SL8_CHECK_ARG(q_dtype == SL8_DTYPE_F16 || q_dtype == SL8_DTYPE_BF16,
+                "fni8 decode_kv8: q must be float16 or bfloat16");
+  SL8_CHECK_ARG(B >= 0 && Hq >= 0 && Hkv > 0 && N >= 0 && B * Hq < (1LL << 31),
+                "fni8 decode_kv8: bad shape");
+  SL8_CHECK_ARG(D == 32 || D == 64 || D == 128 || D == 256,
+                "fni8 decode_kv8: head dim must be 32/64/128/256, got %lld", (long long)D);
+  if (num_splits < 0) num_splits = sl8_choose_num_splits(N, B, Hkv);
   if (B == 0 || Hq == 0) return SL8_OK;
-  SL8_CHECK_ARG(q && q_scale && block_table && context_lens && out && v_codebook &&
-                    (num_blocks == 0 || (k_cache && k_scale && v_packed && v_norm)),
-                "fni8 paged_decode_k8v3: null pointer");
-  SL8_CHECK_ARG(num_blocks * Hkv * block_size < (1LL << 31),
-                "fni8 paged_decode_k8v3: cache too large (rows must fit in 31 bits)");
-  SL8_CHECK_ARG(aligned(q, 4) && aligned(k_cache, 16) && aligned(v_packed, 16),
-                "fni8 paged_decode_k8v3: q must be 4-byte aligned, k_cache/v_packed 16-byte aligned");
-  const size_t need = sl8_attn_int8_decode_workspace(B, Hq, D, num_splits);
-  SL8_CHECK_ARG(workspace && workspace_bytes >= need && aligned(workspace, 16),
-                "fni8 paged_decode_k8v3: workspace needs %zu bytes", need);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const int ns = (int)num_splits, ibhq = (int)bhq, gsz = (int)(Hq / Hkv);
-  const int G = group_width(gsz);
-  float* op = static_cast<float*>(workspace);
-  float* mp = op + (size_t)ns * ibhq * D;
-  float* lp = mp + (size_t)ns * ibhq;
-  const dim3 grid((unsigned)ns, (unsigned)(B * Hkv), (unsigned)((gsz + G - 1) / G));
-  int bs_sh = 0;
-  while ((1LL << bs_sh) < block_size) ++bs_sh;
-  if ((1LL << bs_sh) != block_size) bs_sh = -1;  // not a power of two: divide
-  const PagedArgs pg{block_table, context_lens, (int)max_blocks_per_seq, (int)block_size, bs_sh, 0};
-  const uint32_t* vp = reinterpret_cast<const uint32_t*>(v_packed);
-#define SL8_K3(DD, GG)                                                                      \
-  k8v3_split_kernel<DD, GG><<<grid, DEC_THREADS, 0, st>>>(                                  \
-      q, q_scale, k_cache, k_scale, vp, v_norm, v_codebook, op, mp, lp, (int)max_context_len, \
-      ns, (int)Hq, (int)Hkv, gsz, ibhq, pg)
-#define SL8_K3D(DD)                     \
-  switch (G) {                          \
-    case 1: SL8_K3(DD, 1); break;       \
-    case 2: SL8_K3(DD, 2); break;       \
-    case 4: SL8_K3(DD, 4); break;       \
-    default: SL8_K3(DD, 8); break;      \
-  }
-  if (D == 128) SL8_K3D(128)
-  else SL8_K3D(256)
-#undef SL8_K3D
-#undef SL8_K3
-  SL8_CHECK_LAUNCH("attn_paged_decode_k8v3 split");
-  launch_combine((int)D, ibhq, st, op, mp, lp, static_cast<uint16_t*>(out), ns, ibhq);
-  SL8_CHECK_LAUNCH("attn_paged_decode_k8v3 combine");
-  return SL8_OK;
+  SL8_CHECK_ARG(q && aligned(q, 16), "fni8 decode_kv8: q must be 16-byte aligned");
+  const size_t need = sl8_attn_int8_decode_kv8_q16_workspace(B, Hq, D, num_splits);
+  SL8_CHECK_ARG(workspace && need && workspace_bytes >= need && aligned(workspace, 16),
+                "fni8 decode_kv8: workspace needs %zu bytes", need);
+  const size_t part = (sl8_attn_int8_decode_workspace(B, Hq, D, num_splits) + 15) / 16 * 16;
+  int8_t* qi = static_cast<int8_t*>(workspace) + part;
+  float* qs = reinterpret_cast<float*>(qi + B * Hq * D);
+  if (const int rc = launch_prep(q, q_dtype, B * Hq, D, rotate != 0, q_scale_mul, qi, qs, PlanArgs{},
+                                 static_cast<hipStream_t>(stream)))
+    return rc;
+  return sl8_attn_int8_decode_kv8(qi, qs, k, k_scale, v, v_scale, out, B, Hq, Hkv, N, D, num_splits,
+                                  workspace, part, stream);
 }
 
 namespace sl8 {

@@ -146,13 +146,18 @@ def attn_decode_cached(q: torch.Tensor, k_i8: torch.Tensor, k_scale: torch.Tenso
             "attn_decode_cached received a per-token V scale [B,H,N]; the contiguous int8-V "
             "decode kernel (attn_int8_decode_kv8) supports per-channel V scales [B,H,D] only")
     softmax_scale = (1.0 / (q.shape[-1] ** 0.5)) if scale is None else scale
+    ns = -1 if num_splits is None else int(num_splits)
+    q = q.contiguous()
+    if _C.q16_ok(q):
+        return _C.attn_int8_decode_kv8_q16(q, softmax_scale * LOG2E, rotate, k_i8.contiguous(),
+                                           k_scale.contiguous(), v_i8.contiguous(),
+                                           v_scale.contiguous(), ns)
     if rotate:
         q = rotate_last(q)
     q_shape = q.shape
     q_i8, q_scale = quantize_i8_rowwise(q.reshape(-1, q_shape[-1]).contiguous())
     q_i8 = q_i8.reshape(q_shape)
     q_scale = (q_scale.float() * (softmax_scale * LOG2E)).reshape(q_shape[0], q_shape[1], 1).contiguous()
-    ns = -1 if num_splits is None else int(num_splits)
     return _C.attn_int8_decode_kv8(q_i8.contiguous(), q_scale, k_i8.contiguous(),
                                    k_scale.contiguous(), v_i8.contiguous(), v_scale.contiguous(), ns)
 
@@ -186,6 +191,15 @@ def attn_paged_decode_cached(q: torch.Tensor, k_cache: torch.Tensor, k_scale: to
     if max_context_len is None:
         max_context_len = int(context_lens.max().item())
     softmax_scale = (1.0 / (q.shape[-1] ** 0.5)) if scale is None else scale
+    q = q.contiguous()
+    if num_splits is None and _C.q16_ok(q):
+        out = _C.attn_paged_decode_q16(q, softmax_scale * LOG2E, rotate, k_cache.contiguous(),
+                                       k_scale.contiguous(), v_cache.contiguous(),
+                                       v_scale.contiguous(), block_table.contiguous(),
+                                       context_lens.contiguous(), int(block_size),
+                                       int(max_context_len))
+        if out is not None:
+            return out
     if rotate:
         q = rotate_last(q)
     q_shape = q.shape
@@ -218,6 +232,15 @@ def attn_paged_decode_k8v3(q: torch.Tensor, k_cache: torch.Tensor, k_scale: torc
     if max_context_len is None:
         max_context_len = int(context_lens.max().item())
     softmax_scale = (1.0 / (q.shape[-1] ** 0.5)) if scale is None else scale
+    q = q.contiguous()
+    if num_splits is None and _C.q16_ok(q):
+        out = _C.attn_paged_decode_k8v3_q16(q, softmax_scale * LOG2E, rotate, k_cache.contiguous(),
+                                            k_scale.contiguous(), v_packed.contiguous(),
+                                            v_norm.contiguous(), v_codebook.contiguous(),
+                                            block_table.contiguous(), context_lens.contiguous(),
+                                            int(block_size), int(max_context_len))
+        if out is not None:
+            return out
     if rotate:
         q = rotate_last(q)
     q_shape = q.shape

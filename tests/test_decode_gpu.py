@@ -398,3 +398,55 @@ def test_paged_rejects(device):
         _C.attn_paged_decode(q, qs, kc, ks, vc, vs, bt, ctx, 16, 10 ** 6)
     with pytest.raises(RuntimeError, match="int32"):
         _C.attn_paged_decode(q, qs, kc, ks, vc, vs, bt.long(), ctx, 16, 50)
+
+
+PLAN_CASES = [  # B, Hq, Hkv, D, block size, lengths
+    (1, 8, 2, 128, 16, (1,)), (3, 32, 8, 128, 16, (5000, 0, 257)), (2, 8, 4, 128, 32, (3000, 64)),
+    (2, 16, 2, 64, 16, (4097, 255)), (2, 8, 2, 256, 64, (2000, 1)), (3, 4, 4, 128, 16, (700, 256, 0)),
+    (2, 8, 2, 32, 8, (900, 3)), (2, 16, 1, 128, 12, (1000, 300)), (1, 8, 2, 128, 1, (1800,)),
+    (70, 4, 1, 64, 16, tuple(13 * i % 600 for i in range(70))),
+]
+
+
+@pytest.mark.parametrize("case", PLAN_CASES, ids=lambda c: "B%dH%d_%dD%dbs%d" % c[:5])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_paged_planned_splits(device, case, dtype):
+    """ops.attn_paged_decode_cached with its splits planned on the device (mixed lengths, empty
+    sequences, more sequences than a wave has lanes, blocks that are no power of two, contexts
+    above max_context_len, NaN scales in unwritten slots) against the one-split kernel on the
+    query quantised beforehand. Both round p to fp16 and the output to fp16: the decode bar."""
+    B, Hq, Hkv, D, bs, lens = case
+    _, _, kc, ks, vc, vs, bt, ctx = _paged_cache(case, device, seed=5)
+    ks, vs = ks.clone(), vs.clone()
+    for b, n in enumerate(lens):
+        if n % bs:
+            ks[int(bt[b, n // bs]), :, n % bs:] = float("nan")
+            vs[int(bt[b, n // bs]), :, n % bs:] = float("nan")
+    g = torch.Generator(device="cpu").manual_seed(B + D)
+    q = torch.randn(B, Hq, 1, D, generator=g).to(dtype).to(device)
+    for nmax in (max(lens), max(1, max(lens) * 2 // 3)):
+        out = sl8.attn_paged_decode_cached(q, kc, ks, vc, vs, bt, ctx, bs, max_context_len=nmax,
+                                           rotate=False)
+        q_i8, qs = _C.quantize_i8_rowwise(q.reshape(-1, D))
+        qs = (qs * (quant.LOG2E / D ** 0.5)).reshape(B, Hq, 1)
+        ref = _C.attn_paged_decode(q_i8.reshape(B, Hq, 1, D), qs, kc, ks, vc, vs, bt, ctx, bs, nmax, 1)
+        assert_finite(out)
+        assert_close_abs(out, _np(ref.float()), atol=2e-3, rtol=2e-3, what=f"planned {case} {nmax}")
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+def test_decode_query_rotated_in_the_call(device, D):
+    """The rotation of the 16-bit query inside the decode call against rotate_last before it:
+    a neighbouring fp16 rounding moves a code by at most one step of 127."""
+    case = (2, 8, 2, D, 16, (700, 40))
+    _, _, kc, ks, vc, vs, bt, ctx = _paged_cache(case, device, seed=6)
+    q = torch.randn(2, 8, 1, D, device=device, dtype=torch.float16)
+    rot = quant.rotation.rotate_last(q)
+    a = sl8.attn_paged_decode_cached(q, kc, ks, vc, vs, bt, ctx, 16, max_context_len=700)
+    b = sl8.attn_paged_decode_cached(rot, kc, ks, vc, vs, bt, ctx, 16, max_context_len=700, rotate=False)
+    assert_close_abs(a, _np(b.float()), atol=2e-2, rtol=1e-2, what=f"rotated query D={D}")
+    k, v = (torch.randn(2, 2, 300, D, device=device, dtype=torch.float16) for _ in range(2))
+    cache = sl8.quantize_kv_cache(k, v, rotate=True)
+    a = sl8.attn_decode_cached(q, *cache, rotate=True)
+    b = sl8.attn_decode_cached(rot, *cache, rotate=False)
+    assert_close_abs(a, _np(b.float()), atol=1e-2, rtol=1e-2, what=f"rotated query kv8 D={D}")

@@ -290,3 +290,21 @@ def test_k8v3_rejects(device):
         _C.attn_paged_decode_k8v3(*args[:6], torch.zeros(7, device=device), *args[7:], 16, 8, 1)
     with pytest.raises(RuntimeError, match="num_splits"):
         _C.attn_paged_decode_k8v3(*args, 16, 8, 0)
+
+
+@pytest.mark.parametrize("case", [(1, 8, 2, 128, 16, (1,)), (3, 32, 8, 128, 16, (3000, 0, 257)),
+                                  (2, 8, 4, 256, 32, (1500, 64)), (2, 16, 1, 128, 12, (1000, 300)),
+                                  (70, 2, 2, 128, 16, tuple(17 * i % 500 for i in range(70)))],
+                         ids=lambda c: "B%dH%d_%dD%dbs%d" % c[:5])
+def test_k8v3_planned_splits(device, case):
+    """ops.attn_paged_decode_k8v3 with its splits planned on the device against the one-split
+    kernel on the query quantised beforehand (the K8V3 bar)."""
+    B, Hq, Hkv, D, bs, lens = case
+    _, _, *store = _store(case, device, seed=4)
+    g = torch.Generator(device="cpu").manual_seed(B + D)
+    q = torch.randn(B, Hq, 1, D, generator=g).half().to(device)
+    out = sl8.attn_paged_decode_k8v3(q, *store, bs, max_context_len=max(lens), rotate=False)
+    q_i8, qs = _C.quantize_i8_rowwise(q.reshape(-1, D))
+    qs = (qs * (np.log2(np.e) / D ** 0.5)).reshape(B, Hq, 1)
+    ref = _np(_C.attn_paged_decode_k8v3(q_i8.reshape(B, Hq, 1, D), qs, *store, bs, max(lens), 1).float())
+    assert_close_abs(out, ref, atol=2e-3 * max(1.0, np.abs(ref).max()), rtol=2e-3, what=f"planned {case}")

@@ -111,6 +111,19 @@ int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t qrows, int6
                     int8_t* k_i8, float* k_scale, float* k_mean, int32_t* gate_flag,
                     void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same prologue for other sets of tensors, without the gate: q [qrows, D] (null, qrows 0: none),
+ * k and v [G, N, D] (null: none; at least one of them), all dtype f16 or bf16. v gets per-channel
+ * codes as sl8_quantize_i8_cols. rotate != 0: Q's rows and the smoothed K's are multiplied by the
+ * normalised Hadamard matrix first (fp32, rounded to dtype; D a power of two). k_mean may be NULL.
+ * Replaces quantize_kv_cache's and quantize_qk(rotate=True)'s torch steps (reference
+ * superl8/ops.py:531-584, superl8/quant/core.py:164-196).
+ * workspace: sl8_quantize_qkv_workspace(G, N, D) bytes, 8-byte aligned. */
+size_t sl8_quantize_qkv_workspace(int64_t G, int64_t N, int64_t D);
+int sl8_quantize_qkv(const void* q, const void* k, const void* v, int dtype, int64_t qrows,
+                     int64_t G, int64_t N, int64_t D, int rotate, float q_scale_mul, int8_t* q_i8,
+                     float* q_scale, int8_t* k_i8, float* k_scale, float* k_mean, int8_t* v_i8,
+                     float* v_scale, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Per-channel int8 of V over the key axis (W8A8 path).
  * Replaces quantize_v_perchannel, reference superl8/quant/core.py:98-110

@@ -167,6 +167,54 @@ def quantize_qk_fused(q: torch.Tensor, k: torch.Tensor, q_scale_mul: float,
     return q_i8, q_scale, k_i8, k_scale, k_mean, flag
 
 
+_PROLOGUE_DIMS = (32, 64, 72, 80, 128, 256)
+
+
+def prologue_ok(*ts: torch.Tensor) -> bool:
+    """Whether the fused prologue serves these 16-bit tensors [..., rows, D] (of one type and D)."""
+    t0 = ts[0]
+    return (t0.dtype in (torch.float16, torch.bfloat16) and t0.shape[-1] in _PROLOGUE_DIMS
+            and all(t.is_cuda and t.dtype == t0.dtype and t.dim() >= 2
+                    and t.shape[-1] == t0.shape[-1] and t.numel() > 0
+                    and t.shape[-2] < (1 << 23) and t.numel() < t.shape[-2] * t.shape[-1] * 65536
+                    # 16-byte loads: a contiguous view at an odd offset takes the separate kernels
+                    and (t.data_ptr() % 16 == 0 or not t.is_contiguous()) for t in ts))
+
+
+def quantize_qkv_fused(q, k, v, q_scale_mul: float = 1.0, rotate: bool = False):
+    """The fused prologue without the gate, for what is not None of q [B,Hq,M,D] and k, v
+    [..., N, D] (see prologue_ok): Q and the smoothed K per row (rotated first with `rotate`),
+    V per channel. Returns (q_i8, q_scale [B,Hq,M], k_i8, k_scale [..., N], k_mean [..., 1, D],
+    v_i8, v_scale [..., 1, D]), None for what is absent."""
+    kv = k if k is not None else v
+    _on_gpu(*(t for t in (q, k, v) if t is not None))
+    q, k, v = (t if t is None else t.contiguous() for t in (q, k, v))
+    *lead, N, D = kv.shape
+    _check(k is None or v is None or k.shape == v.shape, "fused prologue: K/V shape mismatch")
+    _check(q is None or q.shape[-1] == D, "fused prologue: Q/K head dims differ")
+    G, dev = math.prod(lead), kv.device
+
+    def outs(t, scale_shape):
+        if t is None:
+            return None, None
+        return (torch.empty(t.shape, device=dev, dtype=torch.int8),
+                torch.empty(scale_shape, device=dev, dtype=torch.float32))
+
+    q_i8, q_scale = outs(q, None if q is None else q.shape[:-1])
+    k_i8, k_scale = outs(k, (*lead, N))
+    v_i8, v_scale = outs(v, (*lead, 1, D))
+    k_mean = None if k is None else torch.empty((*lead, 1, D), device=dev, dtype=torch.float32)
+    ws_bytes = _lib.load().sl8_quantize_qkv_workspace(G, N, D)
+    ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
+    ptr = _lib.ptr
+    with torch.cuda.device(dev):
+        call("sl8_quantize_qkv", ptr(q), ptr(k), ptr(v), dtype_code(kv.dtype),
+             0 if q is None else q.numel() // D, G, N, D, int(bool(rotate)), float(q_scale_mul),
+             ptr(q_i8), ptr(q_scale), ptr(k_i8), ptr(k_scale), ptr(k_mean), ptr(v_i8),
+             ptr(v_scale), ws.data_ptr(), ws_bytes, stream_of(kv))
+    return q_i8, q_scale, k_i8, k_scale, k_mean, v_i8, v_scale
+
+
 _GATE_MAX_D = 256
 
 
@@ -197,6 +245,8 @@ def quantize_v_perchannel(v: torch.Tensor):
     _check(v.is_cuda, "quantize_v_perchannel expects a CUDA tensor")
     _check(v.dtype in (torch.float16, torch.bfloat16, torch.float32),
            "quantize_v_perchannel input must be float16/bfloat16/float32")
+    if v.dim() >= 2 and prologue_ok(v):
+        return quantize_qkv_fused(None, None, v)[5:]
     v = v.contiguous()
     *lead, N, D = v.shape
     G = math.prod(lead)

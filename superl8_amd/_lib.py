@@ -32,6 +32,9 @@ SIGNATURES = {
     "sl8_quantize_qk_workspace": (_SZ, [_I64, _I64, _I64, _I64]),
     "sl8_quantize_qk": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _F, _F, _P, _P, _P, _P, _P, _P,
                              _P, _SZ, _P]),
+    "sl8_quantize_qkv_workspace": (_SZ, [_I64, _I64, _I64]),
+    "sl8_quantize_qkv": (_I, [_P, _P, _P, _I, _I64, _I64, _I64, _I64, _I, _F] + [_P] * 8
+                         + [_SZ, _P]),
     "sl8_quantize_i8_cols": (_I, [_P, _I, _I64, _I64, _I64, _P, _P, _P]),
     "sl8_attn_int8_fwd_workspace": (_SZ, [_I64, _I64, _I64, _I64, _I64, _I64]),
     "sl8_attn_int8_fwd": (_I, [_P, _P, _P, _P, _P, _I, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,

@@ -1053,11 +1053,7 @@ decode_prep_kernel(const uint16_t* __restrict__ q, int64_t rows, float q_mul,
   const bool live = r < rows;
   float f[8];
   VecIO<DT>::unpack(reinterpret_cast<const uint4*>(q + (live ? r : 0) * D)[lane], f);
-  if constexpr (ROT) {
-    hadamard_row<D>(f, lane);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = Elem<DT>::round(f[e]);
-  }
+  if constexpr (ROT) rotate_row<DT, D>(f, lane);
   float amax = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(f[e]));
@@ -1421,9 +1417,9 @@ kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __
     float h[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) h[e] = f[e];
-    hadamard_row<D>(h, lane);
+    rotate_row<SL8_DTYPE_F16, D>(h, lane);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = is_v ? f[e] : Elem<SL8_DTYPE_F16>::round(h[e]);
+    for (int e = 0; e < 8; ++e) f[e] = is_v ? f[e] : h[e];
   }
   float amax = 0.f;
 #pragma unroll

@@ -670,6 +670,10 @@ extern "C" int sl8_q_outlier_gate(const void* q, int dtype, int64_t rows, int64_
 //     2^-18 of max / ratio). A row holding a NaN never fires (torch's amax and
 //     median are NaN there). A block with a firing row ORs 1 into the flag
 //     (atomicOr), so the flag is set iff some row fires.
+// sl8_quantize_qkv adds V's per-channel codes (column maxima in A, codes in B) and the rotation of
+// Q and the smoothed K; without Q it builds a K/V cache. Bound by HBM: K and V are read twice
+// (the second time from the MALL where they fit). 16384 keys of 8 heads, D = 128: 93 us as nine
+// launches (a byte store per element in the column kernel, the smoothed K written and read back), 37 us here.
 // Head dims 72 and 80 take the 16 lanes per row of 128 with 9 and 10 of them
 // holding elements.
 // ---------------------------------------------------------------------------
@@ -756,10 +760,10 @@ __device__ __forceinline__ void mean_chunk(const uint16_t* __restrict__ kg, int6
   }
 }
 
-// Smooth + quantise PRO_KROWS key rows from n0 on, by a 256-thread block: the rows' loads are
-// issued first, the group's mean is formed from its C partials under them.
-template <int DT, int D>
-__device__ __forceinline__ void smooth_rows(const uint16_t* __restrict__ kg, int64_t n0, int64_t N,
+// Smooth (+ rotate) + quantise `rows` key rows from n0 on, by a 256-thread block: the first rows'
+// loads are issued first, the group's mean is formed from its C partials under them.
+template <int DT, int D, bool ROT>
+__device__ __forceinline__ void smooth_rows(const uint16_t* __restrict__ kg, int64_t n0, int rows, int64_t N,
                                             const typename MeanSum<DT>::T* __restrict__ part, int C,
                                             float* __restrict__ mean_out,
                                             int8_t* __restrict__ kq, float* __restrict__ kscale) {
@@ -768,11 +772,15 @@ __device__ __forceinline__ void smooth_rows(const uint16_t* __restrict__ kg, int
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
   const bool on = lane < NL;
   uint4 raw[NP];
+  const int64_t n_end = min(N, n0 + rows);
+  auto load = [&](int64_t b) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int64_t n = n0 + i * RPP + sub;
-    raw[i] = on && n < N ? reinterpret_cast<const uint4*>(kg + n * D)[lane] : make_uint4(0, 0, 0, 0);
-  }
+    for (int i = 0; i < NP; ++i) {
+      const int64_t n = b + i * RPP + sub;
+      raw[i] = on && n < n_end ? reinterpret_cast<const uint4*>(kg + n * D)[lane] : make_uint4(0, 0, 0, 0);
+    }
+  };
+  load(n0);
   // column d summed by PS threads over every PS-th partial, then in LDS
   constexpr int PS = 256 / D;
   __shared__ typename S::T mred[PS][D];
@@ -797,61 +805,192 @@ __device__ __forceinline__ void smooth_rows(const uint16_t* __restrict__ kg, int
   float mv[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) mv[e] = on ? mean_s[lane * 8 + e] : 0.f;
+  auto rows_of = [&](const uint4 (&r)[NP], int64_t b) __attribute__((always_inline)) {
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int64_t n = n0 + i * RPP + sub;
-    float f[8];
-    VecIO<DT>::unpack(raw[i], f);
-    float mx = 0.f;
+    for (int i = 0; i < NP; ++i) {
+      const int64_t n = b + i * RPP + sub;
+      float f[8];
+      VecIO<DT>::unpack(r[i], f);
+      float mx = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      f[e] = Elem<DT>::round(f[e] - mv[e]);
-      mx = fmaxf(mx, fabsf(f[e]));
+      for (int e = 0; e < 8; ++e) f[e] = Elem<DT>::round(f[e] - mv[e]);
+      if constexpr (ROT) rotate_row<DT, D>(f, lane);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
+      mx = lane_group_max<LPR>(mx);
+      const float s = mx * (1.0f / 127.0f);
+      const float safe = (s == 0.f) ? 1.f : s;
+      if (on && n < n_end) {
+        if (lane == 0) kscale[n] = safe;
+        reinterpret_cast<uint2*>(kq + n * D)[lane] = row_codes8<DT>(f, safe);
+      }
     }
-    mx = lane_group_max<LPR>(mx);
-    const float s = mx * (1.0f / 127.0f);
+  };
+  for (int64_t b = n0; b < n_end; b += PRO_KROWS) {
+    uint4 cur[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) cur[i] = raw[i];
+    if (b + PRO_KROWS < n_end) load(b + PRO_KROWS);  // in flight under this pass
+    rows_of(cur, b);
+  }
+}
+
+// Column maxima of |v| over rows [n0, n1) by a 256-thread block -> part[0, D) (NaN elements are
+// skipped, as by fmaxf).
+template <int DT, int D>
+__device__ __forceinline__ void amax_chunk(const uint16_t* __restrict__ vg, int64_t n0, int64_t n1,
+                                           float* __restrict__ part) {
+  constexpr int LPR = row_lanes(D), NL = D / 8, RPP = 256 / LPR;
+  constexpr int NIT = PRO_CHUNK / RPP < 8 ? PRO_CHUNK / RPP : 8;
+  const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
+  const bool on = lane < NL;
+  __shared__ float red[RPP][D];
+  float mx[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) mx[e] = 0.f;
+  for (int64_t b = n0; b < n1; b += NIT * RPP) {
+    uint4 raw[NIT];
+#pragma unroll
+    for (int i = 0; i < NIT; ++i) {
+      const int64_t n = b + sub + i * RPP;
+      raw[i] = on && n < n1 ? reinterpret_cast<const uint4*>(vg + n * D)[lane] : make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < NIT; ++i) {
+      float f[8];
+      VecIO<DT>::unpack(raw[i], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mx[e] = fmaxf(mx[e], fabsf(f[e]));
+    }
+  }
+  if (on) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[sub][lane * 8 + e] = mx[e];
+  }
+  __syncthreads();
+  for (int d = threadIdx.x; d < D; d += 256) {
+    float m = 0.f;
+#pragma unroll 8
+    for (int p = 0; p < RPP; ++p) m = fmaxf(m, red[p][d]);
+    part[d] = m;
+  }
+}
+
+// Per-channel codes of `rows` rows from n0 on, the group's scales formed from its C partial
+// maxima (codes8 with a scale per element).
+template <int DT, int D>
+__device__ __forceinline__ void channel_rows(const uint16_t* __restrict__ vg, int64_t n0, int rows,
+                                             int64_t N, const float* __restrict__ part, int C,
+                                             float* __restrict__ scale_out, int8_t* __restrict__ vq) {
+  constexpr int LPR = row_lanes(D), NL = D / 8, RPP = 256 / LPR, NP = PRO_KROWS / RPP;
+  const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
+  const bool on = lane < NL;
+  uint4 raw[NP];
+  const int64_t n_end = min(N, n0 + rows);
+  auto load = [&](int64_t b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int64_t n = b + i * RPP + sub;
+      raw[i] = on && n < n_end ? reinterpret_cast<const uint4*>(vg + n * D)[lane] : make_uint4(0, 0, 0, 0);
+    }
+  };
+  load(n0);
+  constexpr int PS = 256 / D;
+  __shared__ float mred[PS][D], scale_s[D];
+  if (threadIdx.x < PS * D) {
+    const int d = threadIdx.x % D, ps = threadIdx.x / D;
+    float m = 0.f;
+#pragma unroll 8
+    for (int c = ps; c < C; c += PS) m = fmaxf(m, part[(int64_t)c * D + d]);
+    mred[ps][d] = m;
+  }
+  __syncthreads();
+  if (threadIdx.x < D) {
+    float m = 0.f;
+#pragma unroll
+    for (int p = 0; p < PS; ++p) m = fmaxf(m, mred[p][threadIdx.x]);
+    const float s = m * (1.0f / 127.0f);
     const float safe = (s == 0.f) ? 1.f : s;
-    if (on && n < N) {
-      if (lane == 0) kscale[n] = safe;
-      reinterpret_cast<uint2*>(kq + n * D)[lane] = row_codes8<DT>(f, safe);
+    scale_s[threadIdx.x] = safe;
+    if (scale_out) scale_out[threadIdx.x] = safe;
+  }
+  __syncthreads();
+  float safe[8], inv[8];
+  bool fast = true;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    safe[e] = on ? scale_s[lane * 8 + e] : 1.f;
+    inv[e] = __builtin_amdgcn_rcpf(safe[e]);
+    fast &= DT == SL8_DTYPE_F16 || safe[e] >= 0x1p-120f;
+  }
+  for (int64_t b = n0; b < n_end; b += PRO_KROWS) {
+    uint4 cur[NP];
+#pragma unroll
+    for (int i = 0; i < NP; ++i) cur[i] = raw[i];
+    if (b + PRO_KROWS < n_end) load(b + PRO_KROWS);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int64_t n = b + i * RPP + sub;
+      float f[8];
+      VecIO<DT>::unpack(cur[i], f);
+      if (on && n < n_end)
+        reinterpret_cast<uint2*>(vq + n * D)[lane] = codes8_each(f, safe, inv, fast);
     }
   }
 }
 
-// A: K-mean partials of `chunk`-row chunks, one block per (group, chunk).
-template <int DT, int D>
+// A: K-mean partials of `chunk`-row chunks, one block per (group, chunk), then the column maxima
+// of V's chunks.
+template <int DT, int D, bool HASV>
 __global__ void __launch_bounds__(256)
 prologue_a_kernel(const uint16_t* __restrict__ k, int64_t N, int C, int64_t chunk,
-                  typename MeanSum<DT>::T* __restrict__ part, int32_t* __restrict__ flag) {
+                  typename MeanSum<DT>::T* __restrict__ part, int32_t* __restrict__ flag,
+                  int nka, const uint16_t* __restrict__ v, float* __restrict__ vpart) {
   if (flag && blockIdx.x == 0 && threadIdx.x == 0) *flag = 0;
-  const int64_t g = blockIdx.x / C, c = blockIdx.x % C;
-  mean_chunk<DT, D>(k + g * N * D, c * chunk, min(N, (c + 1) * chunk), part + (g * C + c) * D);
+  const bool is_v = HASV && (int)blockIdx.x >= nka;
+  const int64_t i = blockIdx.x - (is_v ? nka : 0), g = i / C, c = i % C;
+  const int64_t n0 = c * chunk, n1 = min(N, n0 + chunk);
+  if constexpr (HASV) {
+    if (is_v) return amax_chunk<DT, D>(v + g * N * D, n0, n1, vpart + i * D);
+  }
+  mean_chunk<DT, D>(k + g * N * D, n0, n1, part + i * D);
 }
 
-// B: the smoothed K rows (blocks [0, nkb): PRO_KROWS rows of group
-// blockIdx / kbg each) and the Q rows with the outlier gate (the rest). The Q
-// work does not depend on the mean, but sharing this launch keeps it off the
+// B: the smoothed K rows (blocks [0, nkb): krows rows of group
+// blockIdx / kbg each), V's rows (nvb blocks, likewise) and the Q rows with the outlier gate (the
+// rest). The Q work does not depend on the mean, but sharing this launch keeps it off the
 // critical path A -> mean -> B of the K side.
-template <int DT, int D, bool GATE>
+template <int DT, int D, bool GATE, bool ROT, bool HASV>
 __global__ void __launch_bounds__(256)
 prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
                   const typename MeanSum<DT>::T* __restrict__ part,
                   int C, float* __restrict__ k_mean,
-                  int8_t* __restrict__ k_i8, float* __restrict__ k_scale, int kbg, int nkb,
+                  int8_t* __restrict__ k_i8, float* __restrict__ k_scale, int krows, int kbg, int nkb,
                   const uint16_t* __restrict__ q, int64_t qrows, float qmul, float ratio,
                   int8_t* __restrict__ q_i8, float* __restrict__ q_scale,
-                  int32_t* __restrict__ flag) {
+                  int32_t* __restrict__ flag, int nvb, const uint16_t* __restrict__ v,
+                  const float* __restrict__ vpart, int8_t* __restrict__ v_i8,
+                  float* __restrict__ v_scale) {
   constexpr int LPR = row_lanes(D), NL = D / 8, RPP = 256 / LPR;
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
   if ((int)blockIdx.x < nkb) {
     const int64_t g = blockIdx.x / kbg;
     const int b = blockIdx.x % kbg;
-    smooth_rows<DT, D>(k + g * N * D, (int64_t)b * PRO_KROWS, N, part + g * C * D, C,
-                       b == 0 ? k_mean + g * D : nullptr, k_i8 + g * N * D, k_scale + g * N);
+    smooth_rows<DT, D, ROT>(k + g * N * D, (int64_t)b * krows, krows, N, part + g * C * D, C,
+                            b == 0 && k_mean ? k_mean + g * D : nullptr, k_i8 + g * N * D,
+                            k_scale + g * N);
     return;
   }
+  if constexpr (HASV) {
+    if ((int)blockIdx.x < nkb + nvb) {
+      const int64_t g = (blockIdx.x - nkb) / kbg;
+      const int b = (blockIdx.x - nkb) % kbg;
+      return channel_rows<DT, D>(v + g * N * D, (int64_t)b * krows, krows, N, vpart + g * C * D, C,
+                                 b == 0 ? v_scale + g * D : nullptr, v_i8 + g * N * D);
+    }
+  }
   const bool on = lane < NL;
-  const int qb = blockIdx.x - nkb, nqb = gridDim.x - nkb;
+  const int qb = blockIdx.x - nkb - nvb, nqb = gridDim.x - nkb - nvb;
   int fired = 0;
   const float rinv = 1.f / ratio;
   for (int64_t base = (int64_t)qb * RPP * PRO_QP; base < qrows;
@@ -869,6 +1008,7 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
       const bool live = r < qrows;
       float f[8];
       VecIO<DT>::unpack(raw[p], f);
+      if constexpr (ROT) rotate_row<DT, D>(f, lane);
       float mx = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(f[e]));
@@ -886,28 +1026,27 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
         // (t below 2^-100: every element takes the division.)
         const float t = mx * rinv;
         const bool tiny = t < 0x1p-100f;
-        const float tlo = tiny ? 0.f : t * (1.f - 0x1p-18f);
         const float thi = tiny ? INFINITY : t * (1.f + 0x1p-18f);
-        int cnt = 0, nan = 0;
-        bool amb = false;
+        // first an upper bound of the count, |x| <= thi: rows that could fire are rare, and only a
+        // wave that holds one counts exactly
+        int cnt = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) cnt += fabsf(f[e]) <= thi;
+        if (!on) cnt = 0;  // a lane without elements
+        cnt = lane_group_sum<LPR>(cnt);
+        const bool maybe = live && cnt > (D - 1) / 2;
+        if (__builtin_expect(__ballot(maybe) == 0, 1)) continue;
+        const float tlo = tiny ? 0.f : t * (1.f - 0x1p-18f);
+        int nan = 0;
+        cnt = 0;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           const float a = fabsf(f[e]);
           nan |= a != a;
           const float y = a + 1e-10f;
-          cnt += y < tlo;
-          amb |= y >= tlo && y <= thi;
+          cnt += y < tlo || (y <= thi && __fdiv_rn(mx, y) > ratio);
         }
-        if (__builtin_expect(__ballot(amb) != 0, 0)) {
-          if (amb) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-              const float y = fabsf(f[e]) + 1e-10f;
-              if (y >= tlo && y <= thi) cnt += __fdiv_rn(mx, y) > ratio;
-            }
-          }
-        }
-        if (!on) cnt = 0;  // a lane without elements
+        if (!on) cnt = 0;
         cnt = lane_group_sum<LPR>(cnt + (nan << 16));  // NaN count in the high half
         if (live && (cnt >> 16) == 0 && (cnt & 0xFFFF) > (D - 1) / 2) fired = 1;
       }
@@ -926,32 +1065,44 @@ int prologue_nqb(int64_t qrows, int D) {
 
 // The sizes of one prologue call and its launches for a storage type and head dim.
 struct Prologue {
-  const uint16_t *q, *k;
+  const uint16_t *q, *k, *v;  // null: no queries (qrows 0), keys, values
   int64_t qrows, G, N;
   float q_scale_mul, gate_ratio;
-  int8_t *q_i8, *k_i8;
-  float *q_scale, *k_scale, *k_mean;
+  int8_t *q_i8, *k_i8, *v_i8;
+  float *q_scale, *k_scale, *v_scale, *k_mean;
   int32_t* flag;
+  bool rotate;
   void* part;
   hipStream_t st;
   int64_t chunk;
-  int C, kbg;
+  int C, krows, kbg;
 
   // A (K-mean partials) -> B (the mean, K and Q rows, gate): the Q rows, the
   // bulk of the bytes, run beside the K rows in B instead of ahead of the mean
   template <int DT, int D>
   void go() const {
     using S = typename MeanSum<DT>::T;
-    const int nkb = (int)(G * kbg), nqb = prologue_nqb(qrows, D);
+    const int nka = k ? (int)(G * C) : 0, nkb = k ? (int)(G * kbg) : 0;
+    const int nva = v ? (int)(G * C) : 0, nvb = v ? (int)(G * kbg) : 0;
+    const int nqb = qrows ? prologue_nqb(qrows, D) : 0;
     S* pt = static_cast<S*>(part);
-    prologue_a_kernel<DT, D><<<(unsigned)(G * C), 256, 0, st>>>(k, N, C, chunk, pt, flag);
-    auto b = [&](auto gate) {
-      prologue_b_kernel<DT, D, decltype(gate)::value><<<nkb + nqb, 256, 0, st>>>(
-          k, N, pt, C, k_mean, k_i8, k_scale, kbg, nkb, q, qrows, q_scale_mul, gate_ratio, q_i8,
-          q_scale, flag);
+    float* vpt = reinterpret_cast<float*>(pt + (int64_t)nka * D);
+    using T = std::true_type;
+    using F = std::false_type;
+    auto run = [&](auto gate, auto rot, auto hasv) {
+      constexpr bool HV = decltype(hasv)::value;
+      prologue_a_kernel<DT, D, HV><<<nka + nva, 256, 0, st>>>(k, N, C, chunk, pt, flag, nka, v, vpt);
+      prologue_b_kernel<DT, D, decltype(gate)::value, decltype(rot)::value, HV>
+          <<<nkb + nvb + nqb, 256, 0, st>>>(k, N, pt, C, k_mean, k_i8, k_scale, krows, kbg, nkb, q,
+                                            qrows, q_scale_mul, gate_ratio, q_i8, q_scale, flag,
+                                            nvb, v, vpt, v_i8, v_scale);
     };
-    if (flag) b(std::true_type{});
-    else b(std::false_type{});
+    if constexpr ((D & (D - 1)) == 0) {
+      if (rotate) return v ? run(F{}, T{}, T{}) : run(F{}, T{}, F{});
+    }
+    if (flag) run(T{}, F{}, F{});
+    else if (v) run(F{}, F{}, T{});
+    else run(F{}, F{}, F{});
   }
   template <int DT>
   void go(int64_t D) const {
@@ -965,6 +1116,45 @@ struct Prologue {
     }
   }
 };
+
+// Checks and launches shared by the entries (q_i8 .. as in Prologue).
+int prologue(Prologue p, int dtype, int64_t D, void* workspace, size_t workspace_bytes,
+             size_t need, void* stream) {
+  SL8_CHECK_ARG(dtype == SL8_DTYPE_F16 || dtype == SL8_DTYPE_BF16,
+                "fused prologue: q and k must be float16 or bfloat16");
+  SL8_CHECK_ARG(D == 32 || D == 64 || D == 72 || D == 80 || D == 128 || D == 256,
+                "fused prologue: head dim must be 32/64/72/80/128/256, got %lld", (long long)D);
+  SL8_CHECK_ARG(!p.rotate || (D & (D - 1)) == 0,
+                "fused prologue: Hadamard needs a power-of-two dim, got %lld", (long long)D);
+  SL8_CHECK_ARG(p.G > 0 && p.N > 0 && p.N < (1LL << 23),
+                "fused prologue: bad shape (rows %lld, groups %lld, keys %lld)", (long long)p.qrows,
+                (long long)p.G, (long long)p.N);
+  SL8_CHECK_ARG((p.k || p.v) && (!p.k || (p.k_i8 && p.k_scale)) && (!p.qrows || (p.q && p.q_i8 && p.q_scale)) &&
+                    (!p.v || (p.v_i8 && p.v_scale)),
+                "fused prologue: null pointer");
+  SL8_CHECK_ARG(aligned(p.q, 16) && aligned(p.k, 16) && aligned(p.v, 16) && aligned(p.q_i8, 8) &&
+                    aligned(p.k_i8, 8) && aligned(p.v_i8, 8),
+                "fused prologue: q/k/v must be 16-byte and codes 8-byte aligned");
+  SL8_CHECK_ARG(workspace && workspace_bytes >= need && aligned(workspace, 8),
+                "fused prologue: workspace needs %zu bytes", need);
+  // rows per quantise block: up to 256 while two blocks per CU remain (K's alone), since every
+  // block reads all its group's partials: 16384 keys of 8 heads, D = 128, K and V: 64 rows a block
+  // 30.0 us, 128 rows 21.9, 256 rows 20.7 (101 MB at 4.9 TB/s)
+  int64_t krows = PRO_KROWS;
+  while (krows < 4 * PRO_KROWS && p.G * (p.N / (2 * krows)) >= 512) krows *= 2;
+  const int64_t kbg = (p.N + krows - 1) / krows;  // quantise blocks per group
+  p.chunk = pro_chunk_rows(p.N);
+  p.C = (int)((p.N + p.chunk - 1) / p.chunk);
+  p.krows = (int)krows;
+  p.kbg = (int)kbg;
+  SL8_CHECK_ARG(p.G * kbg < (1LL << 29) && p.G < 65536, "fused prologue: too many key groups");
+  p.part = workspace;
+  p.st = static_cast<hipStream_t>(stream);
+  if (dtype == SL8_DTYPE_F16) p.go<SL8_DTYPE_F16>(D);
+  else p.go<SL8_DTYPE_BF16>(D);
+  SL8_CHECK_LAUNCH("fused prologue");
+  return SL8_OK;
+}
 
 }  // namespace
 }  // namespace sl8
@@ -982,31 +1172,32 @@ extern "C" int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t 
                                float* k_mean, int32_t* gate_flag, void* workspace,
                                size_t workspace_bytes, void* stream) {
   clear_error();
-  SL8_CHECK_ARG(dtype == SL8_DTYPE_F16 || dtype == SL8_DTYPE_BF16,
-                "fused prologue: q and k must be float16 or bfloat16");
-  SL8_CHECK_ARG(D == 32 || D == 64 || D == 72 || D == 80 || D == 128 || D == 256,
-                "fused prologue: head dim must be 32/64/72/80/128/256, got %lld", (long long)D);
-  SL8_CHECK_ARG(qrows > 0 && G > 0 && N > 0 && N < (1LL << 23),
-                "fused prologue: bad shape (rows %lld, groups %lld, keys %lld)", (long long)qrows,
-                (long long)G, (long long)N);
-  SL8_CHECK_ARG(q && k && q_i8 && q_scale && k_i8 && k_scale && k_mean, "fused prologue: null pointer");
-  SL8_CHECK_ARG(aligned(q, 16) && aligned(k, 16) && aligned(q_i8, 8) && aligned(k_i8, 8),
-                "fused prologue: q/k must be 16-byte and codes 8-byte aligned");
   const bool gate = gate_ratio > 0.f;
   SL8_CHECK_ARG(!gate || gate_flag, "fused prologue: gate_flag required with a gate ratio");
-  const size_t need = sl8_quantize_qk_workspace(qrows, G, N, D);
-  SL8_CHECK_ARG(workspace && workspace_bytes >= need && aligned(workspace, 8),
-                "fused prologue: workspace needs %zu bytes", need);
-  const int64_t chunk = pro_chunk_rows(N), C = (N + chunk - 1) / chunk;
-  const int64_t kbg = (N + PRO_KROWS - 1) / PRO_KROWS;  // quantise blocks per group
-  SL8_CHECK_ARG(G * C < (1LL << 30) && G * kbg < (1LL << 30) && G < 65536,
-                "fused prologue: too many key groups");
-  const Prologue p{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), qrows, G, N,
-                   q_scale_mul, gate_ratio, q_i8, k_i8, q_scale, k_scale, k_mean,
-                   gate ? gate_flag : nullptr, workspace, static_cast<hipStream_t>(stream), chunk,
-                   (int)C, (int)kbg};
-  if (dtype == SL8_DTYPE_F16) p.go<SL8_DTYPE_F16>(D);
-  else p.go<SL8_DTYPE_BF16>(D);
-  SL8_CHECK_LAUNCH("fused prologue");
-  return SL8_OK;
+  SL8_CHECK_ARG(qrows > 0, "fused prologue: bad shape (rows %lld)", (long long)qrows);
+  SL8_CHECK_ARG(k && k_mean, "fused prologue: null pointer");
+  const Prologue p{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), nullptr, qrows,
+                   G, N, q_scale_mul, gate_ratio, q_i8, k_i8, nullptr, q_scale, k_scale, nullptr,
+                   k_mean, gate ? gate_flag : nullptr, false, nullptr, nullptr, 0, 0, 0, 0};
+  return prologue(p, dtype, D, workspace, workspace_bytes,
+                  sl8_quantize_qk_workspace(qrows, G, N, D), stream);
+}
+
+extern "C" size_t sl8_quantize_qkv_workspace(int64_t G, int64_t N, int64_t D) {
+  return sl8_quantize_qk_workspace(0, G, N, D) / sizeof(long long) * (sizeof(long long) + sizeof(float));
+}
+
+extern "C" int sl8_quantize_qkv(const void* q, const void* k, const void* v, int dtype,
+                                int64_t qrows, int64_t G, int64_t N, int64_t D, int rotate,
+                                float q_scale_mul, int8_t* q_i8, float* q_scale, int8_t* k_i8,
+                                float* k_scale, float* k_mean, int8_t* v_i8, float* v_scale,
+                                void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  SL8_CHECK_ARG(qrows >= 0 && (q || qrows == 0), "fused prologue: bad shape (rows %lld)",
+                (long long)qrows);
+  const Prologue p{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
+                   static_cast<const uint16_t*>(v), qrows, G, N, q_scale_mul, 0.f, q_i8, k_i8, v_i8,
+                   q_scale, k_scale, v_scale, k_mean, nullptr, rotate != 0, nullptr, nullptr, 0, 0, 0, 0};
+  return prologue(p, dtype, D, workspace, workspace_bytes, sl8_quantize_qkv_workspace(G, N, D),
+                  stream);
 }

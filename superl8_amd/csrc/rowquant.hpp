@@ -101,48 +101,55 @@ template <> struct VecIO<SL8_DTYPE_F32> {
 // Eight codes clamp(rint(fl(x / safe))) without a division per element.
 // |x| <= amax, so |x / safe| <= 127 * (1 + 2^-23) and, with inv = v_rcp_f32(safe)
 // (at most 1 ulp from 1 / safe; safe is normal and above 2^-120: fp16 rows always
-// are, 2^-24 / 127 at least, bf16 callers check),
-// r = fl(x * inv) is within 128 * (2^-23 + 2^-24) = 1.5 * 2^-16 of x / safe,
-// and fl(x / safe) within 2^-17 of it: |r - fl(x / safe)| < 2^-14. n = r
-// rounded to nearest-even by the 1.5 * 2^23 magic constant; unless
-// |r - n| > 0.5 - 2^-14 (r near a half-integer) both r and fl(x / safe)
-// round to n. Lanes holding such an element (about 1e-4 of them) take the
-// IEEE division, under a wave-uniform branch so the common path never
-// executes it.
-__device__ __forceinline__ uint2 codes8(const float* f, float safe) {
-  const float inv = __builtin_amdgcn_rcpf(safe);
+// are, 2^-24 / 127 at least, bf16 callers check), the exact product x * inv is within
+// 128 * 2^-23 = 2^-16 of x / safe, and fl(x / safe) within 2^-17 of that. One fma
+// against 1.5 * 2^23 rounds the product to the nearest integer n (ties to even) and
+// leaves n's two's complement in the low bits; a second one gives its distance from
+// n. Unless that exceeds 0.5 - 2^-14, fl(x / safe) rounds to n too. Lanes holding a
+// farther element (about 1e-4 of them) or a NaN take the IEEE division, under a
+// wave-uniform branch so the common path never executes it: 4.3 VALU instructions an
+// element, where a product, its rounding, a comparison, the clamp and the conversion took 8.5.
+// safe, inv: per element (codes8: one scale for all); fast: every scale is in that range, else
+// every element is divided.
+__device__ __forceinline__ uint2 codes8_each(const float* f, const float* safe, const float* inv,
+                                             bool fast) {
   constexpr float MAGIC = 12582912.f;  // 1.5 * 2^23
-  float n[8];
-  bool amb = false;
+  float t[8], far = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float r = f[e] * inv;
-    n[e] = (r + MAGIC) - MAGIC;
-    amb |= !(fabsf(r - n[e]) <= 0.5f - 0x1p-14f);  // also catches inf / NaN
+    t[e] = fmaf(f[e], inv[e], MAGIC);
+    // (maximum: NaN stays)
+    far = __builtin_elementwise_maximum(far, fabsf(fmaf(f[e], inv[e], MAGIC - t[e])));
   }
+  const bool amb = !fast || !(far <= 0.5f - 0x1p-14f);
   if (__builtin_expect(__ballot(amb) != 0, 0)) {
     if (amb) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        n[e] = rintf(__fdiv_rn(f[e], safe));
-        if (n[e] != n[e]) n[e] = -127.f;  // NaN: the clamp of fmaxf / fminf gives -127
+        const float n = rintf(__fdiv_rn(f[e], safe[e]));
+        // NaN: the clamp of fmaxf / fminf gives -127
+        t[e] = (n != n ? -127.f : fminf(fmaxf(n, -127.f), 127.f)) + MAGIC;
       }
     }
   }
-  // n is an integer in [-128, 128] (or the division's result): clamp as int
   uint32_t w[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    int c[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) c[e] = __builtin_amdgcn_fmed3f(n[4 * i + e], -127.f, 127.f);
-    // bytes 0 of c0..c3 -> one dword (v_perm_b32: selectors 0-3 pick the
+    // the low bytes of four words -> one dword (v_perm_b32: selectors 0-3 pick the
     // second operand's bytes, 4-7 the first's, 0x0c a zero byte)
-    const uint32_t lo = __builtin_amdgcn_perm((uint32_t)c[1], (uint32_t)c[0], 0x0c0c0400u);
-    const uint32_t hi = __builtin_amdgcn_perm((uint32_t)c[3], (uint32_t)c[2], 0x04000c0cu);
+    const uint32_t lo = __builtin_amdgcn_perm(__float_as_uint(t[4 * i + 1]), __float_as_uint(t[4 * i]),
+                                              0x0c0c0400u);
+    const uint32_t hi = __builtin_amdgcn_perm(__float_as_uint(t[4 * i + 3]),
+                                              __float_as_uint(t[4 * i + 2]), 0x04000c0cu);
     w[i] = lo | hi;
   }
   return make_uint2(w[0], w[1]);
+}
+__device__ __forceinline__ uint2 codes8(const float* f, float safe) {
+  const float s[8] = {safe, safe, safe, safe, safe, safe, safe, safe};
+  const float r = __builtin_amdgcn_rcpf(safe);
+  const float inv[8] = {r, r, r, r, r, r, r, r};
+  return codes8_each(f, s, inv, true);
 }
 
 // The same codes by IEEE division (any safe).
@@ -208,6 +215,14 @@ __device__ __forceinline__ void hadamard_row(float* f, int lane) {
   const float rs = (float)(1.0 / __builtin_sqrt((double)D));
 #pragma unroll
   for (int e = 0; e < 8; ++e) f[e] *= rs;
+}
+
+// The rotation of a row as its own pass would store it: rounded to its storage type.
+template <int DT, int D>
+__device__ __forceinline__ void rotate_row(float* f, int lane) {
+  hadamard_row<D>(f, lane);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) f[e] = Elem<DT>::round(f[e]);
 }
 
 }  // namespace

@@ -37,6 +37,14 @@ def attn_int8_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: 
     if internal_accuracy_gate:
         fired, qk = quant.quantize_qk_gated(q, k, softmax_scale=scale, rotate=rotate,
                                             defer=not int8_pv)
+    elif int8_pv and window_left < 0 and not rotate and quant.core.fused_ok(q, k, v):
+        # one prologue for Q, K and V
+        s = (1.0 / math.sqrt(q.shape[-1])) if scale is None else scale
+        q_i8, q_scale, k_i8, k_scale, _k_mean, v_i8, v_scale = _C.quantize_qkv_fused(
+            q, k, v, s * quant.LOG2E)
+        return _C.attn_w8a8_fwd(q_i8, q_scale, k_i8, k_scale, v_i8, v_scale.squeeze(-2), causal,
+                                causal_diag=k.shape[-2] - q.shape[-2] if causal else 0,
+                                per_warp_quant=per_warp_quant)
     else:
         fired, qk = False, quant.quantize_qk(q, k, softmax_scale=scale, rotate=rotate)
     if isinstance(fired, torch.Tensor):
@@ -115,6 +123,11 @@ def quantize_kv_cache(k: torch.Tensor, v: torch.Tensor, *, rotate: bool = False,
 
     if v_quant not in ("per_channel", "per_token"):
         raise ValueError(f"v_quant must be 'per_channel' or 'per_token', got {v_quant!r}")
+    if rotate:
+        hadamard_dim(k.shape[-1])
+    if v_quant == "per_channel" and k.shape == v.shape and _C.prologue_ok(k, v):
+        _, _, k_i8, k_scale, _, v_i8, v_scale = _C.quantize_qkv_fused(None, k, v, rotate=rotate)
+        return k_i8, k_scale, v_i8, v_scale.squeeze(-2)
     k_s, _k_mean = smooth_k(k)
     if rotate:
         from .quant.rotation import rotate_last

@@ -91,15 +91,10 @@ def detect_q_outlier_domination(q: torch.Tensor, *, ratio_threshold: float = 12.
     return bool(((row_max / (row_med + 1e-10)) > ratio_threshold).any())
 
 
-def _fused_ok(q: torch.Tensor, k: torch.Tensor) -> bool:
-    """Shapes the fused prologue (sl8_quantize_qk) serves."""
-    return (q.dtype == k.dtype and q.dtype in (torch.float16, torch.bfloat16) and q.dim() == 4
-            and k.dim() == 4 and q.shape[-1] == k.shape[-1]
-            and q.shape[-1] in (32, 64, 72, 80, 128, 256)
-            and q.shape[0] == k.shape[0] and q.numel() > 0 and k.numel() > 0
-            and k.shape[-2] < (1 << 23)
-            # 16-byte loads: a contiguous view at an odd offset takes the separate kernels
-            and all(t.data_ptr() % 16 == 0 or not t.is_contiguous() for t in (q, k)))
+def fused_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None = None) -> bool:
+    """Shapes the fused prologue (sl8_quantize_qk, with V sl8_quantize_qkv) serves."""
+    return (q.dim() == 4 and k.dim() == 4 and q.shape[0] == k.shape[0] and _C.prologue_ok(k, q)
+            and (v is None or (v.shape == k.shape and _C.prologue_ok(k, v))))
 
 
 def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float | None = None,
@@ -121,7 +116,7 @@ def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float 
         capturing = torch.cuda.is_current_stream_capturing()
     except Exception:
         capturing = False
-    if not rotate and not capturing and _fused_ok(q, k):
+    if not rotate and not capturing and fused_ok(q, k):
         s = (1.0 / math.sqrt(q.shape[-1])) if softmax_scale is None else softmax_scale
         q_i8, q_scale, k_i8, k_scale, k_mean, flag = _C.quantize_qk_fused(
             q, k, s * LOG2E, ratio_threshold)
@@ -140,7 +135,7 @@ def quantize_qk(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float | None
     """Quantise Q and smoothed K for the int8 QK^T.
 
     Returns (q_int8, q_scale[..., m, 1] folded with softmax_scale*log2(e),
-    k_int8, k_scale[..., n, 1], k_mean[..., 1, d]). fp16 / bf16 Q/K without rotation
+    k_int8, k_scale[..., n, 1], k_mean[..., 1, d]). fp16 / bf16 Q/K
     take the fused prologue (two launches); otherwise the K mean and the
     smooth-and-quantise of each side are separate kernels (the smoothed K is
     never written either way).
@@ -148,12 +143,17 @@ def quantize_qk(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float | None
     _need_gpu(q, "quantize_qk")
     if softmax_scale is None:
         softmax_scale = 1.0 / math.sqrt(q.shape[-1])
-    if not rotate and _fused_ok(q, k):
+    if not rotate and fused_ok(q, k):
         q_i8, q_scale, k_i8, k_scale, k_mean, _ = _C.quantize_qk_fused(q, k, softmax_scale * LOG2E)
         return q_i8, q_scale.unsqueeze(-1), k_i8, k_scale.unsqueeze(-1), k_mean
     if rotate:
-        from .rotation import rotate_last
+        from .rotation import hadamard_dim, rotate_last
 
+        hadamard_dim(q.shape[-1])
+        if fused_ok(q, k):
+            q_i8, q_scale, k_i8, k_scale, k_mean, _, _ = _C.quantize_qkv_fused(
+                q, k, None, softmax_scale * LOG2E, True)
+            return q_i8, q_scale.unsqueeze(-1), k_i8, k_scale.unsqueeze(-1), k_mean
         k_s, k_mean = smooth_k(k)
         q = rotate_last(q)
         k_src, mean = rotate_last(k_s), None

@@ -246,3 +246,48 @@ def test_public_prefill_gate_read_back_to_back(device):
     torch.cuda.synchronize()
     for x, o in zip((q, q_out, q, q, q_out, q_out, q), outs):
         assert torch.equal(o, quiet if x is q else loud)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("G,N,D", [(2, 1, 128), (3, 63, 64), (2, 777, 72), (1, 6200, 256), (4, 300, 32),
+                                   (2, 4097, 128)])
+def test_cache_build_matches_separate_kernels(device, dtype, G, N, D):
+    """quantize_kv_cache's fused build (and V alone) against k_mean, the centred row quantiser and
+    the element-wise column quantiser (reached with D = 2 D columns viewed apart), bit for bit."""
+    g = torch.Generator(device="cpu").manual_seed(N + D)
+    k, v = ((torch.randn(1, G, N, D, generator=g) * 2 + 1).to(dtype).to(device) for _ in range(2))
+    v[..., 3] = 0            # an all-zero channel: scale 1
+    v[0, 0, N // 2, 5] = float("nan")   # skipped by the maximum, coded -127
+    v[0, G - 1, 0, 7] = float("inf")    # an infinite scale: 0, and -127 for the element itself
+    ki, ks, vi, vs = ops.quantize_kv_cache(k, v)
+    mean = _C.k_mean(k)
+    ki_ref, ks_ref = _C.quantize_rows_centered(k, mean, 1.0)
+    assert torch.equal(ki, ki_ref) and torch.equal(ks, ks_ref)
+    v32 = v.float()
+    vi_ref, vs_ref = _C.quantize_v_perchannel(v32)   # float32 input: the element-wise kernels
+    assert vs.shape == (1, G, D)
+    assert torch.equal(vs, vs_ref.squeeze(-2)) and torch.equal(vi, vi_ref)
+    vi2, vs2 = _C.quantize_v_perchannel(v)
+    assert torch.equal(vi2, vi_ref) and torch.equal(vs2, vs_ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+def test_rotated_prologue_against_64_bits(device, dtype, D):
+    """Q and the smoothed K through the in-register rotation, against the rotation in 64 bits
+    rounded to the storage type: a neighbouring rounding moves a scale by at most one unit in the
+    last place of the type and a code by at most one step."""
+    ulp = 2.0 ** -10 if dtype == torch.float16 else 2.0 ** -7
+    q, k = (torch.randn(1, 2, n, D, device=device).to(dtype) for n in (33, 130))
+    h = torch.ones(1, 1, dtype=torch.float64, device=device)
+    while h.shape[0] < D:
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+    qi, qs, ki, ks, km = quant.quantize_qk(q, k, softmax_scale=1.0 / LOG2E, rotate=True)
+    assert torch.equal(km, _C.k_mean(k))
+    k_s = (k.float() - km).to(dtype)
+    for x, c, s in ((q, qi, qs), (k_s, ki, ks)):
+        ref = (x.double() @ h / D ** 0.5).to(dtype).double()
+        s_ref = ref.abs().amax(-1, keepdim=True) / 127
+        assert ((s.double() / s_ref - 1).abs() <= ulp).all()
+        c_ref = (ref / s_ref).round().clamp(-127, 127)
+        assert ((c.double() - c_ref).abs() <= 1).all() and (c.double() != c_ref).float().mean() <= 0.02

@@ -721,13 +721,11 @@ def kv_write_paged(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scal
 # ---------------------------------------------------------------------------
 # Q4_K (reference csrc/kernel/gemm_dp4a.cu:146-193, gemm_decode_dp4a.cu:375-436)
 # ---------------------------------------------------------------------------
-def _q4k_checks(x, x_scale, w, out_dtype, tag, type_size=Q4K_TYPE_SIZE, x_block_ok=False):
-    _on_gpu(x, x_scale, w)
-    _check(x.dtype == torch.int8, "x must be int8")
+def _kq_weight_checks(x, w, out_dtype, tag, type_size):
+    """The checks shared by the k-quant products: weight bytes against x [M, K]; (M, N, K)."""
     _check(w.dtype == torch.uint8, f"w must be uint8 (native {tag} bytes)")
-    _check(x_scale.dtype == torch.float32, "x_scale must be float32")
     _check(x.dim() == 2 and w.dim() == 2, f"expect x[M,K] and w[N,(K/256)*{type_size}]")
-    _contig(x, x_scale, w)
+    _contig(x, w)
     _check(out_dtype in (torch.float16, torch.bfloat16, torch.float32),
            f"out_dtype must be float16 or bfloat16, got {out_dtype}")
     M, K = x.shape
@@ -735,6 +733,15 @@ def _q4k_checks(x, x_scale, w, out_dtype, tag, type_size=Q4K_TYPE_SIZE, x_block_
     _check(K % 256 == 0, f"{tag} contraction dim K must be %256==0, got {K}")
     _check(w.shape[1] == (K // 256) * type_size,
            f"{tag} weight must be [N, (K/256)*{type_size}], got [{N},{w.shape[1]}] for K={K}")
+    return M, N, K
+
+
+def _q4k_checks(x, x_scale, w, out_dtype, tag, type_size=Q4K_TYPE_SIZE, x_block_ok=False):
+    _on_gpu(x, x_scale, w)
+    _check(x.dtype == torch.int8, "x must be int8")
+    _check(x_scale.dtype == torch.float32, "x_scale must be float32")
+    _contig(x_scale)
+    M, N, K = _kq_weight_checks(x, w, out_dtype, tag, type_size)
     if x_block_ok:
         _check(x_scale.numel() == M or tuple(x_scale.shape) == (M, K // 256),
                f"x_scale must be [M] (per row) or [M, K/256] (per 256-block), got "
@@ -754,9 +761,46 @@ def _q4k(sym, x, x_scale, w, out_dtype, tag="Q4_K", type_size=Q4K_TYPE_SIZE):
     return out
 
 
+def _gemm_kq(fmt, x, x_scale, w, out_dtype, tag, type_size):
+    """The k-quant GEMM of any M, with the scratch of its K splits."""
+    M, N, K = _q4k_checks(x, x_scale, w, out_dtype, tag, type_size)
+    out = torch.empty((M, N), device=x.device, dtype=out_dtype)
+    if M and N:
+        with torch.cuda.device(x.device):
+            ws_bytes = _lib.load().sl8_gemm_kq_workspace(fmt, M, N, K)
+            ws = torch.empty((ws_bytes,), device=x.device, dtype=torch.uint8) if ws_bytes else None
+            call("sl8_gemm_kq", fmt, x.data_ptr(), x_scale.data_ptr(), w.data_ptr(), out.data_ptr(),
+                 dtype_code(out_dtype), M, N, K, None if ws is None else ws.data_ptr(), ws_bytes,
+                 stream_of(x))
+    return out
+
+
+def linear_kq_ok(x: torch.Tensor) -> bool:
+    """Whether linear_kq serves the activation rows x [M, K]: fp16 / bf16, M above the decode cap."""
+    return (x.is_cuda and x.dtype in (torch.float16, torch.bfloat16) and x.dim() == 2
+            and x.shape[0] > DEC_MAX_M and x.is_contiguous() and x.data_ptr() % 16 == 0)
+
+
+def linear_kq(fmt, x, w, out_dtype=torch.float16):
+    """Q4_K / Q5_K linear (fmt 4 / 5) of the 16-bit rows x [M, K] (see linear_kq_ok): quantised
+    and multiplied in one call; the result equals gemm_q4k / gemm_q5k of quantize_i8_rowwise(x)."""
+    tag, type_size = ("Q4_K", Q4K_TYPE_SIZE) if fmt == 4 else ("Q5_K", Q5K_TYPE_SIZE)
+    _on_gpu(x, w)
+    M, N, K = _kq_weight_checks(x, w, out_dtype, tag, type_size)
+    out = torch.empty((M, N), device=x.device, dtype=out_dtype)
+    if N and K:
+        with torch.cuda.device(x.device):
+            ws_bytes = _lib.load().sl8_gemm_kq_workspace(fmt, M, N, K)
+            ws = torch.empty((ws_bytes,), device=x.device, dtype=torch.uint8)
+            call("sl8_linear_kq", fmt, x.data_ptr(), dtype_code(x.dtype), w.data_ptr(),
+                 out.data_ptr(), dtype_code(out_dtype), M, N, K, ws.data_ptr(), ws_bytes,
+                 stream_of(x))
+    return out
+
+
 def gemm_q4k(x, x_scale, w, out_dtype=torch.float16):
     """x int8 [M,K], x_scale fp32 [M], w uint8 [N,(K/256)*144] -> [M,N] out_dtype."""
-    return _q4k("sl8_gemm_q4k", x, x_scale, w, out_dtype)
+    return _gemm_kq(4, x, x_scale, w, out_dtype, "Q4_K", Q4K_TYPE_SIZE)
 
 
 def gemm_decode_q4k(x, x_scale, w, out_dtype=torch.float16):
@@ -793,12 +837,12 @@ def quantize_i8_blockwise(x: torch.Tensor, block: int = 256):
 
 def gemm_q5k(x, x_scale, w, out_dtype=torch.float16):
     """x int8 [M,K], x_scale fp32 [M], w uint8 [N,(K/256)*176] (native Q5_K) -> [M,N]."""
-    return _q4k("sl8_gemm_q5k", x, x_scale, w, out_dtype, "Q5_K", Q5K_TYPE_SIZE)
+    return _gemm_kq(5, x, x_scale, w, out_dtype, "Q5_K", Q5K_TYPE_SIZE)
 
 
 def gemm_q6k(x, x_scale, w, out_dtype=torch.float16):
     """x int8 [M,K], x_scale fp32 [M], w uint8 [N,(K/256)*210] (native Q6_K) -> [M,N]."""
-    return _q4k("sl8_gemm_q6k", x, x_scale, w, out_dtype, "Q6_K", Q6K_TYPE_SIZE)
+    return _gemm_kq(6, x, x_scale, w, out_dtype, "Q6_K", Q6K_TYPE_SIZE)
 
 
 def gemm_decode_q5k(x, x_scale, w, out_dtype=torch.float16):

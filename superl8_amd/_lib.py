@@ -75,6 +75,9 @@ SIGNATURES = {
     "sl8_gemm_decode_q4k_xblock": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),
     "sl8_gemm_q4k": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),
     "sl8_dequant_q4k": (_I, [_P, _P, _I64, _I64, _P]),
+    "sl8_gemm_kq_workspace": (_SZ, [_I, _I64, _I64, _I64]),
+    "sl8_gemm_kq": (_I, [_I, _P, _P, _P, _P, _I, _I64, _I64, _I64, _P, _SZ, _P]),
+    "sl8_linear_kq": (_I, [_I, _P, _I, _P, _P, _I, _I64, _I64, _I64, _P, _SZ, _P]),
     "sl8_gemm_q5k": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),
     "sl8_gemm_q6k": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),
     "sl8_gemm_decode_q5k": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),

@@ -10,28 +10,15 @@
 //         sc_i signed int8.
 // x is the per-row int8 activation with its fp32 scale.
 //
-// Tile GEMM (M > 16; the decode GEMV below serves M <= 16): a 128 x 128 output
-// tile per workgroup, the x tile and the 128 weight super-blocks copied
-// global -> LDS one super-block ahead (double-buffered). Q5_K runs 8 waves,
-// two per SIMD, each owning 32 output columns x 64 rows (each B operand built
-// by the two waves of its columns); Q6_K, whose operand build costs the most,
-// runs 4 waves, one per SIMD, each over 32 columns x all 128 rows (each B
-// operand built once).
-// The integer dot products stay exact:
-//   Q5_K on v_mfma_i32_32x32x32_i8, one K = 32 step per sub-block: with
-//     q = n + 16 b (n the low nibble, b the 5th bit), q * sc_j =
-//     n (sc_j & 7) + 8 (n (sc_j >> 3) + 2 b sc_j), and each of the three B
-//     operands n (sc & 7), n (sc >> 3), 2 b sc is at most 126, so it fits int8
-//     (a 32-bit multiply scales 4 codes at once without carries). Three
-//     MFMAs into T_lo, T_hi, T_hi; per super-block f += d * (T_lo + 8 T_hi).
-//     The min term U = sum_j m_j * sum(x_j) on one fp16 MFMA per row block
-//     and super-block (x half-sums x mins, exact), f -= dmin * U one
-//     super-block later, as in the Q4_K tile kernel.
-//   Q6_K on v_mfma_i32_32x32x32_i8 as well, one K = 32 step per pair of
-//     16-element sub-blocks (each lane half holds one sub-block, so one scale
-//     per lane): P = (q - 32) * sc in [-4096, 4064] is split exactly into two
-//     int8 B operands, P = 256 B_hi + B_lo, two MFMAs into T_lo, T_hi, and
-//     f += d * (T_lo + 256 T_hi) per super-block (details at the kernel).
+// Q6_K tile GEMM (M > 16; Q4_K and Q5_K: gemm_kq_tile.hip; the decode GEMVs below serve M <= 16):
+// 32 RB rows x 128 columns per workgroup of 4 waves, each over 32 columns x all the rows (each B
+// operand built once), the x tile and the 128 weight super-blocks copied global -> LDS one
+// super-block ahead (double-buffered); tiles that do not fill a round of the chip are split over K
+// (plan_tiles). The integer dot products stay exact, on v_mfma_i32_32x32x32_i8, one K = 32 step per
+// pair of 16-element sub-blocks (each lane half holds one sub-block, so one scale per lane): P =
+// (q - 32) * sc in [-4096, 4064] (beyond the integers fp16 holds) is split exactly into two int8 B
+// operands, P = 256 B_hi + B_lo, two MFMAs into T_lo, T_hi, and f += d * (T_lo + 256 T_hi) per
+// super-block (details at the kernel).
 
 #include "kquant.hpp"
 
@@ -45,255 +32,21 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int Q5K_BYTES = 176;
 constexpr int Q6K_BYTES = 210;
-constexpr int KBM = 128, KBN = 128;                       // output tile
-// full k-quant tiles on 8 waves (two per SIMD, RB = 2): config 4's shape at
-// M = 512, same box, Q4_K 143 -> 123 us, Q5_K 174 -> 159 us; Q6_K, whose B
-// operands cost the most VALU to build (each is then built by two waves),
-// 186 -> 205 us, so it keeps 4 waves
-#ifndef SL8_KQ_NW8
-#define SL8_KQ_NW8 1
-#endif
-#ifndef SL8_Q6_NW8
-#define SL8_Q6_NW8 0
-#endif
+constexpr int KBN = 128;  // output tile columns
 
-// x tile copy by NT threads: 128 rows x 256 int8 of super-block sb; 16-byte
+// x tile copy by NT threads: BM rows x 256 int8 of super-block sb; 16-byte
 // chunk c of row r lands at r * 256 + 16 * (c ^ (r & 15)) (rows are one
-// 256-byte bank line). QTR: rows 32 q .. 32 q + 31 only (a last-round
-// quarter workgroup reads no other rows)
-template <int NT, bool QTR>
+// 256-byte bank line)
+template <int NT, int BM>
 __device__ __forceinline__ void copy_x_tile(const int8_t* x, int8_t* xd, int m0, int M, int K, int sb,
-                                            int tid, int wave, int q = 0) {
-  constexpr int XCH = QTR ? 512 : KBM * 16;
+                                            int tid, int wave) {
 #pragma unroll
-  for (int i = 0; i < XCH / NT; ++i) {
-    const int P0 = (QTR ? q * 512 : 0) + i * NT;
-    const int P = P0 + tid, row = P >> 4;
+  for (int i = 0; i < BM * 16 / NT; ++i) {
+    const int P0 = i * NT, P = P0 + tid, row = P >> 4;
     const int c = (P & 15) ^ (row & 15);
     const int8_t* src = x + (int64_t)min(m0 + row, M - 1) * K + (int64_t)sb * 256 + 16 * c;
     __builtin_amdgcn_global_load_lds((kq_gptr_t)src, (kq_lptr_t)(xd + (P0 + wave * 64) * 16), 16, 0, 0);
   }
-}
-
-// ---------------------------------------------------------------------------
-// Q5_K tile GEMM
-// ---------------------------------------------------------------------------
-// RB row blocks (32 rows) per wave, NW waves per workgroup, as the Q4_K tile
-// kernel: full tiles RB = 2, NW = 8 (two waves per SIMD, each over 64 rows)
-// or RB = 4, NW = 4; RB = 1, NW = 4 is a row quarter of a tile
-template <int OUT_DT, int RB, int NW = 4>
-__global__ void __launch_bounds__(64 * NW, 1)
-gemm_q5k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_scale,
-                     const uint8_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
-                     int nt_x, int xcd_m, int tile0) {
-  constexpr bool QTR = RB * NW < 16;
-  constexpr int NT = 64 * NW;
-  constexpr int WCH = (KBN * 11 + NT - 1) / NT * NT;  // weight-tile 16-B chunks, whole copies
-  __shared__ __attribute__((aligned(16))) int8_t xs0[KBM * 256];
-  __shared__ __attribute__((aligned(16))) int8_t xs1[KBM * 256];
-  __shared__ __attribute__((aligned(16))) uint8_t ws0[WCH * 16];
-  __shared__ __attribute__((aligned(16))) uint8_t ws1[WCH * 16];
-  // full tiles: the min-term MFMA's A operands (x half-sums) of one
-  // super-block, [slot][row block][lane]; the scheme of the Q4_K tile kernel
-  __shared__ __attribute__((aligned(16))) uint4 xh_l[QTR ? 1 : 2][QTR ? 1 : 4][64];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, h = lane >> 5;
-  // full tiles: one 128 x 128 tile per workgroup (tiles tile0, tile0 + 1, ...);
-  // quarters: the quarter blockIdx.x & 3 (32 rows) of tile tile0 + blockIdx.x / 4,
-  // so a short last round of tiles spreads over 4x the workgroups
-  const int tile = tile0 + (QTR ? (int)(blockIdx.x >> 2) : (int)blockIdx.x);
-  int ct, rt;
-  kq_tile_coords(tile, nt_x, xcd_m, ct, rt);
-  const int n0 = ct * KBN, m0 = rt * KBM;
-  const int rb0 = QTR ? (int)(blockIdx.x & 3) : 0;
-  const int cg = wave & 3;                                       // the wave's 32 output columns
-  const int rbw = QTR ? rb0 : (NW == 8 ? (wave >> 2) * RB : 0);  // its first row block
-  const int nsb = K >> 8;
-  const int64_t row_bytes = (int64_t)nsb * Q5K_BYTES;
-
-  auto load = [&](int sb, int8_t* xd, uint8_t* wd) __attribute__((always_inline)) {
-    copy_x_tile<NT, QTR>(x, xd, m0, M, K, sb, tid, wave, rb0);
-#pragma unroll
-    for (int i = 0; i < WCH / NT; ++i) {
-      const int P = min(i * NT + tid, KBN * 11 - 1), row = P / 11, c = P - 11 * row;
-      const uint8_t* src = w + (int64_t)min(n0 + row, N - 1) * row_bytes + (int64_t)sb * Q5K_BYTES + 16 * c;
-      __builtin_amdgcn_global_load_lds((kq_gptr_t)src, (kq_lptr_t)(wd + (i * NT + wave * 64) * 16), 16, 0, 0);
-    }
-  };
-
-  // wave (cg, row group) owns weight rows 32 cg .. 32 cg + 31 (output
-  // columns) for its RB row blocks; step j + 1's A reads and B operands are
-  // formed while step j's MFMAs run (one scheduling region per step)
-  float f[RB][16];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) f[rb][e] = 0.f;
-
-  // min term U = sum_j m_j * xsum_j on one fp16 MFMA per row block and
-  // super-block (exact: fp16 half-sums and mins, fp32 integer result); in a
-  // full tile one super-block late through LDS, as in the Q4_K tile kernel
-  float u_dmin = 0.f;
-  v8h u_b = {}, u_a = {};  // its m_j operand and (quarters) its half-sum operand
-  auto u_step = [&](int slot) __attribute__((always_inline)) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      const v8h a = QTR ? u_a : __builtin_bit_cast(v8h, xh_l[slot][rbw + rb][lane]);
-      const v16f_t u = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, u_b, v16f_t{}, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) f[rb][e] -= u_dmin * u[e];
-    }
-  };
-
-  // the half-sums this wave forms: row block urb, sub-blocks ju0 .. ju0 + JN - 1
-  constexpr int JN = (NW == 8 && !QTR) ? 4 : 8;
-  const int urb = QTR ? rb0 : (wave & 3);
-  const int ju0 = (NW == 8 && !QTR) ? 4 * (wave >> 2) : 0;
-  const int urow = 32 * urb + l32;
-
-  auto compute = [&](const int8_t* xt, const uint8_t* wt, int slot) __attribute__((always_inline)) {
-    const uint8_t* wr = wt + (32 * cg + l32) * Q5K_BYTES;
-    const uint4 hd = *reinterpret_cast<const uint4*>(wr);
-    const float d = h2f(hd.x & 0xFFFFu), dmin = h2f(hd.x >> 16);
-    const ScMin sm = unpack_scmin(hd.y, hd.z, hd.w);
-    const uint4 qhv = *reinterpret_cast<const uint4*>(wr + 16 + 16 * h);  // qh of l = 16h..16h+15
-    const uint32_t qh[4] = {qhv.x, qhv.y, qhv.z, qhv.w};
-    uint32_t qw[4][4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const uint4 qv = *reinterpret_cast<const uint4*>(wr + 48 + 32 * g + 16 * h);
-      qw[g][0] = qv.x; qw[g][1] = qv.y; qw[g][2] = qv.z; qw[g][3] = qv.w;
-    }
-    float hsum[8];
-    v4i A[2][RB], bl[2], bh[2], bb[2];
-    auto read_a = [&](int j, int buf) __attribute__((always_inline)) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const int row = 32 * (rbw + rb) + l32;
-        A[buf][rb] = *reinterpret_cast<const v4i*>(xt + row * 256 + 16 * ((2 * j + h) ^ (row & 15)));
-      }
-    };
-    // half-sum of sub-block ju0 + jj (jj < JN) of this lane's row urow, half h
-    auto xsum_half = [&](int jj) __attribute__((always_inline)) {
-      const int j = ju0 + jj;
-      const v4i xv = QTR ? A[jj & 1][0]
-                         : *reinterpret_cast<const v4i*>(xt + urow * 256 + 16 * ((2 * j + h) ^ (urow & 15)));
-      int sacc = __builtin_amdgcn_sdot4(xv[0], 0x01010101, 0, false);
-      sacc = __builtin_amdgcn_sdot4(xv[1], 0x01010101, sacc, false);
-      sacc = __builtin_amdgcn_sdot4(xv[2], 0x01010101, sacc, false);
-      sacc = __builtin_amdgcn_sdot4(xv[3], 0x01010101, sacc, false);
-      hsum[jj] = (float)sacc;
-    };
-    auto build = [&](int j, int buf) __attribute__((always_inline)) {
-      const uint32_t scw = j < 4 ? sm.sc_lo : sm.sc_hi;
-      const uint32_t sc = (scw >> (8 * (j & 3))) & 0xFF;
-      // q = n + 16 b (n the nibble, b the 5th bit): q * sc = n (sc & 7) +
-      // 8 (n (sc >> 3) + 2 b sc); every B byte <= 126
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t nib = (qw[j >> 1][e] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
-        const uint32_t hb = (qh[e] >> j) & 0x01010101u;
-        bl[buf][e] = (int)mul_bytes(nib, sc & 7);  // <= 15 * 7, 15 * 7 and 1 * 126 per byte
-        bh[buf][e] = (int)mul_bytes(nib, sc >> 3);
-        bb[buf][e] = (int)mul_bytes(hb, 2 * sc);
-      }
-    };
-    v16i_t tl[RB], th[RB];
-    read_a(0, 0);
-    build(0, 0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int c = j & 1;
-      __builtin_amdgcn_sched_barrier(0);
-      if (j < 7) read_a(j + 1, c ^ 1);
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        if (j == 0) {
-          tl[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bl[c], v16i_t{}, 0, 0, 0);
-          th[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bh[c], v16i_t{}, 0, 0, 0);
-        } else {
-          tl[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bl[c], tl[rb], 0, 0, 0);
-          th[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bh[c], th[rb], 0, 0, 0);
-        }
-        th[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bb[c], th[rb], 0, 0, 0);
-      }
-      if constexpr (JN == 8) xsum_half(j);
-      else if (j & 1) xsum_half(j >> 1);
-      if (j < 7) build(j + 1, c ^ 1);
-      __builtin_amdgcn_sched_group_barrier(0x100, RB + (QTR ? 0 : 1), 0);  // the LDS reads first
-#pragma unroll
-      for (int k = 0; k < 3 * RB; ++k) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, RB == 4 ? 3 : 8, 0);  // VALU
-      }
-    }
-    v8h ub;
-#pragma unroll
-    for (int jj = 0; jj < 8; ++jj)
-      ub[jj] = (_Float16)(float)(((jj < 4 ? sm.mn_lo : sm.mn_hi) >> (8 * (jj & 3))) & 0xFF);
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) f[rb][e] += d * (float)(tl[rb][e] + 8 * th[rb][e]);
-    // the previous super-block's U (in a full tile its operands were published
-    // before the barrier this compute follows), then this one's goes pending;
-    // both launches apply the same operations in the same order
-    if (slot >= 0) u_step(slot ^ 1);
-    if constexpr (QTR) {
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) u_a[jj] = (_Float16)hsum[jj];
-    } else if constexpr (JN == 8) {
-      v8h ua;
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) ua[jj] = (_Float16)hsum[jj];
-      xh_l[slot & 1][urb][lane] = __builtin_bit_cast(uint4, ua);
-    } else {
-      typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-      v4h ua;
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) ua[jj] = (_Float16)hsum[jj];
-      reinterpret_cast<uint2*>(&xh_l[slot & 1][urb][lane])[ju0 >> 2] = __builtin_bit_cast(uint2, ua);
-    }
-    u_dmin = dmin;
-    u_b = ub;
-  };
-
-  load(0, xs0, ws0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  __syncthreads();
-  int sb = 0;
-  for (; sb + 1 < nsb; sb += 2) {
-    load(sb + 1, xs1, ws1);
-    compute(xs0, ws0, sb == 0 ? -2 : 0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (sb + 2 < nsb) load(sb + 2, xs0, ws0);
-    compute(xs1, ws1, 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  }
-  if (sb < nsb) {
-    compute(xs0, ws0, sb == 0 ? -2 : 0);
-    if constexpr (!QTR) __syncthreads();
-  }
-  u_step((nsb - 1) & 1);  // the last super-block's U
-
-  const int n = n0 + 32 * cg + l32;
-  // the row scales first, unconditionally (clamped rows): one wait, not one per element
-  float xsv[RB][16];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int e = 0; e < 16; ++e)
-      xsv[rb][e] = x_scale[min(m0 + 32 * (rbw + rb) + 8 * (e >> 2) + 4 * h + (e & 3), M - 1)];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int m = m0 + 32 * (rbw + rb) + 8 * (e >> 2) + 4 * h + (e & 3);
-      if (m < M && n < N) st_out<OUT_DT>(out, (int64_t)m * N + n, f[rb][e] * xsv[rb][e]);
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -351,32 +104,22 @@ __device__ __forceinline__ void q6_split4(uint32_t q, v2s_t sc2, v2s_t off2, uin
   hi = __builtin_amdgcn_perm(u1, u0, 0x07050301u);                // high bytes
 }
 
-// RB row blocks per wave, NW waves per workgroup, as the Q4_K tile kernel
-template <int OUT_DT, int RB, int NW = 4>
-__global__ void __launch_bounds__(64 * NW, 1)
+template <int OUT_DT, int RB>
+__global__ void __launch_bounds__(256, RB == 1 ? 2 : 1)
 gemm_q6k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_scale,
                      const uint8_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
-                     int nt_x, int xcd_m, int tile0) {
-  constexpr bool QTR = RB * NW < 16;
-  constexpr int NT = 64 * NW;
-  __shared__ __attribute__((aligned(16))) int8_t xs0[KBM * 256];
-  __shared__ __attribute__((aligned(16))) int8_t xs1[KBM * 256];
+                     const TileWork tw) {
+  constexpr int NT = 256, BM = 32 * RB;
+  __shared__ __attribute__((aligned(16))) int8_t xs0[BM * 256];
+  __shared__ __attribute__((aligned(16))) int8_t xs1[BM * 256];
   __shared__ __attribute__((aligned(16))) uint32_t ws0[t6w<NT>()];
   __shared__ __attribute__((aligned(16))) uint32_t ws1[t6w<NT>()];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, h = lane >> 5;
-  // full tiles: one 128 x 128 tile per workgroup (tiles tile0, tile0 + 1, ...);
-  // quarters: the quarter blockIdx.x & 3 (32 rows) of tile tile0 + blockIdx.x / 4,
-  // so a short last round of tiles spreads over 4x the workgroups
-  const int tile = tile0 + (QTR ? (int)(blockIdx.x >> 2) : (int)blockIdx.x);
-  int ct, rt;
-  kq_tile_coords(tile, nt_x, xcd_m, ct, rt);
-  const int n0 = ct * KBN, m0 = rt * KBM;
-  const int rb0 = QTR ? (int)(blockIdx.x & 3) : 0;
-  const int cg = wave & 3;                                       // the wave's 32 output columns
-  const int rbw = QTR ? rb0 : (NW == 8 ? (wave >> 2) * RB : 0);  // its first row block
   const int nsb = K >> 8;
+  const TileRange tr = tile_range(tw, nsb);
+  const int n0 = tr.ct * KBN, m0 = tr.rt * BM;
   const int64_t row_bytes = (int64_t)nsb * Q6K_BYTES;
   const int rmax = min(KBN, N - n0) - 1;
 
@@ -387,7 +130,7 @@ gemm_q6k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
   // even): 128 rows of < 2^24 bytes
   const uint8_t* wbase = w + (int64_t)n0 * row_bytes;
   auto load = [&](int sb, int8_t* xd, uint32_t* wd) __attribute__((always_inline)) {
-    copy_x_tile<NT, QTR>(x, xd, m0, M, K, sb, tid, wave, rb0);
+    copy_x_tile<NT, BM>(x, xd, m0, M, K, sb, tid, wave);
     const uint32_t sboff = (uint32_t)sb * Q6K_BYTES;
 #pragma unroll
     for (int i = 0; i < (KBN * 14 + NT - 1) / NT; ++i) {
@@ -403,7 +146,7 @@ gemm_q6k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
 #pragma unroll
     for (int e = 0; e < 16; ++e) f[rb][e] = 0.f;
 
-  const int r = 32 * cg + l32;  // this lane's weight row in the tile
+  const int r = 32 * wave + l32;  // this lane's weight row in the tile
   auto compute = [&](int sb, const int8_t* xt, const uint32_t* wt) __attribute__((always_inline)) {
     // the block's misalignment is that of its offset from the row-n0 base
     const uint32_t base = (uint32_t)min(r, rmax) * (uint32_t)row_bytes + (uint32_t)sb * Q6K_BYTES;
@@ -443,7 +186,7 @@ gemm_q6k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
     auto read_a = [&](int s, int buf) __attribute__((always_inline)) {
 #pragma unroll
       for (int rb = 0; rb < RB; ++rb) {
-        const int row = 32 * (rbw + rb) + l32;
+        const int row = 32 * rb + l32;
         A[buf][rb] = *reinterpret_cast<const v4i*>(xt + row * 256 + 16 * ((2 * s + h) ^ (row & 15)));
       }
     };
@@ -472,9 +215,9 @@ gemm_q6k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
 #if SL8_Q6T_SCHED
       __builtin_amdgcn_sched_group_barrier(0x100, 16, 0);  // the LDS reads first
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
+      for (int k = 0; k < 2 * RB; ++k) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // 6 VALU
+        __builtin_amdgcn_sched_group_barrier(0x002, 24 / RB, 0);  // VALU
       }
 #endif
     }
@@ -484,22 +227,30 @@ gemm_q6k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
       for (int e = 0; e < 16; ++e) f[rb][e] += d * (float)(tl[rb][e] + 256 * th[rb][e]);
   };
 
-  load(0, xs0, ws0);
+  load(tr.sb0, xs0, ws0);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
   __syncthreads();
-  int sb = 0;
-  for (; sb + 1 < nsb; sb += 2) {
+  int sb = tr.sb0;
+  for (; sb + 1 < tr.sb1; sb += 2) {
     load(sb + 1, xs1, ws1);
     compute(sb, xs0, ws0);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
-    if (sb + 2 < nsb) load(sb + 2, xs0, ws0);
+    if (sb + 2 < tr.sb1) load(sb + 2, xs0, ws0);
     compute(sb + 1, xs1, ws1);
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __syncthreads();
   }
-  if (sb < nsb) compute(sb, xs0, ws0);
+  if (sb < tr.sb1) compute(sb, xs0, ws0);
 
+  if (tr.part) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        tr.part[(int64_t)BM * KBN * tr.sp + (32 * rb + 8 * (e >> 2) + 4 * h + (e & 3)) * KBN + r] = f[rb][e];
+    return;
+  }
   const int n = n0 + r;
   // the row scales first, unconditionally (clamped rows): one wait, not one per element
   float xsv[RB][16];
@@ -507,12 +258,12 @@ gemm_q6k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
   for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int e = 0; e < 16; ++e)
-      xsv[rb][e] = x_scale[min(m0 + 32 * (rbw + rb) + 8 * (e >> 2) + 4 * h + (e & 3), M - 1)];
+      xsv[rb][e] = x_scale[min(m0 + 32 * rb + 8 * (e >> 2) + 4 * h + (e & 3), M - 1)];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int m = m0 + 32 * (rbw + rb) + 8 * (e >> 2) + 4 * h + (e & 3);
+      const int m = m0 + 32 * rb + 8 * (e >> 2) + 4 * h + (e & 3);
       if (m < M && n < N) st_out<OUT_DT>(out, (int64_t)m * N + n, f[rb][e] * xsv[rb][e]);
     }
 }
@@ -1050,31 +801,7 @@ void launch_gemv_kq(const int8_t* x, const float* xs, const uint8_t* w, void* ou
   else launch_gemv_kq_m<FMT, 2>(x, xs, w, out, odt, M, N, K, st);
 }
 
-template <int FMT>
-void launch_kq_tile(const int8_t* x, const float* xs, const uint8_t* w, void* out, int odt,
-                    int M, int N, int K, hipStream_t st) {
-  // one workgroup per 128 x 128 tile; when the last round of tiles would hold
-  // at most half the CUs, those tiles run as 4 row quarters each (a second
-  // launch), which shortens that round (same per-element arithmetic)
-  const int ntx = (N + KBN - 1) / KBN, T = ntx * ((M + KBM - 1) / KBM), P = cu_count();
-  const int rem = T % P, nfull = (T >= P && rem > 0 && rem <= P / 2) ? T - rem : T;
-  // XCD-aware tile order (kq_tile_coords) when the column tiles split evenly over the 8 XCDs
-  const int xm = (SL8_KQ_XCD && ntx % 8 == 0) ? (M + KBM - 1) / KBM : 0;
-#define SL8_KQT(KERN, RB, NW, G, T0)                                                               \
-  switch (odt) {                                                                                   \
-    case SL8_DTYPE_F16: KERN<SL8_DTYPE_F16, RB, NW><<<G, 64 * NW, 0, st>>>(x, xs, w, out, M, N, K, ntx, xm, T0); break; \
-    case SL8_DTYPE_BF16: KERN<SL8_DTYPE_BF16, RB, NW><<<G, 64 * NW, 0, st>>>(x, xs, w, out, M, N, K, ntx, xm, T0); break; \
-    default: KERN<SL8_DTYPE_F32, RB, NW><<<G, 64 * NW, 0, st>>>(x, xs, w, out, M, N, K, ntx, xm, T0); break;        \
-  }
-  if (FMT == 5) {
-    if (SL8_KQ_NW8) { SL8_KQT(gemm_q5k_tile_kernel, 2, 8, nfull, 0) } else { SL8_KQT(gemm_q5k_tile_kernel, 4, 4, nfull, 0) }
-    if (nfull < T) SL8_KQT(gemm_q5k_tile_kernel, 1, 4, 4 * (T - nfull), nfull)
-  } else {
-    if (SL8_Q6_NW8) { SL8_KQT(gemm_q6k_tile_kernel, 2, 8, nfull, 0) } else { SL8_KQT(gemm_q6k_tile_kernel, 4, 4, nfull, 0) }
-    if (nfull < T) SL8_KQT(gemm_q6k_tile_kernel, 1, 4, 4 * (T - nfull), nfull)
-  }
-#undef SL8_KQT
-}
+constexpr TileShape SHAPES6[] = {{128, 128, 1, 3.5}, {64, 128, 1, 2.7}, {32, 128, 2, 3.1}};  // as SHAPES4
 
 int check_kq(const char* name, const int8_t* x, const float* xs, const uint8_t* w, void* out,
              int odt, int64_t M, int64_t N, int64_t K) {
@@ -1088,14 +815,90 @@ int check_kq(const char* name, const int8_t* x, const float* xs, const uint8_t* 
   SL8_CHECK_ARG(x && xs && w && out, "%s: null pointer", name);
   SL8_CHECK_ARG(aligned(x, 16), "x must be 16-byte aligned for the vectorized int4 loads");
   SL8_CHECK_ARG(aligned(w, 16), "%s: weight must be 16-byte aligned", name);
-  SL8_CHECK_ARG((M + KBM - 1) / KBM * ((N + KBN - 1) / KBN) < (1LL << 28), "%s: M*N too large", name);
+  SL8_CHECK_ARG((M + 31) / 32 * ((N + KBN - 1) / KBN) < (1LL << 28), "%s: M*N too large", name);
   return SL8_OK;
 }
 
 }  // namespace
+
+TilePlan plan_q6_tile(int M, int N, int K, bool may_split) {
+  return plan_tiles(M, N, K, SHAPES6, 3, may_split);
+}
+
+void launch_q6_tile(const TilePlan& p, const int8_t* x, const float* xs, const uint8_t* w, void* out,
+                    int odt, int M, int N, int K, float* part, hipStream_t st) {
+  const TileShape& s = SHAPES6[p.shape];
+  const TileWork tw = tile_work(p, s, M, part);
+  const unsigned grid = (unsigned)(p.nfull + p.nsplit * p.S);
+  auto go = [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    if (p.shape == 0) gemm_q6k_tile_kernel<DT, 4><<<grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
+    else if (p.shape == 1) gemm_q6k_tile_kernel<DT, 2><<<grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
+    else gemm_q6k_tile_kernel<DT, 1><<<grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
+  };
+  if (odt == SL8_DTYPE_F16) go(std::integral_constant<int, SL8_DTYPE_F16>{});
+  else if (odt == SL8_DTYPE_BF16) go(std::integral_constant<int, SL8_DTYPE_BF16>{});
+  else go(std::integral_constant<int, SL8_DTYPE_F32>{});
+  if (p.nsplit) launch_kq_reduce(p, s, tw, xs, out, odt, M, N, st);
+}
+
 }  // namespace sl8
 
 using namespace sl8;
+
+extern "C" size_t sl8_gemm_kq_workspace(int fmt, int64_t M, int64_t N, int64_t K) {
+  if (fmt < 4 || fmt > 6 || M <= 16 || N <= 0 || K <= 0 || K > 65536 || M >= (1LL << 31) || N >= (1LL << 31))
+    return 0;
+  if (fmt == 6) return plan_q6_tile((int)M, (int)N, (int)K, true).part_bytes;
+  return q45_tile_workspace(fmt, (int)M, (int)N, (int)K);
+}
+
+extern "C" int sl8_gemm_kq(int fmt, const int8_t* x, const float* x_scale, const uint8_t* w, void* out,
+                           int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+  clear_error();
+  SL8_CHECK_ARG(fmt >= 4 && fmt <= 6, "gemm_kq: fmt must be 4, 5 or 6, got %d", fmt);
+  const char* name = fmt == 4 ? "gemm_q4k" : fmt == 5 ? "gemm_q5k" : "gemm_q6k";
+  int rc = check_kq(name, x, x_scale, w, out, out_dtype, M, N, K);
+  if (rc != SL8_OK || M == 0 || N == 0 || K == 0) return rc;
+  if (M <= 16)
+    return fmt == 4 ? sl8_gemm_q4k(x, x_scale, w, out, out_dtype, M, N, K, stream)
+         : fmt == 5 ? sl8_gemm_q5k(x, x_scale, w, out, out_dtype, M, N, K, stream)
+                    : sl8_gemm_q6k(x, x_scale, w, out, out_dtype, M, N, K, stream);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const size_t need = sl8_gemm_kq_workspace(fmt, M, N, K);
+  if (!(workspace && workspace_bytes >= need && aligned(workspace, 16))) workspace = nullptr;
+  if (fmt == 6) {
+    const TilePlan p = plan_q6_tile((int)M, (int)N, (int)K, workspace != nullptr);
+    launch_q6_tile(p, x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K,
+                   static_cast<float*>(workspace), st);
+  } else {
+    launch_q45_tile(fmt, x, SL8_KQ_I8, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K, workspace, st);
+  }
+  SL8_CHECK_LAUNCH(name);
+  return SL8_OK;
+}
+
+extern "C" int sl8_linear_kq(int fmt, const void* x, int x_dtype, const uint8_t* w, void* out,
+                             int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace,
+                             size_t workspace_bytes, void* stream) {
+  clear_error();
+  SL8_CHECK_ARG(fmt == 4 || fmt == 5, "linear_kq: fmt must be 4 or 5, got %d", fmt);
+  SL8_CHECK_ARG(x_dtype == SL8_DTYPE_F16 || x_dtype == SL8_DTYPE_BF16,
+                "linear_kq: x must be float16 or bfloat16");
+  SL8_CHECK_ARG(M > 16, "linear_kq: M must be above 16, got %lld", (long long)M);
+  // (x stands in for the scales, which this call makes)
+  int rc = check_kq("linear_kq", static_cast<const int8_t*>(x), static_cast<const float*>(x), w, out,
+                    out_dtype, M, N, K);
+  if (rc != SL8_OK || N == 0 || K == 0) return rc;
+  const size_t need = sl8_gemm_kq_workspace(fmt, M, N, K);
+  SL8_CHECK_ARG(workspace && workspace_bytes >= need && aligned(workspace, 16),
+                "linear_kq: workspace needs %zu bytes", need);
+  launch_q45_tile(fmt, x, x_dtype, nullptr, w, out, out_dtype, (int)M, (int)N, (int)K, workspace,
+                  static_cast<hipStream_t>(stream));
+  SL8_CHECK_LAUNCH("linear_kq");
+  return SL8_OK;
+}
 
 extern "C" int sl8_gemm_q5k(const int8_t* x, const float* x_scale, const uint8_t* w, void* out,
                             int out_dtype, int64_t M, int64_t N, int64_t K, void* stream) {
@@ -1104,8 +907,7 @@ extern "C" int sl8_gemm_q5k(const int8_t* x, const float* x_scale, const uint8_t
   if (rc != SL8_OK || M == 0 || N == 0 || K == 0) return rc;
   if (M <= 16) launch_gemv_kq<5>(x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K,
                                  static_cast<hipStream_t>(stream));
-  else launch_kq_tile<5>(x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K,
-                    static_cast<hipStream_t>(stream));
+  else return sl8_gemm_kq(5, x, x_scale, w, out, out_dtype, M, N, K, nullptr, 0, stream);
   SL8_CHECK_LAUNCH("gemm_q5k");
   return SL8_OK;
 }
@@ -1117,8 +919,7 @@ extern "C" int sl8_gemm_q6k(const int8_t* x, const float* x_scale, const uint8_t
   if (rc != SL8_OK || M == 0 || N == 0 || K == 0) return rc;
   if (M <= 16) launch_gemv_kq<6>(x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K,
                                  static_cast<hipStream_t>(stream));
-  else launch_kq_tile<6>(x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K,
-                    static_cast<hipStream_t>(stream));
+  else return sl8_gemm_kq(6, x, x_scale, w, out, out_dtype, M, N, K, nullptr, 0, stream);
   SL8_CHECK_LAUNCH("gemm_q6k");
   return SL8_OK;
 }

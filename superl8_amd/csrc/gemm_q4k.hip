@@ -570,294 +570,6 @@ gemv_q4k_small_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_
   }
 }
 
-// ---------------------------------------------------------------------------
-// Tiled Q4_K GEMM for M > 16 (prefill; reference csrc/include/gemm_q4k_dp4a.cuh:
-// 60-199, csrc/kernel/gemm_dp4a.cu:146-193): a 128 x 128 output tile per
-// workgroup of 8 waves, two per SIMD, each owning 32 output columns x 64 rows
-// (2 blocks of 32 x 32; each B operand is built by the two waves of its
-// columns: with 4 waves over all 128 rows, one per SIMD, a single wave's VALU
-// issue rate bounded the kernel). Per super-block the
-// x tile (128 x 256 int8) and the 128 weight super-blocks (144 B each) are
-// copied global -> LDS one super-block ahead (double-buffered). The products
-// stay exact integers on v_mfma_i32_32x32x32_i8, one MFMA per 32-element
-// sub-block j (K = 32):
-//   T_j = <x_j, q_j * sc_j> with the 6-bit sc_j split in 3-bit halves so each
-//         B operand fits int8: q * (sc & 7) and q * (sc >> 3) (<= 105; one
-//         32-bit multiply scales 4 nibbles at once, no carries), combined as
-//         T_lo + 8 T_hi;
-// and once per super-block f += d * (T_lo + 8 T_hi) (fp32). The min term
-//   U = sum_j m_j * sum(x_j) is one v_mfma_f32_32x32x16_f16 per row block and
-// super-block on the x half-sums and the mins (both exact in fp16; U is an
-// exact fp32 integer), applied as f -= dmin * U one super-block later (the
-// half-sums of the tile's rows are formed once, spread over the waves, and
-// shared through LDS).
-// x chunks are XOR-swizzled in LDS by row (rows are 256 B = one bank line);
-// weight rows are 144 B apart, which already spreads 16 rows over all banks.
-// ---------------------------------------------------------------------------
-// SL8_KQ_NW8=0: the full tiles on 4 waves (one per SIMD, RB = 4)
-#ifndef SL8_KQ_NW8
-#define SL8_KQ_NW8 1
-#endif
-constexpr int TBM = 128, TBN = 128;  // output tile
-
-template <int OUT_DT, int RB, int NW = 4>
-__global__ void __launch_bounds__(64 * NW, 1)
-gemm_q4k_tile_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_scale,
-                     const uint8_t* __restrict__ w, void* __restrict__ out, int M, int N, int K,
-                     int nt_x, int xcd_m, int tile0) {
-  // RB row blocks (32 rows) per wave, NW waves per workgroup: a full tile is
-  // RB = 4, NW = 4 (one wave per SIMD, every wave over all 128 rows) or RB = 2,
-  // NW = 8 (two waves per SIMD, each over 64 rows); RB = 1, NW = 4 is a row
-  // quarter of a tile (the short last round)
-  constexpr bool QTR = RB * NW < 16;
-  constexpr int NT = 64 * NW;
-  constexpr int WCH = (TBN * 9 + NT - 1) / NT * NT;  // weight-tile 16-B chunks, whole copies
-  __shared__ __attribute__((aligned(16))) int8_t xs0[TBM * 256];
-  __shared__ __attribute__((aligned(16))) int8_t xs1[TBM * 256];
-  __shared__ __attribute__((aligned(16))) uint8_t ws0[WCH * 16];
-  __shared__ __attribute__((aligned(16))) uint8_t ws1[WCH * 16];
-  // full tiles: the fp16 A operands of the min-term MFMA (x half-sums) of one
-  // super-block, [slot][row block][lane], formed by the waves together and
-  // read after the next workgroup barrier
-  __shared__ __attribute__((aligned(16))) uint4 xh_l[QTR ? 1 : 2][QTR ? 1 : 4][64];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, h = lane >> 5;
-  // full tiles: one 128 x 128 tile per workgroup (tiles tile0, tile0 + 1, ...);
-  // quarters: the quarter blockIdx.x & 3 (32 rows) of tile tile0 + blockIdx.x / 4,
-  // so a short last round of tiles spreads over 4x the workgroups
-  const int tile = tile0 + (QTR ? (int)(blockIdx.x >> 2) : (int)blockIdx.x);
-  int ct, rt;
-  kq_tile_coords(tile, nt_x, xcd_m, ct, rt);
-  const int n0 = ct * TBN, m0 = rt * TBM;
-  const int rb0 = QTR ? (int)(blockIdx.x & 3) : 0;
-  const int cg = wave & 3;                                  // the wave's 32 output columns
-  const int rbw = QTR ? rb0 : (NW == 8 ? (wave >> 2) * RB : 0);  // its first row block
-  const int nsb = K >> 8;
-  const int64_t row_bytes = (int64_t)nsb * Q4K_BYTES;
-
-  // copies of super-block sb into (xd, wd); chunk P of the tile lands at P*16
-  auto load = [&](int sb, int8_t* xd, uint8_t* wd) __attribute__((always_inline)) {
-    constexpr int XCH = QTR ? 512 : TBM * 16;  // a quarter copies only its 32 rows
-#pragma unroll
-    for (int i = 0; i < XCH / NT; ++i) {
-      const int P0 = (QTR ? rb0 * 512 : 0) + i * NT;
-      const int P = P0 + tid, row = P >> 4;
-      const int c = (P & 15) ^ (row & 15);
-      const int8_t* src = x + (int64_t)min(m0 + row, M - 1) * K + (int64_t)sb * 256 + 16 * c;
-      __builtin_amdgcn_global_load_lds((q4_gptr_t)src, (q4_lptr_t)(xd + (P0 + wave * 64) * 16), 16, 0, 0);
-    }
-#pragma unroll
-    for (int i = 0; i < WCH / NT; ++i) {
-      const int P = min(i * NT + tid, TBN * 9 - 1), row = P / 9, c = P - 9 * row;
-      const uint8_t* src = w + (int64_t)min(n0 + row, N - 1) * row_bytes + (int64_t)sb * Q4K_BYTES + 16 * c;
-      __builtin_amdgcn_global_load_lds((q4_gptr_t)src, (q4_lptr_t)(wd + (i * NT + wave * 64) * 16), 16, 0, 0);
-    }
-  };
-
-  typedef int v16i_t __attribute__((ext_vector_type(16)));
-  typedef float v16f_t __attribute__((ext_vector_type(16)));
-  // wave (cg, row group) owns weight rows 32 cg .. 32 cg + 31 (output columns)
-  // for the activation rows of its RB row blocks. K step j of a super-block is
-  // sub-block j (lane half h holds its elements 16 h .. 16 h + 15); step j + 1's
-  // A reads and B operands are formed while step j's MFMAs run (one
-  // scheduling region per step).
-  float f[RB][16];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) f[rb][e] = 0.f;
-
-  // Min term U = sum_j m_j * xsum_j on one v_mfma_f32_32x32x16_f16 per row
-  // block and super-block: A = the 16-element half-sums of x (k = 8 h + j,
-  // |sum| <= 16 * 127 = 2032: exact in fp16), B = m_j (6-bit, exact) for both
-  // halves, so U comes out as an exact fp32 integer (|U| <= 8 * 4064 * 63 <
-  // 2^24). In a full tile the half-sums of the 4 row blocks are formed once
-  // (NW = 4: wave w sums row block w; NW = 8: wave w row block w & 3, sub-blocks
-  // 4 (w >> 2) .. +3) and published in LDS; every wave reads its row blocks'
-  // after the next super-block's barrier, so U of super-block sb is formed
-  // (and f -= dmin * U applied) one super-block late. Quarter waves share their
-  // rows and form their operand themselves, and apply U just as late, so the
-  // quarter launch's per-element arithmetic stays that of the full tiles.
-  float u_dmin = 0.f;  // dmin of the super-block whose U is pending
-  v8h u_b = {}, u_a = {};  // its m_j operand and (quarters) its half-sum operand
-  auto u_step = [&](int slot) __attribute__((always_inline)) {
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb) {
-      const v8h a = QTR ? u_a : __builtin_bit_cast(v8h, xh_l[slot][rbw + rb][lane]);
-      const v16f_t u = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, u_b, v16f_t{}, 0, 0, 0);
-#pragma unroll
-      for (int e = 0; e < 16; ++e) f[rb][e] -= u_dmin * u[e];
-    }
-  };
-  // the half-sums this wave forms: row block urb, sub-blocks ju0 .. ju0 + JN - 1
-  constexpr int JN = (NW == 8 && !QTR) ? 4 : 8;
-  const int urb = QTR ? rb0 : (wave & 3);
-  const int ju0 = (NW == 8 && !QTR) ? 4 * (wave >> 2) : 0;
-  const int urow = 32 * urb + l32;
-
-  auto compute = [&](const int8_t* xt, const uint8_t* wt, int slot) __attribute__((always_inline)) {
-    const uint8_t* wr = wt + (32 * cg + l32) * Q4K_BYTES;
-    const uint4 hd = *reinterpret_cast<const uint4*>(wr);
-    const float d = h2f(hd.x & 0xFFFFu), dmin = h2f(hd.x >> 16);
-    const ScMin sm = unpack_scmin(hd.y, hd.z, hd.w);
-    uint32_t qw[4][4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const uint4 qv = *reinterpret_cast<const uint4*>(wr + 16 + 32 * g + 16 * h);
-      qw[g][0] = qv.x; qw[g][1] = qv.y; qw[g][2] = qv.z; qw[g][3] = qv.w;
-    }
-    float hsum[8];
-    v4i A[2][RB], bl[2], bh[2];
-    auto read_a = [&](int j, int buf) __attribute__((always_inline)) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const int row = 32 * (rbw + rb) + l32;
-        A[buf][rb] = *reinterpret_cast<const v4i*>(xt + row * 256 + 16 * ((2 * j + h) ^ (row & 15)));
-      }
-    };
-    // half-sum of sub-block ju0 + jj (jj < JN) of this lane's row urow, half h
-    auto xsum_half = [&](int jj) __attribute__((always_inline)) {
-      const int j = ju0 + jj;
-      const v4i xv = QTR ? A[jj & 1][0]
-                         : *reinterpret_cast<const v4i*>(xt + urow * 256 + 16 * ((2 * j + h) ^ (urow & 15)));
-      int sacc = __builtin_amdgcn_sdot4(xv[0], 0x01010101, 0, false);
-      sacc = __builtin_amdgcn_sdot4(xv[1], 0x01010101, sacc, false);
-      sacc = __builtin_amdgcn_sdot4(xv[2], 0x01010101, sacc, false);
-      sacc = __builtin_amdgcn_sdot4(xv[3], 0x01010101, sacc, false);
-      hsum[jj] = (float)sacc;
-    };
-    auto build = [&](int j, int buf) __attribute__((always_inline)) {
-      const uint32_t scw = j < 4 ? sm.sc_lo : sm.sc_hi;
-      const uint32_t sc = (scw >> (8 * (j & 3))) & 0xFF;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t nib = (qw[j >> 1][e] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
-        bl[buf][e] = (int)mul_bytes(nib, sc & 7);  // <= 15 * 7 per byte
-        bh[buf][e] = (int)mul_bytes(nib, sc >> 3);
-      }
-    };
-    v16i_t tl[RB], th[RB];
-    read_a(0, 0);
-    build(0, 0);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int c = j & 1;
-      __builtin_amdgcn_sched_barrier(0);
-      if (j < 7) read_a(j + 1, c ^ 1);
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        if (j == 0) {
-          tl[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bl[c], v16i_t{}, 0, 0, 0);
-          th[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bh[c], v16i_t{}, 0, 0, 0);
-        } else {
-          tl[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bl[c], tl[rb], 0, 0, 0);
-          th[rb] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[c][rb], bh[c], th[rb], 0, 0, 0);
-        }
-      }
-      // the half-sums: a quarter wave sums step j's own A operand; in a full
-      // tile this wave's JN sub-blocks are spread over the steps
-      if constexpr (JN == 8) xsum_half(j);
-      else if (j & 1) xsum_half(j >> 1);
-      if (j < 7) build(j + 1, c ^ 1);
-      __builtin_amdgcn_sched_group_barrier(0x100, RB + (QTR ? 0 : 1), 0);  // the LDS reads first
-#pragma unroll
-      for (int k = 0; k < 2 * RB; ++k) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, RB == 4 ? 4 : 8, 0);  // VALU
-      }
-    }
-    // the min-term operands of this super-block
-    v8h ub;
-#pragma unroll
-    for (int jj = 0; jj < 8; ++jj)
-      ub[jj] = (_Float16)(float)(((jj < 4 ? sm.mn_lo : sm.mn_hi) >> (8 * (jj & 3))) & 0xFF);
-#pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) f[rb][e] += d * (float)(tl[rb][e] + (th[rb][e] << 3));
-    // the previous super-block's U (in a full tile its operands were published
-    // before the barrier this compute follows), then this one's goes pending;
-    // both launches apply the same operations in the same order
-    if (slot >= 0) u_step(slot ^ 1);
-    if constexpr (QTR) {
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) u_a[jj] = (_Float16)hsum[jj];
-    } else if constexpr (JN == 8) {
-      v8h ua;
-#pragma unroll
-      for (int jj = 0; jj < 8; ++jj) ua[jj] = (_Float16)hsum[jj];
-      xh_l[slot & 1][urb][lane] = __builtin_bit_cast(uint4, ua);
-    } else {
-      typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-      v4h ua;
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) ua[jj] = (_Float16)hsum[jj];
-      reinterpret_cast<uint2*>(&xh_l[slot & 1][urb][lane])[ju0 >> 2] = __builtin_bit_cast(uint2, ua);
-    }
-    u_dmin = dmin;
-    u_b = ub;
-  };
-
-  load(0, xs0, ws0);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-  __syncthreads();
-  // slot: the LDS slot this super-block's half-sums go to (full tiles); -2
-  // for the first super-block (no U pending yet, slot 0)
-  int sb = 0;
-  for (; sb + 1 < nsb; sb += 2) {
-    load(sb + 1, xs1, ws1);
-    compute(xs0, ws0, sb == 0 ? -2 : 0);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (sb + 2 < nsb) load(sb + 2, xs0, ws0);
-    compute(xs1, ws1, 1);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  }
-  if (sb < nsb) {
-    compute(xs0, ws0, sb == 0 ? -2 : 0);
-    if constexpr (!QTR) __syncthreads();
-  }
-  u_step((nsb - 1) & 1);  // the last super-block's U
-
-  const int n = n0 + 32 * cg + l32;
-  // the row scales first, unconditionally (clamped rows): one wait, not one per element
-  float xsv[RB][16];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int e = 0; e < 16; ++e)
-      xsv[rb][e] = x_scale[min(m0 + 32 * (rbw + rb) + 8 * (e >> 2) + 4 * h + (e & 3), M - 1)];
-#pragma unroll
-  for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int m = m0 + 32 * (rbw + rb) + 8 * (e >> 2) + 4 * h + (e & 3);
-      if (m < M && n < N) st_out<OUT_DT>(out, (int64_t)m * N + n, f[rb][e] * xsv[rb][e]);
-    }
-}
-
-void launch_gemm_tile(const int8_t* x, const float* xs, const uint8_t* w, void* out, int odt,
-                      int M, int N, int K, hipStream_t st) {
-  // one workgroup per 128 x 128 tile; when the last round of tiles would hold
-  // at most half the CUs, those tiles run as 4 row quarters each (a second
-  // launch), which shortens that round (same per-element arithmetic)
-  const int ntx = (N + TBN - 1) / TBN, T = ntx * ((M + TBM - 1) / TBM), P = cu_count();
-  const int rem = T % P, nfull = (T >= P && rem > 0 && rem <= P / 2) ? T - rem : T;
-  // XCD-aware tile order (kq_tile_coords) when the column tiles split evenly over the 8 XCDs
-  const int xm = (SL8_KQ_XCD && ntx % 8 == 0) ? (M + TBM - 1) / TBM : 0;
-#define SL8_Q4T(RB, NW, G, T0)                                                                              \
-  switch (odt) {                                                                                            \
-    case SL8_DTYPE_F16: gemm_q4k_tile_kernel<SL8_DTYPE_F16, RB, NW><<<G, 64 * NW, 0, st>>>(x, xs, w, out, M, N, K, ntx, xm, T0); break; \
-    case SL8_DTYPE_BF16: gemm_q4k_tile_kernel<SL8_DTYPE_BF16, RB, NW><<<G, 64 * NW, 0, st>>>(x, xs, w, out, M, N, K, ntx, xm, T0); break; \
-    default: gemm_q4k_tile_kernel<SL8_DTYPE_F32, RB, NW><<<G, 64 * NW, 0, st>>>(x, xs, w, out, M, N, K, ntx, xm, T0); break;        \
-  }
-  if (SL8_KQ_NW8) { SL8_Q4T(2, 8, nfull, 0) } else { SL8_Q4T(4, 4, nfull, 0) }
-  if (nfull < T) SL8_Q4T(1, 4, 4 * (T - nfull), nfull)
-#undef SL8_Q4T
-}
-
 __global__ void dequant_q4k_kernel(const uint8_t* __restrict__ w, float* __restrict__ out,
                                    int64_t N, int K) {
   // one thread per (row, sub-block): 32 outputs
@@ -1030,12 +742,7 @@ extern "C" int sl8_gemm_q4k(const int8_t* x, const float* x_scale, const uint8_t
   SL8_CHECK_ARG(N < (1LL << 31), "gemm_q4k: N too large");
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int esz = out_dtype == SL8_DTYPE_F32 ? 4 : 2;
-  if (M > 16) {
-    SL8_CHECK_ARG(M < (1LL << 31) && (M + TBM - 1) / TBM * ((N + TBN - 1) / TBN) < (1LL << 28), "gemm_q4k: M*N too large");
-    launch_gemm_tile(x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K, st);
-    SL8_CHECK_LAUNCH("gemm_q4k");
-    return SL8_OK;
-  }
+  if (M > 16) return sl8_gemm_kq(4, x, x_scale, w, out, out_dtype, M, N, K, nullptr, 0, stream);
   // M <= 16: one 16-row activation slab through the GEMV MFMA kernel.
   for (int64_t m0 = 0; m0 < M; m0 += 16) {
     const int64_t mt = (M - m0) < 16 ? (M - m0) : 16;

@@ -1,6 +1,8 @@
 // Shared pieces of the GGUF k-quant kernels (Q4_K, Q5_K, Q6_K).
 #pragma once
 
+#include <type_traits>
+
 #include "common.hpp"
 
 #ifndef SL8_KQ_XCD
@@ -57,6 +59,63 @@ void launch_gemv_q5k_small(const int8_t* x, const float* xs, const uint8_t* w, v
 // Q5_K decode GEMV for 3 <= M <= 16 on the int8 MFMA (gemm_q4k.hip)
 void launch_gemv_q5k_mfma(const int8_t* x, const float* xs, const uint8_t* w, void* out, int odt,
                           int M, int N, int K, hipStream_t st);
+
+// Tiled GEMMs (M > 16): a tile shape with the workgroups of it a CU holds and the time one
+// super-block of one takes then, and the plan of a call: tiles [0, nfull) whole, nsplit more
+// tiles split S ways over K into part_bytes of fp32 partials.
+struct TileShape {
+  int bm, bn, wgs_per_cu;
+  double us_per_sb;
+};
+struct TilePlan {
+  int shape, nt_x, S;
+  int64_t nfull, nsplit;
+  size_t part_bytes;
+};
+TilePlan plan_tiles(int M, int N, int K, const TileShape* shapes, int count, bool may_split);
+
+// Which part of the problem a workgroup computes: workgroups below nfull a whole tile, the others
+// a K range of tiles nfull .., S per tile, into part[tile - nfull][split][BM][BN].
+struct TileWork {
+  int nt_x, xcd_m, nfull, S, tile_elems;
+  float* part;
+};
+inline TileWork tile_work(const TilePlan& p, const TileShape& s, int M, float* part) {
+  // XCD-aware tile order (kq_tile_coords) when the column tiles split evenly over the 8 XCDs
+  const int xm = (SL8_KQ_XCD && p.nt_x % 8 == 0) ? (M + s.bm - 1) / s.bm : 0;
+  return TileWork{p.nt_x, xm, (int)p.nfull, p.S, s.bm * s.bn, part};
+}
+struct TileRange {
+  int ct, rt, sb0, sb1, sp;
+  float* part;  // the tile's S partials, null for a whole tile
+};
+__device__ __forceinline__ TileRange tile_range(const TileWork& tw, int nsb) {
+  TileRange r{0, 0, 0, nsb, 0, nullptr};
+  int tile = blockIdx.x;
+  if (tile >= tw.nfull) {
+    const int i = tile - tw.nfull, t = i / tw.S;
+    tile = tw.nfull + t;
+    r.sp = i % tw.S;
+    r.sb0 = r.sp * nsb / tw.S;
+    r.sb1 = (r.sp + 1) * nsb / tw.S;
+    r.part = tw.part + (int64_t)t * tw.S * tw.tile_elems;
+  }
+  kq_tile_coords(tile, tw.nt_x, tw.xcd_m, r.ct, r.rt);
+  return r;
+}
+void launch_kq_reduce(const TilePlan& p, const TileShape& s, const TileWork& tw, const float* xs,
+                      void* out, int odt, int M, int N, hipStream_t st);
+// Q6_K (gemm_kq56.hip)
+TilePlan plan_q6_tile(int M, int N, int K, bool may_split);
+void launch_q6_tile(const TilePlan& p, const int8_t* x, const float* xs, const uint8_t* w, void* out,
+                    int odt, int M, int N, int K, float* part, hipStream_t st);
+// Q4_K / Q5_K (gemm_kq_tile.hip): x int8 codes with their row scales xs (x_dtype SL8_KQ_I8), or
+// fp16 / bf16 rows that are quantised in the call (with a workspace only; 16-byte aligned).
+// workspace: q45_tile_workspace() bytes, or null.
+constexpr int SL8_KQ_I8 = 3;
+size_t q45_tile_workspace(int fmt, int M, int N, int K);
+void launch_q45_tile(int fmt, const void* x, int x_dtype, const float* xs, const uint8_t* w, void* out,
+                     int odt, int M, int N, int K, void* workspace, hipStream_t st);
 
 typedef __attribute__((address_space(1))) const void* kq_gptr_t;
 typedef __attribute__((address_space(3))) void* kq_lptr_t;

@@ -355,14 +355,14 @@ def linear_q4k(x: torch.Tensor, w_bytes: torch.Tensor, *, bias: torch.Tensor | N
                out_dtype: torch.dtype = torch.float16) -> torch.Tensor:
     """GGUF Q4_K linear on native 144-byte super-blocks: x [..., K] -> [..., N]."""
     return _linear_kquant(x, w_bytes, bias, out_dtype, _C.gemm_q4k,
-                          getattr(_C, "gemm_decode_q4k", None))
+                          getattr(_C, "gemm_decode_q4k", None), 4)
 
 
 def linear_q5k(x: torch.Tensor, w_bytes: torch.Tensor, *, bias: torch.Tensor | None = None,
                out_dtype: torch.dtype = torch.float16) -> torch.Tensor:
     """GGUF Q5_K linear on native 176-byte super-blocks (reference ops.py:1328-1336)."""
     return _linear_kquant(x, w_bytes, bias, out_dtype, _C.gemm_q5k,
-                          getattr(_C, "gemm_decode_q5k", None))
+                          getattr(_C, "gemm_decode_q5k", None), 5)
 
 
 def linear_q6k(x: torch.Tensor, w_bytes: torch.Tensor, *, bias: torch.Tensor | None = None,
@@ -388,16 +388,19 @@ def linear(x: torch.Tensor, qt, *, bias: torch.Tensor | None = None,
     raise ValueError(f"superl8.linear: unsupported weight scheme {qt.scheme!r}")
 
 
-def _linear_kquant(x, w_bytes, bias, out_dtype, tile_op, decode_op):
+def _linear_kquant(x, w_bytes, bias, out_dtype, tile_op, decode_op, fmt=None):
     *lead, K = x.shape
     x2 = x.reshape(-1, K).contiguous()
     w_bytes = w_bytes.contiguous()
-    x_i8, x_scale = quantize_i8_rowwise(x2)
     M = x2.shape[0]
-    if decode_op is not None and x2.is_cuda and 0 < M <= _KQUANT_DECODE_MAX_M:
-        y = decode_op(x_i8, x_scale, w_bytes, out_dtype)
+    if M > _KQUANT_DECODE_MAX_M and fmt is not None and _C.linear_kq_ok(x2):  # one call
+        y = _C.linear_kq(fmt, x2, w_bytes, out_dtype)
     else:
-        y = tile_op(x_i8, x_scale, w_bytes, out_dtype)
+        x_i8, x_scale = quantize_i8_rowwise(x2)
+        if decode_op is not None and x2.is_cuda and 0 < M <= _KQUANT_DECODE_MAX_M:
+            y = decode_op(x_i8, x_scale, w_bytes, out_dtype)
+        else:
+            y = tile_op(x_i8, x_scale, w_bytes, out_dtype)
     if bias is not None:
         y = (y.float() + bias.float()).to(y.dtype)
     return y.reshape(*lead, y.shape[-1])

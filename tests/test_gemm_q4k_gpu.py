@@ -215,3 +215,54 @@ def test_gemv_per_row_scale_shaped_m1(device, M):
     assert (err <= 1e-5 * np.abs(ref) + 1e-5 * np.abs(ref).max()).all()
     with pytest.raises(RuntimeError, match=r"\[M\] \(per row\) or \[M, K/256\]"):
         _C.gemm_decode_q4k(x_i8, torch.ones(M, 3, device=device), wd, torch.float32)
+
+
+# Every tile shape of the Q4_K / Q5_K tile GEMM (32, 64, 128 rows), whole and split over K (few
+# tiles; odd counts of super-blocks, which split unevenly), with ragged rows and columns
+SHAPES_KQ = [(17, 40, 2304), (33, 130, 5120), (64, 1000, 2304), (65, 257, 1280), (129, 4100, 768),
+             (300, 600, 3328), (200, 4096, 512)]
+
+
+@pytest.mark.parametrize("fmt", [4, 5])
+@pytest.mark.parametrize("M,N,K", SHAPES_KQ)
+def test_tile_shapes_and_splits(device, fmt, M, N, K):
+    """Against the exact integer sums: fp32 accumulation over K / 256 super-blocks and splits
+    (2^-24 relative to the partial sums per step)."""
+    from oracle import kquant as okq
+    from superl8_amd import _lib
+
+    gen, ref_fn = (oq.random_weights, oq.gemv) if fmt == 4 else (okq.q5k_random, okq.q5k_gemv)
+    w = gen(N, K, seed=M + N)
+    wd = torch.from_numpy(w).to(device)
+    g = torch.Generator(device="cpu").manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(device)
+    x_i8, xs = _C.quantize_i8_rowwise(x.half())
+    ref = np.concatenate([ref_fn(_np(x_i8), _np(xs), w[n:n + 512], K) for n in range(0, N, 512)], axis=1)
+    tol = 1e-5 * np.abs(ref) + 1e-5 * np.abs(ref).max()
+    y = (_C.gemm_q4k if fmt == 4 else _C.gemm_q5k)(x_i8, xs, wd, torch.float32)
+    assert (np.abs(_np(y).astype(np.float64) - ref) <= tol).all()
+    # the C entry without scratch: int8 codes through registers, whole tiles
+    out = torch.empty(M, N, device=device, dtype=torch.float32)
+    lib = _lib.load()
+    rc = getattr(lib, f"sl8_gemm_q{fmt}k")(x_i8.data_ptr(), xs.data_ptr(), wd.data_ptr(), out.data_ptr(),
+                                           2, M, N, K, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, lib.sl8_last_error()
+    assert (np.abs(_np(out).astype(np.float64) - ref) <= tol).all()
+    # the fused linear from 16-bit rows: the same codes, scales and sums, bit for bit
+    for dt in (torch.float16, torch.bfloat16):
+        xd = x.to(dt)
+        c, s = _C.quantize_i8_rowwise(xd)
+        assert torch.equal(_C.linear_kq(fmt, xd, wd, torch.float32),
+                           (_C.gemm_q4k if fmt == 4 else _C.gemm_q5k)(c, s, wd, torch.float32))
+
+
+@pytest.mark.parametrize("K", [2048, 2304, 4352, 8448, 16640, 33024])
+def test_linear_kq_row_lengths(device, K):
+    """The fused linear's row preparation around its thread and vector counts."""
+    M, N = 18, 24
+    wd = torch.from_numpy(oq.random_weights(N, K, seed=K)).to(device)
+    x = torch.randn(M, K, device=device, dtype=torch.float16)
+    x[0] = 0
+    x[1, K - 1] = 60.0
+    c, s = _C.quantize_i8_rowwise(x)
+    assert torch.equal(_C.linear_kq(4, x, wd, torch.float32), _C.gemm_q4k(c, s, wd, torch.float32))

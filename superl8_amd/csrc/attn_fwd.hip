@@ -33,6 +33,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "attn_common.hpp"
 
@@ -168,6 +169,8 @@ struct FwdArgs {
   int xcd_map;         // xcd_mode(): XCD-aware block order
   float w8_excess;     // W8A8: headroom of P above the reference point (log2)
   int dout;            // output row length (= D, or the caller's head dim when D is padded)
+  int paired;          // causal: a workgroup takes query blocks nqb-1-slot and slot, one after the other
+  int fold;            // not paired: slots from here on count their query block up from 0
   const int32_t* skip; // production kernel: nonzero *skip -> every workgroup exits at once
 };
 
@@ -187,9 +190,9 @@ struct QOp {
 
 // ---------------------------------------------------------------------------
 // Production kernel. A wave owns NG x 32 queries (NG = 1: one MFMA column
-// block) for the whole key loop; WV waves per workgroup (8 for D = 128, 4 for
-// D = 64, halved down to 2 while the grid is smaller than the CU count; two
-// waves per SIMD) share each 64-key K / k_scale / V^T tile, copied
+// block) for the whole key loop; WV waves per workgroup (8 or 4 for D = 128, 4 for
+// D = 64 and 256: fwd_geometry; up to two waves per SIMD) share each 64-key K / k_scale / V^T
+// tile, copied
 // global -> LDS one tile ahead, so a larger workgroup means fewer copies per
 // query. Each tile is processed as two 32-key half-steps; half-step h issues
 // QK of half h and PV of half h-2 on the matrix cores while the VALU does the
@@ -200,6 +203,10 @@ struct QOp {
 // operand reads (1 KB per MFMA), ~7 VALU operations per score.
 // ---------------------------------------------------------------------------
 
+// W8A8 at D = 256: 16 queries per wave (attn_w8a8_q16_kernel)
+#ifndef SL8_W8_Q16
+#define SL8_W8_Q16 1
+#endif
 #ifndef SL8_FWD_FAST
 #define SL8_FWD_FAST 1
 #endif
@@ -253,7 +260,7 @@ attn_fwd_wide_kernel(const FwdArgs a) {
   using PV = PvOp<VDT>;
   typedef typename PV::vec pvec;
 
-  const int nslot = CAUSAL ? (a.nqb + 1) / 2 : a.nqb;
+  const int nslot = CAUSAL && a.paired ? (a.nqb + 1) / 2 : a.nqb;
   int bh, slot;
   block_coords(a, nslot, bh, slot);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -274,9 +281,9 @@ attn_fwd_wide_kernel(const FwdArgs a) {
 
   int qbs[2];
   int npass = 1;
-  qbs[0] = a.nqb - 1 - slot;
+  qbs[0] = slot < a.fold ? a.nqb - 1 - slot : slot - a.fold;
   qbs[1] = slot;
-  if (CAUSAL) npass = (qbs[1] != qbs[0]) ? 2 : 1;
+  if (CAUSAL && a.paired) npass = (qbs[1] != qbs[0]) ? 2 : 1;
 
   constexpr int KCPR = D / 16;
   // LDS has 64 four-byte banks (256 B): 16 lanes of a 16-byte read cover 16
@@ -1185,24 +1192,78 @@ void launch_wide(const FwdArgs& a, int grid, hipStream_t st) {
   attn_fwd_wide_kernel<D, CAUSAL, VDT, LSE, wide_ng(D), WV, W8><<<grid, WV * 64, 0, st>>>(a);
 }
 
-// Small grids (short sequences, few heads): fewer waves per workgroup, i.e.
-// fewer queries per workgroup and more workgroups, until the grid covers the
-// CUs (the waves per SIMD stay 2: see the launch bounds). D = 128: 8, 4 or 2
-// waves; D = 64: 4 or 2; D = 256 keeps 4.
-#ifndef SL8_FWD_SMALLGRID
-#define SL8_FWD_SMALLGRID 1
-#endif
-int wide_waves_for(int64_t DP, int64_t B, int64_t Hq, int64_t M, bool causal) {
-  int wv = wide_waves(DP);
-  if (!SL8_FWD_SMALLGRID || (DP != 128 && DP != 64) || wide_ng(DP) != 1) return wv;
+// Launch geometry of a prefill: waves per workgroup (they share every tile copy), and for causal
+// launches which query blocks a workgroup takes: a heavy and a light one in turn (paired: equal
+// workgroups, half as many), or one, the heaviest blocks first.
+//
+// A wave alone on its SIMD runs a 64-key tile in about 1.15 us, two in about 2.0 us together
+// (D = 128), so idle SIMDs and a second pass's fill and drain cost more than narrower workgroups
+// do. Wide and paired launches are faster only where they come out even on the CUs. Call times
+// at D = 128, fp16 V, 32 heads, causal, in us (queries x keys):
+//                         paired, 8 waves   paired, 4   one block, 8   one block, 4
+//   512 x 512                        32.7        22.7           20.8           16.2
+//   2048 x 2048                      62.7        47.3           52.6           45.3 (folded 43.7)
+//   4096 x 4096 (even)              119.6       121.1          120.8          125.3
+//   4500 x 4500                       234         198            160            151
+//   8192 x 8192 (even)                435         442            435            443
+//   1000 x 6121                       245         181            131            101
+//   4096 x 12288 (even)               518         533            513            528
+//   3000, window 1024                74.4        64.8           69.1           57.1
+struct FwdGeom {
+  int wv;
+  bool paired;
+  bool folded;  // one block each, all resident: the second workgroup of a CU light to heavy
+};
+struct FwdKernel {
+  int wave_q;          // queries per wave
+  int wide, narrow;    // waves per workgroup of its instantiations (equal: there is one)
+  int cap;             // workgroups of the narrow one that fit a CU (of the wide one: 1)
+};
+// D = 64: 4 waves. D = 128: 8 or 4; W8A8 4 (at every size measured 4 to 15 % faster than 8).
+// D = 256: 4, a CU's LDS full; its W8A8 kernel (16 queries per wave) 8 or 4.
+FwdKernel fwd_kernel(int64_t D, bool w8) {
+  if (D == 64) return {32, 4, 4, 2};
+  if (D == 128) return {32, w8 ? 4 : 8, 4, 2};
+  if (w8 && SL8_W8_Q16) return {16, 8, 4, 1};
+  return {32 * wide_ng(256), 4, 4, 1};
+}
+
+FwdGeom fwd_geometry(const FwdKernel& kn, int64_t heads, int64_t M, int64_t N, bool causal,
+                     int64_t window_left) {
   const int64_t cus = cu_count();
-  while (wv > 2) {
-    const int64_t bm = (int64_t)wv * 32, nqb = (M + bm - 1) / bm;
-    const int64_t grid = B * Hq * (causal ? (nqb + 1) / 2 : nqb);
-    if (grid >= cus) break;
-    wv /= 2;
+  // the blocks' costs differ (no long prefix, no window that evens them out)
+  const bool windowed = window_left >= 0 && 2 * window_left <= N;
+  const bool ramp = causal && 2 * M > N, skewed = ramp && !windowed;
+  auto grid = [&](int wv, bool paired) {
+    const int64_t nqb = (M + wv * kn.wave_q - 1) / (wv * kn.wave_q);
+    return heads * (paired ? (nqb + 1) / 2 : nqb);
+  };
+  // comes out even: rows in use, of those that the rounds of cap workgroups per CU hold
+  auto even = [&](int wv, bool paired, int64_t cap) {
+    const int64_t rounds = (grid(wv, paired) + cus * cap - 1) / (cus * cap);
+    return heads * M >= 0.9 * (double)(rounds * cus * cap * (paired ? 2 : 1) * wv * kn.wave_q);
+  };
+  if (kn.wide != kn.narrow) {
+    // D = 128: wide where it is even, but for windows, whose edges mask more of a wider block.
+    // D = 256 W8A8: a CU holds one workgroup of either, narrow ones as long as they take one round
+    // (heads x queries 16 x 600: 30.9 against 33.9 us, 16 x 4096: 227 / 152), or, when the second
+    // round's are the short ones, up to 7/4 (16 x 1536: 52 / 60; 32 x 1024, two rounds: 51 / 48)
+    const bool wide = kn.cap == 1 ? 4 * grid(kn.narrow, false) > (skewed ? 7 : 4) * cus
+                                  : !windowed && even(kn.wide, skewed, 1);
+    if (wide) return {kn.wide, skewed && even(kn.wide, true, 1), false};
   }
-  return wv;
+  // Two workgroups to a CU: pairs only as one even round (D = 64, 16 heads x 8192: 193 us against
+  // 199; 32 heads, two rounds: 377 / 369), then with windows too (D = 128, 32 x 4096, window 512:
+  // 49 / 53)
+  const int64_t pairs = grid(kn.narrow, true), blocks = grid(kn.narrow, false);
+  bool paired = ramp && even(kn.narrow, true, kn.cap) && (kn.cap == 1 || pairs <= cus * kn.cap);
+  // D = 128, one pair to a CU: no wave shares its SIMD, and the second pass is paid back from 4096
+  // keys on (8 heads x 8192: 138 / 146 us; 16 x 4096: 78 / 78; 32 x 2048: 47 / 44)
+  if (kn.wide != kn.narrow && kn.cap > 1 && skewed && N >= 4096 && pairs <= cus &&
+      even(kn.narrow, true, 1))
+    paired = true;
+  const bool folded = causal && !paired && kn.cap > 1 && blocks > cus && blocks <= 2 * cus && heads <= cus;
+  return {kn.narrow, paired, folded};
 }
 
 template <int D, int VDT, int WV>
@@ -1218,12 +1279,8 @@ void dispatch_wide_wv(const FwdArgs& a, int grid, bool causal, bool lse, hipStre
 
 template <int D, int VDT>
 void dispatch_wide(const FwdArgs& a, int grid, bool causal, bool lse, int wv, hipStream_t st) {
-  if constexpr (D == 128) {
-    if (wv == 2) return dispatch_wide_wv<D, VDT, 2>(a, grid, causal, lse, st);
+  if constexpr (wide_waves(D) != 4)
     if (wv == 4) return dispatch_wide_wv<D, VDT, 4>(a, grid, causal, lse, st);
-  } else if constexpr (D == 64) {
-    if (wv == 2) return dispatch_wide_wv<D, VDT, 2>(a, grid, causal, lse, st);
-  }
   dispatch_wide_wv<D, VDT, wide_waves(D)>(a, grid, causal, lse, st);
 }
 
@@ -1242,11 +1299,10 @@ int check_fwd_shape(int64_t B, int64_t Hq, int64_t Hkv, int64_t M, int64_t N, in
 }
 
 // launch geometry of the production kernel for (padded) head dim DP: query
-// blocks of wv x 32 x wide_ng(DP) rows (wv = 0: wide_waves(DP)); causal launches pair block qb with nqb-1-qb, so
-// the grid holds (nqb + 1) / 2 slots per head
+// blocks of geom.wv x wave_q rows; paired launches hold (nqb + 1) / 2 slots per head
 FwdArgs make_args(int64_t B, int64_t Hq, int64_t Hkv, int64_t M, int64_t N, int64_t DP,
-                  bool causal, int& grid, int wv = 0) {
-  const int bm = (wv > 0 ? wv : wide_waves(DP)) * 32 * wide_ng(DP);
+                  bool causal, int& grid, const FwdGeom& geom, int wave_q) {
+  const int bm = geom.wv * wave_q;
   FwdArgs a{};
   a.M = (int)M;
   a.N = (int)N;
@@ -1257,7 +1313,9 @@ FwdArgs make_args(int64_t B, int64_t Hq, int64_t Hkv, int64_t M, int64_t N, int6
   a.window_left = -1;
   a.diag = (int)(N - M);
   a.dout = 0;  // set by the callers
-  const int nslot = causal ? (a.nqb + 1) / 2 : a.nqb;
+  a.paired = geom.paired;
+  a.fold = geom.folded ? (int)(cu_count() / (B * Hq)) : a.nqb;  // slots of the first round
+  const int nslot = geom.paired ? (a.nqb + 1) / 2 : a.nqb;
   grid = (int)(B * Hq * nslot);
   a.xcd_map = xcd_mode(B * Hkv, Hq / Hkv, nslot);
   return a;
@@ -1409,9 +1467,6 @@ int w8a8_pad_operands(const int8_t*& q, const int8_t*& k, const int8_t*& v, cons
 // so is the straight-line half-step. Config 5: 1081 -> 986 us (the same
 // kernel with the compiler's schedule, each operand read right before its
 // MFMA: 1633 us). SL8_W8_Q16 = 0 runs attn_fwd_wide_kernel's W8A8 path.
-#ifndef SL8_W8_Q16
-#define SL8_W8_Q16 1
-#endif
 #ifndef SL8_Q16_PD
 #define SL8_Q16_PD 4  // operand reads ahead of their MFMA (2 / 3 / 4 / 6 at config 5: 972 / 969 / 963 / 967 us)
 #endif
@@ -1419,11 +1474,11 @@ typedef float v4f_t __attribute__((ext_vector_type(4)));
 
 namespace {
 
-template <bool CAUSAL>
-__global__ void __launch_bounds__(512, 1)
+template <bool CAUSAL, int WV>
+__global__ void __launch_bounds__(64 * WV, 1)
 attn_w8a8_q16_kernel(const FwdArgs a) {
   if (a.skip != nullptr && *a.skip != 0) return;
-  constexpr int D = 256, WT = 512, WQ = 16, WBM = 128;
+  constexpr int D = 256, WT = 64 * WV, WQ = 16, WBM = WV * WQ;
   constexpr int KCH = BN * D / 16 / WT;      // K tile copies per thread
   constexpr int VCH = D * BN * 2 / 16 / WT;  // V^T tile copies per thread
   constexpr float LOG2_127 = 6.988684686772166f;
@@ -1434,7 +1489,7 @@ attn_w8a8_q16_kernel(const FwdArgs a) {
   __shared__ __attribute__((aligned(16))) float ss0[BN];
   __shared__ __attribute__((aligned(16))) float ss1[BN];
 
-  const int nslot = CAUSAL ? (a.nqb + 1) / 2 : a.nqb;
+  const int nslot = CAUSAL && a.paired ? (a.nqb + 1) / 2 : a.nqb;
   int bh, slot;
   block_coords(a, nslot, bh, slot);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1452,9 +1507,9 @@ attn_w8a8_q16_kernel(const FwdArgs a) {
 
   int qbs[2];
   int npass = 1;
-  qbs[0] = a.nqb - 1 - slot;
+  qbs[0] = slot < a.fold ? a.nqb - 1 - slot : slot - a.fold;
   qbs[1] = slot;
-  if (CAUSAL) npass = (qbs[1] != qbs[0]) ? 2 : 1;
+  if (CAUSAL && a.paired) npass = (qbs[1] != qbs[0]) ? 2 : 1;
 
   // K operand (A, 16 keys x 64 dims): lane (l16, g) reads the 16-byte chunk
   // 4 c + g of key row l16 of the block; the tile keeps chunk c of row r at
@@ -1781,26 +1836,31 @@ int w8a8_wide_launch(const int8_t* q, const float* q_scale, const int8_t* k, con
     SL8_CHECK_LAUNCH("attn_w8a8_fwd v to bf16 V^T");
   }
   int grid;
-  FwdArgs a = make_args(B, Hq, Hkv, M, N, D, causal, grid);
+  const bool q16 = SL8_W8_Q16 && D == 256;
+  const FwdKernel kn = fwd_kernel(D, true);
+  const FwdGeom geom = fwd_geometry(kn, B * Hq, M, N, causal, -1);
+  FwdArgs a = make_args(B, Hq, Hkv, M, N, D, causal, grid, geom, kn.wave_q);
   a.q = q; a.qs = q_scale; a.k = k; a.ks = k_scale;
   a.vt = vt; a.vs = v_scale; a.out = out; a.lse = nullptr;
   a.diag = (int)causal_diag;
   a.dout = (int)dout;
   a.w8_excess = w8_excess_for(N);
   constexpr int F = SL8_DTYPE_BF16;
-  if (SL8_W8_Q16 && D == 256) {
-    if (causal) attn_w8a8_q16_kernel<true><<<grid, 512, 0, st>>>(a);
-    else attn_w8a8_q16_kernel<false><<<grid, 512, 0, st>>>(a);
-  } else if (D == 64) {
-    if (causal) launch_wide<64, true, F, false, true>(a, grid, st);
-    else launch_wide<64, false, F, false, true>(a, grid, st);
-  } else if (D == 128) {
-    if (causal) launch_wide<128, true, F, false, true>(a, grid, st);
-    else launch_wide<128, false, F, false, true>(a, grid, st);
-  } else {
-    if (causal) launch_wide<256, true, F, false, true>(a, grid, st);
-    else launch_wide<256, false, F, false, true>(a, grid, st);
-  }
+  auto wide = [&](auto d) {
+    constexpr int DD = decltype(d)::value;
+    if (causal) launch_wide<DD, true, F, false, true, 4>(a, grid, st);
+    else launch_wide<DD, false, F, false, true, 4>(a, grid, st);
+  };
+  auto q16_waves = [&](auto wv) {
+    constexpr int WV = decltype(wv)::value;
+    if (causal) attn_w8a8_q16_kernel<true, WV><<<grid, 64 * WV, 0, st>>>(a);
+    else attn_w8a8_q16_kernel<false, WV><<<grid, 64 * WV, 0, st>>>(a);
+  };
+  if (q16 && geom.wv == 4) q16_waves(std::integral_constant<int, 4>{});
+  else if (q16) q16_waves(std::integral_constant<int, 8>{});
+  else if (D == 64) wide(std::integral_constant<int, 64>{});
+  else if (D == 128) wide(std::integral_constant<int, 128>{});
+  else wide(std::integral_constant<int, 256>{});
   SL8_CHECK_LAUNCH("attn_w8a8_fwd");
   return SL8_OK;
 }
@@ -1846,8 +1906,10 @@ int attn_int8_fwd_impl(const int8_t* q, const float* q_scale, const int8_t* k,
   }
   const bool c = causal != 0, want_lse = lse != nullptr;
   int grid;
-  const int wv = wide_waves_for(DP, B, Hq, M, c);
-  FwdArgs a = make_args(B, Hq, Hkv, M, N, DP, c, grid, wv);
+  const FwdKernel kn = fwd_kernel(DP, false);
+  const FwdGeom geom = fwd_geometry(kn, B * Hq, M, N, c, window_left);
+  const int wv = geom.wv;
+  FwdArgs a = make_args(B, Hq, Hkv, M, N, DP, c, grid, geom, kn.wave_q);
   a.q = q; a.qs = q_scale; a.k = k; a.ks = k_scale;
   a.vt = static_cast<const uint16_t*>(v);  // V [B*Hkv][N][DP], read in place
   a.out = out; a.lse = lse; a.window_left = (int)window_left;
@@ -1916,7 +1978,7 @@ extern "C" int sl8_attn_int8_qk_scores(const int8_t* q, const int8_t* k, int32_t
   }
   const bool c = causal != 0;
   int grid;
-  FwdArgs a = make_args(B, Hq, Hkv, M, N, DP, c, grid);
+  FwdArgs a = make_args(B, Hq, Hkv, M, N, DP, c, grid, FwdGeom{wide_waves(DP), c, false}, 32 * wide_ng(DP));
   a.q = q; a.k = k; a.scores = scores;
   a.dout = (int)D;
   // V and the scales are never read by the dump instantiation

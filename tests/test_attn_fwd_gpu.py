@@ -362,3 +362,54 @@ def test_small_grid_wave_counts(device, case, vdt):
         # tolerance as test_kernel_matches_oracle: the P rounding of the PV operand
         np.testing.assert_allclose(_np(lse[b:b + 1, h:h + 1]), ref_lse, rtol=0,
                                    atol=5e-4 if f16 else 4e-3)
+
+
+# The launch geometry (waves per workgroup; causal blocks in pairs, heaviest first or folded) follows
+# the sizes; a head's result does not. Each form against the same head launched alone (one
+# narrow workgroup per block), which the oracle tests above cover. Both run the same tiles in the
+# same order per wave, so the results are the same bits.
+GEOMETRIES = [
+    # w8, B, Hq, Hkv, M, N, D, causal, window
+    (False, 4, 32, 8, 1024, 1024, 128, True, -1),    # 8 waves, pairs
+    (False, 4, 32, 8, 500, 500, 128, False, -1),     # 8 waves, one block each
+    (False, 4, 32, 8, 512, 2001, 128, True, -1),     # 8 waves, a long prefix
+    (False, 1, 16, 4, 4096, 4096, 128, True, -1),    # 4 waves, pairs
+    (False, 1, 32, 8, 1100, 1100, 128, True, -1),    # 4 waves, folded
+    (False, 1, 40, 8, 1000, 1000, 128, True, -1),    # 4 waves, folded, heads that do not divide 256
+    (False, 1, 8, 2, 300, 700, 128, True, -1),       # 4 waves, heaviest first
+    (False, 3, 40, 8, 1100, 1100, 128, True, 300),   # 4 waves, window
+    (False, 4, 16, 4, 2048, 2048, 64, True, -1),     # pairs
+    (False, 1, 32, 8, 1100, 1100, 64, True, -1),     # folded
+    (False, 1, 32, 8, 2048, 2048, 256, True, -1),    # pairs
+    (False, 2, 16, 4, 700, 700, 256, True, -1),      # heaviest first
+    (True, 4, 16, 4, 2048, 2048, 128, True, -1),     # W8A8: pairs
+    (True, 1, 32, 8, 1100, 1100, 128, True, -1),     # folded
+    (True, 1, 32, 8, 2048, 2048, 256, True, -1),     # 8 waves, pairs
+    (True, 1, 32, 8, 1030, 1030, 256, True, -1),     # 8 waves, heaviest first
+    (True, 1, 16, 4, 600, 600, 256, True, -1),       # 4 waves
+    (True, 1, 8, 2, 300, 300, 256, False, -1),       # 4 waves, not causal
+]
+
+
+@pytest.mark.parametrize("case", GEOMETRIES, ids=lambda c: "-".join(map(str, c)))
+def test_launch_geometries_match_single_heads(device, case):
+    w8, B, Hq, Hkv, M, N, D, causal, window = case
+    g = torch.Generator(device=device).manual_seed(5)
+    i8 = lambda *s: torch.randint(-127, 128, s, device=device, generator=g, dtype=torch.int8)
+    rnd = lambda *s: torch.rand(s, device=device, generator=g) + 0.5
+    q, k = i8(B, Hq, M, D), i8(B, Hkv, N, D)
+    qs, ks = rnd(B, Hq, M) * 1e-3, rnd(B, Hkv, N) * 1e-2
+    if w8:
+        v, vs = i8(B, Hkv, N, D), rnd(B, Hkv, D) * 1e-2
+        run = lambda b, h, n: _C.attn_w8a8_fwd(q[b, h], qs[b, h], k[b, n], ks[b, n], v[b, n], vs[b, n],
+                                               causal, N - M)
+    else:
+        v = torch.randn(B, Hkv, N, D, device=device, generator=g).half()
+        run = lambda b, h, n: _C.attn_int8_fwd(q[b, h], qs[b, h], k[b, n], ks[b, n], v[b, n], causal, window)
+    all_ = slice(None)
+    out = run(all_, all_, all_)
+    assert_finite(out)
+    for b, h in {(0, 0), (B - 1, Hq - 1), (B // 2, Hq // 2 + 1)}:
+        n = h // (Hq // Hkv)
+        one = run(slice(b, b + 1), slice(h, h + 1), slice(n, n + 1))
+        assert torch.equal(out[b, h], one[0, 0]), (out[b, h].float() - one[0, 0].float()).abs().max()

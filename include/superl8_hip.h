@@ -110,6 +110,14 @@ int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t qrows, int6
                     int64_t D, float q_scale_mul, float gate_ratio, int8_t* q_i8, float* q_scale,
                     int8_t* k_i8, float* k_scale, float* k_mean, int32_t* gate_flag,
                     void* workspace, size_t workspace_bytes, void* stream);
+/* The same; a firing gate also stores 1 to *gate_flag_host (NULL: none), pinned host memory that
+ * the caller has set to 0. The host may read it once an event recorded behind this call is done,
+ * and must keep the memory until then. */
+int sl8_quantize_qk_hostflag(const void* q, const void* k, int dtype, int64_t qrows, int64_t G,
+                             int64_t N, int64_t D, float q_scale_mul, float gate_ratio,
+                             int8_t* q_i8, float* q_scale, int8_t* k_i8, float* k_scale,
+                             float* k_mean, int32_t* gate_flag, int32_t* gate_flag_host,
+                             void* workspace, size_t workspace_bytes, void* stream);
 
 /* The same prologue for other sets of tensors, without the gate: q [qrows, D] (null, qrows 0: none),
  * k and v [G, N, D] (null: none; at least one of them), all dtype f16 or bf16. v gets per-channel

@@ -148,17 +148,21 @@ def quantize_row_groups(x: torch.Tensor, rows_per_group: int, mean: torch.Tensor
 
 
 def quantize_qk_fused(q: torch.Tensor, k: torch.Tensor, q_scale_mul: float,
-                      gate_ratio: float = 0.0):
+                      gate_ratio: float = 0.0, flag_host: torch.Tensor | None = None):
     """Fused fp16 / bf16 prologue: q [B,Hq,M,D], k [B,Hkv,N,D] -> (q_i8, q_scale [B,Hq,M],
     k_i8, k_scale [B,Hkv,N], k_mean fp32 [B,Hkv,1,D], flag int32 [1] or None).
 
     K is smoothed by its per-channel mean (see k_mean), q_scale carries q_scale_mul;
-    with gate_ratio > 0, flag = 1 when some Q row has max/(median+1e-10) above it."""
+    with gate_ratio > 0, flag = 1 when some Q row has max/(median+1e-10) above it; then
+    flag_host (pinned int32 [1], zeroed by the caller), if given, is set to 1 too, readable
+    once an event recorded after this call is done."""
     _on_gpu(q, k)
     _check(q.dtype == k.dtype and q.dtype in (torch.float16, torch.bfloat16),
            "fused prologue expects float16 or bfloat16 q and k")
     _check(q.dim() == 4 and k.dim() == 4 and q.shape[-1] == k.shape[-1],
            "fused prologue expects q[B,Hq,M,D], k[B,Hkv,N,D]")
+    _check(flag_host is None or (flag_host.dtype == torch.int32 and flag_host.is_pinned()),
+           "fused prologue: flag_host must be a pinned int32 tensor")
     q, k = q.contiguous(), k.contiguous()
     B, Hq, M, D = q.shape
     _, Hkv, N, _ = k.shape
@@ -172,10 +176,10 @@ def quantize_qk_fused(q: torch.Tensor, k: torch.Tensor, q_scale_mul: float,
     ws_bytes = _lib.load().sl8_quantize_qk_workspace(qrows, G, N, D)
     ws = q.new_empty((max(ws_bytes, 8),), dtype=torch.uint8)
     with on_device(q):
-        call("sl8_quantize_qk", q.data_ptr(), k.data_ptr(), dtype_code(q.dtype), qrows, G, N, D,
-             float(q_scale_mul), float(gate_ratio), q_i8.data_ptr(), q_scale.data_ptr(),
-             k_i8.data_ptr(), k_scale.data_ptr(), k_mean.data_ptr(),
-             None if flag is None else flag.data_ptr(), ws.data_ptr(), ws_bytes, stream_of(q))
+        call("sl8_quantize_qk_hostflag", q.data_ptr(), k.data_ptr(), dtype_code(q.dtype), qrows, G,
+             N, D, float(q_scale_mul), float(gate_ratio), q_i8.data_ptr(), q_scale.data_ptr(),
+             k_i8.data_ptr(), k_scale.data_ptr(), k_mean.data_ptr(), _lib.ptr(flag),
+             _lib.ptr(flag_host), ws.data_ptr(), ws_bytes, stream_of(q))
     return q_i8, q_scale, k_i8, k_scale, k_mean, flag
 
 

@@ -33,6 +33,8 @@ SIGNATURES = {
     "sl8_quantize_qk_workspace": (_SZ, [_I64, _I64, _I64, _I64]),
     "sl8_quantize_qk": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _F, _F, _P, _P, _P, _P, _P, _P,
                              _P, _SZ, _P]),
+    "sl8_quantize_qk_hostflag": (_I, [_P, _P, _I, _I64, _I64, _I64, _I64, _F, _F, _P, _P, _P, _P, _P,
+                                      _P, _P, _P, _SZ, _P]),
     "sl8_quantize_qkv_workspace": (_SZ, [_I64, _I64, _I64]),
     "sl8_quantize_qkv": (_I, [_P, _P, _P, _I, _I64, _I64, _I64, _I64, _I, _F] + [_P] * 8
                          + [_SZ, _P]),

@@ -669,7 +669,9 @@ extern "C" int sl8_q_outlier_gate(const void* q, int dtype, int64_t rows, int64_
 //     no median search (the division is needed only for elements within
 //     2^-18 of max / ratio). A row holding a NaN never fires (torch's amax and
 //     median are NaN there). A block with a firing row ORs 1 into the flag
-//     (atomicOr), so the flag is set iff some row fires.
+//     (atomicOr), so the flag is set iff some row fires. The caller's host copy of the flag, if
+//     any, is stored to by the same thread: a copy behind the launch cost 4 us on the device and
+//     3.5 us on the host (a prefill of 8 heads x 512, D = 64: 52.0 us, 46.5 here).
 // sl8_quantize_qkv adds V's per-channel codes (column maxima in A, codes in B) and the rotation of
 // Q and the smoothed K; without Q it builds a K/V cache. Bound by HBM: K and V are read twice
 // (the second time from the MALL where they fit). 16384 keys of 8 heads, D = 128: 93 us as nine
@@ -968,8 +970,8 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
                   int8_t* __restrict__ k_i8, float* __restrict__ k_scale, int krows, int kbg, int nkb,
                   const uint16_t* __restrict__ q, int64_t qrows, float qmul, float ratio,
                   int8_t* __restrict__ q_i8, float* __restrict__ q_scale,
-                  int32_t* __restrict__ flag, int nvb, const uint16_t* __restrict__ v,
-                  const float* __restrict__ vpart, int8_t* __restrict__ v_i8,
+                  int32_t* __restrict__ flag, int32_t* flag_host, int nvb,
+                  const uint16_t* __restrict__ v, const float* __restrict__ vpart, int8_t* __restrict__ v_i8,
                   float* __restrict__ v_scale) {
   constexpr int LPR = row_lanes(D), NL = D / 8, RPP = 256 / LPR;
   const int lane = threadIdx.x % LPR, sub = threadIdx.x / LPR;
@@ -1054,7 +1056,11 @@ prologue_b_kernel(const uint16_t* __restrict__ k, int64_t N,
   }
   if constexpr (GATE) {
     fired = __syncthreads_or(fired);
-    if (fired && threadIdx.x == 0) atomicOr(flag, 1);  // cleared by A, earlier on the stream
+    if (fired && threadIdx.x == 0) {
+      atomicOr(flag, 1);  // cleared by A, earlier on the stream
+      if (flag_host)
+        __hip_atomic_store(flag_host, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
   }
 }
 
@@ -1070,7 +1076,7 @@ struct Prologue {
   float q_scale_mul, gate_ratio;
   int8_t *q_i8, *k_i8, *v_i8;
   float *q_scale, *k_scale, *v_scale, *k_mean;
-  int32_t* flag;
+  int32_t *flag, *flag_host;
   bool rotate;
   void* part;
   hipStream_t st;
@@ -1095,7 +1101,7 @@ struct Prologue {
       prologue_b_kernel<DT, D, decltype(gate)::value, decltype(rot)::value, HV>
           <<<nkb + nvb + nqb, 256, 0, st>>>(k, N, pt, C, k_mean, k_i8, k_scale, krows, kbg, nkb, q,
                                             qrows, q_scale_mul, gate_ratio, q_i8, q_scale, flag,
-                                            nvb, v, vpt, v_i8, v_scale);
+                                            flag_host, nvb, v, vpt, v_i8, v_scale);
     };
     if constexpr ((D & (D - 1)) == 0) {
       if (rotate) return v ? run(F{}, T{}, T{}) : run(F{}, T{}, F{});
@@ -1166,11 +1172,12 @@ extern "C" size_t sl8_quantize_qk_workspace(int64_t BHq_M, int64_t G, int64_t N,
   return (size_t)(G * C * D) * sizeof(long long);  // the K-mean partials
 }
 
-extern "C" int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t qrows, int64_t G,
-                               int64_t N, int64_t D, float q_scale_mul, float gate_ratio,
-                               int8_t* q_i8, float* q_scale, int8_t* k_i8, float* k_scale,
-                               float* k_mean, int32_t* gate_flag, void* workspace,
-                               size_t workspace_bytes, void* stream) {
+extern "C" int sl8_quantize_qk_hostflag(const void* q, const void* k, int dtype, int64_t qrows,
+                                        int64_t G, int64_t N, int64_t D, float q_scale_mul,
+                                        float gate_ratio, int8_t* q_i8, float* q_scale,
+                                        int8_t* k_i8, float* k_scale, float* k_mean,
+                                        int32_t* gate_flag, int32_t* gate_flag_host,
+                                        void* workspace, size_t workspace_bytes, void* stream) {
   clear_error();
   const bool gate = gate_ratio > 0.f;
   SL8_CHECK_ARG(!gate || gate_flag, "fused prologue: gate_flag required with a gate ratio");
@@ -1178,9 +1185,20 @@ extern "C" int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t 
   SL8_CHECK_ARG(k && k_mean, "fused prologue: null pointer");
   const Prologue p{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), nullptr, qrows,
                    G, N, q_scale_mul, gate_ratio, q_i8, k_i8, nullptr, q_scale, k_scale, nullptr,
-                   k_mean, gate ? gate_flag : nullptr, false, nullptr, nullptr, 0, 0, 0, 0};
+                   k_mean, gate ? gate_flag : nullptr, gate ? gate_flag_host : nullptr, false, nullptr,
+                   nullptr, 0, 0, 0, 0};
   return prologue(p, dtype, D, workspace, workspace_bytes,
                   sl8_quantize_qk_workspace(qrows, G, N, D), stream);
+}
+
+extern "C" int sl8_quantize_qk(const void* q, const void* k, int dtype, int64_t qrows, int64_t G,
+                               int64_t N, int64_t D, float q_scale_mul, float gate_ratio,
+                               int8_t* q_i8, float* q_scale, int8_t* k_i8, float* k_scale,
+                               float* k_mean, int32_t* gate_flag, void* workspace,
+                               size_t workspace_bytes, void* stream) {
+  return sl8_quantize_qk_hostflag(q, k, dtype, qrows, G, N, D, q_scale_mul, gate_ratio, q_i8, q_scale,
+                                  k_i8, k_scale, k_mean, gate_flag, nullptr, workspace,
+                                  workspace_bytes, stream);
 }
 
 extern "C" size_t sl8_quantize_qkv_workspace(int64_t G, int64_t N, int64_t D) {
@@ -1197,7 +1215,7 @@ extern "C" int sl8_quantize_qkv(const void* q, const void* k, const void* v, int
                 (long long)qrows);
   const Prologue p{static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
                    static_cast<const uint16_t*>(v), qrows, G, N, q_scale_mul, 0.f, q_i8, k_i8, v_i8,
-                   q_scale, k_scale, v_scale, k_mean, nullptr, rotate != 0, nullptr, nullptr, 0, 0, 0, 0};
+                   q_scale, k_scale, v_scale, k_mean, nullptr, nullptr, rotate != 0, nullptr, nullptr, 0, 0, 0, 0};
   return prologue(p, dtype, D, workspace, workspace_bytes, sl8_quantize_qkv_workspace(G, N, D),
                   stream);
 }

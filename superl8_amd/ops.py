@@ -14,7 +14,6 @@ import math
 import torch
 
 from . import _C
-from ._lib import on_device
 from .quant.rotation import hadamard_dim
 
 # Decode-shape M cap for the k-quant linear (reference ops.py:1289).
@@ -37,7 +36,7 @@ def attn_int8_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: 
 
     if internal_accuracy_gate:
         fired, qk = quant.quantize_qk_gated(q, k, softmax_scale=scale, rotate=rotate,
-                                            defer=not int8_pv)
+                                            defer=False if int8_pv else "host")
     elif int8_pv and window_left < 0 and not rotate and quant.core.fused_ok(q, k, v):
         # one prologue for Q, K and V
         s = (1.0 / math.sqrt(q.shape[-1])) if scale is None else scale
@@ -48,23 +47,21 @@ def attn_int8_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: 
                                 per_warp_quant=per_warp_quant)
     else:
         fired, qk = False, quant.quantize_qk(q, k, softmax_scale=scale, rotate=rotate)
-    if isinstance(fired, torch.Tensor):
-        # gate decided on the device: its flag is copied to pinned host memory
-        # right after the prologue, the attention is launched behind the copy
-        # (it exits at once if the gate fired), and the host waits only for the
-        # copy -- not for the attention, so the next call's prologue is queued
-        # while this attention runs (a plain .item() after the launch would
-        # wait for the attention and leave the GPU idle during the next enqueue)
+    if isinstance(fired, tuple):
+        # gate decided on the device: the prologue sets its flag in pinned host
+        # memory too, the attention is launched behind it (it exits at once if
+        # the gate fired), and the host waits only for the prologue -- not for
+        # the attention, so the next call's prologue is queued while this
+        # attention runs (a plain .item() after the launch would wait for the
+        # attention and leave the GPU idle during the next enqueue)
+        flag, flag_host, flag_ready = fired
         q_i8, q_scale, k_i8, k_scale, _k_mean = qk
-        flag_host = torch.empty(1, dtype=torch.int32, pin_memory=True)
-        flag_host.copy_(fired, non_blocking=True)
-        flag_ready = torch.cuda.Event()
-        with on_device(q):
-            flag_ready.record()
-        out = _C.attn_int8_fwd(q_i8, q_scale.squeeze(-1).contiguous(), k_i8,
-                               k_scale.squeeze(-1).contiguous(), v.contiguous(), causal,
-                               window_left, gate_flag=fired)
-        flag_ready.synchronize()
+        try:
+            out = _C.attn_int8_fwd(q_i8, q_scale.squeeze(-1).contiguous(), k_i8,
+                                   k_scale.squeeze(-1).contiguous(), v.contiguous(), causal,
+                                   window_left, gate_flag=flag)
+        finally:
+            flag_ready.synchronize()  # before flag_host is read, or let go
         if int(flag_host[0]) == 0:
             return out
         fired = True

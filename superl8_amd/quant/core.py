@@ -98,7 +98,8 @@ def fused_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None = None) ->
 
 
 def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float | None = None,
-                      rotate: bool = False, ratio_threshold: float = 12.0, defer: bool = False):
+                      rotate: bool = False, ratio_threshold: float = 12.0,
+                      defer: bool | str = False):
     """The attention prologue with the outlier gate (reference ops.py:115-150).
 
     Returns (fired, quantize_qk's five outputs or None). fired is
@@ -110,6 +111,9 @@ def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float 
     detect_q_outlier_domination. With defer=True the fused path returns the
     device flag (int32 [1]) in place of fired, unread, with the quantised
     tensors: the caller reads it later (the other paths still return a bool).
+    defer="host" returns (that flag, a pinned host int32 [1] that the kernel sets
+    with it, an event behind the launch); the caller waits for the event before it
+    reads the host flag or lets go of it.
     """
     _need_gpu(q, "quantize_qk")
     try:
@@ -118,8 +122,16 @@ def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float 
         capturing = False
     if not rotate and not capturing and fused_ok(q, k):
         s = (1.0 / math.sqrt(q.shape[-1])) if softmax_scale is None else softmax_scale
+        flag_host = None
+        if defer == "host":
+            flag_host, ready = torch.zeros(1, dtype=torch.int32, pin_memory=True), torch.cuda.Event()
         q_i8, q_scale, k_i8, k_scale, k_mean, flag = _C.quantize_qk_fused(
-            q, k, s * LOG2E, ratio_threshold)
+            q, k, s * LOG2E, ratio_threshold, flag_host)
+        if defer == "host":
+            with _C.on_device(q):
+                ready.record()
+            return ((flag, flag_host, ready),
+                    (q_i8, q_scale.unsqueeze(-1), k_i8, k_scale.unsqueeze(-1), k_mean))
         if defer:
             return flag, (q_i8, q_scale.unsqueeze(-1), k_i8, k_scale.unsqueeze(-1), k_mean)
         if bool(flag.item()):

@@ -291,3 +291,24 @@ def test_rotated_prologue_against_64_bits(device, dtype, D):
         assert ((s.double() / s_ref - 1).abs() <= ulp).all()
         c_ref = (ref / s_ref).round().clamp(-127, 127)
         assert ((c.double() - c_ref).abs() <= 1).all() and (c.double() != c_ref).float().mean() <= 0.02
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,D", [(1, 1, 64), (300, 77, 128), (64, 512, 72), (700, 33, 256)])
+def test_host_flag_follows_the_device_flag(device, dtype, M, N, D):
+    g = torch.Generator(device=device).manual_seed(3)
+    k = torch.randn(1, 2, N, D, device=device, generator=g).to(dtype)
+    calm = torch.randn(1, 4, M, D, device=device, generator=g).clamp(-2, 2).to(dtype)
+    calm[..., 0] = 2.0
+    last, first = calm.clone(), calm.clone()
+    last[0, -1, -1, -1] = 4000.0  # one row fires, in the last block
+    first[0, 0, 0, 0] = -4000.0
+    for q, fires in ((calm, 0), (last, 1), (calm, 0), (first, 1)):
+        host = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        flag = _C.quantize_qk_fused(q, k, 1.0, 24.0, host)[5]
+        ready = torch.cuda.Event()
+        ready.record()
+        ready.synchronize()
+        assert int(host[0]) == flag.item() == fires
+    with pytest.raises(RuntimeError, match="pinned"):
+        _C.quantize_qk_fused(calm, k, 1.0, 24.0, torch.zeros(1, dtype=torch.int32))

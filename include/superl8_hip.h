@@ -160,6 +160,10 @@ int sl8_quantize_i8_cols(const void* x, int dtype, int64_t G, int64_t N, int64_t
  * ---------------------------------------------------------------------- */
 size_t sl8_attn_int8_fwd_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t M, int64_t N,
                                    int64_t D);
+/* Workspace that also holds the fp32 key parts of launches whose query blocks leave CUs idle (few
+ * heads or queries, many keys). With less, sl8_attn_int8_fwd runs the keys in one part. */
+size_t sl8_attn_int8_fwd_split_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t M, int64_t N,
+                                         int64_t D, int causal, int64_t window_left);
 int sl8_attn_int8_fwd(const int8_t* q, const float* q_scale, const int8_t* k,
                       const float* k_scale, const void* v, int v_dtype, void* out,
                       float* lse, int64_t B, int64_t Hq, int64_t Hkv, int64_t M,

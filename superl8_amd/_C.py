@@ -306,7 +306,8 @@ def _attn_fwd(q, q_scale, k, k_scale, v, causal, window_left, want_lse, gate_fla
     lse = q.new_empty((B, H, M), dtype=torch.float32) if want_lse else None
     if M == 0 or B == 0 or H == 0:
         return out, lse
-    ws_bytes = _lib.load().sl8_attn_int8_fwd_workspace(B, H, Hkv, M, N, D)
+    ws_bytes = _lib.load().sl8_attn_int8_fwd_split_workspace(B, H, Hkv, M, N, D, int(bool(causal)),
+                                                            int(window_left))
     ws = q.new_empty((ws_bytes,), dtype=torch.uint8) if ws_bytes else None
     args = (q.data_ptr(), q_scale.data_ptr(), k.data_ptr(), k_scale.data_ptr(), v.data_ptr(),
             dtype_code(v.dtype), out.data_ptr(), lse.data_ptr() if want_lse else None,

@@ -40,6 +40,7 @@ SIGNATURES = {
                          + [_SZ, _P]),
     "sl8_quantize_i8_cols": (_I, [_P, _I, _I64, _I64, _I64, _P, _P, _P]),
     "sl8_attn_int8_fwd_workspace": (_SZ, [_I64, _I64, _I64, _I64, _I64, _I64]),
+    "sl8_attn_int8_fwd_split_workspace": (_SZ, [_I64, _I64, _I64, _I64, _I64, _I64, _I, _I64]),
     "sl8_attn_int8_fwd": (_I, [_P, _P, _P, _P, _P, _I, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64,
                                _I, _I64, _P, _SZ, _P]),
     "sl8_attn_int8_fwd_gated": (_I, [_P, _P, _P, _P, _P, _I, _P, _P, _I64, _I64, _I64, _I64, _I64,

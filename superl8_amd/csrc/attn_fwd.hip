@@ -171,6 +171,10 @@ struct FwdArgs {
   int dout;            // output row length (= D, or the caller's head dim when D is padded)
   int paired;          // causal: a workgroup takes query blocks nqb-1-slot and slot, one after the other
   int fold;            // not paired: slots from here on count their query block up from 0
+  int parts;           // PARTS: key parts of a query block, a workgroup each
+  float* part_o;       // PARTS: [parts][B*Hq*M][D] fp32, each part's own softmax applied
+  float2* part_ml;     // PARTS: [parts][B*Hq*M] reference point (log2) and row sum
+  int64_t part_rows;   // PARTS: B*Hq*M
   const int32_t* skip; // production kernel: nonzero *skip -> every workgroup exits at once
 };
 
@@ -233,7 +237,10 @@ struct QOp {
 // stored to a.scores [B*Hq][M][N] (the test hook that proves the production
 // MFMA path's Q.K^T bit-exact); V and the scales are not read, nothing else
 // is written.
-template <int D, bool CAUSAL, int VDT, bool LSE, int NG, int WV, bool W8, bool DUMP = false>
+// PARTS = a query block's keys are split over a.parts workgroups, each of which stores its fp32
+// result, reference points and row sums; attn_parts_combine_kernel joins them.
+template <int D, bool CAUSAL, int VDT, bool LSE, int NG, int WV, bool W8, bool DUMP = false,
+          bool PARTS = false>
 __global__ void __launch_bounds__(WV * 64, (NG == 1 && D <= 128) ? SL8_FWD_OCC * 4 / WV : 1)
 attn_fwd_wide_kernel(const FwdArgs a) {
   // the caller's accuracy gate fired: its result is discarded, so do nothing
@@ -260,9 +267,14 @@ attn_fwd_wide_kernel(const FwdArgs a) {
   using PV = PvOp<VDT>;
   typedef typename PV::vec pvec;
 
-  const int nslot = CAUSAL && a.paired ? (a.nqb + 1) / 2 : a.nqb;
+  const int nslot = PARTS ? a.nqb * a.parts : CAUSAL && a.paired ? (a.nqb + 1) / 2 : a.nqb;
   int bh, slot;
   block_coords(a, nslot, bh, slot);
+  int part = 0;
+  if constexpr (PARTS) {
+    part = slot % a.parts;
+    slot /= a.parts;
+  }
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = lane >> 5, l32 = lane & 31;
@@ -354,7 +366,12 @@ attn_fwd_wide_kernel(const FwdArgs a) {
     if (CAUSAL) n_end = max(0, min(N, m_blk + WBM + diag));
     int n_beg = 0;
     if (wl >= 0) n_beg = min(n_end, max(0, m_blk + diag - wl + 1) & ~(BN - 1));
-    const int ntiles = (n_end - n_beg + BN - 1) / BN;
+    int ntiles = (n_end - n_beg + BN - 1) / BN;
+    if constexpr (PARTS) {
+      const int tp = (ntiles + a.parts - 1) / a.parts, t0 = min(part * tp, ntiles);
+      n_beg += t0 * BN;
+      ntiles = min(tp, ntiles - t0);
+    }
     const int wq_lo = q0 + diag, wq_hi = q0 + WQ - 1 + diag;
     auto live = [&](int t) __attribute__((always_inline)) {
       if (t < 0 || t >= ntiles) return false;
@@ -1135,6 +1152,21 @@ attn_fwd_wide_kernel(const FwdArgs a) {
     for (int g = 0; g < NG; ++g) {
       if constexpr (DUMP) break;
       const float l = l_lane[g] + __shfl_xor(l_lane[g], 32, 64);
+      if constexpr (PARTS) {
+        if (!m_ok[g]) continue;
+        const int64_t row = (int64_t)part * a.part_rows + (int64_t)bh * M + mq[g];
+        const float inv = (l > 0.f) ? 1.f / l : 0.f;
+        float* orow = a.part_o + row * D;
+#pragma unroll
+        for (int tt = 0; tt < DC; ++tt)
+#pragma unroll
+          for (int gq = 0; gq < 4; ++gq)
+            *reinterpret_cast<float4*>(orow + 32 * tt + 8 * gq + 4 * h) =
+                make_float4(oacc[g][tt][4 * gq] * inv, oacc[g][tt][4 * gq + 1] * inv,
+                            oacc[g][tt][4 * gq + 2] * inv, oacc[g][tt][4 * gq + 3] * inv);
+        if (h == 0) a.part_ml[row] = make_float2(m_run[g], l);
+        continue;
+      }
       if (m_ok[g]) {
         const float inv = (l > 0.f) ? 1.f / l : 0.f;
         uint16_t* orow = reinterpret_cast<uint16_t*>(a.out) + ((int64_t)bh * M + mq[g]) * a.dout;
@@ -1164,6 +1196,48 @@ attn_fwd_wide_kernel(const FwdArgs a) {
       }
     }
   }
+}
+
+// Joins the key parts of every query row: out = sum_p w_p O_p / sum_p w_p with
+// w_p = l_p 2^(m_p - max m), and the row's LSE where asked for. D / 4 lanes per row.
+template <int D, int VDT>
+__global__ void __launch_bounds__(256)
+attn_parts_combine_kernel(const FwdArgs a) {
+  if (a.skip != nullptr && *a.skip != 0) return;  // the parts were not written
+  constexpr int LPR = D / 4, RPB = 256 / LPR;
+  const int lane = threadIdx.x % LPR;
+  const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
+  if (row >= a.part_rows) return;
+  float mx = -INFINITY;
+  for (int p = 0; p < a.parts; ++p) {
+    const float2 ml = a.part_ml[p * a.part_rows + row];
+    if (ml.y > 0.f) mx = fmaxf(mx, ml.x);
+  }
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  float sum = 0.f;
+  for (int p = 0; p < a.parts; ++p) {
+    const int64_t r = p * a.part_rows + row;
+    const float2 ml = a.part_ml[r];
+    const float w = ml.y > 0.f ? ml.y * exp2f(ml.x - mx) : 0.f;  // no keys: no weight
+    const float4 o = *reinterpret_cast<const float4*>(a.part_o + r * D + 4 * lane);
+    sum += w;
+    acc.x += w * o.x;
+    acc.y += w * o.y;
+    acc.z += w * o.z;
+    acc.w += w * o.w;
+  }
+  const float inv = sum > 0.f ? 1.f / sum : 0.f;
+  if (4 * lane < a.dout) {
+    const float v[4] = {acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+    uint16_t hv[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) hv[e] = VDT == SL8_DTYPE_F16 ? f2h_bits(v[e]) : f2bf_bits(v[e]);
+    uint2 pk;
+    pk.x = hv[0] | ((uint32_t)hv[1] << 16);
+    pk.y = hv[2] | ((uint32_t)hv[3] << 16);
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + row * a.dout + 4 * lane) = pk;
+  }
+  if (a.lse && lane == 0) a.lse[row] = sum > 0.f ? mx * LN2F + logf(sum) : -INFINITY;
 }
 
 // query-column blocks per wave of the production kernel
@@ -1266,6 +1340,43 @@ FwdGeom fwd_geometry(const FwdKernel& kn, int64_t heads, int64_t M, int64_t N, b
   return {kn.narrow, paired, folded};
 }
 
+// Key parts of a prefill whose query blocks leave CUs idle (1: none). A chain of N / 64 tiles bounds
+// such a launch, whatever the number of blocks. Model, in us: a workgroup takes its longest run of
+// tiles and 3 of fill and drain, `pair` times that where two share a CU (fewer do if the causal
+// blocks differ); the parts are written, read and joined by a second launch. Within 8 % of the
+// best count of 1 to 16 at 100 of 105 shapes. Kernel times, causal, one part -> parts taken, in us:
+//   4 heads x 64 queries, 8192 keys, D = 128      124 -> 29 (16)
+//   16 heads, 256 x 16384                         242 -> 53 (7);    D = 256: 573 -> 104 (8)
+//   16 heads, 1000 x 6121                          96 -> 62 (4);    D = 64: 117 -> 54 (4)
+//   16 heads, 2048 x 2048: 40 in one part, 43 in two
+int fwd_parts(const FwdKernel& kn, int64_t DP, int64_t heads, int64_t M, int64_t N, bool causal,
+              int64_t window_left) {
+  const int64_t cus = cu_count(), bm = kn.narrow * kn.wave_q, nqb = (M + bm - 1) / bm;
+  const int64_t grid = heads * nqb;
+  int64_t keys = N;
+  if (window_left >= 0) keys = std::min(N, window_left + bm + BN);
+  const int64_t nt = (keys + BN - 1) / BN;
+  const double tile = DP == 64 ? 1.2 : DP == 128 ? 1.0 : 2.3, pair = DP == 64 ? 0.4 : 0.75;
+  const bool skewed = causal && 2 * M > N && (window_left < 0 || 2 * window_left > N);
+  int best = 1;
+  double best_t = 1e30;
+  for (int p = 1; p <= 16; ++p) {
+    const int64_t g = grid * p, run = (nt + p - 1) / p;
+    if (p > 1 && (g > cus * kn.cap || run < 4)) break;
+    const double share = g <= cus ? 1.0 : 1.0 + pair * (skewed ? 0.5 * (g - cus) / cus : 1.0);
+    double us = tile * (run + 3) * share;
+    if (p > 1) us = 1.1 * us + 5.0 + 8.0 * (double)(heads * M * DP * p) / 3.5e6;
+    if (us < best_t) {
+      best_t = us;
+      best = p;
+    }
+  }
+  return best;
+}
+size_t fwd_parts_bytes(int64_t rows, int64_t DP, int parts) {
+  return parts > 1 ? (size_t)parts * rows * (DP + 2) * sizeof(float) : 0;
+}
+
 template <int D, int VDT, int WV>
 void dispatch_wide_wv(const FwdArgs& a, int grid, bool causal, bool lse, hipStream_t st) {
   if (causal) {
@@ -1279,6 +1390,14 @@ void dispatch_wide_wv(const FwdArgs& a, int grid, bool causal, bool lse, hipStre
 
 template <int D, int VDT>
 void dispatch_wide(const FwdArgs& a, int grid, bool causal, bool lse, int wv, hipStream_t st) {
+  if (a.parts > 1) {
+    constexpr int NG = wide_ng(D);
+    if (causal) attn_fwd_wide_kernel<D, true, VDT, false, NG, 4, false, false, true><<<grid, 256, 0, st>>>(a);
+    else attn_fwd_wide_kernel<D, false, VDT, false, NG, 4, false, false, true><<<grid, 256, 0, st>>>(a);
+    constexpr int rpb = 256 / (D / 4);
+    attn_parts_combine_kernel<D, VDT><<<(unsigned)((a.part_rows + rpb - 1) / rpb), 256, 0, st>>>(a);
+    return;
+  }
   if constexpr (wide_waves(D) != 4)
     if (wv == 4) return dispatch_wide_wv<D, VDT, 4>(a, grid, causal, lse, st);
   dispatch_wide_wv<D, VDT, wide_waves(D)>(a, grid, causal, lse, st);
@@ -1876,6 +1995,16 @@ extern "C" size_t sl8_attn_int8_fwd_workspace(int64_t B, int64_t Hq, int64_t Hkv
   return pad_workspace(B, Hq, Hkv, M, N, D, 2, false);
 }
 
+extern "C" size_t sl8_attn_int8_fwd_split_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t M,
+                                                    int64_t N, int64_t D, int causal,
+                                                    int64_t window_left) {
+  const size_t pad = sl8_attn_int8_fwd_workspace(B, Hq, Hkv, M, N, D);
+  if (B <= 0 || Hq <= 0 || M <= 0 || N <= 0) return pad;
+  const int64_t DP = padded_head_dim(D);
+  const int parts = fwd_parts(fwd_kernel(DP, false), DP, B * Hq, M, N, causal != 0, window_left);
+  return (pad + 15) / 16 * 16 * (parts > 1) + pad * (parts <= 1) + fwd_parts_bytes(B * Hq * M, DP, parts);
+}
+
 namespace {
 int attn_int8_fwd_impl(const int8_t* q, const float* q_scale, const int8_t* k,
                        const float* k_scale, const void* v, int v_dtype, void* out, float* lse,
@@ -1907,9 +2036,22 @@ int attn_int8_fwd_impl(const int8_t* q, const float* q_scale, const int8_t* k,
   const bool c = causal != 0, want_lse = lse != nullptr;
   int grid;
   const FwdKernel kn = fwd_kernel(DP, false);
-  const FwdGeom geom = fwd_geometry(kn, B * Hq, M, N, c, window_left);
+  // key parts, where the caller's workspace has room for them
+  int parts = N > 0 ? fwd_parts(kn, DP, B * Hq, M, N, c, window_left) : 1;
+  const size_t pad = (need + 15) / 16 * 16, part_bytes = fwd_parts_bytes(B * Hq * M, DP, parts);
+  if (!workspace || !aligned(workspace, 16) || workspace_bytes < pad + part_bytes) parts = 1;
+  const FwdGeom geom = parts > 1 ? FwdGeom{kn.narrow, false, false}
+                                 : fwd_geometry(kn, B * Hq, M, N, c, window_left);
   const int wv = geom.wv;
   FwdArgs a = make_args(B, Hq, Hkv, M, N, DP, c, grid, geom, kn.wave_q);
+  a.parts = parts;
+  if (parts > 1) {
+    a.part_rows = B * Hq * M;
+    a.part_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + pad);
+    a.part_ml = reinterpret_cast<float2*>(a.part_o + (int64_t)parts * a.part_rows * DP);
+    grid *= parts;
+    a.xcd_map = xcd_mode(B * Hkv, Hq / Hkv, (int64_t)a.nqb * parts);
+  }
   a.q = q; a.qs = q_scale; a.k = k; a.ks = k_scale;
   a.vt = static_cast<const uint16_t*>(v);  // V [B*Hkv][N][DP], read in place
   a.out = out; a.lse = lse; a.window_left = (int)window_left;

@@ -391,6 +391,22 @@ GEOMETRIES = [
 ]
 
 
+def _one_part(q, qs, k, ks, v, causal, window=-1, want_lse=False):
+    """The prefill through the C ABI without scratch: its keys in one part."""
+    from superl8_amd import _lib
+
+    B, H, M, D = q.shape
+    Hkv, N = k.shape[1], k.shape[2]
+    out, lse = torch.empty(q.shape, device=q.device, dtype=v.dtype), torch.empty_like(qs)
+    need = _lib.load().sl8_attn_int8_fwd_workspace(B, H, Hkv, M, N, D)
+    ws = torch.empty((max(need, 1),), device=q.device, dtype=torch.uint8)
+    _lib.call("sl8_attn_int8_fwd", q.data_ptr(), qs.data_ptr(), k.data_ptr(), ks.data_ptr(),
+              v.data_ptr(), _lib.dtype_code(v.dtype), out.data_ptr(),
+              lse.data_ptr() if want_lse else None, B, H, Hkv, M, N, D, int(causal), window,
+              ws.data_ptr() if need else None, need, _lib.stream_of(q))
+    return (out, lse) if want_lse else out
+
+
 @pytest.mark.parametrize("case", GEOMETRIES, ids=lambda c: "-".join(map(str, c)))
 def test_launch_geometries_match_single_heads(device, case):
     w8, B, Hq, Hkv, M, N, D, causal, window = case
@@ -405,7 +421,7 @@ def test_launch_geometries_match_single_heads(device, case):
                                                causal, N - M)
     else:
         v = torch.randn(B, Hkv, N, D, device=device, generator=g).half()
-        run = lambda b, h, n: _C.attn_int8_fwd(q[b, h], qs[b, h], k[b, n], ks[b, n], v[b, n], causal, window)
+        run = lambda b, h, n: _one_part(q[b, h], qs[b, h], k[b, n], ks[b, n], v[b, n], causal, window)
     all_ = slice(None)
     out = run(all_, all_, all_)
     assert_finite(out)
@@ -413,3 +429,76 @@ def test_launch_geometries_match_single_heads(device, case):
         n = h // (Hq // Hkv)
         one = run(slice(b, b + 1), slice(h, h + 1), slice(n, n + 1))
         assert torch.equal(out[b, h], one[0, 0]), (out[b, h].float() - one[0, 0].float()).abs().max()
+
+
+# Few query blocks and many keys: the keys in parts joined by a second launch, against one part.
+PARTS = [
+    # B, Hq, Hkv, M, N, D, causal, window
+    (1, 4, 1, 64, 8192, 128, True, -1),      # the most parts
+    (1, 2, 2, 1, 1025, 64, False, -1),       # one query, the last part one key over
+    (2, 3, 1, 33, 640, 128, False, -1),
+    (1, 4, 2, 130, 1999, 256, True, -1),
+    (1, 2, 1, 1500, 1100, 128, True, -1),    # rows and whole blocks that see no key
+    (1, 2, 1, 700, 2500, 128, True, 1000),   # window: parts that a wave sees nothing of
+    (1, 2, 1, 200, 2049, 64, True, 1000),
+    (1, 2, 2, 260, 1100, 32, True, -1),      # padded head dims
+    (1, 2, 2, 577, 900, 72, False, -1),
+    (1, 1, 1, 90, 3000, 80, True, -1),
+    (1, 8, 2, 1000, 6121, 128, True, -1),
+]
+
+
+@pytest.mark.parametrize("vdt", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("case", PARTS, ids=lambda c: "-".join(map(str, c)))
+def test_key_parts_match_one_part(device, case, vdt):
+    from superl8_amd import _lib
+
+    B, Hq, Hkv, M, N, D, causal, window = case
+    lib = _lib.load()
+    assert (lib.sl8_attn_int8_fwd_split_workspace(B, Hq, Hkv, M, N, D, int(causal), window)
+            > lib.sl8_attn_int8_fwd_workspace(B, Hq, Hkv, M, N, D))
+    g = torch.Generator(device=device).manual_seed(7)
+    i8 = lambda *s: torch.randint(-127, 128, s, device=device, generator=g, dtype=torch.int8)
+    q, k = i8(B, Hq, M, D), i8(B, Hkv, N, D)
+    qs = (torch.rand(B, Hq, M, device=device, generator=g) + 0.5) * 1e-3
+    ks = (torch.rand(B, Hkv, N, device=device, generator=g) + 0.5) * 1e-2
+    ks[..., N // 2:] *= 3  # later parts hold the larger scores
+    v = torch.randn(B, Hkv, N, D, device=device, generator=g).to(vdt)
+    ref, ref_lse = _one_part(q, qs, k, ks, v, causal, window, True)
+    out = _C.attn_int8_fwd(q, qs, k, ks, v, causal, window)
+    assert_finite(out)
+    # P is rounded to V's type (unit roundoff u) relative to each side's own reference point, and
+    # both results once more: |difference| <= 4 u max |v|; a row sum's relative error is below u
+    u = 2.0 ** (-11 if vdt == torch.float16 else -8)
+    assert (out.float() - ref.float()).abs().max() <= 4 * u * v.float().abs().max()
+    if window < 0:
+        out_t, lse = _C.attn_int8_fwd_train(q, qs, k, ks, v, causal)
+        assert torch.equal(out, out_t)
+        empty = ref_lse == -float("inf")
+        assert torch.equal(lse == -float("inf"), empty)
+        assert (lse - ref_lse)[~empty].abs().max() <= 4 * u
+
+
+def test_key_parts_skip_and_replay(device):
+    """With the gate flag set neither launch reads the parts; captured calls replay to the same bits."""
+    g = torch.Generator(device=device).manual_seed(8)
+    q = torch.randint(-127, 128, (1, 2, 100, 128), device=device, generator=g, dtype=torch.int8)
+    k = torch.randint(-127, 128, (1, 1, 3000, 128), device=device, generator=g, dtype=torch.int8)
+    qs, ks = torch.full((1, 2, 100), 1e-3, device=device), torch.full((1, 1, 3000), 1e-2, device=device)
+    v = torch.randn(1, 1, 3000, 128, device=device, generator=g).half()
+    ref = _C.attn_int8_fwd(q, qs, k, ks, v, True)
+    flag = torch.ones(1, device=device, dtype=torch.int32)
+    _C.attn_int8_fwd(q, qs, k, ks, v, True, gate_flag=flag)
+    flag.zero_()
+    assert torch.equal(_C.attn_int8_fwd(q, qs, k, ks, v, True, gate_flag=flag), ref)
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = _C.attn_int8_fwd(q, qs, k, ks, v, True)
+    for _ in range(3):
+        out.zero_()
+        torch.randn(1 << 20, device=device)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)

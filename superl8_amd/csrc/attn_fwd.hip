@@ -203,6 +203,8 @@ struct QOp {
 // softmax of half h-1, so P stays in registers for one half-step. The
 // reference point of the softmax is set once per row (see settle()) and O is
 // never rescaled inside the loop.
+// D = 64 (VALU-bound: half the MFMAs, as many scores) took 1.2 us a tile when the compiler ordered
+// its half-steps, 0.9 in half_step_fast: 32 heads x 2048 44.8 -> 33.7 us, 8192 372 -> 290.
 // Per wave and tile (D = 128): 8 i8 + 16 f16 32x32 MFMAs, 24 KB of LDS
 // operand reads (1 KB per MFMA), ~7 VALU operations per score.
 // ---------------------------------------------------------------------------
@@ -217,9 +219,6 @@ struct QOp {
 // operand prefetch distance of the straight-line half-steps (MFMAs ahead)
 #ifndef SL8_FWD_PD
 #define SL8_FWD_PD 3
-#endif
-#ifndef SL8_FWD_BAL
-#define SL8_FWD_BAL 1
 #endif
 // balanced slices: the slot whose VALU slice starts the k_scale reads (config 2:
 // slot 4 ~0.5 % faster than slot 6 on two machines)
@@ -246,8 +245,10 @@ attn_fwd_wide_kernel(const FwdArgs a) {
   // the caller's accuracy gate fired: its result is discarded, so do nothing
   if (a.skip != nullptr && *a.skip != 0) return;
   constexpr int WT = WV * 64;                  // threads per workgroup
-  // the straight-line steady-state half-step (half_step_fast): D = 128, NG = 1
-  constexpr bool FAST = SL8_FWD_FAST && D == 128 && NG == 1 && !W8;
+  // the straight-line steady-state half-step (half_step_fast): D = 64 and 128, NG = 1
+  constexpr bool FAST = SL8_FWD_FAST && D <= 128 && NG == 1 && !W8;
+  // its scores start from C0BITS and skip the conversion; D = 64 converts (3 operations, not 2)
+  constexpr bool SEEDED = D == 128;
   // ... and its W8A8 counterpart (half_step_fast_w8): D = 256, NG = 1, lazy rescale
   constexpr bool FAST_W8 = SL8_FWD_FAST && D == 256 && NG == 1 && W8 && W8_LAZY;
   constexpr int WQ = 32 * NG;                  // queries per wave
@@ -722,41 +723,37 @@ attn_fwd_wide_kernel(const FwdArgs a) {
       float4 kv[4];
       v16i sc;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) sc[r] = C0BITS;
+      for (int r = 0; r < 16; ++r) sc[r] = SEEDED ? C0BITS : 0;
       v4i opb[NOP];  // operand i is read SL8_FWD_PD MFMAs ahead of its use
 #pragma unroll
       for (int i = 0; i < SL8_FWD_PD && i < NOP; ++i) opb[i] = load_op(i);
       // Issue order, fixed by scheduling barriers: MFMA i is preceded by the
-      // read of operand i + SL8_FWD_PD and followed by a slice of VALU work --
-      //   QK MFMAs 0..3: P of half h-1, four exp2 each (xi holds the exp2 argument);
-      //   PV MFMAs 0..1: pack P to fp16 + row sums (one 16-key step each);
-      //   PV MFMA 2: k_scale reads; PV MFMAs 3..6: exp2 arguments of half h
-      //   (two fmas each from the seeded accumulator, see C0BITS).
+      // read of operand i + SL8_FWD_PD and followed by a slice of VALU work.
 #pragma unroll
       for (int i = 0; i < NOP; ++i) {
         if (i + SL8_FWD_PD < NOP) opb[i + SL8_FWD_PD] = load_op(i + SL8_FWD_PD);
         __builtin_amdgcn_sched_barrier(0);  // the read goes out before MFMA i
         const v4i cur = opb[i];
-#if SL8_FWD_BAL
-        // Balanced slices (VALU cycles per MFMA slot ~32-40; exp2 is quarter
+        // Balanced slices (D = 128: VALU cycles per MFMA slot ~32-40; exp2 is quarter
         // rate): slots 0..7 exp2 of keys 2i, 2i+1 of half h-1, with the pack +
         // row sum of keys 0..7 after slot 3 and of keys 8..15 after slot 7;
         // slot SL8_FWD_KVS reads k_scale, four slots before its first use;
         // slots 8..11 form the exp2 arguments of half h, four keys each (the QK
-        // chain ended at slot 3).
-        static_assert(NOP == 12, "balanced slices: D = 128");
+        // chain ended at slot 3). D = 64 has half the slots and as much VALU work, which
+        // bounds it: exp2 of four keys in slots 0..3, arguments in slots 3, 4 and 5 (4 + 4 + 8).
+        constexpr int EPS = DC == 2 ? 4 : 2, KVS = DC == 2 ? 1 : SL8_FWD_KVS;
         if (i < DC) sc = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur, qop[0].c[i], sc, 0, 0, 0);
         else oacc[0][(i - DC) % DC] = PV::mfma(__builtin_bit_cast(pvec, cur), p2[0][(i - DC) / DC],
                                                oacc[0][(i - DC) % DC]);
-        if (i < 8) {
+        if (i < 16 / EPS) {
 #pragma unroll
-          for (int e = 2 * i; e < 2 * i + 2; ++e) {
+          for (int e = EPS * i; e < EPS * i + EPS; ++e) {
             pe[e] = __builtin_amdgcn_exp2f(xi[0][e]);  // -inf -> 0
             pin_vgpr(pe[e]);
           }
         }
-        if (i == 3 || i == 7) {
-          const int k = i / 4;
+        if (i == 8 / EPS - 1 || i == 16 / EPS - 1) {
+          const int k = i / (8 / EPS);
           // same packing, row-sum order and overflow test as half_probs
           p1[0][k] = PV::pack(&pe[8 * k]);
           hs = PV::sum(p1[0][k], &pe[8 * k], hs);
@@ -767,66 +764,30 @@ attn_fwd_wide_kernel(const FwdArgs a) {
             ovf = ovf || (hs > 32768.f);
           }
         }
-        if (i == SL8_FWD_KVS) {
+        if (i == KVS) {
 #pragma unroll
           for (int gq = 0; gq < 4; ++gq)
             kv[gq] = *reinterpret_cast<const float4*>(st + 32 * s + 8 * gq + 4 * h);
         }
-        if (i >= 8) {
-          const int gq = i - 8;
+        constexpr int G0 = DC == 2 ? 3 : 8;  // first slot of the arguments
+#pragma unroll
+        for (int gq = 0; gq < 4; ++gq) {
+          if (i != min(G0 + gq, NOP - 1)) continue;
           const float kk[4] = {kv[gq].x, kv[gq].y, kv[gq].z, kv[gq].w};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            const float w = fmaf(__int_as_float(sc[4 * gq + e]), qs26, cq26);
+            const float w = SEEDED ? fmaf(__int_as_float(sc[4 * gq + e]), qs26, cq26)
+                                   : (float)sc[4 * gq + e] * qsc[0];
             xo[0][4 * gq + e] = fmaf(w, kk[e], -msub);
           }
 #pragma unroll
           for (int e = 0; e < 4; ++e) pin_vgpr(xo[0][4 * gq + e]);
         }
-#else
-        if (i < DC) {
-          sc = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur, qop[0].c[i], sc, 0, 0, 0);
-#pragma unroll
-          for (int e = 4 * i; e < 4 * i + 4; ++e) {
-            pe[e] = __builtin_amdgcn_exp2f(xi[0][e]);  // -inf -> 0
-            pin_vgpr(pe[e]);
-          }
-        } else {
-          const int c = (i - DC) / DC, tt = (i - DC) % DC;
-          oacc[0][tt] = PV::mfma(__builtin_bit_cast(pvec, cur), p2[0][c], oacc[0][tt]);
-          const int k = i - DC;
-          if (k < 2) {
-            // same packing, row-sum order and overflow test as half_probs
-            p1[0][k] = PV::pack(&pe[8 * k]);
-            hs = PV::sum(p1[0][k], &pe[8 * k], hs);
-            pin_vgpr(__builtin_bit_cast(v4i, p1[0][k]));
-            pin_vgpr(hs);
-            if (k == 1) {
-              l_lane[0] += hs;
-              ovf = ovf || (hs > 32768.f);
-            }
-          } else if (k == 2) {
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq)
-              kv[gq] = *reinterpret_cast<const float4*>(st + 32 * s + 8 * gq + 4 * h);
-          } else if (k < 7) {
-            const int gq = k - 3;
-            const float kk[4] = {kv[gq].x, kv[gq].y, kv[gq].z, kv[gq].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const float w = fmaf(__int_as_float(sc[4 * gq + e]), qs26, cq26);
-              xo[0][4 * gq + e] = fmaf(w, kk[e], -msub);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) pin_vgpr(xo[0][4 * gq + e]);
-          }
-        }
-#endif
         __builtin_amdgcn_sched_barrier(0);
       }
       if constexpr (DUMP) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[r] -= C0BITS;  // the bits hold C0BITS + acc
+        for (int r = 0; r < 16; ++r) sc[r] -= SEEDED ? C0BITS : 0;  // the bits hold C0BITS + acc
         dump(0, sc, j, s);
       }
       }
@@ -1292,14 +1253,15 @@ struct FwdKernel {
   int wave_q;          // queries per wave
   int wide, narrow;    // waves per workgroup of its instantiations (equal: there is one)
   int cap;             // workgroups of the narrow one that fit a CU (of the wide one: 1)
+  bool pairs;          // whether pairs of its blocks can pay
 };
 // D = 64: 4 waves. D = 128: 8 or 4; W8A8 4 (at every size measured 4 to 15 % faster than 8).
 // D = 256: 4, a CU's LDS full; its W8A8 kernel (16 queries per wave) 8 or 4.
 FwdKernel fwd_kernel(int64_t D, bool w8) {
-  if (D == 64) return {32, 4, 4, 2};
-  if (D == 128) return {32, w8 ? 4 : 8, 4, 2};
-  if (w8 && SL8_W8_Q16) return {16, 8, 4, 1};
-  return {32 * wide_ng(256), 4, 4, 1};
+  if (D == 64) return {32, 4, 4, 2, w8};
+  if (D == 128) return {32, w8 ? 4 : 8, 4, 2, true};
+  if (w8 && SL8_W8_Q16) return {16, 8, 4, 1, true};
+  return {32 * wide_ng(256), 4, 4, 1, true};
 }
 
 FwdGeom fwd_geometry(const FwdKernel& kn, int64_t heads, int64_t M, int64_t N, bool causal,
@@ -1326,11 +1288,11 @@ FwdGeom fwd_geometry(const FwdKernel& kn, int64_t heads, int64_t M, int64_t N, b
                                   : !windowed && even(kn.wide, skewed, 1);
     if (wide) return {kn.wide, skewed && even(kn.wide, true, 1), false};
   }
-  // Two workgroups to a CU: pairs only as one even round (D = 64, 16 heads x 8192: 193 us against
-  // 199; 32 heads, two rounds: 377 / 369), then with windows too (D = 128, 32 x 4096, window 512:
-  // 49 / 53)
+  // Two workgroups to a CU: pairs only as one even round (W8A8, D = 64, 32 heads x 4096: 117 us
+  // against 118, two rounds of them 409 / 391; D = 128, 32 x 4096, window 512: 50 / 53), and never
+  // for D = 64, whose blocks are the shortest (32 x 4096: 92 / 87; 64 x 2048: 54 / 49)
   const int64_t pairs = grid(kn.narrow, true), blocks = grid(kn.narrow, false);
-  bool paired = ramp && even(kn.narrow, true, kn.cap) && (kn.cap == 1 || pairs <= cus * kn.cap);
+  bool paired = kn.pairs && ramp && even(kn.narrow, true, kn.cap) && (kn.cap == 1 || pairs <= cus * kn.cap);
   // D = 128, one pair to a CU: no wave shares its SIMD, and the second pass is paid back from 4096
   // keys on (8 heads x 8192: 138 / 146 us; 16 x 4096: 78 / 78; 32 x 2048: 47 / 44)
   if (kn.wide != kn.narrow && kn.cap > 1 && skewed && N >= 4096 && pairs <= cus &&
@@ -1347,7 +1309,7 @@ FwdGeom fwd_geometry(const FwdKernel& kn, int64_t heads, int64_t M, int64_t N, b
 // best count of 1 to 16 at 100 of 105 shapes. Kernel times, causal, one part -> parts taken, in us:
 //   4 heads x 64 queries, 8192 keys, D = 128      124 -> 29 (16)
 //   16 heads, 256 x 16384                         242 -> 53 (7);    D = 256: 573 -> 104 (8)
-//   16 heads, 1000 x 6121                          96 -> 62 (4);    D = 64: 117 -> 54 (4)
+//   16 heads, 1000 x 6121                          96 -> 62 (4);    D = 64: 72 us a part, 47 (4)
 //   16 heads, 2048 x 2048: 40 in one part, 43 in two
 int fwd_parts(const FwdKernel& kn, int64_t DP, int64_t heads, int64_t M, int64_t N, bool causal,
               int64_t window_left) {
@@ -1356,7 +1318,7 @@ int fwd_parts(const FwdKernel& kn, int64_t DP, int64_t heads, int64_t M, int64_t
   int64_t keys = N;
   if (window_left >= 0) keys = std::min(N, window_left + bm + BN);
   const int64_t nt = (keys + BN - 1) / BN;
-  const double tile = DP == 64 ? 1.2 : DP == 128 ? 1.0 : 2.3, pair = DP == 64 ? 0.4 : 0.75;
+  const double tile = DP == 64 ? 0.9 : DP == 128 ? 1.0 : 2.3, pair = DP == 64 ? 0.3 : 0.75;
   const bool skewed = causal && 2 * M > N && (window_left < 0 || 2 * window_left > N);
   int best = 1;
   double best_t = 1e30;

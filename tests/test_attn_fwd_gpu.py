@@ -378,7 +378,7 @@ GEOMETRIES = [
     (False, 1, 40, 8, 1000, 1000, 128, True, -1),    # 4 waves, folded, heads that do not divide 256
     (False, 1, 8, 2, 300, 700, 128, True, -1),       # 4 waves, heaviest first
     (False, 3, 40, 8, 1100, 1100, 128, True, 300),   # 4 waves, window
-    (False, 4, 16, 4, 2048, 2048, 64, True, -1),     # pairs
+    (False, 4, 16, 4, 2048, 2048, 64, True, -1),     # heaviest first
     (False, 1, 32, 8, 1100, 1100, 64, True, -1),     # folded
     (False, 1, 32, 8, 2048, 2048, 256, True, -1),    # pairs
     (False, 2, 16, 4, 700, 700, 256, True, -1),      # heaviest first

@@ -20,6 +20,8 @@
 // operands, P = 256 B_hi + B_lo, two MFMAs into T_lo, T_hi, and f += d * (T_lo + 256 T_hi) per
 // super-block (details at the kernel).
 
+#include <type_traits>
+
 #include "kquant.hpp"
 
 namespace sl8 {
@@ -594,7 +596,8 @@ void launch_gemv_kq_m(const int8_t* x, const float* xs, const uint8_t* w, void* 
 // up to Q6CH super-blocks; a lane 4 r + c loads 16-byte piece c of each
 // 64-byte part (ql halves, qh) of weight row r. Q6_K blocks are 210 bytes,
 // so odd super-blocks start 2 bytes off a dword: pieces are read as 5
-// aligned dwords and v_alignbyte.
+// aligned dwords and v_alignbyte (PIPE: 2-byte aligned loads, 3 to 7 % slower
+// where nothing runs ahead).
 // ---------------------------------------------------------------------------
 #ifndef SL8_Q6W  // measured at config 4's shape, M = 8: 8 x 3 27.6 us, 10 x 2 33.9, 5 x 4 34.3, 6 x 4 34.2
 #define SL8_Q6W 8
@@ -614,11 +617,25 @@ __device__ __forceinline__ uint4 load16_a2(const uint8_t* p, uint32_t sh) {
   return make_uint4(__builtin_amdgcn_alignbyte(d.y, d.x, sh), __builtin_amdgcn_alignbyte(d.z, d.y, sh),
                     __builtin_amdgcn_alignbyte(d.w, d.z, sh), __builtin_amdgcn_alignbyte(e, d.w, sh));
 }
+// ... and 16 or 4 bytes there in one 2-byte aligned load each, whose result is not touched
+typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32_a2 __attribute__((aligned(2)));
+__device__ __forceinline__ uint4 load16_u(const uint8_t* p) {
+  const u32x4_a2 d = *reinterpret_cast<const u32x4_a2*>(p);
+  return make_uint4(d.x, d.y, d.z, d.w);
+}
 
-template <int OUT_DT, int MB>  // MB blocks of 4 activation rows
+// MB blocks of 4 activation rows. PIPE: chunks of 2 super-blocks, the next one's weights on their
+// way into registers while one is computed; its activations, from L2, are copied after that (a copy
+// into LDS under way makes every LDS read wait). For M <= 8 and K past one chunk per wave: 5120 x
+// 17408, M = 4 / 8: 29.9 / 33.3 us without, 27.9 / 30.9 with it. M > 8 takes chunks of 2 as well,
+// whose activations leave LDS for two workgroups per CU (with PIPE its registers would not): 17408 x
+// 5120, M = 16: 52.8 -> 36.7 us.
+template <int OUT_DT, int MB, bool PIPE>
 __global__ void __launch_bounds__(64 * Q6W)
 gemv_q6k_mfma_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_scale,
                      const uint8_t* __restrict__ w, void* __restrict__ out, int M, int N, int K) {
+  constexpr int CH = PIPE || MB == 4 ? 2 : Q6CH, XP = CH * 256;
   extern __shared__ __attribute__((aligned(16))) int8_t xq6[];  // per wave: M rows + a zero row
   __shared__ float red6[Q6W - 1][MB][16][4];
   const int lane = threadIdx.x & 63;
@@ -630,47 +647,63 @@ gemv_q6k_mfma_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
   const int64_t row_bytes = (int64_t)nsb * Q6K_BYTES;
   const uint8_t* wrow = w + (int64_t)min(n0 + lr, N - 1) * row_bytes;
   const int gA = lj >> 2, mA = lj & 3;       // A row lj = 4 gA + mA
-  const int xarea = (M * Q6XP + 1023) & ~1023;
-  int8_t* xw = xq6 + (int64_t)wave * (xarea + Q6XP);
+  const int xarea = (M * XP + 1023) & ~1023;
+  int8_t* xw = xq6 + (int64_t)wave * (xarea + XP);
   int8_t* xz = xw + xarea;                   // zero row
-  for (int i = lane; i < Q6XP / 16; i += 64) reinterpret_cast<uint4*>(xz)[i] = make_uint4(0, 0, 0, 0);
+  for (int i = lane; i < XP / 16; i += 64) reinterpret_cast<uint4*>(xz)[i] = make_uint4(0, 0, 0, 0);
   const int8_t* xrow[MB];
 #pragma unroll
-  for (int t = 0; t < MB; ++t) xrow[t] = (gA == h && 4 * t + mA < M) ? xw + (4 * t + mA) * Q6XP : xz;
-
+  for (int t = 0; t < MB; ++t) xrow[t] = (gA == h && 4 * t + mA < M) ? xw + (4 * t + mA) * XP : xz;
   float f[MB][4];
 #pragma unroll
   for (int t = 0; t < MB; ++t)
 #pragma unroll
     for (int r = 0; r < 4; ++r) f[t][r] = 0.f;
 
-  auto chunk = [&](const int c0, const int cnt) {
-    uint4 qlp[Q6CH][2], qhp[Q6CH];
-    uint32_t scw[Q6CH], dw[Q6CH];
+  struct Part {
+    uint4 qlp[CH][2], qhp[CH];
+    uint32_t scw[CH], dw[CH];
+  };
+  auto load = [&](const int c0, Part& p) __attribute__((always_inline)) {
+    auto& [qlp, qhp, scw, dw] = p;
 #pragma unroll
-    for (int i = 0; i < Q6CH; ++i) {
+    for (int i = 0; i < CH; ++i) {
       const int sb = min(c0 + i, nsb - 1);
       const uint8_t* blk = wrow + (int64_t)sb * Q6K_BYTES;
-      const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(blk) & 3);
-      qlp[i][0] = load16_a2(blk + 16 * lc, sh);
-      qlp[i][1] = load16_a2(blk + 64 + 16 * lc, sh);
-      qhp[i] = load16_a2(blk + 128 + 16 * lc, sh);
-      const uint32_t* sp = reinterpret_cast<const uint32_t*>(reinterpret_cast<uintptr_t>(blk + 192 + 4 * lc) & ~(uintptr_t)3);
-      // sp[1] only when misaligned (aligned: it lies past the block for lc = 3);
-      // d by a 16-bit load (2-byte aligned), never past the block
-      scw[i] = __builtin_amdgcn_alignbyte(sp[sh ? 1 : 0], sp[0], sh);  // scales 4 lc .. 4 lc + 3
+      if constexpr (PIPE) {
+        qlp[i][0] = load16_u(blk + 16 * lc);
+        qlp[i][1] = load16_u(blk + 64 + 16 * lc);
+        qhp[i] = load16_u(blk + 128 + 16 * lc);
+        scw[i] = *reinterpret_cast<const u32_a2*>(blk + 192 + 4 * lc);  // scales 4 lc .. 4 lc + 3
+      } else {
+        const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(blk) & 3);
+        qlp[i][0] = load16_a2(blk + 16 * lc, sh);
+        qlp[i][1] = load16_a2(blk + 64 + 16 * lc, sh);
+        qhp[i] = load16_a2(blk + 128 + 16 * lc, sh);
+        const uint32_t* sp = reinterpret_cast<const uint32_t*>(reinterpret_cast<uintptr_t>(blk + 192 + 4 * lc) & ~(uintptr_t)3);
+        // sp[1] only when misaligned (aligned: it lies past the block for lc = 3);
+        // d by a 16-bit load (2-byte aligned), never past the block
+        scw[i] = __builtin_amdgcn_alignbyte(sp[sh ? 1 : 0], sp[0], sh);
+      }
       dw[i] = *reinterpret_cast<const uint16_t*>(blk + 208);
     }
-    const int xch = M * (Q6XP / 16);
+    if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);  // issued before the compute that hides them
+  };
+  auto load_x = [&](const int c0, const int cnt) __attribute__((always_inline)) {
+    const int xch = M * (XP / 16);
     for (int j = 0; j * 64 < xch; ++j) {
       const int id = min(j * 64 + lane, xch - 1);
-      const int m = id / (Q6XP / 16), pos = min(id % (Q6XP / 16), cnt * 16 - 1);
+      const int m = id / (XP / 16), pos = min(id % (XP / 16), cnt * 16 - 1);
       __builtin_amdgcn_global_load_lds((kq_gptr_t)(x + (int64_t)m * K + (int64_t)c0 * 256 + 16 * pos),
                                        (kq_lptr_t)(xw + j * 1024), 16, 0, 0);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);
+  };
+  auto compute = [&](const int cnt, const Part& p) __attribute__((always_inline)) {
+    const auto& [qlp, qhp, scw, dw] = p;
 #pragma unroll
-    for (int i = 0; i < Q6CH; ++i) {
+    for (int i = 0; i < CH; ++i) {
       if (i < cnt) {
         const float d = h2f((uint16_t)q6_pull(dw[i], 4 * lj));  // column lj's d (lane 4 lj loaded it)
         // exact integer sums of this lane's 4 sub-blocks of the super-block:
@@ -725,10 +758,35 @@ gemv_q6k_mfma_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
   };
 
   const int sb0 = (wave * nsb) / Q6W, sb1 = ((wave + 1) * nsb) / Q6W;
-  if (sb1 - sb0 <= Q6CH) {
-    if (sb1 > sb0) chunk(sb0, sb1 - sb0);
+  Part pa;
+  if constexpr (PIPE) {
+    Part pb;
+    if (sb0 < sb1) load(sb0, pa);
+    for (int c = sb0; c < sb1; c += 2 * CH) {
+      const int c1 = c + CH, c2 = c + 2 * CH;
+      load_x(c, min(CH, sb1 - c));
+      if (c1 < sb1) load(c1, pb);
+      compute(min(CH, sb1 - c), pa);
+      __builtin_amdgcn_wave_barrier();  // the next chunk's copies overwrite what was read
+      if (c1 >= sb1) break;
+      load_x(c1, min(CH, sb1 - c1));
+      if (c2 < sb1) load(c2, pa);
+      compute(min(CH, sb1 - c1), pb);
+      __builtin_amdgcn_wave_barrier();
+    }
+  } else if (sb1 - sb0 <= CH) {  // one chunk
+    if (sb1 > sb0) {
+      load(sb0, pa);
+      load_x(sb0, sb1 - sb0);
+      compute(sb1 - sb0, pa);
+    }
   } else {
-    for (int c0 = sb0; c0 < sb1; c0 += Q6CH) chunk(c0, min(Q6CH, sb1 - c0));
+    for (int c = sb0; c < sb1; c += CH) {
+      load(c, pa);
+      load_x(c, min(CH, sb1 - c));
+      compute(min(CH, sb1 - c), pa);
+      __builtin_amdgcn_wave_barrier();
+    }
   }
   // C rows 4 g + r (g = lane / 16): sum the 4 sub-block groups, then the waves in fixed order
 #pragma unroll
@@ -762,15 +820,25 @@ gemv_q6k_mfma_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
 void launch_gemv_q6k_mfma(const int8_t* x, const float* xs, const uint8_t* w, void* out, int odt,
                           int M, int N, int K, hipStream_t st) {
   const dim3 grid((unsigned)((N + 15) / 16));
-  const size_t lds = (size_t)Q6W * ((((size_t)M * Q6XP + 1023) & ~(size_t)1023) + Q6XP);
-#define SL8_Q6M(MB)                                                                                   \
-  switch (odt) {                                                                                      \
-    case SL8_DTYPE_F16: gemv_q6k_mfma_kernel<SL8_DTYPE_F16, MB><<<grid, 64 * Q6W, lds, st>>>(x, xs, w, out, M, N, K); break; \
-    case SL8_DTYPE_BF16: gemv_q6k_mfma_kernel<SL8_DTYPE_BF16, MB><<<grid, 64 * Q6W, lds, st>>>(x, xs, w, out, M, N, K); break; \
-    default: gemv_q6k_mfma_kernel<SL8_DTYPE_F32, MB><<<grid, 64 * Q6W, lds, st>>>(x, xs, w, out, M, N, K); break; \
-  }
-  if (M <= 4) { SL8_Q6M(1) } else if (M <= 8) { SL8_Q6M(2) } else { SL8_Q6M(4) }
-#undef SL8_Q6M
+  const bool pipe = M <= 8 && (K >> 8) > Q6W * Q6CH;
+  const size_t xp = pipe || M > 8 ? 512 : Q6XP;  // a chunk's activation row
+  const size_t lds = (size_t)Q6W * ((((size_t)M * xp + 1023) & ~(size_t)1023) + xp);
+  auto go = [&](auto mb, auto pp) {
+    constexpr int MB = decltype(mb)::value;
+    constexpr bool P = decltype(pp)::value;
+    switch (odt) {
+      case SL8_DTYPE_F16: gemv_q6k_mfma_kernel<SL8_DTYPE_F16, MB, P><<<grid, 64 * Q6W, lds, st>>>(x, xs, w, out, M, N, K); break;
+      case SL8_DTYPE_BF16: gemv_q6k_mfma_kernel<SL8_DTYPE_BF16, MB, P><<<grid, 64 * Q6W, lds, st>>>(x, xs, w, out, M, N, K); break;
+      default: gemv_q6k_mfma_kernel<SL8_DTYPE_F32, MB, P><<<grid, 64 * Q6W, lds, st>>>(x, xs, w, out, M, N, K); break;
+    }
+  };
+  auto by_rows = [&](auto pp) {
+    if (M <= 4) go(std::integral_constant<int, 1>{}, pp);
+    else if (M <= 8) go(std::integral_constant<int, 2>{}, pp);
+    else go(std::integral_constant<int, 4>{}, std::false_type{});
+  };
+  if (pipe) by_rows(std::true_type{});
+  else by_rows(std::false_type{});
 }
 
 // smallest M on the int8 MFMA GEMVs (below: the VALU kernels). Config 4's

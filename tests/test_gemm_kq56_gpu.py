@@ -182,3 +182,15 @@ def test_rejects(device, fmt):
         getattr(_C, FMT[fmt][4])(torch.zeros(2, 256, device=device, dtype=torch.int8),
                                  torch.ones(2, device=device),
                                  torch.zeros(8, 144, device=device, dtype=torch.uint8))
+
+
+# chunks per wave of the Q6_K decode GEMV: one chunk and just past it (24 and 25 super-blocks), the
+# last chunk short or whole, waves with unequal counts; M > 8 takes smaller chunks
+@pytest.mark.parametrize("nsb", [16, 17, 24, 25, 33, 47])
+@pytest.mark.parametrize("M", [2, 4, 5, 8, 9, 16])
+def test_q6k_decode_chunks(device, M, nsb):
+    N, K = 33, 256 * nsb
+    x, w, wd = _case("q6k", M, N, K, seed=M * 100 + nsb, device=device)
+    x_i8, xs = _C.quantize_i8_rowwise(x)
+    y = _C.gemm_decode_q6k(x_i8, xs, wd, torch.float32)
+    _check_exact_sum(y, FMT["q6k"][2](_np(x_i8), _np(xs), w, K), torch.float32)

@@ -56,13 +56,18 @@ def attn_int8_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: 
         # attention and leave the GPU idle during the next enqueue)
         flag, flag_host, flag_ready = fired
         q_i8, q_scale, k_i8, k_scale, _k_mean = qk
+        refused = None
         try:
             out = _C.attn_int8_fwd(q_i8, q_scale.squeeze(-1).contiguous(), k_i8,
                                    k_scale.squeeze(-1).contiguous(), v.contiguous(), causal,
                                    window_left, gate_flag=flag)
+        except RuntimeError as e:  # a V that only full precision takes: the gate decides first
+            refused = e
         finally:
             flag_ready.synchronize()  # before flag_host is read, or let go
         if int(flag_host[0]) == 0:
+            if refused is not None:
+                raise refused
             return out
         fired = True
     if fired:

@@ -77,3 +77,24 @@ def test_gate_rejects(device):
         _C.q_outlier_gate(torch.randn(2, 300, device=device, dtype=torch.float16))
     flag, st = _C.q_outlier_gate(torch.empty(0, 64, device=device, dtype=torch.float16), stats=True)
     assert flag.item() == 0 and st.shape == (0, 2)
+
+
+@pytest.mark.parametrize("dtype,D,Dv,v_dtype", [(torch.bfloat16, 128, 128, torch.float32),
+                                                (torch.bfloat16, 64, 32, torch.bfloat16),
+                                                (torch.float16, 72, 72, torch.float32),
+                                                (torch.float16, 128, 128, torch.float32)])
+def test_gate_fires_before_v_is_refused(device, dtype, D, Dv, v_dtype):
+    """A firing gate sends the call to full precision whatever V is; the int8 path refuses a V it
+    does not take only where the gate does not fire."""
+    import torch.nn.functional as F
+
+    import superl8_amd as sl8
+
+    q, k = (torch.randn(1, 2, 40, D, device=device).to(dtype) for _ in range(2))
+    v = torch.randn(1, 2, 40, Dv, device=device).to(v_dtype)
+    with pytest.raises(RuntimeError, match="v must be|K/V shape"):
+        sl8.attn_int8_fwd(q, k, v, causal=True)
+    q[0, 0, 0, 3] = 500.0
+    out = sl8.attn_int8_fwd(q, k, v, causal=True)
+    ref = F.scaled_dot_product_attention(q, k, v.to(dtype), is_causal=True, scale=D ** -0.5)
+    assert out.dtype == v_dtype and torch.equal(out, ref.to(v_dtype))

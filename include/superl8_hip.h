@@ -408,11 +408,15 @@ int sl8_dequant_q4k(const uint8_t* w, float* out, int64_t N, int64_t K, void* st
 /* The k-quant GEMMs with scratch: fmt 4, 5, 6 = Q4_K, Q5_K, Q6_K; otherwise as sl8_gemm_q4k /
  * _q5k / _q6k (below), which are this call without a workspace. With sl8_gemm_kq_workspace()
  * bytes (16-byte aligned, uninitialised; 0: nothing to gain) the activations are prepared once in
- * scratch (Q4_K, Q5_K) and output tiles that do not fill a round of the chip are split over K and
- * summed by a second launch.
+ * scratch (Q4_K, Q5_K: 2 1/8 bytes each) and output tiles that do not fill a round of the chip are
+ * split over K and summed by a second launch. Without, every K sum runs in one workgroup: M = 512,
+ * N = 17408, K = 5120 takes 107 us (Q4_K) with scratch and 125 without, Q5_K 114 and 158.
  * sl8_linear_kq: the same (Q4_K, Q5_K; M > 16; the workspace required) from fp16 / bf16 rows x
  * [M, K], quantised as sl8_quantize_i8_rowwise in that preparation (reference
- * superl8/ops.py:1254-1325). */
+ * superl8/ops.py:1254-1325).
+ * sl8_gemm_kq_plan: how such a call (M > 16) is cut on this device, with scratch or without:
+ * plan[0] rows of an output tile (of 128 columns), [1] whole tiles, [2] tiles split over K, [3]
+ * their K parts, [4] tiles of 128 rows cut in row quarters instead. For tests and tuning. */
 size_t sl8_gemm_kq_workspace(int fmt, int64_t M, int64_t N, int64_t K);
 int sl8_gemm_kq(int fmt, const int8_t* x, const float* x_scale, const uint8_t* w, void* out,
                 int out_dtype, int64_t M, int64_t N, int64_t K, void* workspace,
@@ -420,6 +424,7 @@ int sl8_gemm_kq(int fmt, const int8_t* x, const float* x_scale, const uint8_t* w
 int sl8_linear_kq(int fmt, const void* x, int x_dtype, const uint8_t* w, void* out, int out_dtype,
                   int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
                   void* stream);
+int sl8_gemm_kq_plan(int fmt, int64_t M, int64_t N, int64_t K, int scratch, int64_t* plan);
 
 /* ------------------------------------------------------------------------
  * GGUF Q5_K / Q6_K linear (native 176 / 210-byte super-blocks), same

@@ -82,6 +82,7 @@ SIGNATURES = {
     "sl8_gemm_kq_workspace": (_SZ, [_I, _I64, _I64, _I64]),
     "sl8_gemm_kq": (_I, [_I, _P, _P, _P, _P, _I, _I64, _I64, _I64, _P, _SZ, _P]),
     "sl8_linear_kq": (_I, [_I, _P, _I, _P, _P, _I, _I64, _I64, _I64, _P, _SZ, _P]),
+    "sl8_gemm_kq_plan": (_I, [_I, _I64, _I64, _I64, _I, ctypes.POINTER(_I64)]),
     "sl8_gemm_q5k": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),
     "sl8_gemm_q6k": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),
     "sl8_gemm_decode_q5k": (_I, [_P, _P, _P, _P, _I, _I64, _I64, _I64, _P]),

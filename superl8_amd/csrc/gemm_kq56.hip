@@ -889,25 +889,46 @@ int check_kq(const char* name, const int8_t* x, const float* xs, const uint8_t* 
 
 }  // namespace
 
-TilePlan plan_q6_tile(int M, int N, int K, bool may_split) {
-  return plan_tiles(M, N, K, SHAPES6, 3, may_split);
+TilePlan plan_q6_tile(int M, int N, int K) { return plan_tiles(M, N, K, SHAPES6, 3, true); }
+
+// Without scratch the last round's tiles run as row quarters where that is faster (M = 512, N =
+// 17408, K = 5120: 186 us, 208 with every tile whole; 1000 x 5120 x 17408: 372 / 445).
+TailPlan plan_q6_whole(int M, int N, int K, TilePlan& tiles) {
+  TailPlan p = plan_tail(M, N, K, SHAPES6[0], SHAPES6[2]);
+  tiles = plan_tiles(M, N, K, SHAPES6, 3, false);
+  if (tiles.us <= p.us) p.whole = 0;
+  return p;
 }
 
-void launch_q6_tile(const TilePlan& p, const int8_t* x, const float* xs, const uint8_t* w, void* out,
-                    int odt, int M, int N, int K, float* part, hipStream_t st) {
-  const TileShape& s = SHAPES6[p.shape];
-  const TileWork tw = tile_work(p, s, M, part);
-  const unsigned grid = (unsigned)(p.nfull + p.nsplit * p.S);
-  auto go = [&](auto dt) {
-    constexpr int DT = decltype(dt)::value;
-    if (p.shape == 0) gemm_q6k_tile_kernel<DT, 4><<<grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
-    else if (p.shape == 1) gemm_q6k_tile_kernel<DT, 2><<<grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
-    else gemm_q6k_tile_kernel<DT, 1><<<grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
+void launch_q6_tile(const int8_t* x, const float* xs, const uint8_t* w, void* out, int odt, int M,
+                    int N, int K, float* part, hipStream_t st) {
+  auto go = [&](int shape, int64_t grid, const TileWork& tw) {
+    auto by_dt = [&](auto dt) {
+      constexpr int DT = decltype(dt)::value;
+      if (shape == 0) gemm_q6k_tile_kernel<DT, 4><<<(unsigned)grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
+      else if (shape == 1) gemm_q6k_tile_kernel<DT, 2><<<(unsigned)grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
+      else gemm_q6k_tile_kernel<DT, 1><<<(unsigned)grid, 256, 0, st>>>(x, xs, w, out, M, N, K, tw);
+    };
+    if (odt == SL8_DTYPE_F16) by_dt(std::integral_constant<int, SL8_DTYPE_F16>{});
+    else if (odt == SL8_DTYPE_BF16) by_dt(std::integral_constant<int, SL8_DTYPE_BF16>{});
+    else by_dt(std::integral_constant<int, SL8_DTYPE_F32>{});
   };
-  if (odt == SL8_DTYPE_F16) go(std::integral_constant<int, SL8_DTYPE_F16>{});
-  else if (odt == SL8_DTYPE_BF16) go(std::integral_constant<int, SL8_DTYPE_BF16>{});
-  else go(std::integral_constant<int, SL8_DTYPE_F32>{});
-  if (p.nsplit) launch_kq_reduce(p, s, tw, xs, out, odt, M, N, st);
+  TilePlan p;
+  if (part) {
+    p = plan_q6_tile(M, N, K);
+  } else {
+    const TailPlan tail = plan_q6_whole(M, N, K, p);
+    if (tail.whole) {
+      TileWork tw{tail.nt_x, xcd_rows(tail.nt_x, M, SHAPES6[0].bm), (int)tail.whole, 1, 0, nullptr, -1};
+      go(0, tail.whole, tw);
+      tw.quarter0 = (int)tail.whole;
+      if (tail.cut) go(2, 4 * tail.cut, tw);
+      return;
+    }
+  }
+  const TileWork tw = tile_work(p, SHAPES6[p.shape], M, part);
+  go(p.shape, p.nfull + p.nsplit * p.S, tw);
+  if (p.nsplit) launch_kq_reduce(p, SHAPES6[p.shape], tw, xs, out, odt, M, N, st);
 }
 
 }  // namespace sl8
@@ -917,8 +938,29 @@ using namespace sl8;
 extern "C" size_t sl8_gemm_kq_workspace(int fmt, int64_t M, int64_t N, int64_t K) {
   if (fmt < 4 || fmt > 6 || M <= 16 || N <= 0 || K <= 0 || K > 65536 || M >= (1LL << 31) || N >= (1LL << 31))
     return 0;
-  if (fmt == 6) return plan_q6_tile((int)M, (int)N, (int)K, true).part_bytes;
+  if (fmt == 6) return plan_q6_tile((int)M, (int)N, (int)K).part_bytes;
   return q45_tile_workspace(fmt, (int)M, (int)N, (int)K);
+}
+
+extern "C" int sl8_gemm_kq_plan(int fmt, int64_t M, int64_t N, int64_t K, int scratch, int64_t* plan) {
+  clear_error();
+  SL8_CHECK_ARG(fmt >= 4 && fmt <= 6 && M > 16 && N > 0 && K > 0 && K <= 65536 && K % 256 == 0 &&
+                    M < (1LL << 31) && N < (1LL << 31) && plan,
+                "gemm_kq_plan: bad arguments");
+  const int m = (int)M, n = (int)N, k = (int)K;
+  TilePlan t{};
+  TailPlan tail{};
+  if (!scratch || (fmt == 6 && sl8_gemm_kq_workspace(fmt, M, N, K) == 0))
+    tail = fmt == 6 ? plan_q6_whole(m, n, k, t) : plan_q45_whole(fmt, m, n, k, t);
+  else
+    t = fmt == 6 ? plan_q6_tile(m, n, k) : plan_q45_tile(fmt, m, n, k);
+  const bool cut = tail.whole > 0;
+  plan[0] = cut ? 128 : 128 >> t.shape;  // (every format's shapes are 128, 64 and 32 rows)
+  plan[1] = cut ? tail.whole : t.nfull;
+  plan[2] = cut ? 0 : t.nsplit;
+  plan[3] = cut ? 1 : t.S;
+  plan[4] = cut ? tail.cut : 0;
+  return SL8_OK;
 }
 
 extern "C" int sl8_gemm_kq(int fmt, const int8_t* x, const float* x_scale, const uint8_t* w, void* out,
@@ -937,9 +979,7 @@ extern "C" int sl8_gemm_kq(int fmt, const int8_t* x, const float* x_scale, const
   const size_t need = sl8_gemm_kq_workspace(fmt, M, N, K);
   if (!(workspace && workspace_bytes >= need && aligned(workspace, 16))) workspace = nullptr;
   if (fmt == 6) {
-    const TilePlan p = plan_q6_tile((int)M, (int)N, (int)K, workspace != nullptr);
-    launch_q6_tile(p, x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K,
-                   static_cast<float*>(workspace), st);
+    launch_q6_tile(x, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K, static_cast<float*>(workspace), st);
   } else {
     launch_q45_tile(fmt, x, SL8_KQ_I8, x_scale, w, out, out_dtype, (int)M, (int)N, (int)K, workspace, st);
   }

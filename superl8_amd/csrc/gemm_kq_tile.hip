@@ -24,7 +24,8 @@
 //   * weights: raw super-blocks, global -> LDS by DMA one super-block ahead;
 //   * activations: the codes as fp16 in the order below and their 16-element sums, made once per
 //     call by kq_prep_* and copied global -> LDS by DMA one phase (1 / PH of a super-block) ahead.
-//     XI8: no scratch for those was given; int8 codes go through registers instead;
+//     XI8: no scratch for those was given; int8 codes go through registers instead (64-row tiles
+//     where they are faster than gemm_kq_tile_i8.hip's: plan_q45_whole);
 //   * operand order: lane half h of the MFMA holds the elements of sub-blocks 4 h .. 4 h + 3, so a
 //     lane's weight bytes are contiguous (64 of a super-block's 128) and its scales are one dword.
 //     MFMA step t of a super-block: 8 elements 8 p .. of sub-block 4 h + 2 hs + hi, with t =
@@ -466,10 +467,21 @@ gemm_kq_reduce_kernel(const float* __restrict__ x_scale, void* __restrict__ out,
 // chip, then the remaining tiles, each split over K into S parts (of at least two super-blocks) if
 // that is faster with the partials' traffic. A round that leaves workgroup slots of a CU empty is
 // faster per workgroup, but not in proportion.
+// us of nsb super-blocks of n workgroups of a shape, in rounds over P CUs
+static double rounds_us(int64_t n, int P, int nsb, const TileShape& s) {
+  const int64_t slots = (int64_t)P * s.wgs_per_cu, rem = n % slots;
+  double t = (double)(n / slots) * nsb * s.us_per_sb;
+  if (rem) {
+    const int64_t k = (rem + P - 1) / P;  // workgroups per CU
+    t += (double)nsb * s.us_per_sb * (0.3 + 0.7 * (double)k / s.wgs_per_cu);
+  }
+  return t;
+}
+
 TilePlan plan_tiles(int M, int N, int K, const TileShape* shapes, int count, bool may_split) {
   const int P = cu_count(), nsb = K >> 8;
   TilePlan best{};
-  double best_t = 1e30;
+  best.us = 1e30;
   for (int i = 0; i < count; ++i) {
     const TileShape& s = shapes[i];
     const int nt_x = (N + s.bn - 1) / s.bn;
@@ -477,20 +489,22 @@ TilePlan plan_tiles(int M, int N, int K, const TileShape* shapes, int count, boo
     const int64_t slots = (int64_t)P * s.wgs_per_cu, full = T / slots, rem = T % slots;
     const int smax = may_split && rem ? (int)std::max<int64_t>(1, std::min<int64_t>({slots / rem, nsb / 2, 16})) : 1;
     for (int S = 1; S <= smax; ++S) {
-      double t = (double)full * nsb * s.us_per_sb;
-      if (rem) {
-        const int64_t k = (rem * S + P - 1) / P;  // workgroups per CU
-        t += (double)((nsb + S - 1) / S) * s.us_per_sb * (0.3 + 0.7 * (double)k / s.wgs_per_cu);
-      }
+      double t = rounds_us(full * slots, P, nsb, s) + rounds_us(rem * S, P, (nsb + S - 1) / S, s);
       if (S > 1) t += 3.0 + (double)rem * S * s.bm * s.bn * 8 / 5e6;
-      if (t < best_t) {
-        best_t = t;
-        best = TilePlan{i, nt_x, S, S > 1 ? T - rem : T, S > 1 ? rem : 0, 0};
-      }
+      if (t < best.us) best = TilePlan{i, nt_x, S, S > 1 ? T - rem : T, S > 1 ? rem : 0, 0, t};
     }
   }
   best.part_bytes = (size_t)best.nsplit * best.S * shapes[best.shape].bm * shapes[best.shape].bn * 4;
   return best;
+}
+
+TailPlan plan_tail(int M, int N, int K, const TileShape& tile, const TileShape& quarter) {
+  const int P = cu_count(), nsb = K >> 8, nt_x = (N + tile.bn - 1) / tile.bn;
+  const int64_t T = (int64_t)nt_x * ((M + tile.bm - 1) / tile.bm), rem = T % P;
+  const int64_t cut = T >= P && rem <= P / 2 ? rem : 0;
+  TailPlan p{nt_x, T - cut, cut, rounds_us(T - cut, P, nsb, tile)};
+  if (cut) p.us += 3.0 + rounds_us(4 * cut, P, nsb, quarter);
+  return p;
 }
 
 namespace {
@@ -498,6 +512,16 @@ namespace {
 // us_per_sb: one super-block of one workgroup with every slot of its CU taken (measured)
 constexpr TileShape SHAPES4[] = {{128, 128, 2, 4.7}, {64, 128, 2, 2.7}, {32, 128, 3, 2.5}};
 constexpr TileShape SHAPES5[] = {{128, 128, 2, 5.0}, {64, 128, 2, 3.1}, {32, 128, 2, 2.1}};
+
+// Without scratch: the int8 kernel's 128-row tiles (gemm_kq_tile_i8.hip) and row quarters, or this
+// one's 64-row tiles from int8 codes, whichever the model has faster. The latter win where the CUs
+// are not filled or a last round of the former would be long, the former at even rounds and short
+// last ones. M x N x K, us as 128-row / 64-row tiles: Q4_K 512 x 17408 x 5120 125 / 135, 512 x 5120
+// x 17408 145 / 163, 300 x 17408 x 5120 94 / 84, 32 x 4096 x 4096 35 / 27; Q5_K 512 x 5120 x 17408
+// 185 / 196, 1500 x 4096 x 4096 105 / 84.
+constexpr TileShape I8_TILE[] = {{128, 128, 1, 2.45}, {128, 128, 1, 3.15}};    // Q4_K, Q5_K
+constexpr TileShape I8_QUARTER[] = {{32, 128, 1, 1.2}, {32, 128, 1, 1.47}};
+constexpr TileShape XI8_TILE[] = {{64, 128, 2, 2.6}, {64, 128, 2, 3.2}};
 
 template <int FMT>
 void launch_tiles(const TilePlan& p, const TileX& tx, const uint8_t* w, void* out, int odt, int M,
@@ -549,14 +573,25 @@ TileScratch tile_scratch(int fmt, int M, int N, int K) {
 }  // namespace
 
 size_t q45_tile_workspace(int fmt, int M, int N, int K) { return tile_scratch(fmt, M, N, K).bytes; }
+TilePlan plan_q45_tile(int fmt, int M, int N, int K) { return tile_scratch(fmt, M, N, K).plan; }
+
+TailPlan plan_q45_whole(int fmt, int M, int N, int K, TilePlan& tiles) {
+  const int i = fmt - 4;
+  TailPlan p = plan_tail(M, N, K, I8_TILE[i], I8_QUARTER[i]);
+  tiles = plan_tiles(M, N, K, XI8_TILE + i, 1, false);
+  tiles.shape = 1;
+  if (tiles.us <= p.us) p.whole = 0;
+  return p;
+}
 
 void launch_q45_tile(int fmt, const void* x, int x_dtype, const float* xs, const uint8_t* w, void* out,
                      int odt, int M, int N, int K, void* workspace, hipStream_t st) {
-  if (!workspace) {  // int8 codes through registers, whole tiles
-    const TileShape* shapes = fmt == 4 ? SHAPES4 : SHAPES5;
-    TilePlan p = plan_tiles(M, N, K, shapes + 1, 1, false);
-    p.shape = 1;
-    const TileX tx{static_cast<const int8_t*>(x), nullptr, nullptr, xs};
+  if (!workspace) {
+    TilePlan p;
+    const int8_t* x8 = static_cast<const int8_t*>(x);
+    const TailPlan tail = plan_q45_whole(fmt, M, N, K, p);
+    if (tail.whole) return launch_q45_tile_i8(fmt, tail, x8, xs, w, out, odt, M, N, K, st);
+    const TileX tx{x8, nullptr, nullptr, xs};
     if (fmt == 4) launch_tiles<4>(p, tx, w, out, odt, M, N, K, nullptr, st);
     else launch_tiles<5>(p, tx, w, out, odt, M, N, K, nullptr, st);
     return;

@@ -60,6 +60,9 @@ void launch_gemv_q5k_small(const int8_t* x, const float* xs, const uint8_t* w, v
 void launch_gemv_q5k_mfma(const int8_t* x, const float* xs, const uint8_t* w, void* out, int odt,
                           int M, int N, int K, hipStream_t st);
 
+// XCD-aware tile order (see kq_tile_coords) when the column tiles split evenly over the 8 XCDs
+inline int xcd_rows(int nt_x, int M, int bm) { return SL8_KQ_XCD && nt_x % 8 == 0 ? (M + bm - 1) / bm : 0; }
+
 // Tiled GEMMs (M > 16): a tile shape with the workgroups of it a CU holds and the time one
 // super-block of one takes then, and the plan of a call: tiles [0, nfull) whole, nsplit more
 // tiles split S ways over K into part_bytes of fp32 partials.
@@ -71,19 +74,29 @@ struct TilePlan {
   int shape, nt_x, S;
   int64_t nfull, nsplit;
   size_t part_bytes;
+  double us;  // the model's time
 };
 TilePlan plan_tiles(int M, int N, int K, const TileShape* shapes, int count, bool may_split);
 
+// Without scratch, 128 x 128 tiles whose last round, where it would hold at most half the CUs, runs
+// as 4 row quarters each in a second launch: tiles [0, whole), then `cut` more.
+struct TailPlan {
+  int nt_x;
+  int64_t whole, cut;
+  double us;
+};
+TailPlan plan_tail(int M, int N, int K, const TileShape& tile, const TileShape& quarter);
+
 // Which part of the problem a workgroup computes: workgroups below nfull a whole tile, the others
-// a K range of tiles nfull .., S per tile, into part[tile - nfull][split][BM][BN].
+// a K range of tiles nfull .., S per tile, into part[tile - nfull][split][BM][BN]. quarter0 >= 0:
+// workgroup o computes row quarter o & 3 (the kernel's BM rows) of tile quarter0 + o / 4.
 struct TileWork {
   int nt_x, xcd_m, nfull, S, tile_elems;
   float* part;
+  int quarter0;
 };
 inline TileWork tile_work(const TilePlan& p, const TileShape& s, int M, float* part) {
-  // XCD-aware tile order (kq_tile_coords) when the column tiles split evenly over the 8 XCDs
-  const int xm = (SL8_KQ_XCD && p.nt_x % 8 == 0) ? (M + s.bm - 1) / s.bm : 0;
-  return TileWork{p.nt_x, xm, (int)p.nfull, p.S, s.bm * s.bn, part};
+  return TileWork{p.nt_x, xcd_rows(p.nt_x, M, s.bm), (int)p.nfull, p.S, s.bm * s.bn, part, -1};
 }
 struct TileRange {
   int ct, rt, sb0, sb1, sp;
@@ -92,6 +105,11 @@ struct TileRange {
 __device__ __forceinline__ TileRange tile_range(const TileWork& tw, int nsb) {
   TileRange r{0, 0, 0, nsb, 0, nullptr};
   int tile = blockIdx.x;
+  if (tw.quarter0 >= 0) {
+    kq_tile_coords(tw.quarter0 + (tile >> 2), tw.nt_x, tw.xcd_m, r.ct, r.rt);
+    r.rt = 4 * r.rt + (tile & 3);
+    return r;
+  }
   if (tile >= tw.nfull) {
     const int i = tile - tw.nfull, t = i / tw.S;
     tile = tw.nfull + t;
@@ -105,17 +123,24 @@ __device__ __forceinline__ TileRange tile_range(const TileWork& tw, int nsb) {
 }
 void launch_kq_reduce(const TilePlan& p, const TileShape& s, const TileWork& tw, const float* xs,
                       void* out, int odt, int M, int N, hipStream_t st);
-// Q6_K (gemm_kq56.hip)
-TilePlan plan_q6_tile(int M, int N, int K, bool may_split);
-void launch_q6_tile(const TilePlan& p, const int8_t* x, const float* xs, const uint8_t* w, void* out,
-                    int odt, int M, int N, int K, float* part, hipStream_t st);
+// Q6_K (gemm_kq56.hip). part: the partials of a split plan; null: a plan without (plan_q6_whole)
+TilePlan plan_q6_tile(int M, int N, int K);
+void launch_q6_tile(const int8_t* x, const float* xs, const uint8_t* w, void* out, int odt, int M,
+                    int N, int K, float* part, hipStream_t st);
+// the plan without scratch: 128-row tiles with a cut last round (whole > 0), or one tile shape
+TailPlan plan_q6_whole(int M, int N, int K, TilePlan& tiles);
 // Q4_K / Q5_K (gemm_kq_tile.hip): x int8 codes with their row scales xs (x_dtype SL8_KQ_I8), or
 // fp16 / bf16 rows that are quantised in the call (with a workspace only; 16-byte aligned).
 // workspace: q45_tile_workspace() bytes, or null.
 constexpr int SL8_KQ_I8 = 3;
 size_t q45_tile_workspace(int fmt, int M, int N, int K);
+TilePlan plan_q45_tile(int fmt, int M, int N, int K);
+TailPlan plan_q45_whole(int fmt, int M, int N, int K, TilePlan& tiles);  // as plan_q6_whole
 void launch_q45_tile(int fmt, const void* x, int x_dtype, const float* xs, const uint8_t* w, void* out,
                      int odt, int M, int N, int K, void* workspace, hipStream_t st);
+// gemm_kq_tile_i8.hip: 128-row tiles on the int8 codes
+void launch_q45_tile_i8(int fmt, const TailPlan& p, const int8_t* x, const float* xs, const uint8_t* w,
+                        void* out, int odt, int M, int N, int K, hipStream_t st);
 
 typedef __attribute__((address_space(1))) const void* kq_gptr_t;
 typedef __attribute__((address_space(3))) void* kq_lptr_t;

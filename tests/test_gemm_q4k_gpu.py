@@ -100,11 +100,9 @@ def test_tile_gemm_matches_exact_sum(device, M, N, K, odt):
     assert (err <= rtol * np.abs(ref) + 1e-5 * scale).all(), f"max err {err.max():.3e}"
 
 
-# at least one full round of 128 x 128 tiles on 256 CUs plus a short last
-# round (260 and 258 tiles): the last tiles run as row quarters in a second
-# launch; (257, 10890): the split tiles are the ragged last ones in M and N
+# more tiles than workgroup slots, ragged last ones in M and N (test_kq_tile_gpu.py has the plans)
 @pytest.mark.parametrize("M,N,K", [(160, 16635, 512), (257, 10890, 256)])
-def test_tile_gemm_last_round_split(device, M, N, K):
+def test_tile_gemm_many_tiles(device, M, N, K):
     x, w, wd = _case(M, N, K, seed=M + N, device=device)
     x_i8, xs = _C.quantize_i8_rowwise(x)
     y = _C.gemm_q4k(x_i8, xs, wd, torch.float32)
@@ -112,20 +110,6 @@ def test_tile_gemm_last_round_split(device, M, N, K):
     ref = np.concatenate([oq.gemv(xn, xsn, w[n:n + 1024], K) for n in range(0, N, 1024)], axis=1)
     err = np.abs(_np(y).astype(np.float64) - ref)
     assert (err <= 1e-5 * np.abs(ref) + 1e-5 * np.abs(ref).max()).all(), f"max err {err.max():.3e}"
-
-
-def test_tile_quarters_bit_match_full_tiles(device):
-    """The last-round quarter launch applies the full tiles' per-element
-    operations in the same order: at M = 160, N = 16635 (260 tiles in row-major
-    order on 256 CUs) tiles 256..259 -- rows 128..159, columns 16128.. -- run as
-    quarters; the same columns computed alone (130 full tiles over the sliced
-    weights) must match them bit for bit."""
-    M, N, K, c0 = 160, 16635, 512, 126 * 128
-    x, w, wd = _case(M, N, K, seed=31, device=device)
-    x_i8, xs = _C.quantize_i8_rowwise(x)
-    y = _C.gemm_q4k(x_i8, xs, wd, torch.float32)
-    y_sub = _C.gemm_q4k(x_i8, xs, wd[c0:].contiguous(), torch.float32)
-    assert torch.equal(y[:, c0:], y_sub)
 
 
 def test_tile_min_term_at_its_exactness_limits(device):
@@ -217,8 +201,8 @@ def test_gemv_per_row_scale_shaped_m1(device, M):
         _C.gemm_decode_q4k(x_i8, torch.ones(M, 3, device=device), wd, torch.float32)
 
 
-# Every tile shape of the Q4_K / Q5_K tile GEMM (32, 64, 128 rows), whole and split over K (few
-# tiles; odd counts of super-blocks, which split unevenly), with ragged rows and columns
+# Small Q4_K / Q5_K tile GEMMs, mostly of 32-row tiles split over K (odd counts of super-blocks,
+# which split unevenly), with ragged rows and columns (the other tiles: test_kq_tile_gpu.py)
 SHAPES_KQ = [(17, 40, 2304), (33, 130, 5120), (64, 1000, 2304), (65, 257, 1280), (129, 4100, 768),
              (300, 600, 3328), (200, 4096, 512)]
 
@@ -241,7 +225,7 @@ def test_tile_shapes_and_splits(device, fmt, M, N, K):
     tol = 1e-5 * np.abs(ref) + 1e-5 * np.abs(ref).max()
     y = (_C.gemm_q4k if fmt == 4 else _C.gemm_q5k)(x_i8, xs, wd, torch.float32)
     assert (np.abs(_np(y).astype(np.float64) - ref) <= tol).all()
-    # the C entry without scratch: int8 codes through registers, whole tiles
+    # the C entry without scratch
     out = torch.empty(M, N, device=device, dtype=torch.float32)
     lib = _lib.load()
     rc = getattr(lib, f"sl8_gemm_q{fmt}k")(x_i8.data_ptr(), xs.data_ptr(), wd.data_ptr(), out.data_ptr(),

@@ -189,6 +189,7 @@ int launch_quant(const void* x, const float* mean, int8_t* q, float* scale, int6
     using N1 = std::integral_constant<int, 1>;
     using N2 = std::integral_constant<int, 2>;
     using N4 = std::integral_constant<int, 4>;
+    using N5 = std::integral_constant<int, 5>;
     using N8 = std::integral_constant<int, 8>;
     if (nvec <= 16) gv(B{}, std::integral_constant<int, 16>{}, N1{});
     else if (nvec <= 32) gv(B{}, std::integral_constant<int, 32>{}, N1{});
@@ -198,7 +199,11 @@ int launch_quant(const void* x, const float* mean, int8_t* q, float* scale, int6
     else if (nvec <= 512) gv(B{}, B{}, N2{});
     // longer rows: 1024 threads, so the few rows of a decode batch (one CU each) have 16 waves
     // of loads in flight. 8 bf16 rows of 17408 (past the 16384 that 256 threads of 8 vectors
-    // held): 92.0 us in the element-wise kernel below, about 4 us here
+    // held): 92.0 us in the element-wise kernel below, about 4 us here. Rows that two workgroups a
+    // CU do not hold at once and that would leave many of 1024 threads idle take 256 threads of 4
+    // or 5 vectors: 8192 rows of 5120, fp16 30 us against 44, bf16 27 / 40 (2048 rows: 10 / 13)
+    else if (nvec <= 1024 && rows > 2 * (int64_t)cu_count()) gv(B{}, B{}, N4{});
+    else if (nvec <= 1280 && rows > 2 * (int64_t)cu_count()) gv(B{}, B{}, N5{});
     else if (nvec <= 1024) gv(L{}, L{}, N1{});
     else if (nvec <= 2048) gv(L{}, L{}, N2{});
     else if (nvec <= 4096) gv(L{}, L{}, N4{});

@@ -118,3 +118,17 @@ def test_bf16_tiny_and_huge_rows_bit_exact(device, K):
     rq, rs = oqn.quantize_rows(_np(x.float()))
     np.testing.assert_array_equal(_np(s), rs)
     np.testing.assert_array_equal(_np(q), rq)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rows", [512, 513, 1025])
+@pytest.mark.parametrize("K", [3000, 4104, 5120, 8192, 8200, 10240, 10248])
+def test_many_rows_bit_exact(device, dtype, rows, K):
+    """Rows on either side of what two 1024-thread workgroups a CU hold at once (256 threads a row
+    beyond): a sample of rows against the oracle."""
+    x = (torch.randn(rows, K, device=device) * 3).to(dtype)
+    q, s = _C.quantize_i8_rowwise(x)
+    i = torch.tensor([0, 1, rows // 2, rows - 1], device=device)
+    rq, rs = oqn.quantize_rows(_as_oracle(x[i]))
+    np.testing.assert_array_equal(_np(q[i]), rq)
+    np.testing.assert_array_equal(_np(s[i]), rs)

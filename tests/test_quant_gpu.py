@@ -132,3 +132,15 @@ def test_many_rows_bit_exact(device, dtype, rows, K):
     rq, rs = oqn.quantize_rows(_as_oracle(x[i]))
     np.testing.assert_array_equal(_np(q[i]), rq)
     np.testing.assert_array_equal(_np(s[i]), rs)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("G,N,D", [(1, 1, 8), (3, 64, 130), (3, 65, 130), (511, 70, 64), (512, 70, 64), (257, 300, 72)])
+def test_k_mean_phases(device, dtype, G, N, D):
+    """Few groups (64 row phases) and many or short ones (4): the fp64 sums differ from the exact
+    ones by N * 2^-53, so the fp32 mean by one rounding."""
+    k = (torch.randn(G, N, D, device=device) + 2).to(dtype)
+    ref = k.double().mean(-2, keepdim=True)
+    got = _C.k_mean(k)
+    assert ((got.double() - ref).abs() <= 2.0 ** -23 * ref.abs()).all()
+    assert torch.equal(got, _C.k_mean(k))

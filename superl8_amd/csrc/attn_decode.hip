@@ -1452,7 +1452,8 @@ kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __
 //   * softmax in the MFMA output layout: lane (g4, col) holds keys
 //     16 kb + 4 g4 + i of head col; logit = (acc * k_scale) * q_scale, the
 //     tile max over the lane's 16 values and the 4 lanes of the column; p
-//     stored as fp16 in LDS, one 64-key row per head (rows G..15 stay zero);
+//     stored in LDS as two fp16 parts, p rounded towards zero in
+//     row col and the rest in row G + col, 64 keys each (rows 2G..15 stay zero);
 //   * value tables (key = lane): fp16 of codebook[i] * norm for i = 0..7 per
 //     128-channel block, as a low-byte plane (2 dwords) and a high-byte plane
 //     (2 dwords), handed to the dequantising lanes by v_permlane32_swap;
@@ -1461,12 +1462,17 @@ kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __
 //     0..7, picks the fp16 values out of the table planes with v_perm_b32, and
 //     writes the half row to an 8 KB (D = 128) LDS tile, read back transposed
 //     (ds_read_b64_tr_b16) as the A operand of v_mfma_f32_16x16x32_f16
-//     (16 channels x 32 keys) against P^T (32 keys x 16 heads).
+//     (16 channels x 32 keys) against P^T (32 keys x 16 columns: the heads'
+//     P, then their rests, whose sums are added at the end).
 // Each of the next tile's loads goes into the registers of the current tile's
 // input right after its last use, so they are in flight during the rest of
-// the tile. P enters the MFMA as fp16 (relative rounding 2^-11 per
-// probability; the reference multiplies the fp32 p); the V values are exactly
-// the reference's.
+// the tile. The two parts hold p to 2^-21 (the reference multiplies the fp32 p;
+// the columns of the rests are MFMA columns that G <= 8 heads leave unused); with
+// p rounded to one fp16, whose error is least where a key's p is its tile's exact
+// maximum 1, splits of more tiles were further from 64 bits than short ones: 16
+// sequences of 1024 to 16384 keys 2.7e-4 with planned splits, 2.6e-4 with splits
+// of 256 keys, 2.1e-4 with both parts (the fp16 output alone), for 43 -> 44 us. The V values are
+// exactly the reference's.
 template <int D, int G>
 struct K3Smem {
   static constexpr int PP = 72;  // P row pitch in halves (64 keys + 8: bank spread)
@@ -1477,7 +1483,7 @@ struct K3Smem {
   union alignas(16) {
     struct {
       uint16_t v[DEC_WAVES][32 * D];   // fp16 V half tile [32 keys][D], 32-byte chunks swizzled
-      uint16_t p[DEC_WAVES][16 * PP];  // fp16 P [16 heads][64 keys]
+      uint16_t p[DEC_WAVES][16 * PP];  // fp16 P [heads, then their rests][64 keys]
       float ks[DEC_WAVES][DEC_TILE];   // the tile's k_scale
     } t;
     struct {
@@ -1517,6 +1523,13 @@ __device__ __forceinline__ uint32_t swap32_hi(uint32_t a, uint32_t b) {
   return __builtin_amdgcn_permlane32_swap(a, b, false, false)[1];
 }
 
+// x of another lane of the 16-lane row (a DPP control); lanes it gives no source keep their own
+template <int CTRL>
+__device__ __forceinline__ float row_from(float x) {
+  const int v = __float_as_int(x);
+  return __int_as_float(__builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false));
+}
+
 template <int D, int G>
 // workgroups per CU: the most that fit without spills
 __global__ void __launch_bounds__(DEC_THREADS, (D == 128 && G <= 4) ? 3 : 2)
@@ -1526,7 +1539,7 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
                   const float* __restrict__ codebook, float* __restrict__ o_part,
                   float* __restrict__ m_part, float* __restrict__ l_part, int n_len,
                   int n_splits, int h_q, int h_kv, int gsz, int bhq, const PagedArgs pg) {
-  static_assert(G <= 16, "S^T and P^T have 16 head columns");
+  static_assert(2 * G <= 16, "P^T has 16 columns: the heads' and their rests'");
   using SM = K3Smem<D, G>;
   constexpr int D4 = D / 4;
   constexpr int KS = D / 64;      // 64-channel QK steps
@@ -1563,7 +1576,7 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
     const int64_t hq = (int64_t)b * h_q + kvh * gsz + j0 + tid;
     sm.qs[tid] = tid < ng ? q_scale[hq] : 0.f;
   }
-  // P rows of the unused head columns stay zero
+  // P rows of the unused columns stay zero
   for (int i = lane; i < 16 * PP; i += 64) sm.t.p[wave][i] = 0;
   float cb[8];
 #pragma unroll
@@ -1727,11 +1740,13 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
     }
     mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float mn = fmaxf(m_run, mt * qsl);
+    // the reference point lies 11 below the maximum: p up to 2^11, the rest of a usual p an fp16
+    // normal too
+    const float mn = fmaxf(m_run, fmaf(mt, qsl, -11.f));
     const float resc = __builtin_amdgcn_exp2f(m_run - mn);  // first tile: exp2(-inf) = 0
     m_run = mn;
     float ls = 0.f;
-    uint32_t ph[4][2];
+    typedef __fp16 h2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
       float p[4];
@@ -1740,19 +1755,28 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
         p[i] = __builtin_amdgcn_exp2f(fmaf(x[kb][i], qsl, -mn));  // masked key: -inf -> 0
         ls += p[i];
       }
-      ph[kb][0] = (uint32_t)f2h_bits(p[0]) | ((uint32_t)f2h_bits(p[1]) << 16);
-      ph[kb][1] = (uint32_t)f2h_bits(p[2]) | ((uint32_t)f2h_bits(p[3]) << 16);
+      uint32_t ph[2], pl[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const h2 hi = __builtin_amdgcn_cvt_pkrtz(p[2 * i], p[2 * i + 1]);
+        h2 lo = __builtin_amdgcn_cvt_pkrtz(p[2 * i] - (float)hi[0], p[2 * i + 1] - (float)hi[1]);
+        // above 0, so that an infinite V stays infinite where the rest is 0
+        lo = __builtin_elementwise_max(lo, h2{(__fp16)0x1p-24f, (__fp16)0x1p-24f});
+        ph[i] = __builtin_bit_cast(uint32_t, hi);
+        pl[i] = __builtin_bit_cast(uint32_t, lo);
+      }
+      if (col < G) {
+        uint16_t* pr = pt + col * PP + 16 * kb + 4 * g4;
+        *reinterpret_cast<uint2*>(pr) = uint2{ph[0], ph[1]};
+        *reinterpret_cast<uint2*>(pr + G * PP) = uint2{pl[0], pl[1]};
+      }
     }
     l_lane = l_lane * resc + ls;
-    if (col < G) {
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb)
-        *reinterpret_cast<uint2*>(pt + col * PP + 16 * kb + 4 * g4) = uint2{ph[kb][0], ph[kb][1]};
-    }
     // rescale the accumulators only when some head's running max moved
     if (__builtin_amdgcn_ballot_w64(col < G && resc != 1.f)) {
+      const float ro = row_from<0x110 | G>(resc);  // column G + c takes c's (row_shr)
 #pragma unroll
-      for (int t = 0; t < DT; ++t) oacc[t] *= resc;
+      for (int t = 0; t < DT; ++t) oacc[t] *= ro;
     }
 
     // ---- PV, two 32-key halves ----
@@ -1805,13 +1829,14 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
     sm.r.m[wave][col] = m_run;
     sm.r.l[wave][col] = l_lane;
   }
-  // accumulator lane (g4, col) holds channels 16 t + 4 g4 + i of head col
-  if (col < G) {
+  // accumulator lane (g4, col) holds channels 16 t + 4 g4 + i of column col
 #pragma unroll
-    for (int t = 0; t < DT; ++t)
+  for (int t = 0; t < DT; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sm.r.o[wave][col][16 * t + 4 * g4 + i] = oacc[t][i];
-  }
+    for (int i = 0; i < 4; ++i) {
+      const float o = oacc[t][i] + row_from<0x100 | G>(oacc[t][i]);  // + column G + col's (row_shl)
+      if (col < G) sm.r.o[wave][col][16 * t + 4 * g4 + i] = o;
+    }
   __syncthreads();
 
   for (int i = tid; i < G * D; i += DEC_THREADS) {

@@ -201,7 +201,7 @@ int launch_quant(const void* x, const float* mean, int8_t* q, float* scale, int6
     // of loads in flight. 8 bf16 rows of 17408 (past the 16384 that 256 threads of 8 vectors
     // held): 92.0 us in the element-wise kernel below, about 4 us here. Rows that two workgroups a
     // CU do not hold at once and that would leave many of 1024 threads idle take 256 threads of 4
-    // or 5 vectors: 8192 rows of 5120, fp16 30 us against 44, bf16 27 / 40 (2048 rows: 10 / 13)
+    // or 5 vectors: 8192 rows of 5120, fp16 22 us against 44, bf16 22 / 40 (2048 rows: 8 / 13)
     else if (nvec <= 1024 && rows > 2 * (int64_t)cu_count()) gv(B{}, B{}, N4{});
     else if (nvec <= 1280 && rows > 2 * (int64_t)cu_count()) gv(B{}, B{}, N5{});
     else if (nvec <= 1024) gv(L{}, L{}, N1{});

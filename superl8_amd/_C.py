@@ -186,15 +186,19 @@ def quantize_qk_fused(q: torch.Tensor, k: torch.Tensor, q_scale_mul: float,
 _PROLOGUE_DIMS = (32, 64, 72, 80, 128, 256)
 
 
-def prologue_ok(*ts: torch.Tensor) -> bool:
-    """Whether the fused prologue serves these 16-bit tensors [..., rows, D] (of one type and D)."""
-    t0 = ts[0]
-    return (t0.dtype in (torch.float16, torch.bfloat16) and t0.shape[-1] in _PROLOGUE_DIMS
-            and all(t.is_cuda and t.dtype == t0.dtype and t.dim() >= 2
-                    and t.shape[-1] == t0.shape[-1] and t.numel() > 0
-                    and t.shape[-2] < (1 << 23) and t.numel() < t.shape[-2] * t.shape[-1] * 65536
-                    # 16-byte loads: a contiguous view at an odd offset takes the separate kernels
-                    and (t.data_ptr() % 16 == 0 or not t.is_contiguous()) for t in ts))
+def prologue_ok(*kv: torch.Tensor, q: torch.Tensor | None = None) -> bool:
+    """Whether the fused prologue serves these 16-bit K / V tensors [..., N, D] (of one type, D and
+    device) and the queries q [..., M, D], whose rows it takes as one list."""
+    t0 = kv[0]
+    if t0.dtype not in (torch.float16, torch.bfloat16) or t0.shape[-1] not in _PROLOGUE_DIMS:
+        return False
+    for t in kv if q is None else (*kv, q):
+        if not (t.is_cuda and t.device == t0.device and t.dtype == t0.dtype and t.dim() >= 2
+                and t.shape[-1] == t0.shape[-1] and t.numel() > 0
+                # 16-byte loads: a contiguous view at an odd offset takes the separate kernels
+                and (t.data_ptr() % 16 == 0 or not t.is_contiguous())):
+            return False
+    return all(t.shape[-2] < (1 << 23) and t.numel() < t.shape[-2] * t.shape[-1] * 65536 for t in kv)
 
 
 def quantize_qkv_fused(q, k, v, q_scale_mul: float = 1.0, rotate: bool = False):

@@ -93,8 +93,9 @@ def detect_q_outlier_domination(q: torch.Tensor, *, ratio_threshold: float = 12.
 
 def fused_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor | None = None) -> bool:
     """Shapes the fused prologue (sl8_quantize_qk, with V sl8_quantize_qkv) serves."""
-    return (q.dim() == 4 and k.dim() == 4 and q.shape[0] == k.shape[0] and _C.prologue_ok(k, q)
-            and (v is None or (v.shape == k.shape and _C.prologue_ok(k, v))))
+    return (q.dim() == 4 and k.dim() == 4 and q.shape[0] == k.shape[0]
+            and (v is None or v.shape == k.shape)
+            and _C.prologue_ok(*((k,) if v is None else (k, v)), q=q))
 
 
 def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float | None = None,

@@ -69,3 +69,38 @@ def test_ops_reject_cpu_tensors():
         superl8_amd.attn_int8_fwd(q, q, q, internal_accuracy_gate=False)
     with pytest.raises(RuntimeError):
         superl8_amd.linear_q4k(x, torch.zeros(8, 144, dtype=torch.uint8))
+
+
+class _Cuda:
+    """What prologue_ok looks at in a contiguous GPU tensor."""
+    is_cuda = True
+
+    def __init__(self, *shape, device="cuda:0", dtype=torch.float16, ptr=0):
+        self.shape, self.device, self.dtype, self._ptr = torch.Size(shape), torch.device(device), dtype, ptr
+
+    def dim(self):
+        return len(self.shape)
+
+    def numel(self):
+        return self.shape.numel()
+
+    def data_ptr(self):
+        return self._ptr
+
+    def is_contiguous(self):
+        return True
+
+
+def test_fused_prologue_routing():
+    """What the fused prologue takes: K and V of one type, shape rule and device (on two devices
+    each is quantised by itself); any number of query rows and heads."""
+    k = _Cuda(1, 8, 100, 128)
+    assert _C.prologue_ok(k, _Cuda(1, 8, 100, 128))
+    assert not _C.prologue_ok(k, _Cuda(1, 8, 100, 128, device="cuda:1"))
+    assert not _C.prologue_ok(k, _Cuda(1, 8, 100, 128, dtype=torch.bfloat16))
+    assert not _C.prologue_ok(k, _Cuda(1, 8, 100, 128, ptr=8))
+    assert not _C.prologue_ok(_Cuda(1, 8, 100, 96)) and not _C.prologue_ok(_Cuda(1, 8, 0, 128))
+    assert not _C.prologue_ok(_Cuda(1, 8, 1 << 23, 128)) and not _C.prologue_ok(_Cuda(65536, 1, 4, 128))
+    assert _C.prologue_ok(k, q=_Cuda(1024, 64, 1, 128)) and _C.prologue_ok(k, q=_Cuda(1, 1, 1 << 23, 128))
+    assert not _C.prologue_ok(k, q=_Cuda(1, 8, 1, 128, device="cuda:1"))
+    assert not _C.prologue_ok(k, q=_Cuda(1, 8, 1, 128, ptr=2))

@@ -176,10 +176,18 @@ constexpr int row_lanes(int D) { return D <= 32 ? 4 : D <= 64 ? 8 : D <= 128 ? 1
 // the row's 2-norm per element, where a running sum of D products has up to D * 2^-24 of it.
 // Lane partners by DPP (xor 1, 2; xor 4 and 8 as two mirrors / a rotation inside the 16-lane
 // row), xor 16 by v_permlane16_swap.
-template <int D>
+// WIDE (bf16 rows, whose sums can pass the largest float where the result does not): a power of two
+// of the factor goes first, which changes no rounding.
+template <int D, bool WIDE>
 __device__ __forceinline__ void hadamard_row(float* f, int lane) {
   static_assert(D >= 32 && D <= 256 && (D & (D - 1)) == 0, "power-of-two head dim");
   constexpr int LPR = row_lanes(D);
+  constexpr float PRE = D >= 128 ? 0x1p-4f : 0x1p-3f;
+  static_assert(PRE * PRE * D <= 1.f && PRE * PRE * D >= 0.5f, "the power of two below 1 / sqrt(D)");
+  if constexpr (WIDE) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) f[e] *= PRE;
+  }
 #pragma unroll
   for (int s = 1; s < 8; s <<= 1)
 #pragma unroll
@@ -212,7 +220,7 @@ __device__ __forceinline__ void hadamard_row(float* f, int lane) {
       const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
       return __uint_as_float((lane & 16) ? r[0] : r[1]);
     });
-  const float rs = (float)(1.0 / __builtin_sqrt((double)D));
+  const float rs = (float)(1.0 / __builtin_sqrt((double)D)) * (WIDE ? 1.f / PRE : 1.f);
 #pragma unroll
   for (int e = 0; e < 8; ++e) f[e] *= rs;
 }
@@ -220,7 +228,7 @@ __device__ __forceinline__ void hadamard_row(float* f, int lane) {
 // The rotation of a row as its own pass would store it: rounded to its storage type.
 template <int DT, int D>
 __device__ __forceinline__ void rotate_row(float* f, int lane) {
-  hadamard_row<D>(f, lane);
+  hadamard_row<D, DT != SL8_DTYPE_F16>(f, lane);
 #pragma unroll
   for (int e = 0; e < 8; ++e) f[e] = Elem<DT>::round(f[e]);
 }

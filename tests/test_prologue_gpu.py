@@ -312,3 +312,24 @@ def test_host_flag_follows_the_device_flag(device, dtype, M, N, D):
         assert int(host[0]) == flag.item() == fires
     with pytest.raises(RuntimeError, match="pinned"):
         _C.quantize_qk_fused(calm, k, 1.0, 24.0, torch.zeros(1, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("D", [32, 64, 128, 256])
+def test_rotated_bf16_rows_near_the_largest_float(device, D):
+    """Rows whose unscaled sums pass the largest float while the normalised rotation does not:
+    against the rotation in 64 bits (a bf16 rounding, 2^-8, moves a scale by at most that and a code
+    by one step)."""
+    x = torch.ones(1, 2, 5, D, dtype=torch.float64)
+    x[:, :, 1] *= torch.where(torch.arange(D) % 3 == 0, -1.0, 1.0).double()
+    x[:, :, 2:] = torch.randn(1, 2, 3, D, dtype=torch.float64).clamp(-3, 3) / 3
+    q = (x * 3.0e38 / D ** 0.5).to(torch.bfloat16).to(device)
+    k = torch.randn(1, 2, 5, D, device=device).to(torch.bfloat16)
+    qi, qs, *_ = quant.quantize_qk(q, k, softmax_scale=1.0 / LOG2E, rotate=True)
+    h = torch.ones(1, 1, dtype=torch.float64, device=device)
+    while h.shape[0] < D:
+        h = torch.cat([torch.cat([h, h], 1), torch.cat([h, -h], 1)], 0)
+    ref = (q.double() @ h / D ** 0.5).to(torch.bfloat16).double()
+    assert torch.isfinite(ref).all() and torch.isfinite(qs).all()
+    s_ref = ref.abs().amax(-1) / 127
+    assert ((qs.squeeze(-1).double() / s_ref - 1).abs() <= 2.0 ** -7).all()
+    assert ((qi.double() - (ref / s_ref[..., None]).round()).abs() <= 1).all()

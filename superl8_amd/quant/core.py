@@ -126,11 +126,17 @@ def quantize_qk_gated(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: float 
         flag_host = None
         if defer == "host":
             flag_host, ready = torch.zeros(1, dtype=torch.int32, pin_memory=True), torch.cuda.Event()
-        q_i8, q_scale, k_i8, k_scale, k_mean, flag = _C.quantize_qk_fused(
-            q, k, s * LOG2E, ratio_threshold, flag_host)
+        try:
+            q_i8, q_scale, k_i8, k_scale, k_mean, flag = _C.quantize_qk_fused(
+                q, k, s * LOG2E, ratio_threshold, flag_host)
+            if defer == "host":
+                with _C.on_device(q):
+                    ready.record()
+        except BaseException:
+            if flag_host is not None:  # what was launched may still store to it
+                torch.cuda.synchronize(q.device)
+            raise
         if defer == "host":
-            with _C.on_device(q):
-                ready.record()
             return ((flag, flag_host, ready),
                     (q_i8, q_scale.unsqueeze(-1), k_i8, k_scale.unsqueeze(-1), k_mean))
         if defer:

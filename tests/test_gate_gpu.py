@@ -98,3 +98,21 @@ def test_gate_fires_before_v_is_refused(device, dtype, D, Dv, v_dtype):
     out = sl8.attn_int8_fwd(q, k, v, causal=True)
     ref = F.scaled_dot_product_attention(q, k, v.to(dtype), is_causal=True, scale=D ** -0.5)
     assert out.dtype == v_dtype and torch.equal(out, ref.to(v_dtype))
+
+
+def test_host_flag_outlives_a_failed_prologue(device, monkeypatch):
+    """An error behind the launch that may still store to the pinned flag waits for the GPU before
+    the flag is let go."""
+    q, k = (torch.randn(1, 2, 40, 64, device=device, dtype=torch.float16) for _ in range(2))
+    orig, waits = _C.quantize_qk_fused, []
+
+    def failing(*a):
+        orig(*a)
+        raise RuntimeError("behind the launch")
+
+    monkeypatch.setattr(_C, "quantize_qk_fused", failing)
+    sync = torch.cuda.synchronize
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda *a: (waits.append(a), sync(*a)))
+    with pytest.raises(RuntimeError, match="behind the launch"):
+        quant.quantize_qk_gated(q, k, defer="host")
+    assert waits == [(q.device,)]

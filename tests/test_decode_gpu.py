@@ -450,3 +450,23 @@ def test_decode_query_rotated_in_the_call(device, D):
     a = sl8.attn_decode_cached(q, *cache, rotate=True)
     b = sl8.attn_decode_cached(rot, *cache, rotate=False)
     assert_close_abs(a, _np(b.float()), atol=1e-2, rtol=1e-2, what=f"rotated query kv8 D={D}")
+
+
+def test_batch_too_large_to_plan(device):
+    """Above 1024 sequences (and for contexts of more splits than the block-table staging holds) the
+    device plan is refused and the call takes the equal splits: against the same sequences in two
+    calls that are planned (the decode bar)."""
+    from superl8_amd import _lib
+
+    lib = _lib.load()
+    assert lib.sl8_attn_paged_decode_q16_workspace(1024, 4, 1, 64, 8, 16, 100, 0) > 0
+    assert lib.sl8_attn_paged_decode_q16_workspace(1025, 4, 1, 64, 8, 16, 100, 0) == 0
+    assert lib.sl8_attn_paged_decode_q16_workspace(1, 4, 1, 64, 8, 1, 300000, 0) == 0
+    B, D = 1030, 64
+    lens = tuple(1 + 7 * i % 90 for i in range(B))
+    _, _, *store, bt, ctx = _paged_cache((B, 4, 1, D, 16, lens), device, seed=7)
+    q = torch.randn(B, 4, 1, D, device=device, dtype=torch.float16)
+    out = sl8.attn_paged_decode_cached(q, *store, bt, ctx, 16, max_context_len=90)
+    for half in (slice(0, 515), slice(515, B)):
+        ref = sl8.attn_paged_decode_cached(q[half], *store, bt[half], ctx[half], 16, max_context_len=90)
+        assert_close_abs(out[half], _np(ref.float()), atol=2e-2, rtol=1e-2, what="1030 sequences")

@@ -296,13 +296,14 @@ def test_k8v3_rejects(device):
                                   (2, 8, 4, 256, 32, (1500, 64)), (2, 16, 1, 128, 12, (1000, 300)),
                                   (70, 2, 2, 128, 16, tuple(17 * i % 500 for i in range(70)))],
                          ids=lambda c: "B%dH%d_%dD%dbs%d" % c[:5])
-def test_k8v3_planned_splits(device, case):
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_k8v3_planned_splits(device, case, dtype):
     """ops.attn_paged_decode_k8v3 with its splits planned on the device against the one-split
     kernel on the query quantised beforehand (the K8V3 bar)."""
     B, Hq, Hkv, D, bs, lens = case
     _, _, *store = _store(case, device, seed=4)
     g = torch.Generator(device="cpu").manual_seed(B + D)
-    q = torch.randn(B, Hq, 1, D, generator=g).half().to(device)
+    q = torch.randn(B, Hq, 1, D, generator=g).to(dtype).to(device)
     out = sl8.attn_paged_decode_k8v3(q, *store, bs, max_context_len=max(lens), rotate=False)
     q_i8, qs = _C.quantize_i8_rowwise(q.reshape(-1, D))
     qs = (qs * (np.log2(np.e) / D ** 0.5)).reshape(B, Hq, 1)

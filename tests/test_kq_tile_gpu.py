@@ -134,3 +134,32 @@ def test_whole_tiles_beside_split_ones(device, fmt):
     _, wd, x_i8, xs = _case(device, fmt, M, N, K)
     y = _gemm(fmt, x_i8, xs, wd, True)
     assert torch.equal(y[:, :n], _gemm(fmt, x_i8, xs, wd[:n].contiguous(), True))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fmt,q_max", [(4, 15), (5, 31)])
+@pytest.mark.parametrize("scratch", [True, False])
+@pytest.mark.parametrize("M", [40, 512])
+def test_largest_sums(device, fmt, q_max, scratch, M):
+    """Every code, scale and min at its largest and x rows of all +127, all -127 and halves that
+    cancel: the running sums of a super-block reach 256 * 127 * 63 * q_max (6.3e7, above 2^24). The
+    int8 kernel (M = 512 without scratch) holds them exactly, the fp16 one rounds 16 times per
+    super-block at 2^-23 of the largest; then fp32 sums over the super-blocks."""
+    N, K = 4864, 1024
+    nsb = K // 256
+    one = np.ones((N, nsb), np.float16)
+    sc = np.full((N, nsb, 8), 63, np.uint8)
+    q = np.full((N, nsb, 8, 32), q_max, np.uint8)
+    q[1::2, :, :, ::3] = 0
+    make = oq.make_blocks if fmt == 4 else okq.q5k_make
+    w = make(one, one, sc, sc.copy(), q).reshape(N, -1)
+    x = np.full((M, K), 127, np.int8)
+    x[1::3] = -127
+    x[2::3] = np.where(np.arange(K) % 256 < 128, 127, -127)
+    xt, wd = torch.from_numpy(x).to(device), torch.from_numpy(w).to(device)
+    y = _gemm(fmt, xt, torch.ones(M, device=device), wd, scratch)
+    ref = GEMV[fmt](x[:3], np.ones(3, np.float32), w[:2], K)  # rows and columns repeat
+    ref = np.tile(ref, (-(-M // 3), N // 2))[:M]
+    top = 256 * 127 * 63.0 * q_max
+    tol = nsb * 16 * 2.0 ** -23 * top + nsb * 2.0 ** -23 * nsb * top
+    assert np.abs(y.cpu().numpy().astype(np.float64) - ref).max() <= tol

@@ -1087,21 +1087,15 @@ int launch_prep(const void* q, int dtype, int64_t rows, int64_t D, bool rotate, 
   return SL8_OK;
 }
 
-template <int D, int G, bool VI8, bool PG, bool KS16>
-void launch_split(dim3 grid, const int8_t* q, const float* qs, const int8_t* k, const void* ks,
-                  const void* v, const float* vsc, float* op, float* mp, float* lp, int N, int ns,
-                  int hq, int hkv, int gsz, int bhq, const PagedArgs& pg, hipStream_t st) {
-  decode_split_kernel<D, G, VI8, PG, KS16><<<grid, DEC_THREADS, 0, st>>>(
-      q, qs, k, ks, v, vsc, op, mp, lp, N, ns, hq, hkv, gsz, bhq, pg);
-}
-
-template <int D, bool VI8, bool PG = false, bool KS16 = false>
+// the splits of a contiguous cache
+template <int D, bool VI8, bool KS16>
 void launch_d(int G, dim3 grid, const int8_t* q, const float* qs, const int8_t* k,
               const void* ks, const void* v, const float* vsc, float* op, float* mp, float* lp,
-              int N, int ns, int hq, int hkv, int gsz, int bhq, hipStream_t st,
-              const PagedArgs& pg = PagedArgs{nullptr, nullptr, 0, 1, 0, 0, nullptr}) {
-#define SL8_SPLIT(GG) \
-  launch_split<D, GG, VI8, PG, KS16>(grid, q, qs, k, ks, v, vsc, op, mp, lp, N, ns, hq, hkv, gsz, bhq, pg, st)
+              int N, int ns, int hq, int hkv, int gsz, int bhq, hipStream_t st) {
+  const PagedArgs pg{nullptr, nullptr, 0, 1, 0, 0, nullptr};
+#define SL8_SPLIT(GG)                                                             \
+  decode_split_kernel<D, GG, VI8, false, KS16><<<grid, DEC_THREADS, 0, st>>>(     \
+      q, qs, k, ks, v, vsc, op, mp, lp, N, ns, hq, hkv, gsz, bhq, pg)
   switch (G) {
     case 1: SL8_SPLIT(1); break;
     case 2: SL8_SPLIT(2); break;
@@ -1175,10 +1169,10 @@ int decode_launch(const int8_t* q, const float* q_scale, const int8_t* k, const 
 #undef SL8_WAVE_D
 #undef SL8_WAVE
   } else switch (D) {
-    case 32: launch_d<32, VI8, false, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
-    case 64: launch_d<64, VI8, false, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
-    case 128: launch_d<128, VI8, false, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
-    default: launch_d<256, VI8, false, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
+    case 32: launch_d<32, VI8, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
+    case 64: launch_d<64, VI8, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
+    case 128: launch_d<128, VI8, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
+    default: launch_d<256, VI8, KS16>(G, grid, q, q_scale, k, k_scale, v, vsc, op, mp, lp, (int)N, ns, (int)Hq, (int)Hkv, gsz, bhq, st); break;
   }
   SL8_CHECK_LAUNCH("attn_int8_decode split");
   launch_combine((int)D, bhq, st, op, mp, lp, static_cast<uint16_t*>(out), ns, bhq);

@@ -209,10 +209,6 @@ struct QOp {
 // operand reads (1 KB per MFMA), ~7 VALU operations per score.
 // ---------------------------------------------------------------------------
 
-// W8A8 at D = 256: 16 queries per wave (attn_w8a8_q16_kernel)
-#ifndef SL8_W8_Q16
-#define SL8_W8_Q16 1
-#endif
 #ifndef SL8_FWD_FAST
 #define SL8_FWD_FAST 1
 #endif
@@ -249,8 +245,7 @@ attn_fwd_wide_kernel(const FwdArgs a) {
   constexpr bool FAST = SL8_FWD_FAST && D <= 128 && NG == 1 && !W8;
   // its scores start from C0BITS and skip the conversion; D = 64 converts (3 operations, not 2)
   constexpr bool SEEDED = D == 128;
-  // ... and its W8A8 counterpart (half_step_fast_w8): D = 256, NG = 1, lazy rescale
-  constexpr bool FAST_W8 = SL8_FWD_FAST && D == 256 && NG == 1 && W8 && W8_LAZY;
+  static_assert(!(W8 && D == 256), "W8A8 at D = 256: attn_w8a8_q16_kernel");
   constexpr int WQ = 32 * NG;                  // queries per wave
   constexpr int WBM = WV * WQ;                 // queries per workgroup
   constexpr int DC = D / 32;
@@ -661,12 +656,6 @@ attn_fwd_wide_kernel(const FwdArgs a) {
 
     xblk xA, xB;  // scores of the last two halves (alternating)
     pblk pA, pB;  // P of the last two halves (alternating)
-    float xmA = -INFINITY, xmB = -INFINITY;  // W8A8 fast path: their row maxima (NG = 1)
-    auto row_max = [&](const xblk& xo) __attribute__((always_inline)) {
-      float t[NG];
-      half_max(xo, t);
-      return t[0];
-    };
     // One half-step, a single straight-line block per variant: xi/p1 = the
     // half before (scores in, P out), xo = this half (scores out), p2 = P of
     // the half two back (consumed by PV). dead = this half has no tile (all
@@ -793,116 +782,6 @@ attn_fwd_wide_kernel(const FwdArgs a) {
       }
     };
 
-    // W8A8 steady-state half-step (D = 256, one wave per SIMD, so the schedule
-    // inside the wave is all there is): the structure of half_step_fast with
-    // half_probs_w8's arithmetic, including its lazy rescale (a branch taken
-    // before the straight-line part, rarely).
-    // xmi: the row max of xi (both lane halves), formed by the step that
-    // produced xi (or by the fixup that changed it); this step forms xmo for
-    // xo in the slices after its scores, so no max and no cross-lane round
-    // trip stands between two half-steps.
-    // pf: the first SL8_FWD_PD operands of half-step s, already read by the
-    // step before it in the same tile (s = 1); step 0 reads them for step 1
-    // in its last slices, so that no half-step inside a tile starts with a
-    // full LDS round trip (one wave per SIMD: nothing else covers it).
-    auto half_step_fast_w8 = [&](int s, const int8_t* kt, const float* st, const uint16_t* vt,
-                                 xblk& xi, float xmi, pblk& p1, xblk& xo, float& xmo,
-                                 pblk& p2, v4i (&pf)[SL8_FWD_PD]) __attribute__((always_inline)) {
-      if constexpr (FAST_W8) {
-      static_assert(SL8_FWD_PD <= DC, "the prefetched operands are K operands");
-      constexpr float LOG2_127 = 6.988684686772166f;
-      const uint16_t* vr = vt + l32 * BN;
-      auto load_op = [&](int i) __attribute__((always_inline)) -> v4i {
-        if (i < DC) return *reinterpret_cast<const v4i*>(kt + (32 * s + l32) * D + koff[i]);
-        const int c = (i - DC) / DC, tt = (i - DC) % DC;
-        return *reinterpret_cast<const v4i*>(vr + 32 * tt * BN + voff[2 * s + c]);
-      };
-      constexpr int NOP = 3 * DC;  // 8 QK + 16 PV MFMAs
-      v4i opb[NOP];  // operand i is read SL8_FWD_PD MFMAs ahead of its use
-      // the first operands go out before the reference-point arithmetic
-#pragma unroll
-      for (int i = 0; i < SL8_FWD_PD && i < NOP; ++i) opb[i] = s ? pf[i] : load_op(i);
-      __builtin_amdgcn_sched_barrier(0);
-      const float tm0 = xmi * qsc[0];
-      // lazy rescale: the row's new reference point is used for this half's
-      // codes now; O (which still gets half h-2's products, relative to the old
-      // point, from the PV MFMAs below) and l are scaled after them
-      const bool ug = tm0 > m_run[0] + a.w8_excess;
-      const bool any_up = __any(ug);
-      const float fr = ug ? __builtin_amdgcn_exp2f(m_run[0] - tm0) : 1.f;
-      if (ug) m_run[0] = tm0;
-      const bool any_key = tm0 != -INFINITY;
-      const float sub = any_key ? tm0 - LOG2_127 : 0.f;
-      const float fac = any_key ? __builtin_amdgcn_exp2f(tm0 - m_run[0]) * (1.0f / 127.0f) : 0.f;
-      float pe[16];
-      float hs = 0.f;
-      float4 kv[4];
-      float xm = -INFINITY;
-      v16i sc;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sc[r] = 0;
-      // slices: QK MFMA i: P codes of keys 2i, 2i+1 of half h-1; PV MFMAs
-      // 0..1: pack them (bf16) + row sum; PV 2: k_scale reads; PV 3..10:
-      // scores of half h, two keys each; PV 11: their max in this lane;
-      // PV 12: the max over both lane halves (xmo)
-#pragma unroll
-      for (int i = 0; i < NOP; ++i) {
-        if (i + SL8_FWD_PD < NOP) opb[i + SL8_FWD_PD] = load_op(i + SL8_FWD_PD);
-        __builtin_amdgcn_sched_barrier(0);  // the read goes out before MFMA i
-        const v4i cur = opb[i];
-        if (i < DC) {
-          sc = __builtin_amdgcn_mfma_i32_32x32x32_i8(cur, qop[0].c[i], sc, 0, 0, 0);
-#pragma unroll
-          for (int e = 2 * i; e < 2 * i + 2; ++e) {
-            const float y = __builtin_amdgcn_exp2f(fmaf(xi[0][e], qsc[0], -sub));
-            hs += y;
-            pe[e] = rintf(y) * fac;
-            pin_vgpr(pe[e]);
-            pin_vgpr(hs);
-          }
-        } else {
-          const int c = (i - DC) / DC, tt = (i - DC) % DC;
-          oacc[0][tt] = PV::mfma(__builtin_bit_cast(pvec, cur), p2[0][c], oacc[0][tt]);
-          const int k = i - DC;
-          if (k < 2) {
-            p1[0][k] = PV::pack(&pe[8 * k]);
-            pin_vgpr(__builtin_bit_cast(v4i, p1[0][k]));
-            if (k == 1) l_lane[0] = l_lane[0] * fr + hs * fac;
-          } else if (k == 2) {
-#pragma unroll
-            for (int gq = 0; gq < 4; ++gq)
-              kv[gq] = *reinterpret_cast<const float4*>(st + 32 * s + 8 * gq + 4 * h);
-          } else if (k < 11) {
-            const int e0 = 2 * (k - 3);
-            const float ka[4] = {kv[e0 >> 2].x, kv[e0 >> 2].y, kv[e0 >> 2].z, kv[e0 >> 2].w};
-            xo[0][e0] = (float)sc[e0] * ka[e0 & 3];
-            xo[0][e0 + 1] = (float)sc[e0 + 1] * ka[(e0 + 1) & 3];
-            pin_vgpr(xo[0][e0]);
-            pin_vgpr(xo[0][e0 + 1]);
-          } else if (k == 11) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) xm = fmaxf(xm, xo[0][e]);
-            pin_vgpr(xm);
-          } else if (k == 12) {
-            xmo = max_xor32(xm);
-            pin_vgpr(xmo);
-          } else if (k >= 16 - SL8_FWD_PD && s == 0) {
-            // the next half-step's first K operand (same tile, keys 32..63)
-            const int n = k - (16 - SL8_FWD_PD);
-            pf[n] = *reinterpret_cast<const v4i*>(kt + (32 + l32) * D + koff[n]);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (any_up) {
-#pragma unroll
-        for (int t = 0; t < DC; ++t)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) oacc[0][t][r] *= fr;
-      }
-      }
-    };
-
     // FAST path: xo already holds the exp2 argument logit - m (logit itself for a
     // row whose reference point is not set yet); a row set here shifts its xo
     auto settle_fast = [&](xblk& xo) __attribute__((always_inline)) {
@@ -1006,8 +885,8 @@ attn_fwd_wide_kernel(const FwdArgs a) {
       // first half-step 126.4 us, split 124.9 us (V first, K after it: 125.9);
       // config 5: all at the start 1100 us, all after the first half-step
       // 1128 us, split 1082 us (V first, K after it: 1135 us).
-      if constexpr (!FAST && !FAST_W8) copies();
-      if constexpr (FAST || FAST_W8) copies_k();
+      if constexpr (FAST) copies_k();
+      else copies();
       const bool dead = !live(j);
       const bool mask = dead || masked(j);
       // A dead tile after a dead tile has nothing to do: the one before already
@@ -1015,26 +894,10 @@ attn_fwd_wide_kernel(const FwdArgs a) {
       // is P = 0 and scores of -inf (in the diagonal block, the waves whose
       // queries end early skip their last tiles this way).
       if (dead && !live(j - 1)) {
-        if constexpr (FAST || FAST_W8) copies_v();
+        if constexpr (FAST) copies_v();
       } else if constexpr (W8) {
-        if constexpr (FAST_W8) {
-          // a fixup may mask scores: the carried max is formed again
-          v4i pf[SL8_FWD_PD];
-          half_step_fast_w8(0, kcur, scur, vprev, xB, xmB, pB, xA, xmA, pA, pf);
-          if (mask || !all_set) {
-            half_fixup(j, 0, mask, dead, xA);
-            xmA = row_max(xA);
-          }
-          copies_v();
-          half_step_fast_w8(1, kcur, scur, vprev, xA, xmA, pA, xB, xmB, pB, pf);
-          if (mask || !all_set) {
-            half_fixup(j, 1, mask, dead, xB);
-            xmB = row_max(xB);
-          }
-        } else {
-          half_step_w8(j, 0, kcur, scur, vprev, mask, dead, xB, pB, xA, pA);
-          half_step_w8(j, 1, kcur, scur, vprev, mask, dead, xA, pA, xB, pB);
-        }
+        half_step_w8(j, 0, kcur, scur, vprev, mask, dead, xB, pB, xA, pA);
+        half_step_w8(j, 1, kcur, scur, vprev, mask, dead, xA, pA, xB, pB);
       } else {
         if constexpr (FAST) {
           // a masked half, or one that may fix some row's reference point,
@@ -1087,7 +950,6 @@ attn_fwd_wide_kernel(const FwdArgs a) {
       for (int g = 0; g < NG; ++g) {
   #pragma unroll
         for (int e = 0; e < 16; ++e) xA[g][e] = xB[g][e] = -INFINITY;
-        xmA = xmB = -INFINITY;
   #pragma unroll
         for (int c = 0; c < 2; ++c) {
           float z[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -1220,7 +1082,6 @@ constexpr int wide_waves(int64_t D) { return D == 128 ? SL8_FWD_WV128 : (D == 64
 #define SL8_FWD_NG256 1
 #endif
 constexpr int wide_ng(int64_t D) { return D == 256 ? SL8_FWD_NG256 : WIDE_NG; }
-constexpr int wide_bm(int64_t D) { return wide_waves(D) * 32 * wide_ng(D); }
 
 template <int D, bool CAUSAL, int VDT, bool LSE, bool W8 = false, int WV = wide_waves(D)>
 void launch_wide(const FwdArgs& a, int grid, hipStream_t st) {
@@ -1260,7 +1121,7 @@ struct FwdKernel {
 FwdKernel fwd_kernel(int64_t D, bool w8) {
   if (D == 64) return {32, 4, 4, 2, w8};
   if (D == 128) return {32, w8 ? 4 : 8, 4, 2, true};
-  if (w8 && SL8_W8_Q16) return {16, 8, 4, 1, true};
+  if (w8) return {16, 8, 4, 1, true};
   return {32 * wide_ng(256), 4, 4, 1, true};
 }
 
@@ -1524,8 +1385,8 @@ int w8a8_pad_operands(const int8_t*& q, const int8_t*& k, const int8_t*& v, cons
 // supported width (64/128/256); dout = the output row length (the caller's
 // head dim when the operands were padded).
 // ---------------------------------------------------------------------------
-// W8A8 prefill at D = 256 with 16 queries per wave (SL8_W8_Q16). The 32-query
-// waves of attn_fwd_wide_kernel hold O in 128 accumulators and run one wave
+// W8A8 prefill at D = 256 with 16 queries per wave. 32-query waves (as in
+// attn_fwd_wide_kernel) would hold O in 128 accumulators and run one wave
 // per SIMD, where nothing covers a wave's own latencies or the per-tile
 // barrier. Here a wave owns 16 queries on the 16x16 MFMAs: O^T is 16 blocks
 // of 16 dims x 16 queries (64 accumulators), and a workgroup of 8 waves (two
@@ -1545,9 +1406,9 @@ int w8a8_pad_operands(const int8_t*& q, const int8_t*& k, const int8_t*& v, cons
 //       launch at config 5).
 // The arithmetic per row is the wide kernel's W8A8 path (P re-quantised per
 // 32-key half against the half's max, the lazy reference-point rescale), and
-// so is the straight-line half-step. Config 5: 1081 -> 986 us (the same
-// kernel with the compiler's schedule, each operand read right before its
-// MFMA: 1633 us). SL8_W8_Q16 = 0 runs attn_fwd_wide_kernel's W8A8 path.
+// so is the straight-line half-step. Config 5: 1081 us with 32-query waves, 986
+// here (the same kernel with the compiler's schedule, each operand read right
+// before its MFMA: 1633 us).
 #ifndef SL8_Q16_PD
 #define SL8_Q16_PD 4  // operand reads ahead of their MFMA (2 / 3 / 4 / 6 at config 5: 972 / 969 / 963 / 967 us)
 #endif
@@ -1713,8 +1574,8 @@ attn_w8a8_q16_kernel(const FwdArgs a) {
       pA[e] = pB[e] = (__bf16)0.f;
     }
     bool all_set = false;  // every row's reference point is fixed (wave-uniform)
-    // Straight-line half-step (the wide kernel's half_step_fast_w8 in this
-    // layout): MFMA i (QK of half h: i < 8; PV of half h - 2: i >= 8) is
+    // Straight-line half-step (the wide kernel's half_step_fast with W8A8's arithmetic
+    // and this layout): MFMA i (QK of half h: i < 8; PV of half h - 2: i >= 8) is
     // preceded by the LDS read of operand i + 3 and followed by a slice of
     // VALU work: P code of key i of half h - 1 (i < 8); the k_scale reads and
     // the pack of P (i = 8); the score of key i - 9 of half h (i = 9..16);
@@ -1917,7 +1778,6 @@ int w8a8_wide_launch(const int8_t* q, const float* q_scale, const int8_t* k, con
     SL8_CHECK_LAUNCH("attn_w8a8_fwd v to bf16 V^T");
   }
   int grid;
-  const bool q16 = SL8_W8_Q16 && D == 256;
   const FwdKernel kn = fwd_kernel(D, true);
   const FwdGeom geom = fwd_geometry(kn, B * Hq, M, N, causal, -1);
   FwdArgs a = make_args(B, Hq, Hkv, M, N, D, causal, grid, geom, kn.wave_q);
@@ -1937,11 +1797,10 @@ int w8a8_wide_launch(const int8_t* q, const float* q_scale, const int8_t* k, con
     if (causal) attn_w8a8_q16_kernel<true, WV><<<grid, 64 * WV, 0, st>>>(a);
     else attn_w8a8_q16_kernel<false, WV><<<grid, 64 * WV, 0, st>>>(a);
   };
-  if (q16 && geom.wv == 4) q16_waves(std::integral_constant<int, 4>{});
-  else if (q16) q16_waves(std::integral_constant<int, 8>{});
-  else if (D == 64) wide(std::integral_constant<int, 64>{});
+  if (D == 64) wide(std::integral_constant<int, 64>{});
   else if (D == 128) wide(std::integral_constant<int, 128>{});
-  else wide(std::integral_constant<int, 256>{});
+  else if (geom.wv == 4) q16_waves(std::integral_constant<int, 4>{});
+  else q16_waves(std::integral_constant<int, 8>{});
   SL8_CHECK_LAUNCH("attn_w8a8_fwd");
   return SL8_OK;
 }

@@ -29,8 +29,6 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i_t __attribute__((ext_vector_type(16)));
-typedef float v16f_t __attribute__((ext_vector_type(16)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int Q5K_BYTES = 176;
 constexpr int Q6K_BYTES = 210;

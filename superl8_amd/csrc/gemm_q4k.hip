@@ -35,7 +35,6 @@ namespace sl8 {
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
 constexpr int Q4K_BYTES = 144;
 constexpr int GEMV_ROWS = 16;

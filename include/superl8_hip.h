@@ -94,8 +94,11 @@ int sl8_quantize_i8_row_groups(const void* x, int x_dtype, int64_t G, int64_t N,
  * Fused fp16 / bf16 attention prologue: quantize_qk (no rotation) plus, optionally,
  * the outlier gate, in two launches (six unfused). Replaces superl8/quant/core.py:164-196
  * (smooth_k + quantize_qk) and detect_q_outlier_domination (core.py:113-145)
- * as called from superl8/ops.py:115-150; results equal sl8_k_mean,
- * sl8_quantize_i8_rows_centered and sl8_q_outlier_gate bit for bit.
+ * as called from superl8/ops.py:115-150. fp16: results equal sl8_k_mean,
+ * sl8_quantize_i8_rows_centered and sl8_q_outlier_gate bit for bit. bf16: so do q, the flag and,
+ * while a K column spans no more than about 2^30 in magnitude (its fp64 sums are then exact), the
+ * mean, k and k_scale; beyond, the two means add in different orders and may differ in their last
+ * fp32 bit, and a code of k with them.
  *   q [qrows, D] (qrows = B*Hq*M), k [G, N, D] (G = B*Hkv), both dtype f16 or bf16,
  *   D in {32,64,72,80,128,256}
  *   -> q_i8 [qrows, D], q_scale [qrows] (x q_scale_mul), k_i8 [G, N, D],

@@ -82,7 +82,8 @@ def quantize_i8_rowwise(x: torch.Tensor):
 
 
 def k_mean(k: torch.Tensor) -> torch.Tensor:
-    """fp32 mean over the key axis of k[..., N, D] -> [..., 1, D] (order-independent)."""
+    """fp32 mean over the key axis of k[..., N, D] -> [..., 1, D]: fp16 by exact integer sums (no
+    order), bf16 / fp32 by fp64 sums in a fixed order."""
     _check(k.is_cuda, "k_mean expects a CUDA tensor")
     _check(k.dtype in (torch.float16, torch.bfloat16, torch.float32),
            "k_mean input must be float16/bfloat16/float32")

@@ -698,6 +698,8 @@ gemv_q6k_mfma_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     if constexpr (PIPE) __builtin_amdgcn_sched_barrier(0);
   };
+  // the next chunk's copies overwrite what compute read: its LDS reads are done
+  auto reads_done = [] { __builtin_amdgcn_s_waitcnt(0xC07F); __builtin_amdgcn_wave_barrier(); };
   auto compute = [&](const int cnt, const Part& p) __attribute__((always_inline)) {
     const auto& [qlp, qhp, scw, dw] = p;
 #pragma unroll
@@ -765,12 +767,12 @@ gemv_q6k_mfma_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
       load_x(c, min(CH, sb1 - c));
       if (c1 < sb1) load(c1, pb);
       compute(min(CH, sb1 - c), pa);
-      __builtin_amdgcn_wave_barrier();  // the next chunk's copies overwrite what was read
+      reads_done();
       if (c1 >= sb1) break;
       load_x(c1, min(CH, sb1 - c1));
       if (c2 < sb1) load(c2, pa);
       compute(min(CH, sb1 - c1), pb);
-      __builtin_amdgcn_wave_barrier();
+      reads_done();
     }
   } else if (sb1 - sb0 <= CH) {  // one chunk
     if (sb1 > sb0) {
@@ -783,7 +785,7 @@ gemv_q6k_mfma_kernel(const int8_t* __restrict__ x, const float* __restrict__ x_s
       load(c, pa);
       load_x(c, min(CH, sb1 - c));
       compute(min(CH, sb1 - c), pa);
-      __builtin_amdgcn_wave_barrier();
+      reads_done();
     }
   }
   // C rows 4 g + r (g = lane / 16): sum the 4 sub-block groups, then the waves in fixed order

@@ -8,9 +8,9 @@
 // most 256 * 127 * 1953 = 6.3e7 in magnitude (Q4_K: half of it), held in the fp32 accumulator: exact
 // while every running sum stays below 2^24 = 1.7e7, as those of usual activations do (at most 2.5e6
 // over 1e7 sums of N(0, 1) rows and random Q5_K blocks); beyond, each of the 16 steps rounds at 2^-24
-// of the running sum, where an int32 sum would be rounded once. Against 64 bits, fp32 outputs: M = 17 / 512, N = K = 4096 / 17408
-// x 5120 0.8e-7 / 1.2e-7 of the result (the int8 kernels 1.1e-7 / 1.2e-7, whose fp32 sums over the
-// super-blocks have no K split).
+// of the running sum, where an int32 sum would be rounded once. Relative error against 64 bits of fp32
+// outputs, M x N x K: 17 x 4096 x 4096 0.8e-7, 512 x 17408 x 5120 1.2e-7 (the int8 kernels, which sum
+// the super-blocks in one run, 1.1e-7 and 1.2e-7).
 // One fp16 MFMA per 16 elements costs what the two int8 MFMAs (Q4_K: the 6-bit scale in 3-bit
 // halves; Q5_K: three) per 32 elements did, but it leaves one accumulator instead of two: a wave
 // owns 32 columns x 128 rows at two waves per SIMD, so a weight operand is built once per 128 rows,

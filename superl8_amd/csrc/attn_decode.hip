@@ -962,7 +962,7 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
 // ---------------------------------------------------------------------------
 // Preparation of a decode step that starts from the 16-bit query, one launch: the query rows
 // (optionally rotated, rounded to their type, quantised; the scale carries q_mul) and, for a
-// paged cache, the split plan, made by block 0.
+// paged cache, the split plan, made by the first `plan.blocks` workgroups.
 //
 // The plan: keys per split L is the smallest multiple of `unit` with no more than `target` splits
 // over all (sequence, KV head) pairs (target: the workgroups that are resident at once), within
@@ -973,10 +973,11 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
 // ---------------------------------------------------------------------------
 constexpr int PLAN_MAX_B = 1024;  // sequences (LDS of the plan block); larger batches: no plan
 struct PlanArgs {
-  const int32_t* ctx;  // null: no plan
+  const int32_t* ctx;
   int B, h_kv, n_len;
   int target, unit, lmin, lcap;
   int max_items;
+  int blocks;   // workgroups that make the plan, each for its part of the items
   int4* items;  // [max_items]: (b * h_kv + kvh, first key, end, -), empty past the last
   int2* seq;    // [B]: (first item, splits per KV head)
 };
@@ -1015,7 +1016,7 @@ __device__ __forceinline__ void plan_block(const PlanArgs& p) {
       }
       if (b < p.B) {
         pre_s[b] = base + x - c;
-        p.seq[b] = make_int2((base + x - c) * p.h_kv, c);
+        if (blockIdx.x == 0) p.seq[b] = make_int2((base + x - c) * p.h_kv, c);
       }
       base += __shfl(x, 63, 64);
     }
@@ -1023,7 +1024,7 @@ __device__ __forceinline__ void plan_block(const PlanArgs& p) {
   }
   __syncthreads();
   const int total = pre_s[p.B] * p.h_kv;
-  for (int i = threadIdx.x; i < p.max_items; i += 256) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < p.max_items; i += 256 * p.blocks) {
     int4 it = make_int4(0, 0, 0, 0);
     if (i < total) {
       int a = 0, z = p.B;  // the sequence with pre[b] * h_kv <= i < pre[b + 1] * h_kv
@@ -1046,10 +1047,10 @@ template <int DT, int D, bool ROT>
 __global__ void __launch_bounds__(256)
 decode_prep_kernel(const uint16_t* __restrict__ q, int64_t rows, float q_mul,
                    int8_t* __restrict__ q_i8, float* __restrict__ q_scale, const PlanArgs plan) {
-  if (plan.ctx && blockIdx.x == 0) return plan_block(plan);
+  if ((int)blockIdx.x < plan.blocks) return plan_block(plan);
   constexpr int LPR = row_lanes(D), RPB = 256 / LPR;
   const int lane = threadIdx.x % LPR;
-  const int64_t r = (int64_t)(blockIdx.x - (plan.ctx ? 1 : 0)) * RPB + threadIdx.x / LPR;
+  const int64_t r = (int64_t)(blockIdx.x - plan.blocks) * RPB + threadIdx.x / LPR;
   const bool live = r < rows;
   float f[8];
   VecIO<DT>::unpack(reinterpret_cast<const uint4*>(q + (live ? r : 0) * D)[lane], f);
@@ -1070,7 +1071,7 @@ int launch_prep(const void* q, int dtype, int64_t rows, int64_t D, bool rotate, 
   auto go = [&](auto dt, auto d) {
     constexpr int DT = decltype(dt)::value, DD = decltype(d)::value;
     constexpr int RPB = 256 / row_lanes(DD);
-    const unsigned grid = (unsigned)((rows + RPB - 1) / RPB) + (plan.ctx ? 1 : 0);
+    const unsigned grid = (unsigned)((rows + RPB - 1) / RPB) + (unsigned)plan.blocks;
     const uint16_t* qh = static_cast<const uint16_t*>(q);
     if (rotate) decode_prep_kernel<DT, DD, true><<<grid, 256, 0, st>>>(qh, rows, q_mul, q_i8, q_scale, plan);
     else decode_prep_kernel<DT, DD, false><<<grid, 256, 0, st>>>(qh, rows, q_mul, q_i8, q_scale, plan);
@@ -2098,7 +2099,8 @@ PagedPlan paged_plan(const Paged& p) {
   const int64_t items = std::min(groups * ((nmax + lmin - 1) / lmin),
                                  std::max(target, groups * ((nmax + lcap - 1) / lcap)));
   r.a = PlanArgs{p.ctx, (int)p.B, (int)p.Hkv, (int)p.nmax, (int)target, (int)unit, (int)lmin,
-                 (int)lcap, (int)items, nullptr, nullptr};
+                 (int)lcap, (int)items, (int)std::min<int64_t>(64, (items + 255) / 256),
+                 nullptr, nullptr};
   auto at = [&](size_t n) { const size_t o = r.bytes; r.bytes += (n + 15) / 16 * 16; return o; };
   at((size_t)items * gsz * (p.D + 2) * sizeof(float));
   r.items_at = at((size_t)items * sizeof(int4));

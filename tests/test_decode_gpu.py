@@ -434,6 +434,14 @@ def test_paged_planned_splits(device, case, dtype):
         assert_close_abs(out, _np(ref.float()), atol=2e-3, rtol=2e-3, what=f"planned {case} {nmax}")
 
 
+@pytest.mark.parametrize("case", [(130, 4, 4, 64, 16, tuple(7 * i % 900 for i in range(130))),
+                                  (40, 16, 4, 128, 16, tuple(61 * i % 2400 for i in range(40)))],
+                         ids=lambda c: "B%dH%d_%dD%dbs%d" % c[:5])
+def test_paged_plan_by_several_workgroups(device, case):
+    """More planned splits than one workgroup writes, for both kernels of the int8 cache."""
+    test_paged_planned_splits(device, case, torch.float16)
+
+
 @pytest.mark.parametrize("D", [32, 64, 128, 256])
 def test_decode_query_rotated_in_the_call(device, D):
     """The rotation of the 16-bit query inside the decode call against rotate_last before it:

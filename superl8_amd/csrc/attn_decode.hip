@@ -970,39 +970,66 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
 // sized on the longest sequence alone (256 keys and up to 256 splits of every sequence) left most
 // workgroups of a batch of mixed lengths empty and the rest too short to stream: 32 sequences of
 // 512..8192 keys, 8 KV heads, D = 128: 95 us for 191 MB, 44 with the plan (the call 114 -> 53 us).
+//
+// Where a pair gets only a few splits, whole units of L can leave many workgroups without work: 53
+// sequences of 3393 keys and 4 heads at D = 256 get 4 splits of 1024 keys, 848 for 1024 places. A
+// second target of several rounds of workgroups (paged_plan: round_target) is then taken where its
+// shorter splits are sooner done if the workgroups went in step (plan_time): 194 -> 156 us there.
 // ---------------------------------------------------------------------------
+constexpr int PLAN_SPLIT_KEYS = 33;  // what a split costs besides its keys, in keys
 constexpr int PLAN_MAX_B = 1024;  // sequences (LDS of the plan block); larger batches: no plan
 struct PlanArgs {
   const int32_t* ctx;
   int B, h_kv, n_len;
   int target, unit, lmin, lcap;
+  int slots;         // workgroups resident at once
+  int round_target;  // 0: none
   int max_items;
   int blocks;   // workgroups that make the plan, each for its part of the items
   int4* items;  // [max_items]: (b * h_kv + kvh, first key, end, -), empty past the last
   int2* seq;    // [B]: (first item, splits per KV head)
 };
 
-__device__ __forceinline__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
+__host__ __device__ __forceinline__ int ceil_div(int a, int b) { return (a + b - 1) / b; }
+
+// Time of `items` splits of L keys in rounds of `slots` workgroups, in keys.
+__host__ __device__ __forceinline__ float plan_time(int items, int L, int slots) {
+  return (float)ceil_div(items, slots) * (float)(L + PLAN_SPLIT_KEYS);
+}
+// A second target is taken for a gain of more than the difference between runs.
+constexpr float PLAN_ROUND_GAIN = 0.95f;
 
 __device__ __forceinline__ void plan_block(const PlanArgs& p) {
-  __shared__ int n_s[PLAN_MAX_B], pre_s[PLAN_MAX_B + 1];
+  __shared__ int n_s[PLAN_MAX_B], pre_s[PLAN_MAX_B + 1], len_s[4];
+  __shared__ float time_s[4];
   for (int b = threadIdx.x; b < p.B; b += 256) n_s[b] = max(0, min(p.ctx[b], p.n_len));
   __syncthreads();
   const int lane = threadIdx.x & 63;
-  // every wave searches for itself (no barriers): smallest L = unit * u in the bounds with
-  // splits(L) <= target
+  const int wave = threadIdx.x >> 6;
   auto splits = [&](int L) {
     int s = 0;
     for (int b = lane; b < p.B; b += 64) s += ceil_div(n_s[b], L);
     return __builtin_amdgcn_readfirstlane(lane_group_sum<64>(s)) * p.h_kv;
   };
+  // every wave searches for itself (no barriers): smallest L = unit * u in the bounds with
+  // splits(L) <= target; odd waves for the second target, if there is one
+  const int target = (wave & 1) && p.round_target ? p.round_target : p.target;
   int lo = p.lmin / p.unit, hi = p.lcap / p.unit;
   while (lo < hi) {
     const int mid = (lo + hi) >> 1;
-    if (splits(mid * p.unit) <= p.target) hi = mid;
+    if (splits(mid * p.unit) <= target) hi = mid;
     else lo = mid + 1;
   }
-  const int L = lo * p.unit;
+  int L = lo * p.unit;
+  if (p.round_target) {
+    const float t = plan_time(splits(L), L, p.slots);
+    if (lane == 0) {
+      len_s[wave] = L;
+      time_s[wave] = t;
+    }
+    __syncthreads();
+    L = time_s[1] < PLAN_ROUND_GAIN * time_s[0] ? len_s[1] : len_s[0];
+  }
   if (threadIdx.x < 64) {
     int base = 0;
     for (int b0 = 0; b0 < p.B; b0 += 64) {
@@ -2091,16 +2118,35 @@ PagedPlan paged_plan(const Paged& p) {
   PagedPlan r{};
   // one round of resident workgroups; a batch whose (sequence, KV head) pairs nearly fill that
   // alone gets two splits per pair on average, so that its longest sequences are still cut
-  const int64_t target = std::max<int64_t>((int64_t)cu_count() * wgs / chunks, 2 * groups);
+  const int64_t slots = std::max<int64_t>((int64_t)cu_count() * wgs / chunks, 1);
+  const int64_t target = std::max(slots, 2 * groups);
   int64_t lmin = std::max<int64_t>(256, up((nmax + DEC_MAX_SPLITS - 1) / DEC_MAX_SPLITS));
   int64_t lcap = up(nmax);
   if (streams) lcap = std::min<int64_t>(lcap, (DEC_BT_MAX - 2) * p.bs / unit * unit);
   lcap = std::max(lcap, lmin);
+  // 2, 3 or 6 rounds, the soonest done if every sequence is as long as nmax, where one gains. Only
+  // for the split kernel of the int8 cache, and at D = 64 not for the wider groups: the other two
+  // kernels and those forms lost by shorter splits. Of 526 batches (1 to 64 heads, 4 to 100
+  // sequences of 900 to 6000 keys) 30 take more rounds, in 0.80 to 1.02 of their time in one.
+  int64_t round_target = 0;
+  if (!p.k8v3 && !streams && (p.D >= 128 || (p.D == 64 && G <= 2))) {
+    auto time = [&](int64_t t) {
+      const int64_t per = t / groups;
+      const int64_t L = std::min(std::max(up((nmax + per - 1) / per), lmin), lcap);
+      return plan_time((int)(groups * ((nmax + L - 1) / L)), (int)L, (int)slots);
+    };
+    float best = PLAN_ROUND_GAIN * time(target);
+    for (const int rounds : {2, 3, 6}) {
+      const int64_t t = std::max(slots * rounds, target);
+      if (time(t) < best) best = time(round_target = t);
+    }
+  }
   const int64_t items = std::min(groups * ((nmax + lmin - 1) / lmin),
-                                 std::max(target, groups * ((nmax + lcap - 1) / lcap)));
+                                 std::max({target, round_target,
+                                           groups * ((nmax + lcap - 1) / lcap)}));
   r.a = PlanArgs{p.ctx, (int)p.B, (int)p.Hkv, (int)p.nmax, (int)target, (int)unit, (int)lmin,
-                 (int)lcap, (int)items, (int)std::min<int64_t>(64, (items + 255) / 256),
-                 nullptr, nullptr};
+                 (int)lcap, (int)slots, (int)round_target, (int)items,
+                 (int)std::min<int64_t>(64, (items + 255) / 256), nullptr, nullptr};
   auto at = [&](size_t n) { const size_t o = r.bytes; r.bytes += (n + 15) / 16 * 16; return o; };
   at((size_t)items * gsz * (p.D + 2) * sizeof(float));
   r.items_at = at((size_t)items * sizeof(int4));

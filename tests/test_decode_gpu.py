@@ -442,6 +442,14 @@ def test_paged_plan_by_several_workgroups(device, case):
     test_paged_planned_splits(device, case, torch.float16)
 
 
+@pytest.mark.parametrize("lens", [(1000,) * 65, tuple(1000 - 15 * i for i in range(65))],
+                         ids=["equal", "mixed"])
+def test_paged_plan_of_several_rounds(device, lens):
+    """Few splits per pair: the plan takes several rounds of workgroups, or one for mixed lengths."""
+    for Hq, Hkv, D in ((16, 1, 256), (8, 4, 256), (12, 4, 128)):
+        test_paged_planned_splits(device, (len(lens), Hq, Hkv, D, 16, lens), torch.float16)
+
+
 @pytest.mark.parametrize("D", [32, 64, 128, 256])
 def test_decode_query_rotated_in_the_call(device, D):
     """The rotation of the 16-bit query inside the decode call against rotate_last before it:

@@ -607,6 +607,13 @@ def main():
 PREFILL_KERNEL = "attn_fwd_wide_kernel<128, true, 0, false, 1, 8, false, false>"
 
 
+def _is_prefill(name: str) -> bool:
+    """Whether name is config 2's prefill kernel: PREFILL_KERNEL, or with further switches, all off."""
+    import re
+
+    return re.fullmatch(re.escape(PREFILL_KERNEL[:-1]) + "(, false)*>", name) is not None
+
+
 def _short_kernel_name(name: str) -> str:
     """'void sl8::(anonymous namespace)::k<..>(sl8::..)' -> 'k<..>' (full template
     arguments kept)."""
@@ -646,11 +653,12 @@ def trace_summary(path: str, steps: int) -> str:
         nm = n if len(n) <= 120 else n[:117] + "..."
         lines.append(f"| {nm} | {len(d)} | {np.mean(d):.2f} | {np.median(d):.2f} | {min(d):.2f} | "
                      f"{max(d):.2f} |")
-    if PREFILL_KERNEL in by:
-        v = sorted(by[PREFILL_KERNEL])[-steps:]
+    prefill = next((n for n in by if _is_prefill(n)), None)
+    if prefill:
+        v = sorted(by[prefill])[-steps:]
         d = [x for _, x in v]
         span = (v[-1][0] - v[0][0]) / 1e3 / max(1, len(v) - 1) if len(v) > 1 else float("nan")
-        lines += ["", f"Timed calls ({len(d)}: the last {steps} dispatches of `{PREFILL_KERNEL}`): "
+        lines += ["", f"Timed calls ({len(d)}: the last {steps} dispatches of `{prefill}`): "
                       f"mean {np.mean(d):.2f} us, median {np.median(d):.2f} us, min {min(d):.2f}, "
                       f"max {max(d):.2f}; start-to-start spacing {span:.2f} us."]
     return "\n".join(lines)

@@ -1,8 +1,10 @@
 """CPU checks of bench.py's profile summarisers (the tables under profiles/ come
 from them) and of its refusal to run on more than one GPU."""
 import csv
+import shutil
 import subprocess
 import sys
+from pathlib import Path
 
 import pytest
 
@@ -39,6 +41,22 @@ def test_trace_summary_takes_the_last_steps_dispatches(tmp_path):
     assert "| other_kernel | 1 |" in out
     assert "mean 110.00 us, median 110.00 us, min 100.00, max 120.00" in out
     assert "start-to-start spacing 1000.00 us" in out
+
+
+def test_trace_summary_finds_the_built_prefill_kernel(tmp_path):
+    # under the name that the library's own kernel has in a trace
+    lib = Path(bench.HERE) / "superl8_amd" / "libsuperl8_hip.so"
+    if not lib.exists() or shutil.which("nm") is None:
+        pytest.skip("needs the built library and nm")
+    syms = subprocess.run(["nm", "-C", str(lib)], capture_output=True, text=True, check=True).stdout
+    names = {ln.split(" ", 2)[2].replace("__device_stub__", "") for ln in syms.splitlines()
+             if "__device_stub__attn_fwd_wide_kernel<" in ln}
+    hits = [n for n in names if bench._is_prefill(bench._short_kernel_name(n))]
+    assert len(hits) == 1
+    p = tmp_path / "t.csv"
+    _write_trace(p, [(n, 1000, 50_000) for n in names - set(hits)] + [(hits[0], 9000, 100_000)])
+    assert "Timed calls (1: " in bench.trace_summary(str(p), 1)
+    assert "mean 100.00 us" in bench.trace_summary(str(p), 1)
 
 
 def test_pmc_summary_sums_rows_per_dispatch(tmp_path):

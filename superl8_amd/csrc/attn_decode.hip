@@ -1474,8 +1474,9 @@ kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __
 //   * softmax in the MFMA output layout: lane (g4, col) holds keys
 //     16 kb + 4 g4 + i of head col; logit = (acc * k_scale) * q_scale, the
 //     tile max over the lane's 16 values and the 4 lanes of the column; p
-//     stored in LDS as two fp16 parts, p rounded towards zero in
-//     row col and the rest in row G + col, 64 keys each (rows 2G..15 stay zero);
+//     stored as fp16 in LDS, one 64-key row per head, or (TWO) as two fp16
+//     parts, p rounded towards zero in row col and the rest in row G + col (the
+//     other rows stay zero);
 //   * value tables (key = lane): fp16 of codebook[i] * norm for i = 0..7 per
 //     128-channel block, as a low-byte plane (2 dwords) and a high-byte plane
 //     (2 dwords), handed to the dequantising lanes by v_permlane32_swap;
@@ -1485,16 +1486,18 @@ kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __
 //     writes the half row to an 8 KB (D = 128) LDS tile, read back transposed
 //     (ds_read_b64_tr_b16) as the A operand of v_mfma_f32_16x16x32_f16
 //     (16 channels x 32 keys) against P^T (32 keys x 16 columns: the heads'
-//     P, then their rests, whose sums are added at the end).
+//     P, then (TWO) their rests, whose sums are added at the end).
 // Each of the next tile's loads goes into the registers of the current tile's
 // input right after its last use, so they are in flight during the rest of
-// the tile. The two parts hold p to 2^-21 (the reference multiplies the fp32 p;
-// the columns of the rests are MFMA columns that G <= 8 heads leave unused); with
-// p rounded to one fp16, whose error is least where a key's p is its tile's exact
-// maximum 1, splits of more tiles were further from 64 bits than short ones: 16
-// sequences of 1024 to 16384 keys 2.7e-4 with planned splits, 2.6e-4 with splits
-// of 256 keys, 2.1e-4 with both parts (the fp16 output alone), for 43 -> 44 us. The V values are
-// exactly the reference's.
+// the tile. P enters the MFMA as fp16 (relative rounding 2^-11 per probability,
+// least where a key's p is its tile's exact maximum 1; the reference multiplies
+// the fp32 p). TWO: two parts hold p to 2^-21, in MFMA columns that G <= 8 heads
+// leave unused. It is for planned splits, which are longer than the 256 keys that
+// serve such batches otherwise, and with one part further from 64 bits: 16
+// sequences of 1024 to 16384 keys 2.7e-4, 2.6e-4 with splits of 256 keys, 2.1e-4
+// with both parts (the fp16 output alone), for 43 -> 44 us. Splits that the caller
+// chose keep one part (16 x 32768 keys in 16 splits: 150 us, two parts 157). The V
+// values are exactly the reference's.
 template <int D, int G>
 struct K3Smem {
   static constexpr int PP = 72;  // P row pitch in halves (64 keys + 8: bank spread)
@@ -1505,7 +1508,7 @@ struct K3Smem {
   union alignas(16) {
     struct {
       uint16_t v[DEC_WAVES][32 * D];   // fp16 V half tile [32 keys][D], 32-byte chunks swizzled
-      uint16_t p[DEC_WAVES][16 * PP];  // fp16 P [heads, then their rests][64 keys]
+      uint16_t p[DEC_WAVES][16 * PP];  // fp16 P [heads, then (TWO) their rests][64 keys]
       float ks[DEC_WAVES][DEC_TILE];   // the tile's k_scale
     } t;
     struct {
@@ -1552,7 +1555,7 @@ __device__ __forceinline__ float row_from(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false));
 }
 
-template <int D, int G>
+template <int D, int G, bool TWO>
 // workgroups per CU: the most that fit without spills
 __global__ void __launch_bounds__(DEC_THREADS, (D == 128 && G <= 4) ? 3 : 2)
 k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scale,
@@ -1762,12 +1765,13 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
     }
     mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    // the reference point lies 11 below the maximum: p up to 2^11, the rest of a usual p an fp16
-    // normal too
-    const float mn = fmaxf(m_run, fmaf(mt, qsl, -11.f));
+    // TWO: the reference point lies 11 below the maximum: p up to 2^11, the rest of a usual p an
+    // fp16 normal too
+    const float mn = fmaxf(m_run, TWO ? fmaf(mt, qsl, -11.f) : mt * qsl);
     const float resc = __builtin_amdgcn_exp2f(m_run - mn);  // first tile: exp2(-inf) = 0
     m_run = mn;
     float ls = 0.f;
+    uint32_t ph[4][2];
     typedef __fp16 h2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
@@ -1777,26 +1781,36 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
         p[i] = __builtin_amdgcn_exp2f(fmaf(x[kb][i], qsl, -mn));  // masked key: -inf -> 0
         ls += p[i];
       }
-      uint32_t ph[2], pl[2];
+      if constexpr (TWO) {
+        uint32_t pl[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const h2 hi = __builtin_amdgcn_cvt_pkrtz(p[2 * i], p[2 * i + 1]);
-        h2 lo = __builtin_amdgcn_cvt_pkrtz(p[2 * i] - (float)hi[0], p[2 * i + 1] - (float)hi[1]);
-        // above 0, so that an infinite V stays infinite where the rest is 0
-        lo = __builtin_elementwise_max(lo, h2{(__fp16)0x1p-24f, (__fp16)0x1p-24f});
-        ph[i] = __builtin_bit_cast(uint32_t, hi);
-        pl[i] = __builtin_bit_cast(uint32_t, lo);
-      }
-      if (col < G) {
-        uint16_t* pr = pt + col * PP + 16 * kb + 4 * g4;
-        *reinterpret_cast<uint2*>(pr) = uint2{ph[0], ph[1]};
-        *reinterpret_cast<uint2*>(pr + G * PP) = uint2{pl[0], pl[1]};
+        for (int i = 0; i < 2; ++i) {
+          const h2 hi = __builtin_amdgcn_cvt_pkrtz(p[2 * i], p[2 * i + 1]);
+          h2 lo = __builtin_amdgcn_cvt_pkrtz(p[2 * i] - (float)hi[0], p[2 * i + 1] - (float)hi[1]);
+          // above 0, so that an infinite V stays infinite where the rest is 0
+          lo = __builtin_elementwise_max(lo, h2{(__fp16)0x1p-24f, (__fp16)0x1p-24f});
+          ph[kb][i] = __builtin_bit_cast(uint32_t, hi);
+          pl[i] = __builtin_bit_cast(uint32_t, lo);
+        }
+        if (col < G) {
+          uint16_t* pr = pt + col * PP + 16 * kb + 4 * g4;
+          *reinterpret_cast<uint2*>(pr) = uint2{ph[kb][0], ph[kb][1]};
+          *reinterpret_cast<uint2*>(pr + G * PP) = uint2{pl[0], pl[1]};
+        }
+      } else {
+        ph[kb][0] = (uint32_t)f2h_bits(p[0]) | ((uint32_t)f2h_bits(p[1]) << 16);
+        ph[kb][1] = (uint32_t)f2h_bits(p[2]) | ((uint32_t)f2h_bits(p[3]) << 16);
       }
     }
     l_lane = l_lane * resc + ls;
+    if (!TWO && col < G) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+        *reinterpret_cast<uint2*>(pt + col * PP + 16 * kb + 4 * g4) = uint2{ph[kb][0], ph[kb][1]};
+    }
     // rescale the accumulators only when some head's running max moved
     if (__builtin_amdgcn_ballot_w64(col < G && resc != 1.f)) {
-      const float ro = row_from<0x110 | G>(resc);  // column G + c takes c's (row_shr)
+      const float ro = TWO ? row_from<0x110 | G>(resc) : resc;  // column G + c takes c's (row_shr)
 #pragma unroll
       for (int t = 0; t < DT; ++t) oacc[t] *= ro;
     }
@@ -1856,7 +1870,8 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float o = oacc[t][i] + row_from<0x100 | G>(oacc[t][i]);  // + column G + col's (row_shl)
+      float o = oacc[t][i];
+      if constexpr (TWO) o += row_from<0x100 | G>(o);  // + column G + col's (row_shl)
       if (col < G) sm.r.o[wave][col][16 * t + 4 * g4 + i] = o;
     }
   __syncthreads();
@@ -2029,15 +2044,15 @@ auto with_paged_kernel(const Paged& p, int64_t per, F&& f) {
 #undef SL8_PSPLIT
 }
 
-template <typename F>
+template <bool PLANNED, typename F>
 auto with_k8v3_kernel(const Paged& p, F&& f) {
   const int G = group_width(p.gsz());
-#define SL8_K3D(DD)                                                  \
-  switch (G) {                                                       \
-    case 1: return f(KernelTag<k8v3_split_kernel<DD, 1>>{});         \
-    case 2: return f(KernelTag<k8v3_split_kernel<DD, 2>>{});         \
-    case 4: return f(KernelTag<k8v3_split_kernel<DD, 4>>{});         \
-    default: return f(KernelTag<k8v3_split_kernel<DD, 8>>{});        \
+#define SL8_K3D(DD)                                                     \
+  switch (G) {                                                          \
+    case 1: return f(KernelTag<k8v3_split_kernel<DD, 1, PLANNED>>{});   \
+    case 2: return f(KernelTag<k8v3_split_kernel<DD, 2, PLANNED>>{});   \
+    case 4: return f(KernelTag<k8v3_split_kernel<DD, 4, PLANNED>>{});   \
+    default: return f(KernelTag<k8v3_split_kernel<DD, 8, PLANNED>>{});  \
   }
   if (p.D == 128) { SL8_K3D(128) }
   SL8_K3D(256)
@@ -2059,11 +2074,13 @@ int paged_launch(const Paged& p, const int8_t* q, const float* q_scale, void* ou
   dim3 grid = items ? dim3((unsigned)max_items) : dim3((unsigned)ns, (unsigned)(p.B * p.Hkv));
   if (p.k8v3) {
     grid.z = (unsigned)((gsz + G - 1) / G);
-    with_k8v3_kernel(p, [&](auto kt) {
+    auto go = [&](auto kt) {
       decltype(kt)::kernel<<<grid, DEC_THREADS, 0, st>>>(
           q, q_scale, p.k, p.ks, static_cast<const uint32_t*>(p.v), p.vs, p.codebook, op, mp, lp,
           nmax, ns, (int)p.Hq, (int)p.Hkv, gsz, bhq, pg);
-    });
+    };
+    if (items) with_k8v3_kernel<true>(p, go);
+    else with_k8v3_kernel<false>(p, go);
   } else {
     // planned splits are multiples of the streaming tiles and bounded by its block-table staging
     const int64_t per = items ? 256 : (p.nmax + ns - 1) / ns;
@@ -2111,7 +2128,7 @@ PagedPlan paged_plan(const Paged& p) {
   // keys a workgroup's 4 waves take in one round of tiles
   const int64_t unit = streams ? 4 * p.tile_keys() : 4 * DEC_TILE;
   const int chunks = streams ? 1 : (gsz + G - 1) / G;
-  const int wgs = p.k8v3 ? with_k8v3_kernel(p, [](auto kt) { return decltype(kt)::wgs_per_cu(); })
+  const int wgs = p.k8v3 ? with_k8v3_kernel<true>(p, [](auto kt) { return decltype(kt)::wgs_per_cu(); })
                          : with_paged_kernel(p, 256, [](auto kt) { return decltype(kt)::wgs_per_cu(); });
   auto up = [&](int64_t n) { return (n + unit - 1) / unit * unit; };
   const int64_t nmax = std::max<int64_t>(p.nmax, 1);

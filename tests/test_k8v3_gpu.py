@@ -313,30 +313,34 @@ def test_k8v3_planned_splits(device, case, dtype):
 
 @pytest.mark.parametrize("D,Hq,Hkv", [(128, 2, 2), (128, 4, 2), (128, 8, 2), (128, 16, 2), (256, 8, 2), (256, 8, 8)])
 def test_k8v3_probabilities_keep_their_precision(device, D, Hq, Hkv):
-    """Keys and queries of N(0, 1), one long split (many tiles a wave): the kernel holds p to 2^-21,
-    so its error against 64 bits is that of the fp16 output alone."""
-    N, bs = 3000, 16
+    """Keys and queries of N(0, 1), a batch that shares its keys and whose planned splits are long
+    (1536 keys and more, many tiles a wave): the kernel holds p to 2^-21, so its error against
+    64 bits is that of the fp16 output alone."""
+    B, N, bs = 512, 3000, 16
     nb = -(-N // bs)
     g = torch.Generator(device=device).manual_seed(D + Hq)
     kc, ks = _C.quantize_i8_rowwise(torch.randn(nb * Hkv * bs, D, device=device, generator=g).half())
     kc, ks = kc.reshape(nb, Hkv, bs, D), ks.reshape(nb, Hkv, bs)
-    q, qs = _C.quantize_i8_rowwise(torch.randn(Hq, D, device=device, generator=g).half())
-    qs = (qs * (np.log2(np.e) / D ** 0.5)).reshape(1, Hq, 1)
+    q = torch.randn(B, Hq, 1, D, device=device, generator=g).half()
     codes = torch.randint(0, 8, (nb, Hkv, bs, D), device=device, generator=g)
     vp = torch.from_numpy(olm.pack3(codes.cpu().numpy().astype(np.uint8))).to(device)
     vn = torch.rand(nb, Hkv, bs, D // 128, device=device, generator=g) * 4 + 9
     cb = torch.from_numpy(olm.gaussian_codebook(128)).to(device)
-    bt = torch.arange(nb, device=device, dtype=torch.int32)[None]
-    ctx = torch.tensor([N], device=device, dtype=torch.int32)
-    out = _C.attn_paged_decode_k8v3(q.reshape(1, Hq, 1, D), qs, kc, ks, vp, vn, cb, bt, ctx, bs, N, 1)
+    bt = torch.arange(nb, device=device, dtype=torch.int32)[None].repeat(B, 1)
+    ctx = torch.full((B,), N, device=device, dtype=torch.int32)
+    out = sl8.attn_paged_decode_k8v3(q, kc, ks, vp, vn, cb, bt, ctx, bs, max_context_len=N, rotate=False)
     v = (cb[codes] * vn.repeat_interleave(128, -1)).half()
 
     def rows(x):  # [Hkv, N, ...] in 64 bits
         return x.transpose(0, 1).flatten(1, 2)[:, :N].double()
 
+    def heads(x):  # [Hkv, B * group, ...]
+        return x.reshape(B, Hkv, Hq // Hkv, -1).transpose(0, 1).flatten(1, 2)
+
+    q_i8, qs = _C.quantize_i8_rowwise(q.reshape(-1, D))
     k = rows(kc) * rows(ks)[..., None]
-    s = torch.matmul(q.double().reshape(Hkv, Hq // Hkv, D), k.transpose(1, 2).contiguous())
-    p = torch.softmax(s * qs.double().reshape(Hkv, -1, 1) * np.log(2.0), -1)
-    ref = torch.matmul(p, rows(v)).reshape(1, Hq, 1, D)
+    s = torch.matmul(heads(q_i8.double()), k.transpose(1, 2).contiguous())
+    p = torch.softmax(s * heads(qs.double()) / D ** 0.5, -1)
+    ref = torch.matmul(p, rows(v))
     rounding = (ref.half().double() - ref).norm()
-    assert (out.double() - ref).norm() <= 1.05 * rounding
+    assert (heads(out.double()) - ref).norm() <= 1.05 * rounding

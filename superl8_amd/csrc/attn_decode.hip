@@ -71,8 +71,8 @@ struct PagedArgs {
   int bs_sh;           // log2(bs) (streaming kernels: bs a power of two; K8V3: -1 if not)
   int cache_rows;      // num_blocks * Hkv * bs (streaming kernel, block-aligned tiles)
   // splits planned on the device (see decode_prep_kernel): workgroup x serves keys [y, z) of
-  // (batch, KV head) x of items[x] and writes partial rows x * gsz ..; null = the grid's
-  // (split, batch * KV head) with equal splits of the launch's maximum
+  // (batch, KV head) x of items[x] and writes partial rows x * gsz .. (PLANNED kernels); null: the
+  // grid's (split, batch * KV head) with equal splits of the launch's maximum
   const int4* items;
 };
 
@@ -81,10 +81,13 @@ struct SplitWork {
   int bkv, n0, n1;
   int64_t row;  // partial row of the group's first query head
 };
+// PLANNED: from the launch's items (a template switch: the kernels whose splits the caller chose
+// keep their registers; K8V3 at D = 256 spilled with both forms in one).
+template <bool PLANNED>
 __device__ __forceinline__ SplitWork split_work(int n_len, int n_splits, int h_q, int h_kv, int gsz,
                                                 int bhq, bool paged, const PagedArgs& pg) {
   SplitWork w;
-  if (paged && pg.items) {
+  if constexpr (PLANNED) {
     const int4 it = pg.items[blockIdx.x];
     w.bkv = __builtin_amdgcn_readfirstlane(it.x);
     w.n0 = __builtin_amdgcn_readfirstlane(it.y);
@@ -114,7 +117,7 @@ __device__ __forceinline__ float load_ks(const void* base, int64_t r) {
   else return static_cast<const float*>(base)[r];
 }
 
-template <int D, int G, bool VI8, bool PG, bool KS16 = false>
+template <int D, int G, bool VI8, bool PG, bool KS16 = false, bool PLANNED = false>
 __global__ void __launch_bounds__(DEC_THREADS)
 decode_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scale,
                     const int8_t* __restrict__ k, const void* __restrict__ k_scale,
@@ -130,9 +133,9 @@ decode_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sc
   __shared__ DecSmem<D, G> sm;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const SplitWork sw = split_work(n_len, n_splits, h_q, h_kv, gsz, bhq, PG, pg);
+  const SplitWork sw = split_work<PLANNED>(n_len, n_splits, h_q, h_kv, gsz, bhq, PG, pg);
   const int bkv = sw.bkv, n0 = sw.n0, n1 = sw.n1;
-  if (PG && pg.items && n1 <= n0) return;  // an unused item
+  if (PLANNED && n1 <= n0) return;  // an unused item
   const int b = bkv / h_kv, kvh = bkv % h_kv;
   const int j0 = blockIdx.z * G;  // first head of this chunk within the group
   const int ng = min(G, gsz - j0);
@@ -484,7 +487,8 @@ struct WaveCfg {
 // PGA (paged, block-aligned tiles): every T-key tile lies inside one cache
 // block, so a tile's physical rows are one uniform base plus the lane's fixed
 // offset and its copies go through buffer resources like the contiguous ones.
-template <int D, int GS, int NB, bool VI8, bool PG, bool KS16 = false, bool PGA = false>
+template <int D, int GS, int NB, bool VI8, bool PG, bool KS16 = false, bool PGA = false,
+          bool PLANNED = false>
 __global__ void __launch_bounds__(DEC_THREADS, (SL8_DEC_PV4 && VI8 && DEC_PAIR && D == 128 && GS == 4) ? 3 : 1)
 decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scale,
                    const int8_t* __restrict__ k, const void* __restrict__ k_scale,
@@ -513,9 +517,9 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
     return s + wave * STAGE;
   };
 
-  const SplitWork sw = split_work(n_len, n_splits, h_q, h_kv, GS, bhq, PG, pg);
+  const SplitWork sw = split_work<PLANNED>(n_len, n_splits, h_q, h_kv, GS, bhq, PG, pg);
   const int bkv = sw.bkv, n0 = sw.n0, n1 = sw.n1;
-  if (PG && pg.items && n1 <= n0) return;  // an unused item
+  if (PLANNED && n1 <= n0) return;  // an unused item
   const int b = bkv / h_kv, kvh = bkv % h_kv;
   const int ntiles = n1 > n0 ? (n1 - n0 + T - 1) / T : 0;
   const int nt = ntiles > wave ? (ntiles - wave + DEC_WAVES - 1) / DEC_WAVES : 0;  // this wave's
@@ -1474,7 +1478,7 @@ kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __
 //   * softmax in the MFMA output layout: lane (g4, col) holds keys
 //     16 kb + 4 g4 + i of head col; logit = (acc * k_scale) * q_scale, the
 //     tile max over the lane's 16 values and the 4 lanes of the column; p
-//     stored as fp16 in LDS, one 64-key row per head, or (TWO) as two fp16
+//     stored as fp16 in LDS, one 64-key row per head, or (PLANNED) as two fp16
 //     parts, p rounded towards zero in row col and the rest in row G + col (the
 //     other rows stay zero);
 //   * value tables (key = lane): fp16 of codebook[i] * norm for i = 0..7 per
@@ -1486,12 +1490,12 @@ kv_write_paged_vec_kernel(const uint16_t* __restrict__ k_new, const uint16_t* __
 //     writes the half row to an 8 KB (D = 128) LDS tile, read back transposed
 //     (ds_read_b64_tr_b16) as the A operand of v_mfma_f32_16x16x32_f16
 //     (16 channels x 32 keys) against P^T (32 keys x 16 columns: the heads'
-//     P, then (TWO) their rests, whose sums are added at the end).
+//     P, then (PLANNED) their rests, whose sums are added at the end).
 // Each of the next tile's loads goes into the registers of the current tile's
 // input right after its last use, so they are in flight during the rest of
 // the tile. P enters the MFMA as fp16 (relative rounding 2^-11 per probability,
 // least where a key's p is its tile's exact maximum 1; the reference multiplies
-// the fp32 p). TWO: two parts hold p to 2^-21, in MFMA columns that G <= 8 heads
+// the fp32 p). PLANNED: two parts hold p to 2^-21, in MFMA columns that G <= 8 heads
 // leave unused. It is for planned splits, which are longer than the 256 keys that
 // serve such batches otherwise, and with one part further from 64 bits: 16
 // sequences of 1024 to 16384 keys 2.7e-4, 2.6e-4 with splits of 256 keys, 2.1e-4
@@ -1508,7 +1512,7 @@ struct K3Smem {
   union alignas(16) {
     struct {
       uint16_t v[DEC_WAVES][32 * D];   // fp16 V half tile [32 keys][D], 32-byte chunks swizzled
-      uint16_t p[DEC_WAVES][16 * PP];  // fp16 P [heads, then (TWO) their rests][64 keys]
+      uint16_t p[DEC_WAVES][16 * PP];  // fp16 P [heads, then (PLANNED) their rests][64 keys]
       float ks[DEC_WAVES][DEC_TILE];   // the tile's k_scale
     } t;
     struct {
@@ -1555,7 +1559,7 @@ __device__ __forceinline__ float row_from(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(v, v, CTRL, 0xF, 0xF, false));
 }
 
-template <int D, int G, bool TWO>
+template <int D, int G, bool PLANNED>
 // workgroups per CU: the most that fit without spills
 __global__ void __launch_bounds__(DEC_THREADS, (D == 128 && G <= 4) ? 3 : 2)
 k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scale,
@@ -1581,9 +1585,9 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
   __shared__ SM sm;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const SplitWork sw = split_work(n_len, n_splits, h_q, h_kv, gsz, bhq, true, pg);
+  const SplitWork sw = split_work<PLANNED>(n_len, n_splits, h_q, h_kv, gsz, bhq, true, pg);
   const int bkv = sw.bkv, n0 = sw.n0, n1 = sw.n1;
-  if (pg.items && n1 <= n0) return;  // an unused item
+  if (PLANNED && n1 <= n0) return;  // an unused item
   const int b = bkv / h_kv, kvh = bkv % h_kv;
   const int j0 = blockIdx.z * G;
   const int ng = min(G, gsz - j0);
@@ -1765,9 +1769,9 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
     }
     mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    // TWO: the reference point lies 11 below the maximum: p up to 2^11, the rest of a usual p an
+    // PLANNED: the reference point lies 11 below the maximum: p up to 2^11, the rest of a usual p an
     // fp16 normal too
-    const float mn = fmaxf(m_run, TWO ? fmaf(mt, qsl, -11.f) : mt * qsl);
+    const float mn = fmaxf(m_run, PLANNED ? fmaf(mt, qsl, -11.f) : mt * qsl);
     const float resc = __builtin_amdgcn_exp2f(m_run - mn);  // first tile: exp2(-inf) = 0
     m_run = mn;
     float ls = 0.f;
@@ -1781,7 +1785,7 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
         p[i] = __builtin_amdgcn_exp2f(fmaf(x[kb][i], qsl, -mn));  // masked key: -inf -> 0
         ls += p[i];
       }
-      if constexpr (TWO) {
+      if constexpr (PLANNED) {
         uint32_t pl[2];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -1803,14 +1807,14 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
       }
     }
     l_lane = l_lane * resc + ls;
-    if (!TWO && col < G) {
+    if (!PLANNED && col < G) {
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
         *reinterpret_cast<uint2*>(pt + col * PP + 16 * kb + 4 * g4) = uint2{ph[kb][0], ph[kb][1]};
     }
     // rescale the accumulators only when some head's running max moved
     if (__builtin_amdgcn_ballot_w64(col < G && resc != 1.f)) {
-      const float ro = TWO ? row_from<0x110 | G>(resc) : resc;  // column G + c takes c's (row_shr)
+      const float ro = PLANNED ? row_from<0x110 | G>(resc) : resc;  // column G + c takes c's (row_shr)
 #pragma unroll
       for (int t = 0; t < DT; ++t) oacc[t] *= ro;
     }
@@ -1871,7 +1875,7 @@ k8v3_split_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_scal
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float o = oacc[t][i];
-      if constexpr (TWO) o += row_from<0x100 | G>(o);  // + column G + col's (row_shl)
+      if constexpr (PLANNED) o += row_from<0x100 | G>(o);  // + column G + col's (row_shl)
       if (col < G) sm.r.o[wave][col][16 * t + 4 * g4 + i] = o;
     }
   __syncthreads();
@@ -2005,14 +2009,14 @@ template <auto K> struct KernelTag {
 };
 
 // f(KernelTag) of the int8-V paged kernel that serves p with splits of `per` keys.
-template <typename F>
+template <bool PLANNED, typename F>
 auto with_paged_kernel(const Paged& p, int64_t per, F&& f) {
   const int gsz = p.gsz();
   if (p.streams(per)) {
     const bool al = p.aligned_tiles(per);
-#define SL8_PWAVE(DD, GS, NB)                                                                 \
-    return al ? f(KernelTag<decode_wave_kernel<DD, GS, NB, true, true, false, true>>{})       \
-              : f(KernelTag<decode_wave_kernel<DD, GS, NB, true, true>>{})
+#define SL8_PWAVE(DD, GS, NB)                                                                      \
+    return al ? f(KernelTag<decode_wave_kernel<DD, GS, NB, true, true, false, true, PLANNED>>{})  \
+              : f(KernelTag<decode_wave_kernel<DD, GS, NB, true, true, false, false, PLANNED>>{})
 // D = 128: a two-stage ring (37 KB of LDS per workgroup, so 4 workgroups
 // per CU instead of 2) measured 210 us against 227 us with three stages at
 // config 3's shape with 16-key blocks scattered over the pool: more
@@ -2028,12 +2032,12 @@ auto with_paged_kernel(const Paged& p, int64_t per, F&& f) {
 #undef SL8_PWAVE
   }
   const int G = group_width(gsz);
-#define SL8_PSPLIT(DD)                                                                   \
-  switch (G) {                                                                           \
-    case 1: return f(KernelTag<decode_split_kernel<DD, 1, true, true>>{});               \
-    case 2: return f(KernelTag<decode_split_kernel<DD, 2, true, true>>{});               \
-    case 4: return f(KernelTag<decode_split_kernel<DD, 4, true, true>>{});               \
-    default: return f(KernelTag<decode_split_kernel<DD, 8, true, true>>{});              \
+#define SL8_PSPLIT(DD)                                                                      \
+  switch (G) {                                                                              \
+    case 1: return f(KernelTag<decode_split_kernel<DD, 1, true, true, false, PLANNED>>{});    \
+    case 2: return f(KernelTag<decode_split_kernel<DD, 2, true, true, false, PLANNED>>{});    \
+    case 4: return f(KernelTag<decode_split_kernel<DD, 4, true, true, false, PLANNED>>{});    \
+    default: return f(KernelTag<decode_split_kernel<DD, 8, true, true, false, PLANNED>>{});   \
   }
   switch (p.D) {
     case 32: SL8_PSPLIT(32)
@@ -2085,11 +2089,13 @@ int paged_launch(const Paged& p, const int8_t* q, const float* q_scale, void* ou
     // planned splits are multiples of the streaming tiles and bounded by its block-table staging
     const int64_t per = items ? 256 : (p.nmax + ns - 1) / ns;
     if (!p.streams(per)) grid.z = (unsigned)((gsz + G - 1) / G);
-    with_paged_kernel(p, per, [&](auto kt) {
+    auto go = [&](auto kt) {
       decltype(kt)::kernel<<<grid, DEC_THREADS, 0, st>>>(q, q_scale, p.k, p.ks, p.v, p.vs, op, mp,
                                                          lp, nmax, ns, (int)p.Hq, (int)p.Hkv, gsz,
                                                          bhq, pg);
-    });
+    };
+    if (items) with_paged_kernel<true>(p, per, go);
+    else with_paged_kernel<false>(p, per, go);
   }
   SL8_CHECK_LAUNCH(p.tag);
   launch_combine((int)p.D, bhq, st, op, mp, lp, static_cast<uint16_t*>(out), ns, bhq, seq,
@@ -2129,7 +2135,7 @@ PagedPlan paged_plan(const Paged& p) {
   const int64_t unit = streams ? 4 * p.tile_keys() : 4 * DEC_TILE;
   const int chunks = streams ? 1 : (gsz + G - 1) / G;
   const int wgs = p.k8v3 ? with_k8v3_kernel<true>(p, [](auto kt) { return decltype(kt)::wgs_per_cu(); })
-                         : with_paged_kernel(p, 256, [](auto kt) { return decltype(kt)::wgs_per_cu(); });
+                         : with_paged_kernel<true>(p, 256, [](auto kt) { return decltype(kt)::wgs_per_cu(); });
   auto up = [&](int64_t n) { return (n + unit - 1) / unit * unit; };
   const int64_t nmax = std::max<int64_t>(p.nmax, 1);
   PagedPlan r{};

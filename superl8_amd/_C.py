@@ -411,8 +411,8 @@ def attn_int8_decode(q, q_scale, k, k_scale, v, num_splits=-1):
     """q int8 [B,Hq,1,D], q_scale fp32 [B,Hq,1], k int8 [B,Hkv,N,D], k_scale fp32
     [B,Hkv,N], v fp16 [B,Hkv,N,D] -> fp16 [B,Hq,1,D].
 
-    k_scale may also be fp16 (a cache with half-size per-token scales, BASELINE
-    config 3): the kernels widen it to fp32 exactly and compute as before."""
+    k_scale may also be fp16 (a cache with half-size per-token scales): the
+    kernels widen it to fp32 exactly and compute as before."""
     _on_gpu(q, q_scale, k, k_scale, v)
     _check(q.dtype == torch.int8 and k.dtype == torch.int8, "decode: q/k must be int8")
     _check(q_scale.dtype == torch.float32 and k_scale.dtype in (torch.float32, torch.float16),
@@ -863,7 +863,7 @@ def gemm_decode_q4k(x, x_scale, w, out_dtype=torch.float16):
 
     x_scale [M] is the reference's per-row activation scale; x_scale [M, K/256]
     (one scale per 256-element block, from quantize_i8_blockwise) scales each
-    super-block's integer sums instead (BASELINE config 4's activation format)."""
+    super-block's integer sums instead."""
     if not (x.dim() == 2 and x.shape[0] <= DEC_MAX_M):
         _fail(f"gemm_decode_q4k supports M<={DEC_MAX_M}, got M={x.shape[0] if x.dim() else 0}"
               " -- use the tile gemm_q4k for prefill")

@@ -110,7 +110,7 @@ __device__ __forceinline__ SplitWork split_work(int n_len, int n_splits, int h_q
 constexpr int DEC_BT_MAX = 1024;
 
 // Per-token K scale of key row r: fp32 (the reference contract) or, with
-// KS16, fp16 (half the scale bytes; BASELINE config 3's cache format).
+// KS16, fp16 (half the scale bytes).
 template <bool KS16>
 __device__ __forceinline__ float load_ks(const void* base, int64_t r) {
   if constexpr (KS16) return h2f(static_cast<const uint16_t*>(base)[r]);
@@ -973,7 +973,7 @@ decode_wave_kernel(const int8_t* __restrict__ q, const float* __restrict__ q_sca
 // [lmin, lcap]; each sequence of n keys then gets ceil(n / L) splits of equal length. Splits
 // sized on the longest sequence alone (256 keys and up to 256 splits of every sequence) left most
 // workgroups of a batch of mixed lengths empty and the rest too short to stream: 32 sequences of
-// 512..8192 keys, 8 KV heads, D = 128: 95 us for 191 MB, 44 with the plan (the call 114 -> 53 us).
+// 512..8192 keys, 8 KV heads, D = 128: 95 us for 191 MB, 38 with the plan (the call 114 -> 52 us).
 //
 // Where a pair gets only a few splits, whole units of L can leave many workgroups without work: 53
 // sequences of 3393 keys and 4 heads at D = 256 get 4 splits of 1024 keys, 848 for 1024 places. A
@@ -1242,10 +1242,9 @@ extern "C" int sl8_attn_int8_decode(const int8_t* q, const float* q_scale, const
                               num_splits, workspace, static_cast<hipStream_t>(stream));
 }
 
-// fp16 per-token K scales (BASELINE config 3's cache format: half the scale
-// bytes of the reference's fp32 contract, attn_decode.cu:174-175). Otherwise
-// identical to sl8_attn_int8_decode: the scale is widened to fp32 exactly
-// before the same arithmetic.
+// fp16 per-token K scales (half the scale bytes of the reference's fp32
+// contract, attn_decode.cu:174-175). Otherwise identical to sl8_attn_int8_decode: the
+// scale is widened to fp32 exactly before the same arithmetic.
 extern "C" int sl8_attn_int8_decode_ks16(const int8_t* q, const float* q_scale, const int8_t* k,
                                          const void* k_scale_f16, const void* v, void* out,
                                          int64_t B, int64_t Hq, int64_t Hkv, int64_t N, int64_t D,

@@ -709,9 +709,8 @@ extern "C" int sl8_gemm_decode_q4k(const int8_t* x, const float* x_scale, const 
   return SL8_OK;
 }
 
-// Decode GEMV with one activation scale per 256-element block (BASELINE
-// config 4's activation format): x_scale [M, K/256] multiplies each
-// super-block's exact integer sums instead of the row total.
+// Decode GEMV with one activation scale per 256-element block:
+// x_scale [M, K/256] multiplies each super-block's exact integer sums instead of the row total.
 extern "C" int sl8_gemm_decode_q4k_xblock(const int8_t* x, const float* x_scale, const uint8_t* w,
                                           void* out, int out_dtype, int64_t M, int64_t N, int64_t K,
                                           void* stream) {

@@ -452,7 +452,7 @@ namespace {
 // ---------------------------------------------------------------------------
 // Row-group quantisation (one scale per R consecutive rows of a [G][N][K]
 // tensor, groups restarting at every G slice): the per-wavefront Q / per-tile
-// K scheme of BASELINE config 5. One workgroup per group: pass 1 takes the
+// K scheme. One workgroup per group: pass 1 takes the
 // amax of the (optionally mean-shifted, dtype-rounded) values over the R x K
 // block, pass 2 writes the codes (the block is re-read from L2). The scale,
 // safe value and code follow the row-wise contract above with the group's

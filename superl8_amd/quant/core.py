@@ -188,8 +188,8 @@ def quantize_qk_per_wave(q: torch.Tensor, k: torch.Tensor, *, softmax_scale: flo
                          q_rows: int = 32, k_rows: int = 64):
     """quantize_qk with one scale per tile of rows instead of per row: Q per
     `q_rows` queries (one wavefront's query tile of the prefill kernels, 32) and
-    the smoothed K per `k_rows` keys (one key tile, 64) -- the per-wavefront
-    scheme of BASELINE config 5 (the reference quantises Q/K per row,
+    the smoothed K per `k_rows` keys (one key tile, 64) -- a
+    per-wavefront scheme (the reference quantises Q/K per row,
     core.py:164-196). Same outputs as quantize_qk; every row carries its tile's
     scale, so the attention kernels run unchanged."""
     _need_gpu(q, "quantize_qk_per_wave")
